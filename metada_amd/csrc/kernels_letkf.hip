@@ -184,21 +184,67 @@ void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* k
   }
 }
 
-// start[b] = first sorted position whose key >= b, for b in [0, nbuckets]
-__global__ void k_bucket_ranges(const uint32_t* __restrict__ sk, int64_t p, int nbuckets,
-                                int* __restrict__ start) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t <= p;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    int lo = (t == 0) ? 0 : (int)sk[t - 1] + 1;
-    int hi = (t == p) ? nbuckets : (int)sk[t];
-    for (int b = lo; b <= hi; ++b) start[b] = (int)t;
+// start[b] = first sorted position whose key >= b, for b in [0, nbuckets].  A
+// block owns BR_N consecutive buckets: waves 0 and 1 find the positions of
+// its first bucket and of the bucket past its last by a 64-way search (one
+// load per lane and level), and every bucket is then a binary search inside
+// that range, in LDS when it holds at most BR_LDS keys.  Bound by the search's
+// dependent loads, whatever the gaps between the keys: filling the gap before
+// each key from that key's thread wrote the 250,000 buckets north and south of
+// observations on one parallel one after the other, 7.6 ms at 4,000 columns
+// and 2,000 observations against under 10 us here.
+constexpr int BR_N = 256, BR_LDS = 4096;
+
+// first t in [0, p] with sk[t] >= key (sk[p] taken as +inf), wave-wide
+__device__ inline int64_t wave_lower_bound(const uint32_t* __restrict__ sk, int64_t p,
+                                           uint32_t key) {
+  const int lane = threadIdx.x & 63;
+  int64_t lo = 0, hi = p;  // the answer is in [lo, hi]
+  while (hi > lo) {
+    const int64_t step = (hi - lo + 63) / 64;
+    // lane i looks at the last position of slice i
+    const int64_t t = lo + (lane + 1) * step - 1;
+    const bool ge = t >= hi || sk[t] >= key;
+    const uint64_t m = __ballot(ge);
+    const int f = m ? __builtin_ctzll(m) : 64;  // first slice whose end is >= key
+    const int64_t nlo = lo + (int64_t)f * step;
+    const int64_t nhi = nlo + step - 1;
+    lo = nlo < hi ? nlo : hi;
+    hi = nhi < hi ? nhi : hi;
   }
+  return lo;
+}
+
+__global__ __launch_bounds__(BR_N) void k_bucket_ranges(const uint32_t* __restrict__ sk, int64_t p,
+                                                       int nbuckets, int* __restrict__ start) {
+  __shared__ int64_t ends[2];
+  __shared__ uint32_t ks[BR_LDS];
+  const int tid = threadIdx.x, wv = tid >> 6;
+  const int64_t b0 = (int64_t)blockIdx.x * BR_N;
+  if (wv < 2) {
+    const int64_t t = wave_lower_bound(sk, p, (uint32_t)(b0 + (int64_t)wv * BR_N));
+    if ((tid & 63) == 0) ends[wv] = t;
+  }
+  __syncthreads();
+  const int64_t t0 = ends[0];
+  const int cnt = (int)(ends[1] - t0);
+  const bool in_lds = cnt <= BR_LDS;
+  if (in_lds)
+    for (int i = tid; i < cnt; i += BR_N) ks[i] = sk[t0 + i];
+  __syncthreads();
+  const int64_t b = b0 + tid;
+  int lo = 0, hi = cnt;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if ((in_lds ? ks[mid] : sk[t0 + mid]) >= (uint32_t)b) hi = mid; else lo = mid + 1;
+  }
+  if (b <= nbuckets) start[b] = (int)(t0 + lo);
 }
 
 void launch_bucket_ranges(hipStream_t s, const uint32_t* sorted_keys, int64_t p, int nbuckets,
                           int* start) {
-  hipLaunchKernelGGL(k_bucket_ranges, dim3(grid_for(p + 1, 256, 8192)), dim3(256), 0, s,
-                     sorted_keys, p, nbuckets, start);
+  const unsigned nb = (unsigned)((nbuckets + (int64_t)BR_N) / BR_N);  // buckets 0 .. nbuckets
+  hipLaunchKernelGGL(k_bucket_ranges, dim3(nb), dim3(BR_N), 0, s, sorted_keys, p, nbuckets, start);
   MDA_LAUNCH_CHECK();
 }
 
