@@ -250,8 +250,8 @@ typedef struct {
                                   (split-precision bf16 products, FP32 accumulation; k a
                                   multiple of 16, at most 64) */
   int32_t keep_transforms;     /* 1: keep every column's T for mda_letkf_last_transforms.
-                                  0 (the default): at k in {16, 32, 48, 64} with the
-                                  tridiagonal eigensolver, the matrix combination and an
+                                  0 (the default): at k in 9..16 and 21..64 but 33..40
+                                  with the tridiagonal eigensolver, the matrix combination and an
                                   FP64 transform, the eigenvector kernel applies
                                   X_a = X T' itself and T is not stored */
 } mda_letkf_params;
@@ -335,7 +335,9 @@ int mda_letkf_last_local_counts(mda_ctx* ctx, int32_t* counts);
 /* Per-column eigensolver status of the last LETKF call, [nx*ny] (host):
  * 0 = tridiagonal path, otherwise the column was re-solved by Jacobi and the
  * bits say why (1 QL non-convergence, 2 eigen-residual, 4 orthogonality of a
- * close eigenpair, 8 eigenvalue below (k-1)/rho). */
+ * close eigenpair, 8 eigenvalue below (k-1)/rho, 16 fewer than k local
+ * observations with an FP32 Gram at a k without a tridiagonal
+ * kernel of its own size). */
 int mda_letkf_last_column_flags(mda_ctx* ctx, int32_t* flags);
 
 /* ---- observation operator and files around the analysis ------------------------ */

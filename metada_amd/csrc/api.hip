@@ -696,7 +696,7 @@ struct letkf_plan {
   dev_ensemble de;
   dev_obs o;
   dev_hop h;
-  int k = 0;
+  int k = 0, ks = 0;  // members, size of the per-column blocks (letkf_gram_args::ks)
   int64_t p = 0, n = 0, nx = 0, ny = 0, nlev = 0, ncol = 0;
   // columns per pass of Gram -> solve -> transform: the k x k per-column
   // buffers (C, U, T) hold one pass; ncol when the whole grid fits
@@ -752,10 +752,10 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   P.o = stage_obs(c, obs, true, /*allow_empty=*/true);
   if (P.o.p > 0) P.h = stage_hop(c, hop, P.de.k, P.o.p, P.de.n);
   const int k = P.k = P.de.k;
+  MDA_REQUIRE(k <= 128, "LETKF supports k <= 128 in this build");
   const int64_t p = P.p = P.o.p;
   P.n = P.de.n; P.nx = ens->nx; P.ny = ens->ny; P.nlev = ens->nlev;
   const int64_t ncol = P.ncol = P.nx * P.ny;
-  MDA_REQUIRE(k <= 128, "LETKF supports k <= 128 in this build");
   MDA_REQUIRE(prm->transform_precision != MDA_PREC_BF16X3 || (k % 16 == 0 && k <= 64),
               "a BF16x3 transform needs k a multiple of 16, at most 64");
   const bool gd = geom->on_device != 0;
@@ -824,8 +824,17 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   }
   P.bstart = c->get<int>(pre + "bk_start", P.nbuckets + 1);
 
+  // The tridiagonal eigensolver, in the next larger of its block sizes.  A
+  // BF16x3 Gram is symmetric only to its FP32 accumulation (hi lo^T + lo hi^T
+  // rounds differently in the two triangles), so its result depends at 1e-9
+  // on which entries a solver reads: sizes without a kernel of their own stay
+  // with Jacobi there.
+  const int ke = letkf_eig_size(k);
+  P.eig_path = prm->sqrt_form == MDA_SQRT_SYMMETRIC && prm->eig_method == MDA_EIG_AUTO &&
+               (ke == k || prm->precision != MDA_PREC_BF16X3);
+  const int ks = P.ks = P.eig_path ? ke : k;
   letkf_gram_args& ga = P.ga;
-  ga.k = k; ga.ncol = ncol; ga.nx = P.nx; ga.coord = geom->coord;
+  ga.k = k; ga.ks = ks; ga.ncol = ncol; ga.nx = P.nx; ga.coord = geom->coord;
   ga.col_a = ca; ga.col_b = cb; ga.col_c = cc;
   ga.grid = bg; ga.bstart = P.bstart;
   ga.yp = c->get<double>(pre + "s_yp", (size_t)p * k);
@@ -845,16 +854,16 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   // Column passes: at k > 64 the per-column k x k buffers of the whole grid
   // would not fit in HBM next to the ensemble (3 x 69 GB at k = 128 and
   // 524,288 columns), so the columns run in passes of 65,536.
-  P.chunk = k > 64 ? std::min<int64_t>(ncol, 65536) : ncol;
+  P.chunk = ks > 64 ? std::min<int64_t>(ncol, 65536) : ncol;
   if (const char* ev = std::getenv("MDA_LETKF_CHUNK_COLS")) {
     const long long v = std::atoll(ev);
     if (v > 0) P.chunk = std::min<int64_t>(ncol, v);
   }
   const int64_t nck = P.chunk;
-  ga.C = c->get<double>(pre + "col_C", (size_t)nck * k * k);
+  ga.C = c->get<double>(pre + "col_C", (size_t)nck * ks * ks);
   ga.c32 = prm->precision != MDA_PREC_FP64;
   ga.crec = c->get<int>(pre + "col_rec", (size_t)ncol * LETKF_CREC_INTS);
-  ga.b = c->get<double>(pre + "col_bvec", (size_t)ncol * k);
+  ga.b = c->get<double>(pre + "col_bvec", (size_t)ncol * ks);
   ga.nloc = c->get<int>(pre + "col_nloc", ncol);
   if (geom->coord == MDA_COORD_GEOGRAPHIC) {
     ga.shell_cap = std::max<int64_t>(65536, 4 * nck);
@@ -873,18 +882,16 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   }
 
   letkf_solve_args& sa = P.sa;
-  sa.k = k; sa.ncol = ncol; sa.C = ga.C; sa.c32 = ga.c32; sa.b = ga.b; sa.nloc = ga.nloc;
+  sa.k = k; sa.ks = ks; sa.ncol = ncol; sa.C = ga.C; sa.c32 = ga.c32; sa.b = ga.b; sa.nloc = ga.nloc;
   sa.rho = prm->inflation; sa.rho_col = rho_col;
   sa.inflation_form = prm->inflation_form; sa.sqrt_form = prm->sqrt_form;
   sa.combine = prm->combine;
-  sa.T = c->get<double>(pre + "col_T", (size_t)nck * k * k);
+  sa.T = c->get<double>(pre + "col_T", (size_t)nck * ks * ks);
   P.sweeps = sa.sweeps = c->get<int>(pre + "col_sweeps", ncol);
   sa.status = c->get<int>(pre + "col_status", 1);
-  sa.de = c->get<double>(pre + "eig_de", (size_t)ncol * 2 * k);
-  sa.lam = c->get<double>(pre + "eig_lam", (size_t)ncol * k);
-  P.eig_path = prm->sqrt_form == MDA_SQRT_SYMMETRIC && letkf_eig_supported(k) &&
-               prm->eig_method == MDA_EIG_AUTO;
-  sa.U = P.eig_path ? c->get<double>(pre + "eig_U", (size_t)nck * k * k) : nullptr;
+  sa.de = c->get<double>(pre + "eig_de", (size_t)ncol * 2 * ks);
+  sa.lam = c->get<double>(pre + "eig_lam", (size_t)ncol * ks);
+  sa.U = P.eig_path ? c->get<double>(pre + "eig_U", (size_t)nck * ks * ks) : nullptr;
   sa.flag = c->get<int>(pre + "eig_flag", ncol);
   sa.wlist = c->get<int>(pre + "solve_list", ncol);
   sa.wcount = c->get<unsigned>(pre + "solve_count", 1);
@@ -897,13 +904,24 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
       sa.jscratch = c->get<double>(pre + "jac_scratch", (size_t)sa.jblocks * 2 * kp * (kp + 1));
     }
   }
-  sa.method = prm->eig_method;
+  sa.method = P.eig_path ? MDA_EIG_AUTO : MDA_EIG_JACOBI;
   // eigenvalue noise of the Gram relative to ||A||: FP32 products with FP32
   // accumulation, or BF16x3 products (2^-16 relative) with FP32 accumulation
   sa.null_rel = prm->precision == MDA_PREC_FP32 ? 0x1p-22
                 : prm->precision == MDA_PREC_BF16X3 ? 0x1p-17 : 0.0;
+  // An FP32 Gram in a block larger than k keeps every eigenpair, noise
+  // included, so that those sizes give what the Jacobi solve gives to FP64
+  // rounding (leaving the noise out moves X_a by about 1e-6).  A column
+  // with fewer than k observations has a cluster of noise eigenvalues at
+  // sigma, whose vectors a twisted factorisation does not separate: it goes
+  // to Jacobi at once (as most of them would after the checks; 60 % of the
+  // tridiagonal kernels' time is then not spent on them).
+  if (P.eig_path && ks != k && prm->precision == MDA_PREC_FP32) {
+    sa.null_rel = 0.0;
+    sa.eig_nloc = c->get<int>(pre + "eig_nloc", ncol);
+  }
   // E3 applies the transform itself unless T is to be kept
-  sa.fuse = P.eig_path && letkf_eig_fusable(k) && prm->combine == MDA_COMBINE_MATRIX &&
+  sa.fuse = P.eig_path && !sa.eig_nloc && letkf_eig_fusable(ks) && prm->combine == MDA_COMBINE_MATRIX &&
             prm->transform_precision == MDA_PREC_FP64 && !prm->keep_transforms;
   P.stats = c->get<int64_t>(pre + "col_stats", 9);
   return P;
@@ -971,7 +989,7 @@ static letkf_gram_args gram_pass(const letkf_plan& P, int64_t c0, int64_t nc) {
   if (ga.col_a) ga.col_a += c0;
   if (ga.col_b) ga.col_b += c0;
   if (ga.col_c) ga.col_c += c0;
-  ga.b += c0 * P.k;
+  ga.b += c0 * P.ks;
   ga.nloc += c0;
   if (ga.crec) ga.crec += c0 * LETKF_CREC_INTS;
   return ga;
@@ -980,12 +998,13 @@ static letkf_gram_args gram_pass(const letkf_plan& P, int64_t c0, int64_t nc) {
 static letkf_solve_args solve_pass(const letkf_plan& P, int64_t c0, int64_t nc) {
   letkf_solve_args sa = P.sa;
   sa.ncol = nc;
-  sa.b += c0 * P.k;
+  sa.b += c0 * P.ks;
   sa.nloc += c0;
   if (sa.rho_col) sa.rho_col += c0;
   sa.sweeps += c0;
-  sa.de += c0 * 2 * P.k;
-  sa.lam += c0 * P.k;
+  sa.de += c0 * 2 * P.ks;
+  sa.lam += c0 * P.ks;
+  if (sa.eig_nloc) sa.eig_nloc += c0;
   sa.flag += c0;
   sa.X = P.de.X;
   sa.x_ncol = P.ncol;
@@ -1037,7 +1056,7 @@ static void enqueue_columns(hipStream_t s, letkf_plan& P, std::pair<int, int> cf
     launch_letkf_solve(s, sa);
     if (m) MDA_HIP(hipEventRecord(m->e[5], s));
     // fused: only the columns E3 left to the fallback remain
-    launch_letkf_transform(s, P.de.X, P.k, P.ncol, P.nlev, P.sa.T, P.sa.status, c0, nc,
+    launch_letkf_transform(s, P.de.X, P.k, P.ks, P.ncol, P.nlev, P.sa.T, P.sa.status, c0, nc,
                            P.prm->transform_precision, sa.fuse ? sa.flag : nullptr);
     if (m) MDA_HIP(hipEventRecord(m->e[6], s));
   }
@@ -1059,7 +1078,7 @@ static void finish_letkf(mda_ctx* c, letkf_plan& P, mda_letkf_diag* diag) {
   d2h(c, &hstat, P.sa.status, sizeof(int));
   // the transforms stay readable only when one pass covered every column
   c->last_T = P.chunk == P.ncol && !P.sa.fuse ? P.sa.T : nullptr;
-  c->last_k = P.k; c->last_ncol = P.ncol; c->last_nloc = P.ga.nloc;
+  c->last_k = P.k; c->last_ks = P.ks; c->last_ncol = P.ncol; c->last_nloc = P.ga.nloc;
   c->last_flag = P.eig_path ? P.sa.flag : nullptr;
   throw_status(hstat & MDA_ST_SKIP_UPDATE, "LETKF");
   unstage_ensemble(c, P.ens, P.de);
@@ -1192,7 +1211,7 @@ static std::string plan_signature(const letkf_plan& P) {
                           (const void*)P.ckeys2, (const void*)P.ccols2, (const void*)P.chist,
                           (const void*)P.qcount})
     sig_add(sg, ptr);
-  for (int64_t v : {(int64_t)P.k, P.p, P.n, P.nx, P.ny, P.nlev, P.ncol, P.chunk,
+  for (int64_t v : {(int64_t)P.k, (int64_t)P.ks, P.p, P.n, P.nx, P.ny, P.nlev, P.ncol, P.chunk,
                     (int64_t)P.nbuckets, (int64_t)P.key_bits, P.hist_cap, (int64_t)P.tap_bits,
                     (int64_t)P.geo, (int64_t)P.eig_path, (int64_t)P.queue, P.chist_cap})
     sig_add(sg, v);
@@ -1393,10 +1412,13 @@ int mda_letkf_last_transforms(mda_ctx* c, const int64_t* cols, int64_t ncols, do
                 "the transforms of that analysis were not kept (set keep_transforms = 1; "
                 "an analysis run in column passes never keeps them)");
     MDA_REQUIRE(cols && T_out, "cols and T_out are required");
-    const size_t kk = (size_t)c->last_k * c->last_k;
+    const size_t k = (size_t)c->last_k, ks = (size_t)c->last_ks;
+    std::vector<double> blk(ks * ks);
     for (int64_t i = 0; i < ncols; ++i) {
       MDA_REQUIRE(cols[i] >= 0 && cols[i] < c->last_ncol, "column index out of range");
-      d2h(c, T_out + i * kk, c->last_T + cols[i] * kk, sizeof(double) * kk);
+      d2h(c, blk.data(), c->last_T + cols[i] * ks * ks, sizeof(double) * ks * ks);
+      for (size_t r = 0; r < k; ++r)
+        std::copy_n(blk.data() + r * ks, k, T_out + (i * k + r) * k);
     }
     MDA_HIP(hipStreamSynchronize(c->stream));
   });

@@ -14,6 +14,14 @@
 //       wbar = s Z L^-1 Z^T b, T = wbar 1^T + W (or the element-wise form).
 // A column that fails a check (or QL non-convergence) is flagged and
 // re-solved by the parallel-order Jacobi kernel.
+//
+// The kernels are compiled for block sizes N; an ensemble of km < N members
+// runs in the next larger block.  The Gram's zeros past km make the block
+// diag(A, sigma I): the padding decouples (zero reflector entries, e_i = 0),
+// its eigenvalues are sigma exactly, which E3 leaves out as it does the null
+// space, and km enters only sigma and the scale of W.  Measured at 200 x 160
+// columns of 30 levels, k = 50 (N = 64): Jacobi and the stored transform took
+// 68.4 ms, these kernels with the transform in E3 take 4.5 ms.
 #include "mda_device.hpp"
 #include "mda_internal.hpp"
 #include "mda_xform.hpp"
@@ -95,8 +103,9 @@ constexpr int E1_CH = 2;  // step chunk of k_trd (static column ranges start at 
 template <int N>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 void k_trd(int64_t ncol, const double* __restrict__ C, int c32,
-           const int* __restrict__ nloc, double rho, const double* __restrict__ rho_col,
-           int prior, double* __restrict__ de, double* __restrict__ Uout) {
+           const int* __restrict__ nloc, int km, double rho,
+           const double* __restrict__ rho_col, int prior, double* __restrict__ de,
+           double* __restrict__ Uout) {
   constexpr int n = N;
   __shared__ double row[EIG_N], ub[EIG_N], wb[EIG_N];
   const int lane = threadIdx.x;
@@ -106,7 +115,7 @@ void k_trd(int64_t ncol, const double* __restrict__ C, int c32,
     const int64_t g = blockIdx.x;
     if (g >= ncol || nloc[g] == 0) return;
     const double r = rho_col ? rho_col[g] : rho;
-    const double sigma = prior ? (double)(n - 1) / r : (double)(n - 1);
+    const double sigma = prior ? (double)(km - 1) / r : (double)(km - 1);
     const int rl = lane < n ? lane : n - 1;  // clamped row: loads stay in bounds
     double ar[N];
     if (c32) {  // FP32 entries, widened
@@ -475,8 +484,8 @@ template <int N, bool FUSED, class Pre>
 __device__ __forceinline__ bool e3_column(
     int64_t g, double* __restrict__ slice, const int* __restrict__ nloc,
     const double* __restrict__ de, const double* __restrict__ lam,
-    const double* __restrict__ bvec, double rho, const double* __restrict__ rho_col, int prior,
-    int combine, double null_rel, const double* __restrict__ Ug, double* __restrict__ T,
+    const double* __restrict__ bvec, int km, double rho, const double* __restrict__ rho_col,
+    int prior, int combine, double null_rel, const double* __restrict__ Ug, double* __restrict__ T,
     int* __restrict__ flag, double (&tb)[e3_shape<N>::NP / 4][e3_shape<N>::NP / 16],
     Pre&& pre) {
   constexpr int n = N;
@@ -580,7 +589,7 @@ __device__ __forceinline__ bool e3_column(
   // each would change W by at most 1e-12 relative.  With a reduced-precision
   // Gram the window widens to the Gram's own rounding level, null_rel ||A||.
   const bool pri = prior != 0;
-  const double sigma = pri ? (double)(n - 1) / r : (double)(n - 1);
+  const double sigma = pri ? (double)(km - 1) / r : (double)(km - 1);
   const double null_tol = fmax(2e-12 * sigma, null_rel * tnorm);
   const bool skip = lane >= n || fabs(l - sigma) <= null_tol;
   // weight of eigenpair j in W and wbar: 1 - sigma/lambda_j (0 at sigma)
@@ -770,7 +779,7 @@ __device__ __forceinline__ bool e3_column(
     for (int e2 = 0; e2 < N; ++e2) acc += Z[lane * ld + e2] * sy[e2];
     wbar = sc * (sb[lane] / sigma - acc);
   }
-  const double coef = sqrt((double)(n - 1)) * sqrt(sc);
+  const double coef = sqrt((double)(km - 1)) * sqrt(sc);
   const double fs = 1.0 / sqrt(sigma);
   if (combine == MDA_COMBINE_ELEMENTWISE) {
     // t_i = wbar_i + coef (f(sigma) - sum_a U_s[i][a] (sum_j U_s[j][a]))
@@ -874,7 +883,7 @@ __device__ __forceinline__ bool e3_column(
 template <int N>
 __global__ __launch_bounds__(64) void k_trd_vectors(
     int64_t ncol, const int* __restrict__ nloc, const double* __restrict__ de,
-    const double* __restrict__ lam, const double* __restrict__ bvec, double rho,
+    const double* __restrict__ lam, const double* __restrict__ bvec, int km, double rho,
     const double* __restrict__ rho_col, int prior, int combine, double null_rel,
     const double* __restrict__ Ug, double* __restrict__ T, int* __restrict__ flag) {
   // one column per block: no loop-carried state (a grid-stride loop here
@@ -883,8 +892,8 @@ __global__ __launch_bounds__(64) void k_trd_vectors(
   double tb[e3_shape<N>::NP / 4][e3_shape<N>::NP / 16];
   const int64_t g = blockIdx.x;
   if (g < ncol)
-    e3_column<N, false>(g, slice, nloc, de, lam, bvec, rho, rho_col, prior, combine, null_rel, Ug,
-                        T, flag, tb, [] {});
+    e3_column<N, false>(g, slice, nloc, de, lam, bvec, km, rho, rho_col, prior, combine, null_rel,
+                        Ug, T, flag, tb, [] {});
 }
 
 constexpr int E3_PRE = 2;  // 16-level chunks of X loaded during E3's W products
@@ -900,7 +909,7 @@ constexpr int E3_PRE = 2;  // 16-level chunks of X loaded during E3's W products
 template <int N>
 __global__ __launch_bounds__(256) void k_trd_vectors_x(
     int64_t ncol, const int* __restrict__ nloc, const double* __restrict__ de,
-    const double* __restrict__ lam, const double* __restrict__ bvec, double rho,
+    const double* __restrict__ lam, const double* __restrict__ bvec, int km, double rho,
     const double* __restrict__ rho_col, int prior, double null_rel,
     const double* __restrict__ Ug, int* __restrict__ flag, double* __restrict__ X,
     int64_t x_ncol, int64_t nlev, int64_t col0, int* __restrict__ status) {
@@ -929,12 +938,12 @@ __global__ __launch_bounds__(256) void k_trd_vectors_x(
     if (loaded) return;
 #pragma unroll
     for (int ci = 0; ci < E3_PRE; ++ci)
-      xm_load<N>(pre[ci], X, x_ncol, nlev, col0 + g0, ncl, (int64_t)XM_L * ci);
+      xm_load<N>(pre[ci], X, km, x_ncol, nlev, col0 + g0, ncl, (int64_t)XM_L * ci);
     loaded = true;
   };
   bool ok = false;
   if (wv < ncl)
-    ok = e3_column<N, true>(g0 + wv, lds + wv * SL, nloc, de, lam, bvec, rho, rho_col, prior,
+    ok = e3_column<N, true>(g0 + wv, lds + wv * SL, nloc, de, lam, bvec, km, rho, rho_col, prior,
                             MDA_COMBINE_MATRIX, null_rel, Ug, nullptr, flag, tb, preload);
   preload();
   if ((tid & 63) == 0) sok[wv] = ok ? 1 : 0;
@@ -942,8 +951,8 @@ __global__ __launch_bounds__(256) void k_trd_vectors_x(
   unsigned store = 0u;
   for (int c = 0; c < ncl; ++c) store |= sok[c] ? 1u << c : 0u;
   if (store == 0u || (*status & MDA_ST_SKIP_UPDATE)) return;  // block-uniform
-  xm_tprime<N>(tb);
-  xm_apply<N, E3_PRE>(X, x_ncol, nlev, col0 + g0, ncl, store, tb, lds, status, pre);
+  xm_tprime<N>(tb, km);
+  xm_apply<N, E3_PRE>(X, km, x_ncol, nlev, col0 + g0, ncl, store, tb, lds, status, pre);
 }
 
 // ---------------------------------------------------------------------------
@@ -1108,7 +1117,7 @@ __device__ inline double block_total(double v, double* red) {
 template <int N, int R>
 __global__ __launch_bounds__(2 * N, 2) void k_trd_wr(int64_t ncol, const double* __restrict__ C,
                                                      int c32, const int* __restrict__ nloc,
-                                                     double rho,
+                                                     int km, double rho,
                                                      const double* __restrict__ rho_col,
                                                      int prior, double* __restrict__ de,
                                                      double* __restrict__ Uout) {
@@ -1121,7 +1130,7 @@ __global__ __launch_bounds__(2 * N, 2) void k_trd_wr(int64_t ncol, const double*
   const int64_t g = blockIdx.x;
   if (g >= ncol || nloc[g] == 0) return;  // block-uniform
   const double rr = rho_col ? rho_col[g] : rho;
-  const double sigma = prior ? (double)(n - 1) / rr : (double)(n - 1);
+  const double sigma = prior ? (double)(km - 1) / rr : (double)(km - 1);
   double a[R][M];  // a[i][m] = A[rb + i][G m + h]
   if (c32) {  // FP32 entries, widened
     const float* Cg = reinterpret_cast<const float*>(C) + (size_t)g * n * n;
@@ -1271,7 +1280,7 @@ __global__ __launch_bounds__(2 * N, 2) void k_trd_wr(int64_t ncol, const double*
 template <int N>
 __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
     int64_t ncol, const int* __restrict__ nloc, const double* __restrict__ de,
-    const double* __restrict__ lam, const double* __restrict__ bvec, double rho,
+    const double* __restrict__ lam, const double* __restrict__ bvec, int km, double rho,
     const double* __restrict__ rho_col, int prior, int combine, double null_rel,
     const double* __restrict__ Ug, double* __restrict__ T, int* __restrict__ flag) {
   // N = 64 (two wavefronts, four columns per CU) measured slower than the
@@ -1409,7 +1418,7 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
     for (int m = 0; m < M; ++m) z[m] *= inv;
   }
   const bool pri = prior != 0;
-  const double sigma = pri ? (double)(n - 1) / r : (double)(n - 1);
+  const double sigma = pri ? (double)(km - 1) / r : (double)(km - 1);
   const double null_tol = fmax(2e-12 * sigma, null_rel * tnorm);
   const bool skip = fabs(l - sigma) <= null_tol;
   const double wj = skip ? 0.0 : 1.0 - sigma / l;
@@ -1634,7 +1643,7 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
     }
   }
   __syncthreads();
-  const double coef = sqrt((double)(n - 1)) * sqrt(sc);
+  const double coef = sqrt((double)(km - 1)) * sqrt(sc);
   const double fs = 1.0 / sqrt(sigma);
   // wbar_j = s [ b_j / sigma - sum_e U_s[j][e] y'_e ], row j by its pair
   double wbar;
@@ -1690,15 +1699,15 @@ template <int N>
 static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, double* lam,
                          int* flag) {
   const int prior = a.inflation_form == MDA_INFLFORM_PRIOR;
-  launch_zero(s, flag, sizeof(int) * a.ncol);
+  const int* nloc = a.eig_nloc ? a.eig_nloc : a.nloc;
   MDA_REQUIRE(a.ncol < (int64_t)1 << 31, "eigensolver grid too large");
   const unsigned nb = (unsigned)a.ncol;  // one column per block
-  hipLaunchKernelGGL(k_trd<N>, dim3(nb), dim3(64), 0, s, a.ncol, a.C, a.c32, a.nloc, a.rho,
-                     a.rho_col, prior, de, a.U);
+  hipLaunchKernelGGL(k_trd<N>, dim3(nb), dim3(64), 0, s, a.ncol, a.C, a.c32, nloc, a.k,
+                     a.rho, a.rho_col, prior, de, a.U);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[0]) MDA_HIP(hipEventRecord(a.ev_stage[0], s));
   hipLaunchKernelGGL(k_trd_eigvals<N>, dim3((unsigned)((a.ncol + 63) / 64)), dim3(64), 0, s,
-                     a.ncol, a.nloc, de, lam, flag);
+                     a.ncol, nloc, de, lam, flag);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[1]) MDA_HIP(hipEventRecord(a.ev_stage[1], s));
   if constexpr (N % 16 == 0) {
@@ -1708,18 +1717,18 @@ static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, d
       const int64_t ngrp = (a.ncol + XM_C - 1) / XM_C;
       MDA_REQUIRE(ngrp < (int64_t)1 << 31, "eigenvector grid too large");
       const unsigned nbx = (unsigned)((ngrp + 7) / 8 * 8);
-      hipLaunchKernelGGL(k_trd_vectors_x<N>, dim3(nbx), dim3(256), 0, s, a.ncol, a.nloc, de, lam,
-                         a.b, a.rho, a.rho_col, prior, a.null_rel, a.U, flag, a.X, a.x_ncol,
+      hipLaunchKernelGGL(k_trd_vectors_x<N>, dim3(nbx), dim3(256), 0, s, a.ncol, nloc, de, lam,
+                         a.b, a.k, a.rho, a.rho_col, prior, a.null_rel, a.U, flag, a.X, a.x_ncol,
                          a.x_nlev, a.x_col0, a.status);
       MDA_LAUNCH_CHECK();
       if (a.ev_stage[2]) MDA_HIP(hipEventRecord(a.ev_stage[2], s));
       return;
     }
   }
-  MDA_REQUIRE(!a.fuse, "fused eigenvector transform: no kernel for this k");
+  MDA_REQUIRE(!a.fuse, "fused eigenvector transform: no kernel for this block size");
   MDA_REQUIRE(a.ncol < (int64_t)1 << 31, "eigenvector grid too large");
-  hipLaunchKernelGGL(k_trd_vectors<N>, dim3((unsigned)a.ncol), dim3(64), 0, s, a.ncol, a.nloc, de, lam, a.b,
-                     a.rho, a.rho_col, prior, a.combine, a.null_rel, a.U, a.T, flag);
+  hipLaunchKernelGGL(k_trd_vectors<N>, dim3((unsigned)a.ncol), dim3(64), 0, s, a.ncol, nloc, de, lam, a.b,
+                     a.k, a.rho, a.rho_col, prior, a.combine, a.null_rel, a.U, a.T, flag);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[2]) MDA_HIP(hipEventRecord(a.ev_stage[2], s));
 }
@@ -1728,38 +1737,57 @@ static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, d
 template <int N>
 static void launch_eig_w(hipStream_t s, const letkf_solve_args& a, double* de, double* lam,
                          int* flag) {
-  MDA_REQUIRE(!a.fuse, "fused eigenvector transform: no kernel for this k");
+  MDA_REQUIRE(!a.fuse, "fused eigenvector transform: no kernel for this block size");
   const int prior = a.inflation_form == MDA_INFLFORM_PRIOR;
-  launch_zero(s, flag, sizeof(int) * a.ncol);
+  const int* nloc = a.eig_nloc ? a.eig_nloc : a.nloc;
   MDA_REQUIRE(a.ncol < (int64_t)1 << 31, "eigensolver grid too large");
   const unsigned nb = (unsigned)a.ncol;  // one column per block
-  hipLaunchKernelGGL((k_trd_wr<N, 2>), dim3(nb), dim3(2 * N), 0, s, a.ncol, a.C, a.c32, a.nloc,
-                     a.rho, a.rho_col, prior, de, a.U);
+  hipLaunchKernelGGL((k_trd_wr<N, 2>), dim3(nb), dim3(2 * N), 0, s, a.ncol, a.C, a.c32, nloc,
+                     a.k, a.rho, a.rho_col, prior, de, a.U);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[0]) MDA_HIP(hipEventRecord(a.ev_stage[0], s));
   hipLaunchKernelGGL(k_trd_eigvals_bisect<N>, dim3((unsigned)((a.ncol + 3) / 4)), dim3(256), 0,
-                     s, a.ncol, a.nloc, de, lam, flag);
+                     s, a.ncol, nloc, de, lam, flag);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[1]) MDA_HIP(hipEventRecord(a.ev_stage[1], s));
   MDA_REQUIRE(a.ncol < (int64_t)1 << 31, "eigenvector grid too large");
-  hipLaunchKernelGGL(k_trd_vectors_w4<N>, dim3((unsigned)a.ncol), dim3(2 * N), 0, s, a.ncol, a.nloc, de, lam, a.b,
-                     a.rho, a.rho_col, prior, a.combine, a.null_rel, a.U, a.T, flag);
+  hipLaunchKernelGGL(k_trd_vectors_w4<N>, dim3((unsigned)a.ncol), dim3(2 * N), 0, s, a.ncol, nloc, de, lam, a.b,
+                     a.k, a.rho, a.rho_col, prior, a.combine, a.null_rel, a.U, a.T, flag);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[2]) MDA_HIP(hipEventRecord(a.ev_stage[2], s));
 }
 
-bool letkf_eig_fusable(int k) { return k == 16 || k == 32 || k == 48 || k == 64; }
+bool letkf_eig_fusable(int ks) { return ks == 16 || ks == 32 || ks == 48 || ks == 64; }
 
-bool letkf_eig_supported(int k) {
-  switch (k) {
-    case 8: case 16: case 20: case 32: case 40: case 48: case 64: case 128: return true;
-    default: return false;
+int letkf_eig_size(int k) {
+  for (int n : {8, 16, 20, 32, 40, 48, 64, 128})
+    if (k <= n) return n;
+  throw mda_error(MDA_E_UNSUPPORTED, "tridiagonal eigensolver supports k <= 128");
+}
+
+// Columns with fewer than k observations leave the tridiagonal path: their
+// count in eig_nloc is 0 (its kernels then skip them) and their flag is set.
+__global__ void k_eig_select(int64_t ncol, int k, const int* __restrict__ nloc,
+                             int* __restrict__ eig_nloc, int* __restrict__ flag) {
+  for (int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < ncol;
+       g += (int64_t)gridDim.x * blockDim.x) {
+    const int nl = nloc[g];
+    eig_nloc[g] = nl >= k ? nl : 0;
+    flag[g] = nl > 0 && nl < k ? 16 : 0;
   }
 }
 
 void launch_letkf_eig(hipStream_t s, const letkf_solve_args& a, double* de, double* lam,
                       int* flag) {
-  switch (a.k) {
+  if (a.eig_nloc) {
+    MDA_REQUIRE(!a.fuse, "columns left out of the eigenvector kernel need a stored transform");
+    hipLaunchKernelGGL(k_eig_select, dim3(grid_for(a.ncol, 256, 4096)), dim3(256), 0, s, a.ncol,
+                       a.k, a.nloc, a.eig_nloc, flag);
+    MDA_LAUNCH_CHECK();
+  } else {
+    launch_zero(s, flag, sizeof(int) * a.ncol);
+  }
+  switch (a.ks) {
     case 8: launch_eig_n<8>(s, a, de, lam, flag); break;
     case 16: launch_eig_n<16>(s, a, de, lam, flag); break;
     case 20: launch_eig_n<20>(s, a, de, lam, flag); break;
@@ -1768,7 +1796,7 @@ void launch_letkf_eig(hipStream_t s, const letkf_solve_args& a, double* de, doub
     case 48: launch_eig_n<48>(s, a, de, lam, flag); break;
     case 64: launch_eig_n<64>(s, a, de, lam, flag); break;
     case 128: launch_eig_w<128>(s, a, de, lam, flag); break;
-    default: throw mda_error(MDA_E_UNSUPPORTED, "tridiagonal eigensolver: no kernel for this k");
+    default: throw mda_error(MDA_E_UNSUPPORTED, "tridiagonal eigensolver: no kernel for this block size");
   }
 }
 

@@ -666,10 +666,11 @@ __device__ __forceinline__ void gram_f64_body(const letkf_gram_args& a) {
       bp[ta] += __shfl_xor(bp[ta], 16);
       bp[ta] += __shfl_xor(bp[ta], 32);
     }
-    double* Cg = a.C + (size_t)g * k * k;
-    // k and the lane coordinates through opaque copies: the element offsets
-    // below are recomputed per column, not kept live across the search
-    int ko = k, kk_e = kk, i16_e = i16;
+    double* Cg = a.C + (size_t)g * a.ks * a.ks;
+    // the block size (rows and columns past k are sums of zeros) and the lane
+    // coordinates through opaque copies: the element offsets below are
+    // recomputed per column, not kept live across the search
+    int ko = a.ks, kk_e = kk, i16_e = i16;
     __asm__ volatile("" : "+s"(ko), "+v"(kk_e), "+v"(i16_e));
     int tile = 0;
 #pragma unroll
@@ -694,7 +695,7 @@ __device__ __forceinline__ void gram_f64_body(const letkf_gram_args& a) {
 #pragma unroll
       for (int ta = 0; ta < KT; ++ta) {
         int e = 16 * ta + i16;
-        if (e < k) a.b[(size_t)g * k + e] = bp[ta];
+        if (e < a.ks) a.b[(size_t)g * a.ks + e] = bp[ta];
       }
     }
     if (lane == 0) a.nloc[g] = nl;
@@ -1169,14 +1170,17 @@ __device__ __forceinline__ void gram_mixed_body(const letkf_gram_args& a) {
     if (kq_e == 0) {
 #pragma unroll
       for (int t = 0; t < KT; ++t)
-        if (16 * t + i16_e < k) a.b[(size_t)g * k + 16 * t + i16_e] = bacc[t] - bsum * rk;
+        if (16 * t + i16_e < a.ks)
+          a.b[(size_t)g * a.ks + 16 * t + i16_e] =
+              16 * t + i16_e < k ? bacc[t] - bsum * rk : 0.0;
     }
-    double* Cg = a.C + (size_t)g * k * k;
-    float* Cf = reinterpret_cast<float*>(a.C) + (size_t)g * k * k;
+    double* Cg = a.C + (size_t)g * a.ks * a.ks;
+    float* Cf = reinterpret_cast<float*>(a.C) + (size_t)g * a.ks * a.ks;
     const bool c32 = a.c32 != 0;
-    // k through an opaque copy: the element offsets below are recomputed per
-    // column instead of being kept live across the candidate loop
-    int ko = k;
+    // the block size through an opaque copy: the element offsets below are
+    // recomputed per column instead of being kept live across the candidate
+    // loop; entries past k are zero
+    int ko = a.ks;
     __asm__ volatile("" : "+s"(ko));
     int tile = 0;
 #pragma unroll
@@ -1187,7 +1191,9 @@ __device__ __forceinline__ void gram_mixed_body(const letkf_gram_args& a) {
         for (int r = 0; r < 4; ++r) {
           const int row = 16 * ta + 4 * kq_e + r, col = 16 * tb + i16_e;
           if (row < ko && col < ko) {
-            const double v = (double)acc[tile][r] - (rsum[row] + rsum[col]) * rk + tot;
+            const double v = row < k && col < k
+                                 ? (double)acc[tile][r] - (rsum[row] + rsum[col]) * rk + tot
+                                 : 0.0;
             if (c32) {
               Cf[row * ko + col] = (float)v;
               if (ta != tb) Cf[col * ko + row] = (float)v;
@@ -1254,15 +1260,16 @@ __global__ __launch_bounds__(256) void k_letkf_shell_fixup(letkf_gram_args a,
     if (sg == 0.0) continue;
     const double* y = a.yp + (size_t)t * k;
     if (a.c32) {
-      float* Cf = reinterpret_cast<float*>(a.C) + (size_t)g * k * k;
+      float* Cf = reinterpret_cast<float*>(a.C) + (size_t)g * a.ks * a.ks;
       for (int idx = lane; idx < k * k; idx += 64)
-        atomicAdd(&Cf[idx], (float)(sg * y[idx / k] * y[idx % k]));
+        atomicAdd(&Cf[(idx / k) * a.ks + idx % k], (float)(sg * y[idx / k] * y[idx % k]));
     } else {
-      double* Cg = a.C + (size_t)g * k * k;
+      double* Cg = a.C + (size_t)g * a.ks * a.ks;
       for (int idx = lane; idx < k * k; idx += 64)
-        atomicAdd(&Cg[idx], sg * y[idx / k] * y[idx % k]);
+        atomicAdd(&Cg[(idx / k) * a.ks + idx % k], sg * y[idx / k] * y[idx % k]);
     }
-    for (int i = lane; i < k; i += 64) atomicAdd(&a.b[(size_t)g * k + i], sg * y[i] * a.d[t]);
+    for (int i = lane; i < k; i += 64)
+      atomicAdd(&a.b[(size_t)g * a.ks + i], sg * y[i] * a.d[t]);
   }
 }
 
@@ -1406,6 +1413,8 @@ void launch_column_setup(hipStream_t s, const letkf_gram_args& a) {
 
 void launch_letkf_gram(hipStream_t s, const letkf_gram_args& a) {
   MDA_REQUIRE(a.k >= 1 && a.k <= 128, "LETKF Gram supports k <= 128");
+  MDA_REQUIRE(a.ks >= a.k && a.ks <= (a.k > 64 ? 128 : (a.k + 15) / 16 * 16),
+              "the Gram's tiles cover its column blocks");
   // FP32 entries of C exactly for the FP32 / BF16x3 contractions (the FP64
   // kernels write doubles)
   MDA_REQUIRE((a.c32 != 0) == (a.precision != MDA_PREC_FP64), "Gram storage precision mismatch");
@@ -1493,7 +1502,7 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
   __shared__ double rc[64], rs[64], red[256], bv[128], yv[128], wb[128];
   __shared__ int rp[64], rq[64], flag;
   const int k = a.k, tid = threadIdx.x, nt = blockDim.x;
-  const int kp = (k + 1) & ~1, ld = kp + 1;
+  const int kp = (k + 1) & ~1, ld = kp + 1, ks = a.ks;
   double* A = use_lds ? sh : gscratch + (size_t)blockIdx.x * 2 * kp * ld;
   double* V = A + kp * ld;
   // fallback mode: the listed columns (flagged, or empty: sqrt(rho) I);
@@ -1503,27 +1512,32 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
     const int64_t g = list ? (int64_t)list[it] : it;
     if (only && only[g] == 0 && a.nloc[g] != 0) continue;
     const double rho = a.rho_col ? a.rho_col[g] : a.rho;
-    double* Tg = a.T + (size_t)g * k * k;
+    double* Tg = a.T + (size_t)g * ks * ks;
+    // the block's entries past k (block sizes above k) are zero
+    if (ks > k)
+      for (int idx = tid; idx < ks * ks; idx += nt)
+        if (idx / ks >= k || idx % ks >= k) Tg[idx] = 0.0;
     if (a.nloc[g] == 0) {
       const double sr = sqrt(rho);
-      for (int idx = tid; idx < k * k; idx += nt) Tg[idx] = (idx / k == idx % k) ? sr : 0.0;
+      for (int idx = tid; idx < k * k; idx += nt)
+        Tg[(idx / k) * ks + idx % k] = (idx / k == idx % k) ? sr : 0.0;
       if (tid == 0 && a.sweeps) a.sweeps[g] = 0;
       continue;
     }
     const bool prior = a.inflation_form == MDA_INFLFORM_PRIOR;
     const double sigma = prior ? (double)(k - 1) / rho : (double)(k - 1);
     const double sc = prior ? 1.0 : rho;
-    const double* Cg = a.C + (size_t)g * k * k;
-    const float* Cf = reinterpret_cast<const float*>(a.C) + (size_t)g * k * k;
+    const double* Cg = a.C + (size_t)g * ks * ks;
+    const float* Cf = reinterpret_cast<const float*>(a.C) + (size_t)g * ks * ks;
     for (int idx = tid; idx < kp * kp; idx += nt) {
       int i = idx / kp, j = idx % kp;
       double v;
       if (i < k && j < k)
-        v = (a.c32 ? (double)Cf[i * k + j] : Cg[i * k + j]) + (i == j ? sigma : 0.0);
+        v = (a.c32 ? (double)Cf[i * ks + j] : Cg[i * ks + j]) + (i == j ? sigma : 0.0);
       else v = (i == j) ? 1.0 : 0.0;  // decoupled pad index (odd k)
       A[i * ld + j] = v;
     }
-    for (int i = tid; i < k; i += nt) bv[i] = a.b[(size_t)g * k + i];
+    for (int i = tid; i < k; i += nt) bv[i] = a.b[(size_t)g * ks + i];
     __syncthreads();
     const double sq = sqrt((double)(k - 1));
     if (a.sqrt_form == MDA_SQRT_SYMMETRIC) {
@@ -1554,7 +1568,7 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
           int i = idx / k, j = idx % k;
           double s = 0.0;
           for (int e = 0; e < k; ++e) s += V[i * ld + e] * V[j * ld + e];
-          Tg[idx] = wb[i] + coef * s;
+          Tg[i * ks + j] = wb[i] + coef * s;
         }
       } else {
         for (int i = tid; i < k; i += nt) {
@@ -1568,7 +1582,7 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
         }
         __syncthreads();
         for (int idx = tid; idx < k * k; idx += nt)
-          Tg[idx] = (idx / k == idx % k) ? yv[idx / k] : 0.0;
+          Tg[(idx / k) * ks + idx % k] = (idx / k == idx % k) ? yv[idx / k] : 0.0;
       }
     } else {
       bool ok = block_cholesky(A, ld, k, &flag);
@@ -1586,7 +1600,7 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
       if (a.combine == MDA_COMBINE_MATRIX) {
         for (int idx = tid; idx < k * k; idx += nt) {
           int i = idx / k, j = idx % k;
-          Tg[idx] = wb[i] + sq * A[i * ld + j];
+          Tg[i * ks + j] = wb[i] + sq * A[i * ld + j];
         }
       } else {
         for (int i = tid; i < k; i += nt) {
@@ -1596,7 +1610,7 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
         }
         __syncthreads();
         for (int idx = tid; idx < k * k; idx += nt)
-          Tg[idx] = (idx / k == idx % k) ? yv[idx / k] : 0.0;
+          Tg[(idx / k) * ks + idx % k] = (idx / k == idx % k) ? yv[idx / k] : 0.0;
       }
       if (tid == 0 && a.sweeps) a.sweeps[g] = 0;
     }
@@ -1620,7 +1634,7 @@ void launch_letkf_solve(hipStream_t s, const letkf_solve_args& a) {
   const int* only = nullptr;
   const int* list = nullptr;
   const unsigned* cnt = nullptr;
-  if (a.sqrt_form == MDA_SQRT_SYMMETRIC && letkf_eig_supported(a.k) && a.method == 0) {
+  if (a.sqrt_form == MDA_SQRT_SYMMETRIC && a.method == MDA_EIG_AUTO) {
     // tridiagonal eigensolver; flagged columns fall back to Jacobi below
     launch_letkf_eig(s, a, a.de, a.lam, a.flag);
     only = a.flag;
@@ -1745,7 +1759,8 @@ constexpr int XT_C = 4, XT_L = 20;
 
 template <int K>
 __global__ __launch_bounds__(256) void k_letkf_transform_reg(double* __restrict__ X,
-                                                             int64_t ncol, int64_t nlev,
+                                                             int km, int64_t ncol,
+                                                             int64_t nlev,
                                                              const double* __restrict__ T,
                                                              int64_t col0, int64_t nc,
                                                              int* __restrict__ status) {
@@ -1760,7 +1775,7 @@ __global__ __launch_bounds__(256) void k_letkf_transform_reg(double* __restrict_
   const int64_t g0 = vb * XT_C;  // within the chunk [col0, col0 + nc)
   if (g0 >= nc) return;
   const int ncl = (int)(nc - g0 < XT_C ? nc - g0 : XT_C);
-  const bool own = j < K && c < ncl;
+  const bool own = j < km && c < ncl;
   double t[K];
   double colsum = 0.0;
   {
@@ -1771,7 +1786,7 @@ __global__ __launch_bounds__(256) void k_letkf_transform_reg(double* __restrict_
       colsum += t[m];
     }
   }
-  const double rk = 1.0 / (double)K;
+  const double rk = 1.0 / (double)km;
   const double cmean = 1.0 - colsum;
   for (int64_t l0 = 0; l0 < nlev; l0 += XT_L) {
     const int nll = (int)(nlev - l0 < XT_L ? nlev - l0 : XT_L);
@@ -1779,7 +1794,8 @@ __global__ __launch_bounds__(256) void k_letkf_transform_reg(double* __restrict_
     for (int idx = tid; idx < K * XT_L * XT_C; idx += 256) {
       const int cc = idx % XT_C, l = (idx / XT_C) % XT_L, m = idx / (XT_C * XT_L);
       if (cc < ncl && l < nll)
-        xs[(l * XT_C + cc) * KP + m] = X[(size_t)m * n + (l0 + l) * ncol + col0 + g0 + cc];
+        xs[(l * XT_C + cc) * KP + m] =
+            m < km ? X[(size_t)m * n + (l0 + l) * ncol + col0 + g0 + cc] : 0.0;
     }
     __syncthreads();
     if (own) {
@@ -1810,7 +1826,7 @@ __global__ __launch_bounds__(256) void k_letkf_transform_reg(double* __restrict_
 // the columns the eigenvector kernel left to the Jacobi fallback.
 template <int K>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void k_letkf_transform_mfma(double* __restrict__ X, int64_t ncol, int64_t nlev,
+void k_letkf_transform_mfma(double* __restrict__ X, int km, int64_t ncol, int64_t nlev,
                             const double* __restrict__ T, int64_t col0, int64_t nc,
                             int* __restrict__ status, const int* __restrict__ only) {
   static_assert(K % 16 == 0 && K <= 64, "K must be a multiple of 16, at most 64");
@@ -1842,8 +1858,8 @@ void k_letkf_transform_mfma(double* __restrict__ X, int64_t ncol, int64_t nlev,
       for (int tj = 0; tj < NTJ; ++tj)
         tb[s4][tj] = own ? Tg[(size_t)(4 * s4 + kk) * K + 16 * tj + i16] : 0.0;
   }
-  xm_tprime<K>(tb);
-  xm_apply<K>(X, ncol, nlev, col0 + g0, ncl, store, tb, xs, status);
+  xm_tprime<K>(tb, km);
+  xm_apply<K>(X, km, ncol, nlev, col0 + g0, ncl, store, tb, xs, status);
 }
 
 // 4''''. X_a = X T' for K = 128 on FP64 MFMA: a block of 8 wavefronts takes
@@ -1856,7 +1872,7 @@ constexpr int X2_C = 2;
 
 template <int K>
 __global__ __launch_bounds__(512) void k_letkf_transform_mfma2(
-    double* __restrict__ X, int64_t ncol, int64_t nlev, const double* __restrict__ T,
+    double* __restrict__ X, int km, int64_t ncol, int64_t nlev, const double* __restrict__ T,
     int64_t col0, int64_t nc, int* __restrict__ status, const int* __restrict__ only) {
   static_assert(K == 128, "eight 16-member tiles over four wavefronts");
   if (*status & MDA_ST_SKIP_UPDATE) return;
@@ -1897,7 +1913,7 @@ __global__ __launch_bounds__(512) void k_letkf_transform_mfma2(
         tb[s4][tt] = own ? Tg[(size_t)(4 * s4 + kk) * K + 16 * (2 * tp + tt) + i16] : 0.0;
         cs[tt] += tb[s4][tt];
       }
-    const double rk = 1.0 / (double)K;
+    const double rk = 1.0 / (double)km;
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
       cs[tt] += __shfl_xor(cs[tt], 16);
@@ -1915,7 +1931,7 @@ __global__ __launch_bounds__(512) void k_letkf_transform_mfma2(
       const int idx = tid + 512 * q;
       const int cc = idx % X2_C, l = (idx / X2_C) % XM_L, m = idx / (X2_C * XM_L);
       double v = 0.0;
-      if (cc < ncl && l < nll) v = X[(size_t)m * n + (l0 + l) * ncol + col0 + g0 + cc];
+      if (cc < ncl && l < nll && m < km) v = X[(size_t)m * n + (l0 + l) * ncol + col0 + g0 + cc];
       pv[q] = v;
     }
   };
@@ -1964,7 +1980,7 @@ __global__ __launch_bounds__(512) void k_letkf_transform_mfma2(
       const int idx = tid + 512 * q;
       const int cc = idx % X2_C, w = idx / 64;
       const int j = 32 * (w % (K / 32)) + (idx / X2_C) % 32, l = w / (K / 32);
-      if (cc < ncl && l < nll && ((store >> cc) & 1u))
+      if (cc < ncl && l < nll && j < km && ((store >> cc) & 1u))
         X[(size_t)j * n + (l0 + l) * ncol + col0 + g0 + cc] = xs[cc * CSO + l * LJ + j];
     }
   }
@@ -2110,32 +2126,32 @@ void k_letkf_transform_bf16x3(double* __restrict__ X, int64_t ncol, int64_t nlev
   }
 }
 
-bool letkf_transform_reg_supported(int k) {
-  switch (k) {
+bool letkf_transform_reg_supported(int ks) {
+  switch (ks) {
     case 8: case 16: case 20: case 32: case 40: case 48: case 64: return true;
     default: return false;
   }
 }
 
-void launch_letkf_transform(hipStream_t s, double* X, int k, int64_t ncol, int64_t nlev,
-                            const double* T, int* status, int64_t col0, int64_t nc,
+void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t ncol,
+                            int64_t nlev, const double* T, int* status, int64_t col0, int64_t nc,
                             int precision, const int* only) {
   MDA_REQUIRE(status != nullptr, "transform needs the analysis status word");
-  MDA_REQUIRE(k <= 128, "transform supports k <= 128");
+  MDA_REQUIRE(k <= ks && ks <= 128, "transform supports k <= 128");
   if (nc < 0) nc = ncol;
   MDA_REQUIRE(col0 >= 0 && col0 + nc <= ncol, "transform column range out of bounds");
   if (nc == 0) return;
-  MDA_REQUIRE(!only || (precision != MDA_PREC_BF16X3 && ((k % 16 == 0 && k <= 64) || k == 128)),
+  MDA_REQUIRE(!only || (precision != MDA_PREC_BF16X3 && ((ks % 16 == 0 && ks <= 64) || ks == 128)),
               "a column-restricted transform needs the FP64 MFMA path");
-  if (k == 128 && precision != MDA_PREC_BF16X3) {
+  if (ks == 128 && precision != MDA_PREC_BF16X3) {
     MDA_REQUIRE((nc + X2_C - 1) / X2_C < (int64_t)1 << 31, "transform grid too large");
     const unsigned nb2 = (unsigned)(((nc + X2_C - 1) / X2_C + 7) / 8 * 8);
-    hipLaunchKernelGGL(k_letkf_transform_mfma2<128>, dim3(nb2), dim3(512), 0, s, X, ncol, nlev, T,
-                       col0, nc, status, only);
+    hipLaunchKernelGGL(k_letkf_transform_mfma2<128>, dim3(nb2), dim3(512), 0, s, X, k, ncol, nlev,
+                       T, col0, nc, status, only);
     MDA_LAUNCH_CHECK();
     return;
   }
-  if (precision == MDA_PREC_BF16X3 && k % 16 == 0 && k <= 64) {
+  if (precision == MDA_PREC_BF16X3 && k == ks && k % 16 == 0 && k <= 64) {
     MDA_REQUIRE((nc + XM_C - 1) / XM_C < (int64_t)1 << 31, "transform grid too large");
     const unsigned nbm = (unsigned)(((nc + XM_C - 1) / XM_C + 7) / 8 * 8);
     switch (k) {
@@ -2147,32 +2163,33 @@ void launch_letkf_transform(hipStream_t s, double* X, int k, int64_t ncol, int64
     MDA_LAUNCH_CHECK();
     return;
   }
-  if (k % 16 == 0 && k <= 64) {
+  if (ks % 16 == 0 && ks <= 64) {
     MDA_REQUIRE((nc + XM_C - 1) / XM_C < (int64_t)1 << 31, "transform grid too large");
     const unsigned nbm = (unsigned)(((nc + XM_C - 1) / XM_C + 7) / 8 * 8);
-    switch (k) {
-      case 16: hipLaunchKernelGGL(k_letkf_transform_mfma<16>, dim3(nbm), dim3(256), 0, s, X, ncol, nlev, T, col0, nc, status, only); break;
-      case 32: hipLaunchKernelGGL(k_letkf_transform_mfma<32>, dim3(nbm), dim3(256), 0, s, X, ncol, nlev, T, col0, nc, status, only); break;
-      case 48: hipLaunchKernelGGL(k_letkf_transform_mfma<48>, dim3(nbm), dim3(256), 0, s, X, ncol, nlev, T, col0, nc, status, only); break;
-      default: hipLaunchKernelGGL(k_letkf_transform_mfma<64>, dim3(nbm), dim3(256), 0, s, X, ncol, nlev, T, col0, nc, status, only); break;
+    switch (ks) {
+      case 16: hipLaunchKernelGGL(k_letkf_transform_mfma<16>, dim3(nbm), dim3(256), 0, s, X, k, ncol, nlev, T, col0, nc, status, only); break;
+      case 32: hipLaunchKernelGGL(k_letkf_transform_mfma<32>, dim3(nbm), dim3(256), 0, s, X, k, ncol, nlev, T, col0, nc, status, only); break;
+      case 48: hipLaunchKernelGGL(k_letkf_transform_mfma<48>, dim3(nbm), dim3(256), 0, s, X, k, ncol, nlev, T, col0, nc, status, only); break;
+      default: hipLaunchKernelGGL(k_letkf_transform_mfma<64>, dim3(nbm), dim3(256), 0, s, X, k, ncol, nlev, T, col0, nc, status, only); break;
     }
     MDA_LAUNCH_CHECK();
     return;
   }
-  if (letkf_transform_reg_supported(k)) {
+  if (letkf_transform_reg_supported(ks)) {
     MDA_REQUIRE((nc + XT_C - 1) / XT_C < (int64_t)1 << 31, "transform grid too large");
     const unsigned nbr = (unsigned)(((nc + XT_C - 1) / XT_C + 7) / 8 * 8);
-    const size_t shr = sizeof(double) * XT_L * XT_C * (k + 2);
+    const size_t shr = sizeof(double) * XT_L * XT_C * (ks + 2);
 #define MDA_XT(KK)                                                                          \
   case KK:                                                                                 \
-    hipLaunchKernelGGL(k_letkf_transform_reg<KK>, dim3(nbr), dim3(256), shr, s, X, ncol, nlev, T, \
-                       col0, nc, status);                                                    \
+    hipLaunchKernelGGL(k_letkf_transform_reg<KK>, dim3(nbr), dim3(256), shr, s, X, k, ncol, nlev,  \
+                       T, col0, nc, status);                                                 \
     break;
-    switch (k) { MDA_XT(8) MDA_XT(16) MDA_XT(20) MDA_XT(32) MDA_XT(40) MDA_XT(48) MDA_XT(64) }
+    switch (ks) { MDA_XT(8) MDA_XT(16) MDA_XT(20) MDA_XT(32) MDA_XT(40) MDA_XT(48) MDA_XT(64) }
 #undef MDA_XT
     MDA_LAUNCH_CHECK();
     return;
   }
+  MDA_REQUIRE(ks == k, "transform: no kernel for this block size");
   size_t shm = sizeof(double) * TR_L * TR_C * (k + 1);
   const int64_t tiles = ((nc + TR_C - 1) / TR_C) * ((nlev + TR_L - 1) / TR_L);
   MDA_REQUIRE(tiles < (int64_t)1 << 31, "transform grid too large");

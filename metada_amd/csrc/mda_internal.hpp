@@ -79,7 +79,8 @@ struct mda_ctx {
   // state of the last LETKF call (for mda_letkf_last_transforms)
   int last_k = 0;
   int64_t last_ncol = 0;
-  double* last_T = nullptr;  // device, [ncol][k][k]
+  int last_ks = 0;           // block size of last_T
+  double* last_T = nullptr;  // device, [ncol][last_ks][last_ks]
   int* last_nloc = nullptr;  // device, [ncol]
   int* last_flag = nullptr;  // device, [ncol] (tridiagonal path only)
 
@@ -235,6 +236,9 @@ void launch_gather_rows(hipStream_t s, const uint32_t* order, int64_t p, int k,
                         float* y32);
 struct letkf_gram_args {
   int k;
+  // size of the per-column blocks C [ks][ks] and b [ks]: k, or the padded
+  // size of the eigensolver's kernels (letkf_eig_size), zeros past k
+  int ks;
   int64_t ncol, nx;
   int coord;
   const double* col_a;
@@ -255,11 +259,11 @@ struct letkf_gram_args {
   const double* ux;    // sorted unit vectors of GEOGRAPHIC observation locations (any precision)
   const double* uy;
   const double* uz;
-  double* C;    // out [ncol][k][k]
+  double* C;    // out [ncol][ks][ks]
   // C holds FP32 entries (the FP32 / BF16x3 contractions, whose products are
   // accumulated in FP32): half the buffer is used, E1 widens them to FP64
   int c32;
-  double* b;    // out [ncol][k]
+  double* b;    // out [ncol][ks]
   int* nloc;    // out [ncol]
   // per-column setup records [ncol][96] of the Gram (window rows, row table,
   // reference point), from launch_column_setup
@@ -308,6 +312,7 @@ void launch_mlp_adam(hipStream_t s, float* params, float* m1, float* m2, const f
                      int64_t step, float lr, float b1, float b2, float eps);
 struct letkf_solve_args {
   int k;
+  int ks;  // size of the per-column blocks C, T, U, b, lam (letkf_gram_args::ks)
   int64_t ncol;
   const double* C;
   int c32;  // C holds FP32 entries (letkf_gram_args::c32)
@@ -319,10 +324,10 @@ struct letkf_solve_args {
   double* T;
   int* sweeps;
   int* status;
-  // tridiagonal eigensolver workspace (symmetric square root, k <= 64)
-  double* de;    // [ncol][2k]
-  double* lam;   // [ncol][k]
-  double* U;     // [ncol][k][k] Householder reflectors
+  // tridiagonal eigensolver workspace (symmetric square root)
+  double* de;    // [ncol][2 ks]
+  double* lam;   // [ncol][ks]
+  double* U;     // [ncol][ks][ks] Householder reflectors
   int* flag;     // [ncol] columns re-solved by the Jacobi fallback
   // Jacobi in global memory (k too large for LDS): per-block scratch of
   // 2 kp (kp + 1) doubles for jblocks blocks
@@ -333,11 +338,15 @@ struct letkf_solve_args {
   int* wlist;
   unsigned* wcount;
   int method;    // 0: tridiagonal + Jacobi fallback, 1: Jacobi only
+  // set: the columns the tridiagonal kernels work on [ncol], nloc where
+  // nloc >= k and 0 elsewhere; the others with observations go to the
+  // fallback (k < ks with a reduced-precision Gram, see launch_letkf_solve)
+  int* eig_nloc;
   hipEvent_t ev_stage[3];  // recorded after E1, E2, E3 when set (timing)
   // Reduced-precision Gram: eigenvalues within null_rel * ||A|| of (k-1)/rho
   // are treated as the null space of Y'^T R^-1 Y' (0 for FP64)
   double null_rel;
-  // Fused eigenvectors + transform (tridiagonal path, k in {16, 32, 48, 64},
+  // Fused eigenvectors + transform (tridiagonal path, ks in {16, 32, 48, 64},
   // matrix combination, FP64 transform): E3 applies X_a = X T' to the pass's
   // columns [x_col0, x_col0 + ncol) of X (x_ncol columns of x_nlev levels)
   // and writes T only for the columns it leaves to the fallback (flag != 0)
@@ -346,21 +355,24 @@ struct letkf_solve_args {
   double* X;
   int64_t x_ncol, x_nlev, x_col0;
 };
-// true when the tridiagonal eigensolver can apply the transform itself
-bool letkf_eig_fusable(int k);
+// true when the tridiagonal eigensolver of block size ks can apply the
+// transform itself
+bool letkf_eig_fusable(int ks);
 void launch_letkf_solve(hipStream_t s, const letkf_solve_args& a);
-// ensemble sizes with a compiled tridiagonal eigensolver (others use Jacobi)
-bool letkf_eig_supported(int k);
+// block size of the tridiagonal eigensolver for k members: the smallest
+// compiled size >= k
+int letkf_eig_size(int k);
 void launch_letkf_eig(hipStream_t s, const letkf_solve_args& a, double* de, double* lam,
                       int* flag);
 // X_a = xbar + X' T for the columns [col0, col0 + nc) of X (ncol columns in
-// all; nc < 0: every column); T holds the nc columns' transforms.  Skipped
+// all; nc < 0: every column); T holds the nc columns' transforms, blocks of
+// ks x ks (ks = k, or letkf_eig_size(k)).  Skipped
 // when the status word holds a MDA_ST_SKIP_UPDATE bit.  MDA_PREC_BF16X3
 // runs X' T as split-precision bf16 products with FP32 accumulation (k a
 // multiple of 16, at most 64); otherwise FP64.  `only` ([nc], FP64 MFMA path
 // only) restricts the update to the columns with only[g] != 0.
-void launch_letkf_transform(hipStream_t s, double* X, int k, int64_t ncol, int64_t nlev,
-                            const double* T, int* status, int64_t col0 = 0, int64_t nc = -1,
+void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t ncol,
+                            int64_t nlev, const double* T, int* status, int64_t col0 = 0, int64_t nc = -1,
                             int precision = MDA_PREC_FP64, const int* only = nullptr);
 void launch_reduce_int(hipStream_t s, const int* v, int64_t n, int64_t* out2 /* sum,max */,
                        int64_t* out_empty);

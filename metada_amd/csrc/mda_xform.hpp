@@ -3,9 +3,11 @@
 // eigenvector kernel that applies its own transforms.  Both go through the
 // functions below, so a column gets bit-identical X_a either way.
 //
-// With T'[m][j] = T[m][j] + (1 - sum_m T[m][j]) / K,
+// K is the block size of T; the ensemble has km <= K members, and the staged
+// X holds zeros for the members past km, whose X_a is not written.
+// With T'[m][j] = T[m][j] + (1 - sum_m T[m][j]) / km,
 //   X_a[lev][j] = sum_m X[lev][m] T'[m][j]
-// (xbar = sum_m X[lev][m] / K), i.e. X_a = xbar + X' T = X T'.  The wavefront
+// (xbar = sum_m X[lev][m] / km), i.e. X_a = xbar + X' T = X T'.  The wavefront
 // keeps T' of its column in registers in the MFMA B layout (tb[s][tj] =
 // T'[4s + kk][16 tj + i16], lane = i16 + 16 kk) and runs
 // v_mfma_f64_16x16x4f64 over 16-level chunks.  X is staged through LDS as
@@ -47,9 +49,9 @@ typedef double xm_d4 __attribute__((ext_vector_type(4)));
 
 // T -> T' in place: column sums over the member index (each lane's K/4
 // entries in order, then the four kk groups by xor-shuffles) and the
-// correction (1 - colsum) / K.
+// correction (1 - colsum) / km.
 template <int K>
-__device__ __forceinline__ void xm_tprime(double (&tb)[K / 4][K / 16]) {
+__device__ __forceinline__ void xm_tprime(double (&tb)[K / 4][K / 16], int km) {
   constexpr int NTJ = K / 16, NS = K / 4;
   double cs[NTJ];
 #pragma unroll
@@ -58,7 +60,7 @@ __device__ __forceinline__ void xm_tprime(double (&tb)[K / 4][K / 16]) {
   for (int s4 = 0; s4 < NS; ++s4)
 #pragma unroll
     for (int tj = 0; tj < NTJ; ++tj) cs[tj] += tb[s4][tj];
-  const double rk = 1.0 / (double)K;
+  const double rk = 1.0 / (double)km;
 #pragma unroll
   for (int tj = 0; tj < NTJ; ++tj) {
     cs[tj] += __shfl_xor(cs[tj], 16);
@@ -76,11 +78,12 @@ constexpr int xm_nv() { return XM_C * XM_L * K / 256; }
 
 // Loads chunk c (levels 16c .. 16c + 15 of X[m][level][colbase + col]) into
 // v: element q of thread tid is (col, level, member) = (idx % 4, idx / 4 %
-// 16, idx / 64) with idx = tid + 256 q; zeros outside the columns and levels.
+// 16, idx / 64) with idx = tid + 256 q; zeros outside the columns, levels
+// and members.
 template <int K>
 __device__ __forceinline__ void xm_load(double (&v)[xm_nv<K>()], const double* __restrict__ X,
-                                        int64_t ncol, int64_t nlev, int64_t colbase, int ncl,
-                                        int64_t l0) {
+                                        int km, int64_t ncol, int64_t nlev, int64_t colbase,
+                                        int ncl, int64_t l0) {
   const int tid = threadIdx.x;
   const int64_t n = ncol * nlev;
   const int nll = (int)(nlev - l0 < XM_L ? (nlev - l0 > 0 ? nlev - l0 : 0) : XM_L);
@@ -89,7 +92,7 @@ __device__ __forceinline__ void xm_load(double (&v)[xm_nv<K>()], const double* _
     const int idx = tid + 256 * q;
     const int c = idx % XM_C, l = (idx / XM_C) % XM_L, m = idx / (XM_C * XM_L);
     double v0 = 0.0;
-    if (c < ncl && l < nll) v0 = X[(size_t)m * n + (l0 + l) * ncol + colbase + c];
+    if (c < ncl && l < nll && m < km) v0 = X[(size_t)m * n + (l0 + l) * ncol + colbase + c];
     v[q] = v0;
   }
 }
@@ -103,8 +106,8 @@ __device__ __forceinline__ void xm_load(double (&v)[xm_nv<K>()], const double* _
 // chunks are loaded one ahead of their products.  A non-finite X_a sets
 // MDA_ST_NONFINITE_STATE.
 template <int K, int NPC = 0>
-__device__ __forceinline__ void xm_apply(double* __restrict__ X, int64_t ncol, int64_t nlev,
-                                         int64_t colbase, int ncl, unsigned store,
+__device__ __forceinline__ void xm_apply(double* __restrict__ X, int km, int64_t ncol,
+                                         int64_t nlev, int64_t colbase, int ncl, unsigned store,
                                          const double (&tb)[K / 4][K / 16], double* xs,
                                          int* __restrict__ status,
                                          const double (*pre)[xm_nv<K>()] = nullptr) {
@@ -127,7 +130,7 @@ __device__ __forceinline__ void xm_apply(double* __restrict__ X, int64_t ncol, i
       xs[c * CSI + m * XM_L + l] = src[q];
     }
     __syncthreads();
-    if (load_next) xm_load<K>(pv, X, ncol, nlev, colbase, ncl, l0 + XM_L);
+    if (load_next) xm_load<K>(pv, X, km, ncol, nlev, colbase, ncl, l0 + XM_L);
     xm_d4 acc[NTJ];
 #pragma unroll
     for (int tj = 0; tj < NTJ; ++tj) acc[tj] = xm_d4{0.0, 0.0, 0.0, 0.0};
@@ -161,7 +164,7 @@ __device__ __forceinline__ void xm_apply(double* __restrict__ X, int64_t ncol, i
       const int idx = tid + 256 * q;
       const int c = idx % XM_C, w = idx / 64;
       const int j = 16 * (w % (K / 16)) + (idx / XM_C) % 16, l = w / (K / 16);
-      if (c < ncl && l < nll && ((store >> c) & 1u))
+      if (c < ncl && l < nll && j < km && ((store >> c) & 1u))
         X[(size_t)j * n + (l0 + l) * ncol + colbase + c] = xs[c * CSO + l * LJ + j];
     }
   };
@@ -171,7 +174,7 @@ __device__ __forceinline__ void xm_apply(double* __restrict__ X, int64_t ncol, i
     if (l0 >= nlev) return;  // block-uniform
     chunk(pre[ci], l0, ci == NPC - 1 && l0 + XM_L < nlev);
   }
-  if (NPC == 0) xm_load<K>(pv, X, ncol, nlev, colbase, ncl, 0);
+  if (NPC == 0) xm_load<K>(pv, X, km, ncol, nlev, colbase, ncl, 0);
   for (int64_t l0 = (int64_t)XM_L * NPC; l0 < nlev; l0 += XM_L) chunk(pv, l0, l0 + XM_L < nlev);
 }
 

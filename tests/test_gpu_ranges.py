@@ -3,7 +3,7 @@ chooses it can go wrong, against the oracle."""
 import numpy as np
 import pytest
 
-from cases import rel_err
+from cases import latlon_case, rel_err
 
 pytestmark = pytest.mark.gpu
 TOL = 1e-10
@@ -55,3 +55,52 @@ def test_bucket_ranges_match_oracle(mda, ctx, orc, p, where):
     np.testing.assert_array_equal(f.local_counts(), nloc)
     assert nloc.max() > 0
     assert rel_err(ens.data, Xo) < TOL
+
+
+# ---- ensemble sizes between the eigensolver's block sizes -----------------------------------
+def _latlon(mda, ctx, case, X, radius, **kw):
+    ens = mda.Ensemble(X.copy(), case["nlon"], case["nlat"], case["nlev"])
+    f = mda.LETKF(ens, mda.Observation(case["yo"], case["var"], case["lat"], case["lon"],
+                                       coord=mda._lib.COORD_GEOGRAPHIC), case["H"],
+                  mda.Config({"inflation": 1.05, "localization_radius": radius}),
+                  geometry=mda.ColumnGeometry(mda._lib.COORD_GEOGRAPHIC, case["col_lat"],
+                                              case["col_lon"]), ctx=ctx, **kw)
+    f.Analyse()
+    return f, ens.data
+
+
+@pytest.mark.parametrize("k", [2, 3, 7, 9, 15, 17, 19, 21, 31, 33, 39, 41, 47, 49, 50, 63, 65,
+                               76, 77, 100, 127])
+def test_letkf_every_k_matches_oracle(mda, ctx, orc, k):
+    """k runs in the next larger block (8, 16, 20, 32, 40, 48, 64, 128): the
+    transforms and the analysis (T kept, and applied by the eigenvector
+    kernel) equal the oracle's."""
+    case = latlon_case(nlon=18, nlat=9, nlev=2, k=k, p=700, seed=300 + k, nmodes=96)
+    prob = orc.Problem(k, 18, 9, 2, orc.COORD_GEOGRAPHIC, case["col_lat"], case["col_lon"],
+                       case["lat"], case["lon"], case["yo"], case["var"],
+                       float(np.float32(1.05)), 3000.0)
+    Xo, To, _ = orc.letkf_standard(prob, case["X"], case["H"].apply_host(case["X"]), want_T=True)
+    f, Xk = _latlon(mda, ctx, case, case["X"], 3000.0, keep_transforms=True)
+    cols = np.array([0, 40, 161])
+    assert rel_err(f.transforms(cols), To[cols]) < TOL
+    assert rel_err(Xk, Xo) < TOL
+    assert f.diag["max_jacobi_sweeps"] == 0
+    assert rel_err(_latlon(mda, ctx, case, case["X"], 3000.0)[1], Xo) < TOL
+
+
+@pytest.mark.parametrize("prec", ["FP32", "BF16X3"])
+@pytest.mark.parametrize("k,radius", [(10, 500.0), (25, 3000.0), (50, 1500.0), (50, 6000.0),
+                                      (100, 1500.0), (100, 9000.0)])
+def test_letkf_reduced_precision_blocks_match_jacobi(mda, ctx, k, radius, prec):
+    """The same reduced-precision Gram through the padded block and through
+    Jacobi, with columns of fewer and of more than k observations: equal to
+    the eigensolvers' FP64 rounding."""
+    case = latlon_case(nlon=18, nlat=9, nlev=2, k=k, p=700, seed=400 + k, nmodes=96)
+    L = mda._lib
+    kw = dict(precision=getattr(L, "PREC_" + prec))
+    fa, Xa = _latlon(mda, ctx, case, case["X"], radius, **kw)
+    fj, Xj = _latlon(mda, ctx, case, case["X"], radius, eig_method=L.EIG_JACOBI, **kw)
+    few = int(((fa.local_counts() > 0) & (fa.local_counts() < k)).sum())
+    if prec == "FP32":  # BF16x3 stays with Jacobi at these sizes
+        assert fa.diag["n_fallback_columns"] >= few
+    assert rel_err(Xa, Xj) < TOL
