@@ -443,24 +443,20 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
     dg.analysis_increment_norm = 0.0;
     double* part2 = c->get<double>("sumsq_part", 1024);
     if (diag) {
-      launch_dev_sumsq(s, de.X, k, n, scale, part2, 512);
-      dg.background_spread = std::sqrt(host_sum(c, part2, 512) / ((double)n * k));
       launch_sumsq(s, dd, p, part2, 512);
       dg.innovation_norm = std::sqrt(host_sum(c, part2, 512));
-      // max / min Kalman gain over the n x p entries of K (EnKF.hpp:202-203);
-      // O(n p k) work, as in the reference
-      {
-        double* G = c->get<double>("enkf_G", (size_t)p * k);
-        double* mm = c->get<double>("enkf_mm", 2 * 512);
-        launch_enkf_gain_minmax_ws(s, de.X, k, n, scale, Minv, yp, o.var, p, G, mm, 512);
-        std::vector<double> hm(2 * 512);
-        d2h(c, hm.data(), mm, sizeof(double) * 1024);
-        MDA_HIP(hipStreamSynchronize(s));
-        double mx = -std::numeric_limits<double>::infinity(), mn = -mx;
-        for (int b = 0; b < 512; ++b) { mx = std::max(mx, hm[2 * b]); mn = std::min(mn, hm[2 * b + 1]); }
-        dg.max_kalman_gain = mx;
-        dg.min_kalman_gain = mn;
-      }
+      // max / min Kalman gain over the n x p entries of K (EnKF.hpp:202-203;
+      // O(n p k) work, as in the reference) and the background spread
+      const enkf_gain_shape gs = enkf_gain_plan(k, n, p);
+      double* Gf = c->get<double>("enkf_G", gs.gf_doubles());
+      double* mm = c->get<double>("enkf_mm", gs.partial_doubles());
+      double* out3 = c->get<double>("enkf_mm_out", 3);
+      launch_enkf_gain_minmax(s, de.X, k, n, scale, Minv, yp, o.var, p, gs, Gf, mm, out3);
+      double h3[3] = {0.0, 0.0, 0.0};
+      d2h(c, h3, out3, sizeof(h3));
+      dg.max_kalman_gain = h3[0];
+      dg.min_kalman_gain = h3[1];
+      dg.background_spread = std::sqrt(h3[2] / ((double)n * k));
       // cond(S) = ratio of the extreme singular values of the SPD
       // S = Y'Y'^T/(k-1) + R (EnKF.hpp:205-209)
       dg.condition_number = enkf_condition_number(c, yp, o.var, k, p, EB);

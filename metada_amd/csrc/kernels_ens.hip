@@ -2,6 +2,8 @@
 // pieces: ensemble mean and perturbations, H x with observation-space
 // statistics, Y'^T R^-1 [Y' | d] reductions, the k x k solves, the global
 // transform and Metrics.
+#include <algorithm>
+
 #include "mda_device.hpp"
 #include "mda_internal.hpp"
 
@@ -480,67 +482,206 @@ void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double 
 }
 
 // ---------------------------------------------------------------------------
-// EnKF diagnostics: max / min of K = X' G with G = M^-1 Y'^T R^-1 (k x p),
-// EnKF.hpp:202-203.  G is formed first (obs-major [p][k]).
+// FP64 MFMA over state points (v_mfma_f64_16x16x4f64, one wavefront per
+// 16 MT points): lane (i16, kk) holds members 4s + kk of point i16 of each
+// tile, the layout of either operand (A[l%16][l/16], B[l/16][l%16]).  Member
+// loads are 128-byte segments.  An ensemble of k members takes NS = k / 4
+// steps, rounded up to a compiled size; the values past k are zero.
 // ---------------------------------------------------------------------------
-__global__ void k_enkf_G(const double* __restrict__ Minv, const double* __restrict__ yp_om,
-                         const double* __restrict__ var, int k, int64_t p,
-                         double* __restrict__ G) {
-  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < p * k;
-       e += (int64_t)gridDim.x * blockDim.x) {
-    int64_t o = e / k;
-    int a = (int)(e % k);
-    double s = 0.0;
-    for (int b = 0; b < k; ++b) s += Minv[a * k + b] * yp_om[(size_t)o * k + b];
-    G[e] = s / var[o];
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// v[t][s] = (x - mean) scale of the tile's points (0 past n and k); mean[t]
+// the mean over the members of point i0 + 16 t + i16
+template <int NS, int MT>
+__device__ __forceinline__ void load_pert(const double* __restrict__ X, int k, int64_t n,
+                                          double scale, int64_t i0, double (&v)[MT][NS],
+                                          double (&mean)[MT]) {
+  const int lane = threadIdx.x & 63, i16 = lane & 15, kk = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int64_t i = i0 + 16 * t + i16;
+    double sum = 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int m = 4 * s + kk;
+      v[t][s] = m < k && i < n ? X[(size_t)m * n + i] : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) sum += v[t][s];
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    mean[t] = sum * (1.0 / (double)k);
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      v[t][s] = 4 * s + kk < k && i < n ? (v[t][s] - mean[t]) * scale : 0.0;
   }
 }
 
-__global__ __launch_bounds__(256) void k_enkf_gain_minmax(
-    const double* __restrict__ X, int k, int64_t n, double scale,
-    const double* __restrict__ G, int64_t p, double* __restrict__ partial) {
-  __shared__ double rmax[256], rmin[256];
-  double mx = -1.0e308, mn = 1.0e308;
-  const double rk = 1.0 / (double)k;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double xp[128];
-    double s = 0.0;
-    for (int j = 0; j < k; ++j) { xp[j] = X[(size_t)j * n + i]; s += xp[j]; }
-    double m = s * rk;
-    for (int j = 0; j < k; ++j) xp[j] = (xp[j] - m) * scale;
-    for (int64_t o = 0; o < p; ++o) {
-      double v = 0.0;
-      for (int a = 0; a < k; ++a) v += xp[a] * G[(size_t)o * k + a];
-      mx = v > mx ? v : mx;
-      mn = v < mn ? v : mn;
+// the compiled step counts: k <= 16, 32, ..., 128
+#define MDA_MEMBER_STEPS(k, CALL)        \
+  switch (((k) + 15) / 16) {             \
+    case 1: { CALL(4); } break;          \
+    case 2: { CALL(8); } break;          \
+    case 3: { CALL(12); } break;         \
+    case 4: { CALL(16); } break;         \
+    case 5: { CALL(20); } break;         \
+    case 6: { CALL(24); } break;         \
+    case 7: { CALL(28); } break;         \
+    default: { CALL(32); } break;        \
+  }
+
+// ---------------------------------------------------------------------------
+// EnKF diagnostics: max / min of K = X' G with G = M^-1 Y'^T R^-1 (k x p),
+// EnKF.hpp:202-203, and the background's sum of squares (:334).  G is formed
+// first in fragment order, Gf[tile of 16 observations][step][lane] =
+// G[4 step + kk][16 tile + i16], 512 contiguous bytes per MFMA step.  Then K
+// is formed tile by tile on the matrix cores and folded into the extremes at
+// once; it never reaches memory.  Bound by the FP64 matrix rate (2 n p k
+// FLOP): one 16x16x4 product takes 64 cycles of its SIMD, so a fragment load
+// per two products (two tiles of points per wavefront) leaves the caches
+// idle.  The observation tiles are split over gridDim.y when the points alone
+// leave SIMDs empty.  n = 262,144, p = 1,500, k = 80: 73.7 ms with one thread
+// per point (its perturbations in scratch memory), 1.11 ms here (57 TFLOP/s; a
+// large FP64 matrix product reaches 72 on this card).
+// ---------------------------------------------------------------------------
+__global__ void k_enkf_G(const double* __restrict__ Minv, const double* __restrict__ yp_om,
+                         const double* __restrict__ var, int k, int64_t p, int ns,
+                         int64_t ntile, double* __restrict__ Gf) {
+  const int64_t total = ntile * ns * 64;
+  for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total;
+       e += (int64_t)gridDim.x * blockDim.x) {
+    const int lane = (int)(e & 63);
+    const int64_t ts = e >> 6;
+    const int64_t o = ts / ns * 16 + (lane & 15);
+    const int a = 4 * (int)(ts % ns) + (lane >> 4);
+    double g = 0.0;
+    if (o < p && a < k) {
+      const double* mr = Minv + (size_t)a * k;
+      const double* yr = yp_om + (size_t)o * k;
+      double s0 = 0.0, s1 = 0.0;
+      int b = 0;
+#pragma unroll 4
+      for (; b + 1 < k; b += 2) {
+        s0 = fma(mr[b], yr[b], s0);
+        s1 = fma(mr[b + 1], yr[b + 1], s1);
+      }
+      if (b < k) s0 = fma(mr[b], yr[b], s0);
+      g = (s0 + s1) / var[o];
+    }
+    Gf[e] = g;
+  }
+}
+
+template <int NS>
+__global__ __launch_bounds__(256) void k_enkf_gain_minmax(const double* __restrict__ X, int k,
+                                                          int64_t n, double scale,
+                                                          const double* __restrict__ Gf,
+                                                          int64_t p, int64_t ntile, int64_t per,
+                                                          double* __restrict__ partial) {
+  __shared__ double red[3][4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i16 = lane & 15, kk = lane >> 4;
+  const int64_t i0 = ((int64_t)blockIdx.x * 4 + wv) * 32;
+  double a[2][NS], mean[2];
+  load_pert<NS, 2>(X, k, n, scale, i0, a, mean);
+  double mx = -1.0e308, mn = 1.0e308, ss = 0.0;
+  if (blockIdx.y == 0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) ss = fma(a[t][s], a[t][s], ss);
+  }
+  const int64_t t0 = blockIdx.y * per, t1 = t0 + per < ntile ? t0 + per : ntile;
+  if (i0 < n) {
+    for (int64_t ot = t0; ot < t1; ++ot) {
+      const double* gf = Gf + (size_t)ot * NS * 64 + lane;
+      d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        const double b = gf[64 * s];
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[0][s], b, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[1][s], b, acc[1], 0, 0, 0);
+      }
+      // D[kk + 4r][i16]: point kk + 4r of the tile, observation i16
+      const bool ov = 16 * ot + i16 < p;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const double v = acc[t][r];
+          const bool in = ov && i0 + 16 * t + kk + 4 * r < n;
+          mx = in && v > mx ? v : mx;
+          mn = in && v < mn ? v : mn;
+        }
     }
   }
-  rmax[threadIdx.x] = mx;
-  rmin[threadIdx.x] = mn;
+  for (int off = 32; off > 0; off >>= 1) {
+    mx = fmax(mx, __shfl_xor(mx, off));
+    mn = fmin(mn, __shfl_xor(mn, off));
+    ss += __shfl_xor(ss, off);
+  }
+  if (lane == 0) { red[0][wv] = mx; red[1][wv] = mn; red[2][wv] = ss; }
   __syncthreads();
-  for (int s2 = 128; s2 > 0; s2 >>= 1) {
-    if (threadIdx.x < s2) {
-      rmax[threadIdx.x] = fmax(rmax[threadIdx.x], rmax[threadIdx.x + s2]);
-      rmin[threadIdx.x] = fmin(rmin[threadIdx.x], rmin[threadIdx.x + s2]);
+  if (threadIdx.x == 0) {
+    double* out = partial + 3 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x);
+    out[0] = fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3]));
+    out[1] = fmin(fmin(red[1][0], red[1][1]), fmin(red[1][2], red[1][3]));
+    out[2] = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);
+  }
+}
+
+// [max, min, sum] of nb partial triples, one block, in a fixed order
+__global__ __launch_bounds__(256) void k_fold_minmaxsum(const double* __restrict__ partial,
+                                                        int64_t nb, double* __restrict__ out) {
+  __shared__ double r0[256], r1[256], r2[256];
+  const int tid = threadIdx.x;
+  double mx = -1.0e308, mn = 1.0e308, ss = 0.0;
+  for (int64_t b = tid; b < nb; b += 256) {
+    mx = fmax(mx, partial[3 * b]);
+    mn = fmin(mn, partial[3 * b + 1]);
+    ss += partial[3 * b + 2];
+  }
+  r0[tid] = mx; r1[tid] = mn; r2[tid] = ss;
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if (tid < st) {
+      r0[tid] = fmax(r0[tid], r0[tid + st]);
+      r1[tid] = fmin(r1[tid], r1[tid + st]);
+      r2[tid] += r2[tid + st];
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    partial[2 * blockIdx.x] = rmax[0];
-    partial[2 * blockIdx.x + 1] = rmin[0];
-  }
+  if (tid == 0) { out[0] = r0[0]; out[1] = r1[0]; out[2] = r2[0]; }
 }
 
-void launch_enkf_gain_minmax_ws(hipStream_t s, const double* X, int k, int64_t n, double scale,
-                                const double* Minv, const double* yp_om, const double* var,
-                                int64_t p, double* G, double* partial, int nblocks) {
+// Launch shape: one block per 128 points; with fewer than 1024 blocks (one
+// wavefront per SIMD of the chip) the observation tiles are split further.
+enkf_gain_shape enkf_gain_plan(int k, int64_t n, int64_t p) {
+  enkf_gain_shape g;
+  g.ns = (k + 15) / 16 * 4;
+  g.ntile = (p + 15) / 16;
+  g.nbx = (n + 127) / 128;
+  const int64_t want = std::max<int64_t>(1, 1024 / g.nbx);
+  g.per = (g.ntile + want - 1) / want;
+  g.nby = (g.ntile + g.per - 1) / g.per;
+  return g;
+}
+
+void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, double scale,
+                             const double* Minv, const double* yp_om, const double* var,
+                             int64_t p, const enkf_gain_shape& g, double* Gf, double* partial,
+                             double* out3) {
   MDA_REQUIRE(k <= 128, "gain diagnostics support k <= 128");
-  hipLaunchKernelGGL(k_enkf_G, dim3(grid_for(p * k, 256, 4096)), dim3(256), 0, s, Minv, yp_om,
-                     var, k, p, G);
+  MDA_REQUIRE(g.nbx < (int64_t)1 << 31 && g.nby < 65536, "gain grid too large");
+  hipLaunchKernelGGL(k_enkf_G, dim3(grid_for(g.ntile * g.ns * 64, 256, 4096)), dim3(256), 0, s,
+                     Minv, yp_om, var, k, p, g.ns, g.ntile, Gf);
   MDA_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_enkf_gain_minmax, dim3(nblocks), dim3(256), 0, s, X, k, n, scale, G, p,
-                     partial);
+#define MDA_GAIN(NS)                                                                              \
+  hipLaunchKernelGGL(k_enkf_gain_minmax<NS>, dim3((unsigned)g.nbx, (unsigned)g.nby), dim3(256),  \
+                     0, s, X, k, n, scale, Gf, p, g.ntile, g.per, partial)
+  MDA_MEMBER_STEPS(k, MDA_GAIN)
+#undef MDA_GAIN
+  MDA_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_fold_minmaxsum, dim3(1), dim3(256), 0, s, partial, g.nbx * g.nby, out3);
   MDA_LAUNCH_CHECK();
 }
 

@@ -200,9 +200,19 @@ void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* 
 void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double scale,
                              const double* T, int* status);
 // EnKF diagnostics
-void launch_enkf_gain_minmax_ws(hipStream_t s, const double* X, int k, int64_t n, double scale,
-                                const double* Minv, const double* yp_om, const double* var,
-                                int64_t p, double* G, double* partial, int nblocks);
+struct enkf_gain_shape {
+  int ns;              // MFMA steps over the members
+  int64_t ntile, per;  // tiles of 16 observations, tiles per block
+  int64_t nbx, nby;    // blocks over state points and over observation tiles
+  int64_t gf_doubles() const { return ntile * ns * 64; }
+  int64_t partial_doubles() const { return 3 * nbx * nby; }
+};
+enkf_gain_shape enkf_gain_plan(int k, int64_t n, int64_t p);
+// out3 = [max K, min K, sum over state and members of ((x - mean) scale)^2]
+void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, double scale,
+                             const double* Minv, const double* yp_om, const double* var,
+                             int64_t p, const enkf_gain_shape& g, double* Gf, double* partial,
+                             double* out3);
 void launch_cond_small(hipStream_t s, const double* yp_om, const double* var, int k, int p,
                        double* S, double* out);
 void launch_sym_maxeig(hipStream_t s, const double* EB, int k, double* S, double* out);

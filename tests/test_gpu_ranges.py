@@ -104,3 +104,28 @@ def test_letkf_reduced_precision_blocks_match_jacobi(mda, ctx, k, radius, prec):
     if prec == "FP32":  # BF16x3 stays with Jacobi at these sizes
         assert fa.diag["n_fallback_columns"] >= few
     assert rel_err(Xa, Xj) < TOL
+
+
+# ---- EnKF gain and spread diagnostics: tiles of 16 observations, 32 points, 16 members ------
+@pytest.mark.parametrize("k,n,p", [(2, 1, 1), (16, 31, 15), (17, 33, 16), (33, 128, 17),
+                                   (50, 129, 33), (64, 1000, 40), (80, 257, 100),
+                                   (100, 64, 31), (112, 300, 48), (113, 65, 20),
+                                   (128, 4100, 60)])
+def test_enkf_diagnostics_match_oracle(mda, ctx, orc, k, n, p):
+    rng = np.random.default_rng(1000 * k + p)
+    X = 3.0 + rng.standard_normal((k, n))
+    Yb, yo = rng.standard_normal((k, p)), rng.standard_normal(p)
+    var, Z = rng.uniform(0.5, 2.0, p), rng.standard_normal((p, k))
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    f = mda.EnKF(ens, mda.Observation(yo, var, np.zeros(p), np.zeros(p)),
+                 mda.ObsOperator(hx=Yb), mda.Config({"analysis": {"inflation": 1.1}}), ctx=ctx)
+    f.Analyse(Z=Z)
+    Xo, d = orc.enkf_analyse(X, Yb, yo, var, Z, f.inflation_factor)
+    assert rel_err(ens.data, Xo) < TOL
+    r = f.getAnalysisResults()
+    for key in ("max_kalman_gain", "min_kalman_gain", "background_spread", "analysis_spread",
+                "innovation_norm", "condition_number"):
+        # the gain's rounding scales with its largest entry
+        scale = max(abs(d["max_kalman_gain"]), abs(d["min_kalman_gain"])) \
+            if "gain" in key else abs(d[key])
+        assert abs(r[key] - d[key]) <= 1e-10 * scale, (key, r[key], d[key])
