@@ -306,39 +306,31 @@ int mda_obs_innovations(mda_ctx* c, const mda_ensemble* ens, const mda_obs* obs,
 // ---------------------------------------------------------------------------
 // cond(S) of the EnKF, S = Y'Y'^T/(k-1) + diag(var) (EnKF.hpp:205-209,
 // JacobiSVD singular values; S is SPD, so they are its eigenvalues):
-//   p <= 128                  Jacobi on the dense S (one workgroup);
+//   p <= 128                  tridiagonalisation of the dense S in LDS;
 //   constant var, p > k - 1   S = s^2 (I + Y'Y'^T/(s^2 (k-1))): the smallest
 //                             eigenvalue is s^2 (rank deficiency) and the
 //                             largest s^2 (1 + mu/(k-1)), mu the largest
 //                             eigenvalue of E = Y'^T R^-1 Y' (from [E | b]);
-//   otherwise                 Householder tridiagonalisation of the dense S
-//                             and bisection for its extreme eigenvalues
-//                             (p <= MDA_DENSE_MAX).
+//   otherwise                 both extremes by multisection on k x k
+//                             factorisations (p <= MDA_DENSE_MAX, NaN beyond).
 static double enkf_condition_number(mda_ctx* c, const double* yp, const double* var, int k,
-                                    int64_t p, const double* EB) {
+                                    int64_t p, double* EB) {
   hipStream_t s = c->stream;
-  double* cnd = c->get<double>("enkf_cond", 1);
   std::vector<double> hv(p);
   d2h(c, hv.data(), var, sizeof(double) * p);
   // an invalid observation (var = +inf) is an infinite singular value of S
   if (std::any_of(hv.begin(), hv.end(), [](double v) { return std::isinf(v); }))
     return std::numeric_limits<double>::infinity();
   if (p <= 128) {
-    double* S = c->get<double>("enkf_S", (size_t)130 * 130);
-    launch_cond_small(s, yp, var, k, (int)p, S, cnd);
-    double v = 0.0;
-    d2h(c, &v, cnd, sizeof(double));
-    return v;
+    double* S = c->get<double>("enkf_S", (size_t)128 * 128);
+    launch_form_enkf_S(s, yp, var, k, p, S);
+    const dense_extremes x = dense_sym_extremes(c, S, p);
+    return x.absmax / x.absmin;
   }
   const bool constant = std::all_of(hv.begin(), hv.end(), [&](double v) { return v == hv[0]; });
-  if (constant) {
-    double* S = c->get<double>("enkf_S", (size_t)130 * 130);
-    launch_sym_maxeig(s, EB, k, S, cnd);
-    double mu = 0.0;
-    d2h(c, &mu, cnd, sizeof(double));
-    return 1.0 + mu / (double)(k - 1);
-  }
-  return dense_spd_condition(c, yp, var, k, p);
+  if (constant) return 1.0 + dense_sym_extremes(c, EB, k, k + 1).lmax / (double)(k - 1);
+  if (p > MDA_DENSE_MAX) return std::numeric_limits<double>::quiet_NaN();
+  return lowrank_spd_condition(c, yp, var, hv, k, p);
 }
 
 }  // extern "C"

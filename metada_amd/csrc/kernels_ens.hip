@@ -686,75 +686,6 @@ void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, d
 }
 
 // ---------------------------------------------------------------------------
-// cond(S), S = Y'Y'^T/(k-1) + diag(var), p <= 128 (EnKF.hpp:205-209): S is
-// SPD, so its singular values are its eigenvalues (parallel Jacobi, no V).
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_cond_small(const double* __restrict__ yp_om,
-                                                    const double* __restrict__ var, int k,
-                                                    int p, double* __restrict__ S,
-                                                    double* __restrict__ out) {
-  __shared__ double rc[64], rs[64], red[256];
-  __shared__ int rp[64], rq[64];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int n = (p + 1) & ~1;  // even size; the pad row/column is decoupled
-  for (int idx = tid; idx < n * n; idx += nt) {
-    int a = idx / n, b = idx % n;
-    double v = 0.0;
-    if (a < p && b < p) {
-      for (int j = 0; j < k; ++j) v += yp_om[a * k + j] * yp_om[b * k + j];
-      v = v / (double)(k - 1) + (a == b ? var[a] : 0.0);
-    } else if (a == b) {
-      v = 1.0;
-    }
-    S[idx] = v;
-  }
-  __syncthreads();
-  block_jacobi(S, n, nullptr, 0, n, rc, rs, rp, rq, red, 60, 1e-16);
-  if (tid == 0) {
-    double mx = 0.0, mn = 1.0e308;
-    for (int a = 0; a < p; ++a) {
-      double v = fabs(S[a * n + a]);
-      mx = v > mx ? v : mx;
-      mn = v < mn ? v : mn;
-    }
-    out[0] = mx / mn;
-  }
-}
-
-void launch_cond_small(hipStream_t s, const double* yp_om, const double* var, int k, int p,
-                       double* S, double* out) {
-  MDA_REQUIRE(p <= 128, "direct cond(S) supports p <= 128");
-  hipLaunchKernelGGL(k_cond_small, dim3(1), dim3(256), 0, s, yp_om, var, k, p, S, out);
-  MDA_LAUNCH_CHECK();
-}
-
-// largest eigenvalue of a k x k symmetric matrix (cond(S) for R = sigma^2 I)
-__global__ __launch_bounds__(256) void k_sym_maxeig(const double* __restrict__ EB, int k,
-                                                    double* __restrict__ S,
-                                                    double* __restrict__ out) {
-  __shared__ double rc[128], rs[128], red[256];
-  __shared__ int rp[128], rq[128];
-  const int n = (k + 1) & ~1;
-  for (int idx = threadIdx.x; idx < n * n; idx += blockDim.x) {
-    int a = idx / n, b = idx % n;
-    S[idx] = (a < k && b < k) ? EB[a * (k + 1) + b] : (a == b ? 0.0 : 0.0);
-  }
-  __syncthreads();
-  block_jacobi(S, n, nullptr, 0, n, rc, rs, rp, rq, red, 60, 1e-16);
-  if (threadIdx.x == 0) {
-    double mx = 0.0;
-    for (int a = 0; a < k; ++a) mx = fmax(mx, S[a * n + a]);
-    out[0] = mx;
-  }
-}
-
-void launch_sym_maxeig(hipStream_t s, const double* EB, int k, double* S, double* out) {
-  MDA_REQUIRE(k <= 255, "k too large");
-  hipLaunchKernelGGL(k_sym_maxeig, dim3(1), dim3(256), 0, s, EB, k, S, out);
-  MDA_LAUNCH_CHECK();
-}
-
-// ---------------------------------------------------------------------------
 // Metrics::CalculateAll (Metrics.hpp:74-94): per-block partial sums of
 // [rmse^2, bias, sum mean, sum truth, sum mean*truth, sum mean^2,
 //  sum truth^2, spread, crps], reduced on the host in block order.

@@ -213,9 +213,6 @@ void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, d
                              const double* Minv, const double* yp_om, const double* var,
                              int64_t p, const enkf_gain_shape& g, double* Gf, double* partial,
                              double* out3);
-void launch_cond_small(hipStream_t s, const double* yp_om, const double* var, int k, int p,
-                       double* S, double* out);
-void launch_sym_maxeig(hipStream_t s, const double* EB, int k, double* S, double* out);
 void launch_metrics(hipStream_t s, const double* X, int k, int64_t n, const double* truth,
                     double* partial, int nblocks);
 
@@ -421,11 +418,13 @@ void launch_form_enkf_S(hipStream_t s, const double* yp, const double* var, int 
                         double* S);
 void dense_tridiagonalise(hipStream_t s, int64_t p, double* A, double* d, double* e, double* u,
                           double* pv, double* w, double* sc);
-dense_extremes tridiag_extremes(const std::vector<double>& d, const std::vector<double>& e);
-// extreme eigenvalues of the symmetric device matrix A (destroyed)
-dense_extremes dense_sym_extremes(mda_ctx* c, double* A, int64_t p);
-// cond(S) of S = Y'Y'^T/(k-1) + diag(var); NaN beyond MDA_DENSE_MAX
-double dense_spd_condition(mda_ctx* c, const double* yp, const double* var, int k, int64_t p);
+// extreme eigenvalues of the symmetric device matrix A (destroyed beyond 128
+// rows); lda: row stride, 0 = p (rows beyond 128 are contiguous)
+dense_extremes dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda = 0);
+// cond(S) of S = Y'Y'^T/(k-1) + diag(var) through k x k factorisations
+// (hvar: the finite variances on the host)
+double lowrank_spd_condition(mda_ctx* c, const double* yp, const double* var,
+                             const std::vector<double>& hvar, int k, int64_t p);
 // B <- A^-1 B by Gauss-Jordan with partial pivoting (A destroyed); a zero
 // pivot sets MDA_ST_NOT_SPD in *status
 void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* B,

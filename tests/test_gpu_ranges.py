@@ -129,3 +129,30 @@ def test_enkf_diagnostics_match_oracle(mda, ctx, orc, k, n, p):
         scale = max(abs(d["max_kalman_gain"]), abs(d["min_kalman_gain"])) \
             if "gain" in key else abs(d[key])
         assert abs(r[key] - d[key]) <= 1e-10 * scale, (key, r[key], d[key])
+
+
+# ---- cond(S) of the EnKF: dense in LDS (p <= 128), from E (one variance), by inertia --------
+@pytest.mark.parametrize("k,p,var", [
+    (2, 2, "mixed"), (5, 3, "mixed"), (40, 63, "mixed"), (20, 127, "constant"),
+    (64, 128, "mixed"), (2, 129, "mixed"), (17, 129, "constant"), (17, 130, "mixed"),
+    (64, 300, "mixed"), (64, 700, "constant"), (113, 500, "mixed"), (128, 257, "mixed"),
+    (128, 1000, "few"), (30, 400, "few"), (30, 200, "pair"), (40, 131, "spread")])
+def test_enkf_condition_number(mda, ctx, k, p, var):
+    """cond(S) against a dense eigenvalue solve: all variances distinct, one,
+    three (multiplicities above k), one pair of smallest ones, or spread over
+    four decades."""
+    rng = np.random.default_rng(7 * k + p)
+    Yb = rng.standard_normal((k, p)) @ (np.eye(p) + 0.3 * np.eye(p, k=1))
+    R = {"mixed": rng.uniform(0.1, 1.5, p), "constant": np.full(p, 0.25),
+         "few": rng.choice([0.1, 0.4, 2.0], p), "spread": 10.0 ** rng.uniform(-3, 1, p),
+         "pair": np.r_[0.05, 0.05, rng.uniform(0.2, 1.0, p - 2)]}[var]
+    ens = mda.Ensemble(rng.standard_normal((k, 24)), 24, 1, 1)
+    f = mda.EnKF(ens, mda.Observation(rng.standard_normal(p), R, np.zeros(p), np.zeros(p)),
+                 mda.ObsOperator(hx=Yb), mda.Config({"analysis": {"inflation": 1.0}}), ctx=ctx)
+    f.Analyse()
+    Y = Yb - Yb.mean(0)
+    lam = np.linalg.eigvalsh(Y.T @ Y / (k - 1) + np.diag(R))
+    want = lam[-1] / lam[0]
+    # both sides carry the rounding of the smallest eigenvalue: cond * eps
+    assert abs(f.getAnalysisResults()["condition_number"] - want) <= \
+        want * max(1e-11, 64 * want * 2.2e-16)
