@@ -453,10 +453,15 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
       // S = Y'Y'^T/(k-1) + R (EnKF.hpp:205-209)
       dg.condition_number = enkf_condition_number(c, yp, o.var, k, p, EB);
     }
-    launch_transform_global(s, de.X, k, n, scale, T, st);
     if (diag) {
-      launch_dev_sumsq(s, de.X, k, n, 1.0, part2, 512);
-      dg.analysis_spread = std::sqrt(host_sum(c, part2, 512) / ((double)n * k));
+      double* pa = c->get<double>("enkf_xa_part", (size_t)3 * transform_global_blocks(n));
+      double* out3 = c->get<double>("enkf_mm_out", 3);
+      launch_transform_global(s, de.X, k, n, scale, T, st, pa, out3);
+      double h3[3] = {0.0, 0.0, 0.0};
+      d2h(c, h3, out3, sizeof(h3));
+      dg.analysis_spread = std::sqrt(h3[2] / ((double)n * k));
+    } else {
+      launch_transform_global(s, de.X, k, n, scale, T, st);
     }
     int hs = 0;
     d2h(c, &hs, st, sizeof(int));

@@ -427,61 +427,6 @@ void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* 
 }
 
 // ---------------------------------------------------------------------------
-// Global transform: X_a[j][i] = xbar_i + sum_m (scale (x_m,i - xbar_i)) T[m][j]
-// (ETKF.hpp:163-169, EnKF.hpp:216-227).  T in LDS; one thread per state index.
-// Nothing is written when an earlier stage of the analysis failed (status bits
-// MDA_ST_SKIP_UPDATE); a non-finite background value sets
-// MDA_ST_NONFINITE_STATE (the analysis at that index is then non-finite, as
-// the reference's arithmetic makes it).
-// ---------------------------------------------------------------------------
-template <int KMAX>
-__global__ __launch_bounds__(256) void k_transform_global(double* __restrict__ X, int k,
-                                                          int64_t n, double scale,
-                                                          const double* __restrict__ T,
-                                                          int* __restrict__ status) {
-  if (status && (*status & MDA_ST_SKIP_UPDATE)) return;
-  extern __shared__ double Ts[];
-  for (int idx = threadIdx.x; idx < k * k; idx += blockDim.x) Ts[idx] = T[idx];
-  __syncthreads();
-  const double rk = 1.0 / (double)k;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double xp[KMAX];
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < KMAX; ++j)
-      if (j < k) { xp[j] = X[(size_t)j * n + i]; s += xp[j]; }
-    double m = s * rk;
-    if (status && !isfinite(m)) atomicOr(status, MDA_ST_NONFINITE_STATE);
-#pragma unroll
-    for (int j = 0; j < KMAX; ++j)
-      if (j < k) xp[j] = (xp[j] - m) * scale;
-    for (int j = 0; j < k; ++j) {
-      double acc = 0.0;
-#pragma unroll
-      for (int a = 0; a < KMAX; ++a)
-        if (a < k) acc += xp[a] * Ts[a * k + j];
-      X[(size_t)j * n + i] = m + acc;
-    }
-  }
-}
-
-void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double scale,
-                             const double* T, int* status) {
-  size_t shm = sizeof(double) * k * k;
-  unsigned g = grid_for(n, 256, 16384);
-  if (k <= 32)
-    hipLaunchKernelGGL(k_transform_global<32>, dim3(g), dim3(256), shm, s, X, k, n, scale, T, status);
-  else if (k <= 64)
-    hipLaunchKernelGGL(k_transform_global<64>, dim3(g), dim3(256), shm, s, X, k, n, scale, T, status);
-  else if (k <= 128)
-    hipLaunchKernelGGL(k_transform_global<128>, dim3(g), dim3(256), shm, s, X, k, n, scale, T, status);
-  else
-    throw mda_error(MDA_E_UNSUPPORTED, "global transform supports k <= 128");
-  MDA_LAUNCH_CHECK();
-}
-
-// ---------------------------------------------------------------------------
 // FP64 MFMA over state points (v_mfma_f64_16x16x4f64, one wavefront per
 // 16 MT points): lane (i16, kk) holds members 4s + kk of point i16 of each
 // tile, the layout of either operand (A[l%16][l/16], B[l/16][l%16]).  Member
@@ -529,6 +474,144 @@ __device__ __forceinline__ void load_pert(const double* __restrict__ X, int k, i
     case 7: { CALL(28); } break;         \
     default: { CALL(32); } break;        \
   }
+
+// [max, min, sum] of nb partial triples, one block, in a fixed order
+__global__ __launch_bounds__(256) void k_fold_minmaxsum(const double* __restrict__ partial,
+                                                        int64_t nb, double* __restrict__ out) {
+  __shared__ double r0[256], r1[256], r2[256];
+  const int tid = threadIdx.x;
+  double mx = -1.0e308, mn = 1.0e308, ss = 0.0;
+  for (int64_t b = tid; b < nb; b += 256) {
+    mx = fmax(mx, partial[3 * b]);
+    mn = fmin(mn, partial[3 * b + 1]);
+    ss += partial[3 * b + 2];
+  }
+  r0[tid] = mx; r1[tid] = mn; r2[tid] = ss;
+  __syncthreads();
+  for (int st = 128; st > 0; st >>= 1) {
+    if (tid < st) {
+      r0[tid] = fmax(r0[tid], r0[tid + st]);
+      r1[tid] = fmin(r1[tid], r1[tid + st]);
+      r2[tid] += r2[tid + st];
+    }
+    __syncthreads();
+  }
+  if (tid == 0) { out[0] = r0[0]; out[1] = r1[0]; out[2] = r2[0]; }
+}
+
+// ---------------------------------------------------------------------------
+// Global transform: X_a[j][i] = xbar_i + sum_m (scale (x_m,i - xbar_i)) T[m][j]
+// (ETKF.hpp:163-169, EnKF.hpp:216-227) on FP64 MFMA, in place.  T sits in LDS
+// in fragment order (one 512-byte read per two products: A = T^T, rows =
+// analysis members), a wavefront takes 32 points with all their members in
+// registers (B, columns = points), so X is read and written once in 128-byte
+// segments.  Bound by HBM: n = 2,097,152, k = 64 moves 2.15 GB in 0.55 ms
+// (3.9 TB/s; one LDS broadcast per FMA took 2.50 ms).
+// Nothing is written when an earlier stage of the analysis failed (status bits
+// MDA_ST_SKIP_UPDATE); a non-finite background value sets
+// MDA_ST_NONFINITE_STATE (the analysis at that index is then non-finite, as
+// the reference's arithmetic makes it).  With `partial`, each block leaves
+// [-1e308, 1e308, sum of (x_a - mean_a)^2] for the analysis spread
+// (EnKF.hpp:246-253): sums of the deviations from member 0's increment, which
+// are of the spread's own size.
+// ---------------------------------------------------------------------------
+constexpr int TG_THREADS = 512, TG_POINTS = TG_THREADS / 64 * 32;
+
+template <int NS>
+__global__ __launch_bounds__(TG_THREADS) void k_transform_global(
+    double* __restrict__ X, int k, int64_t n, double scale, const double* __restrict__ T,
+    int* __restrict__ status, double* __restrict__ partial) {
+  constexpr int NT = NS / 4;
+  extern __shared__ double Tf[];  // [NS][NT][64]
+  __shared__ double red[TG_THREADS / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, i16 = lane & 15, kk = lane >> 4;
+  double ss = 0.0;
+  if (!(status && (*status & MDA_ST_SKIP_UPDATE))) {
+    for (int e = tid; e < NS * NT * 64; e += TG_THREADS) {
+      const int l = e & 63, tj = (e >> 6) % NT, st = (e >> 6) / NT;
+      const int m = 4 * st + (l >> 4), j = 16 * tj + (l & 15);
+      Tf[e] = m < k && j < k ? T[m * k + j] : 0.0;
+    }
+    __syncthreads();
+    for (int64_t b0 = (int64_t)blockIdx.x * TG_POINTS; b0 < n;
+         b0 += (int64_t)gridDim.x * TG_POINTS) {
+      const int64_t i0 = b0 + 32 * wv;
+      if (i0 >= n) continue;
+      double v[2][NS], mean[2], sh[2] = {0.0, 0.0}, s1[2] = {0.0, 0.0}, s2[2] = {0.0, 0.0};
+      load_pert<NS, 2>(X, k, n, scale, i0, v, mean);
+      if (status && (!isfinite(mean[0]) || !isfinite(mean[1])))
+        atomicOr(status, MDA_ST_NONFINITE_STATE);
+#pragma unroll 1
+      for (int tj = 0; tj < NT; ++tj) {
+        d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+        const double* tf = Tf + tj * 64 + lane;
+#pragma unroll
+        for (int st = 0; st < NS; ++st) {
+          const double a = tf[st * NT * 64];
+          acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v[0][st], acc[0], 0, 0, 0);
+          acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v[1][st], acc[1], 0, 0, 0);
+        }
+        // D[kk + 4r][i16]: member 16 tj + kk + 4r, point i16
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int64_t i = i0 + 16 * t + i16;
+          if (tj == 0) sh[t] = __shfl(acc[t][0], i16);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int j = 16 * tj + kk + 4 * r;
+            if (j < k && i < n) {
+              X[(size_t)j * n + i] = mean[t] + acc[t][r];
+              const double dv = acc[t][r] - sh[t];
+              s1[t] += dv;
+              s2[t] = fma(dv, dv, s2[t]);
+            }
+          }
+        }
+      }
+      if (partial) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          for (int off = 16; off < 64; off <<= 1) {
+            s1[t] += __shfl_xor(s1[t], off);
+            s2[t] += __shfl_xor(s2[t], off);
+          }
+          if (kk == 0) ss += s2[t] - s1[t] * s1[t] / (double)k;
+        }
+      }
+    }
+  }
+  if (!partial) return;
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+  if (lane == 0) red[wv] = ss;
+  __syncthreads();
+  if (tid == 0) {
+    double t = 0.0;
+    for (int w = 0; w < TG_THREADS / 64; ++w) t += red[w];
+    partial[3 * (size_t)blockIdx.x] = -1.0e308;
+    partial[3 * (size_t)blockIdx.x + 1] = 1.0e308;
+    partial[3 * (size_t)blockIdx.x + 2] = t;
+  }
+}
+
+unsigned transform_global_blocks(int64_t n) {
+  return grid_for(n, TG_POINTS, 4096);
+}
+
+void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double scale,
+                             const double* T, int* status, double* partial, double* out3) {
+  MDA_REQUIRE(k <= 128, "global transform supports k <= 128");
+  const unsigned g = transform_global_blocks(n);
+#define MDA_TG(NS)                                                                           \
+  hipLaunchKernelGGL(k_transform_global<NS>, dim3(g), dim3(TG_THREADS),                      \
+                     sizeof(double) * NS * (NS / 4) * 64, s, X, k, n, scale, T, status, partial)
+  MDA_MEMBER_STEPS(k, MDA_TG)
+#undef MDA_TG
+  MDA_LAUNCH_CHECK();
+  if (partial) {
+    hipLaunchKernelGGL(k_fold_minmaxsum, dim3(1), dim3(256), 0, s, partial, (int64_t)g, out3);
+    MDA_LAUNCH_CHECK();
+  }
+}
 
 // ---------------------------------------------------------------------------
 // EnKF diagnostics: max / min of K = X' G with G = M^-1 Y'^T R^-1 (k x p),
@@ -627,30 +710,6 @@ __global__ __launch_bounds__(256) void k_enkf_gain_minmax(const double* __restri
     out[1] = fmin(fmin(red[1][0], red[1][1]), fmin(red[1][2], red[1][3]));
     out[2] = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);
   }
-}
-
-// [max, min, sum] of nb partial triples, one block, in a fixed order
-__global__ __launch_bounds__(256) void k_fold_minmaxsum(const double* __restrict__ partial,
-                                                        int64_t nb, double* __restrict__ out) {
-  __shared__ double r0[256], r1[256], r2[256];
-  const int tid = threadIdx.x;
-  double mx = -1.0e308, mn = 1.0e308, ss = 0.0;
-  for (int64_t b = tid; b < nb; b += 256) {
-    mx = fmax(mx, partial[3 * b]);
-    mn = fmin(mn, partial[3 * b + 1]);
-    ss += partial[3 * b + 2];
-  }
-  r0[tid] = mx; r1[tid] = mn; r2[tid] = ss;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) {
-      r0[tid] = fmax(r0[tid], r0[tid + st]);
-      r1[tid] = fmin(r1[tid], r1[tid + st]);
-      r2[tid] += r2[tid + st];
-    }
-    __syncthreads();
-  }
-  if (tid == 0) { out[0] = r0[0]; out[1] = r1[0]; out[2] = r2[0]; }
 }
 
 // Launch shape: one block per 128 points; with fewer than 1024 blocks (one

@@ -196,9 +196,13 @@ void launch_etkf_solve_ws(hipStream_t s, int k, const double* EB, double* T, dou
 void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* F, double* T,
                           double* Minv, double* scratch, int* status);
 // X_a = xbar + scale * X' T for all state points (global T); skipped when
-// the status word holds a MDA_ST_SKIP_UPDATE bit
+// the status word holds a MDA_ST_SKIP_UPDATE bit.  With partial (3 doubles per
+// block, transform_global_blocks(n) of them), out3[2] = sum over state and
+// members of (x_a - mean_a)^2
+unsigned transform_global_blocks(int64_t n);
 void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double scale,
-                             const double* T, int* status);
+                             const double* T, int* status, double* partial = nullptr,
+                             double* out3 = nullptr);
 // EnKF diagnostics
 struct enkf_gain_shape {
   int ns;              // MFMA steps over the members

@@ -156,3 +156,19 @@ def test_enkf_condition_number(mda, ctx, k, p, var):
     # both sides carry the rounding of the smallest eigenvalue: cond * eps
     assert abs(f.getAnalysisResults()["condition_number"] - want) <= \
         want * max(1e-11, 64 * want * 2.2e-16)
+
+
+# ---- global transform: 32 points a wavefront, 256 a block, members in steps of 16 -----------
+@pytest.mark.parametrize("k,n", [(2, 1), (3, 15), (16, 17), (17, 31), (32, 33), (48, 255),
+                                 (49, 256), (64, 257), (65, 511), (96, 1000), (113, 70),
+                                 (128, 300)])
+def test_etkf_transform_matches_oracle(mda, ctx, orc, k, n):
+    rng = np.random.default_rng(50 * k + n)
+    p = 37
+    X, Yb = 5.0 + rng.standard_normal((k, n)), rng.standard_normal((k, p))
+    yo, var = rng.standard_normal(p), rng.uniform(0.5, 2.0, p)
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    f = mda.ETKF(ens, mda.Observation(yo, var, np.zeros(p), np.zeros(p)),
+                 mda.ObsOperator(hx=Yb), mda.Config({"inflation": 1.1}), ctx=ctx)
+    f.Analyse()
+    assert rel_err(ens.data, orc.etkf_analyse(X, Yb, yo, var, f.inflation)) < TOL
