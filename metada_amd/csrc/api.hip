@@ -360,7 +360,6 @@ void etkf_run(mda_ctx* c, double inflation, mda_ensemble* ens, const mda_obs* ob
     b.part = c->get<double>("gg_part", (size_t)ETKF_GG_BLOCKS * k * (k + 1));
     b.EB = c->get<double>("gg_EB", (size_t)k * (k + 1));
     b.T = c->get<double>("gT", (size_t)k * k);
-    b.scr = c->get<double>("g_scr", (size_t)2 * k * k);
     b.status = c->get<int>("g_status", 1);
   }
   hipStream_t s = c->stream;
@@ -369,7 +368,7 @@ void etkf_run(mda_ctx* c, double inflation, mda_ensemble* ens, const mda_obs* ob
   launch_obs_stats(s, de.X, k, de.n, p, h.row_ptr, h.col, h.w, h.hx, o.yo, nullptr, b.yp, b.dd,
                    nullptr, nullptr, nullptr, nullptr, b.status);
   launch_global_gram(s, b.yp, b.dd, o.var, nullptr, k, p, 0, b.part, ETKF_GG_BLOCKS, b.EB);
-  launch_etkf_solve_ws(s, k, b.EB, b.T, b.scr, b.status);
+  launch_etkf_solve_ws(s, k, b.EB, b.T, b.status);
   launch_transform_global(s, de.X, k, de.n, inflation, b.T, b.status);
   int hs = 0;
   MDA_HIP(hipMemcpyAsync(&hs, b.status, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -418,8 +417,7 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
     launch_global_gram(s, yp, dd, o.var, dZ, k, p, 1, part, nb, F);
     double* T = c->get<double>("gT", (size_t)k * k);
     double* Minv = c->get<double>("gMinv", (size_t)k * k);
-    double* scr = c->get<double>("g_scr", (size_t)2 * k * k);
-    launch_enkf_solve_ws(s, k, EB, F, T, Minv, scr, st);
+    launch_enkf_solve_ws(s, k, EB, F, T, Minv, st);
     {
       // a failed factorisation or non-finite input ends the call before any
       // diagnostics or update

@@ -377,7 +377,7 @@ dense_extremes dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda)
 // (256 workgroups, one per CU): the weighted Gram on FP64 MFMA, the rows of
 // Y_- carried through the factorisation of A, all in LDS.  Eight rounds narrow
 // each bracket by 129^8 = 8e16.  At p = 1,500, k = 80 the dense reduction of S
-// took 33 ms (four launches per column), this 2.9 ms.
+// took 33 ms (four launches per column), this 1.8 ms.
 // ---------------------------------------------------------------------------
 constexpr int CE_PTS = 128, CE_ROUNDS = 8;
 
@@ -443,45 +443,6 @@ __device__ inline void ce_bracket(int kind, int rounds, int k, int64_t p,
     if (i > 0) lo = a + w * ((double)i / (CE_PTS + 1));
     if (i < CE_PTS) hi = a + w * ((double)(i + 1) / (CE_PTS + 1));
   }
-}
-
-// Row-wise Cholesky of the leading n columns of `rows` >= n rows, row i at
-// row(i): entry j of row i becomes (a_ij - sum_c l_ic l_jc) / l_jj.  Thread i
-// owns row i (rows <= blockDim.x); every thread forms the pivot of row j for
-// itself, so a column costs one barrier.  False when a pivot is not positive.
-template <class Row>
-__device__ inline bool ce_cholesky(int n, int rows, Row row) {
-  const int i = threadIdx.x;
-  bool ok = true;
-  for (int j = 0; j < n; ++j) {
-    const double* lj = row(j);
-    double* li = row(i < rows ? i : rows - 1);
-    const bool own = i >= j && i < rows;
-    double pj = lj[j], s = own ? li[j] : 0.0;
-    double p1 = 0.0, s1 = 0.0;
-    int c = 0;
-    for (; c + 1 < j; c += 2) {
-      const double v0 = lj[c], v1 = lj[c + 1];
-      pj = fma(-v0, v0, pj);
-      p1 = fma(-v1, v1, p1);
-      if (own) {
-        s = fma(-li[c], v0, s);
-        s1 = fma(-li[c + 1], v1, s1);
-      }
-    }
-    if (c < j) {
-      pj = fma(-lj[c], lj[c], pj);
-      if (own) s = fma(-li[c], lj[c], s);
-    }
-    pj += p1;
-    s += s1;
-    if (!(pj > 0.0)) { ok = false; break; }  // the same in every thread
-    __syncthreads();                          // row j's entry j has been read
-    if (own) li[j] = i == j ? sqrt(pj) : s / sqrt(pj);
-    __syncthreads();
-  }
-  __syncthreads();
-  return ok;
 }
 
 template <int KT>
@@ -561,7 +522,8 @@ __global__ __launch_bounds__(256) void k_ce_round(const double* __restrict__ Yf,
     }
   }
   if (kind == 0) {
-    const bool spd = ce_cholesky(k, k, [&](int i) { return M + (size_t)i * (i + 1) / 2; });
+    const bool spd = block_row_cholesky(k, k, [&](int i) { return M + (size_t)i * (i + 1) / 2; },
+                                        [](int) { return 0; });
     if (tid == 0) *flag = spd ? 1 : 0;
     return;
   }
@@ -572,9 +534,10 @@ __global__ __launch_bounds__(256) void k_ce_round(const double* __restrict__ Yf,
     W[t * wld + m] = Yf[((size_t)(t / 4) * KT + m / 16) * 64 + (t % 4) * 16 + m % 16];
   }
   __syncthreads();
-  bool below = ce_cholesky(k, k + nq, [&](int i) {
-    return i < k ? M + (size_t)i * (i + 1) / 2 : W + (size_t)(i - k) * wld;
-  });
+  bool below = block_row_cholesky(
+      k, k + nq,
+      [&](int i) { return i < k ? M + (size_t)i * (i + 1) / 2 : W + (size_t)(i - k) * wld; },
+      [](int) { return 0; });
   if (below) {
     // N = W W^T - D in the triangle's place
     for (int e = tid; e < nq * nq; e += 256) {
@@ -591,7 +554,8 @@ __global__ __launch_bounds__(256) void k_ce_round(const double* __restrict__ Yf,
       M[(size_t)a * (a + 1) / 2 + b] = s0 + s1 - (a == b ? x - rs[a] : 0.0);
     }
     __syncthreads();
-    below = ce_cholesky(nq, nq, [&](int i) { return M + (size_t)i * (i + 1) / 2; });
+    below = block_row_cholesky(nq, nq, [&](int i) { return M + (size_t)i * (i + 1) / 2; },
+                               [](int) { return 0; });
   }
   if (tid == 0) *flag = below ? 0 : 1;
 }

@@ -264,6 +264,8 @@ void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32
   MDA_LAUNCH_CHECK();
 }
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+
 // ---------------------------------------------------------------------------
 // Global Gram over all observations (ETKF.hpp:150-155; EnKF via Woodbury):
 //   mode 0: G[a][c] = sum_o Y'[o][a] Y'[o][c] / var_o (c < k), and
@@ -271,158 +273,289 @@ void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32
 //   mode 1: G[a][j] = sum_o Y'[o][a] D[o][j] / var_o with the perturbed
 //           innovation D[o][j] = d_o + sqrt(var_o) Z[o][j] - Y'[o][j]
 //           (EnKF.hpp:212-224; Z is [p][k]).
-// Fixed grid, per-block partials, then a fixed-order reduction.  Blocks of
-// 256 threads take 32 observations at a time up to k (k+1) = 5120 entries;
-// beyond (64 < k <= 128) blocks of 1024 threads take 16.
+// On FP64 MFMA, four observations a step (lane (i16, kk): member 16t + i16 of
+// observation 4 step + kk, 128-byte row segments): mode 0 on the lower 16 x 16
+// tiles, mode 1 on all.  KT = ceil(k / 16) tile rows; up to 4 the block's four
+// wavefronts take different steps, beyond that two take each step, with the
+// even and the odd tile rows.  The wavefronts' sums meet in LDS, one partial
+// per block, then a fixed-order reduction (none for a single block).
+// p = 100,000, k = 64: 48 us (451 us with one product per thread and
+// observation out of LDS, and 64 us for a serial sum of the partials).
 // ---------------------------------------------------------------------------
-constexpr int GG_ACC = 20;  // entries per thread
-
-__global__ __launch_bounds__(1024) void k_global_gram_partial(
-    const double* __restrict__ yp_om, const double* __restrict__ d,
-    const double* __restrict__ var, const double* __restrict__ Z, int k, int64_t p, int mode,
-    int chunk, double* __restrict__ partial) {
-  extern __shared__ double sh[];
-  const int kq = mode == 0 ? k + 1 : k;
-  double* ys = sh;                  // [chunk][k]
-  double* qs = ys + chunk * k;      // [chunk][kq]
-  double* rs = qs + chunk * kq;     // [chunk]
-  const int tid = threadIdx.x, nt = blockDim.x;
-  const int ne = k * kq;
-  double acc[GG_ACC];
-  for (int t = 0; t < GG_ACC; ++t) acc[t] = 0.0;
-  for (int64_t o0 = (int64_t)blockIdx.x * chunk; o0 < p; o0 += (int64_t)gridDim.x * chunk) {
-    int nob = (int)((p - o0) < chunk ? (p - o0) : chunk);
-    __syncthreads();
-    for (int e = tid; e < nob * k; e += nt) ys[e] = yp_om[(size_t)o0 * k + e];
-    for (int ob = tid; ob < nob; ob += nt) rs[ob] = 1.0 / var[o0 + ob];
-    __syncthreads();
-    for (int e = tid; e < nob * kq; e += nt) {
-      int ob = e / kq, c = e % kq;
-      int64_t o = o0 + ob;
-      double v;
-      if (mode == 0)
-        v = (c < k) ? ys[ob * k + c] : d[o];
-      else  // an invalid observation (var = +inf, weight 0) contributes nothing
-        v = isinf(var[o]) ? 0.0 : d[o] + sqrt(var[o]) * Z[(size_t)o * k + c] - ys[ob * k + c];
-      qs[e] = v;
+template <int KT, int MODE>
+__global__ __launch_bounds__(256) void k_global_gram(const double* __restrict__ yp_om,
+                                                     const double* __restrict__ d,
+                                                     const double* __restrict__ var,
+                                                     const double* __restrict__ Z, int k,
+                                                     int64_t p, double* __restrict__ partial) {
+  constexpr int NG = KT > 4 ? 2 : 1, WS = 4 / NG;  // row groups, wavefronts over steps
+  constexpr int NR = (KT + NG - 1) / NG;           // tile rows of a group
+  constexpr int NA = NR * KT;
+  extern __shared__ double out[];  // [k][kq]
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, i16 = lane & 15, kk = lane >> 4;
+  const int grp = wv % NG, ws = wv / NG;
+  const int kq = MODE == 0 ? k + 1 : k;
+  const int64_t nstep = (p + 3) / 4;
+  d4 acc[NA];
+#pragma unroll
+  for (int t = 0; t < NA; ++t) acc[t] = d4{0.0, 0.0, 0.0, 0.0};
+  double bp[NR];
+#pragma unroll
+  for (int t = 0; t < NR; ++t) bp[t] = 0.0;
+  for (int64_t st = (int64_t)blockIdx.x * WS + ws; st < nstep; st += (int64_t)gridDim.x * WS) {
+    const int64_t o = 4 * st + kk;
+    const bool in = o < p;
+    const double vr = in ? var[o] : INFINITY, dv = in ? d[o] : 0.0;
+    const double rinv = 1.0 / vr;  // 0 for an invalid observation (var = +inf)
+    double y[KT], z[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      const int m = 16 * t + i16;
+      const bool mv = in && m < k;
+      y[t] = mv ? yp_om[(size_t)o * k + m] : 0.0;
+      if (MODE == 1) z[t] = mv && !isinf(vr) ? Z[(size_t)o * k + m] : 0.0;
     }
-    __syncthreads();
-    int t = 0;
-    for (int e = tid; e < ne; e += nt, ++t) {
-      int a = e / kq, c = e % kq;
-      double s = 0.0;
-      for (int ob = 0; ob < nob; ++ob) s += rs[ob] * ys[ob * k + a] * qs[ob * kq + c];
-      acc[t] += s;
+    if (MODE == 1) {
+      const double sr = isinf(vr) ? 0.0 : sqrt(vr);
+#pragma unroll
+      for (int t = 0; t < KT; ++t) z[t] = isinf(vr) ? 0.0 : dv + sr * z[t] - y[t];
+    }
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+      // tile row t NG + grp, by selects on the uniform grp (static indices)
+      double ya = y[t * NG];
+      if (NG == 2) ya = grp ? (t * NG + 1 < KT ? y[t * NG + 1 < KT ? t * NG + 1 : 0] : 0.0) : ya;
+      const double aw = rinv * ya;
+      if (MODE == 0) bp[t] = fma(aw, dv, bp[t]);
+#pragma unroll
+      for (int tb = 0; tb < KT; ++tb)
+        if (MODE == 1 || tb <= t * NG + NG - 1)
+          acc[t * KT + tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+              aw, MODE == 0 ? y[tb] : z[tb], acc[t * KT + tb], 0, 0, 0);
     }
   }
-  int t = 0;
-  for (int e = tid; e < ne; e += nt, ++t) partial[(size_t)blockIdx.x * ne + e] = acc[t];
+#pragma unroll
+  for (int t = 0; t < NR; ++t) {
+    bp[t] += __shfl_xor(bp[t], 16);
+    bp[t] += __shfl_xor(bp[t], 32);
+  }
+  for (int w = 0; w < WS; ++w) {
+    if (ws == w) {
+#pragma unroll
+      for (int t = 0; t < NR; ++t) {
+        const int ta = t * NG + grp;
+#pragma unroll
+        for (int tb = 0; tb < KT; ++tb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int row = 16 * ta + kk + 4 * r, col = 16 * tb + i16;
+            const bool use = row < k && col < k && (MODE == 1 || col <= row);
+            if (use && (MODE == 1 || tb <= t * NG + NG - 1)) {
+              const double v = acc[t * KT + tb][r] + (w == 0 ? 0.0 : out[row * kq + col]);
+              out[row * kq + col] = v;
+              if (MODE == 0 && row != col) out[col * kq + row] = v;
+            }
+          }
+        if (MODE == 0 && kk == 0 && 16 * ta + i16 < k) {
+          const int row = 16 * ta + i16;
+          out[row * kq + k] = bp[t] + (w == 0 ? 0.0 : out[row * kq + k]);
+        }
+      }
+    }
+    __syncthreads();
+  }
+  double* pb = partial + (size_t)blockIdx.x * k * kq;
+  for (int e = tid; e < k * kq; e += 256) pb[e] = out[e];
 }
 
-__global__ void k_reduce_partials(const double* __restrict__ partial, int nblocks, int ne,
-                                  double* __restrict__ out) {
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < ne; e += gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (int b = 0; b < nblocks; ++b) s += partial[(size_t)b * ne + e];
-    out[e] = s;
+// out[e] = sum over blocks of partial[b][e]: eight threads per entry, each a
+// contiguous eighth of the blocks, added in order
+__global__ __launch_bounds__(512) void k_reduce_partials(const double* __restrict__ partial,
+                                                         int nblocks, int ne,
+                                                         double* __restrict__ out) {
+  __shared__ double red[8][64];
+  const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int e = blockIdx.x * 64 + lane;
+  const int per = (nblocks + 7) / 8, b0 = q * per,
+            b1 = b0 + per < nblocks ? b0 + per : nblocks;
+  double s = 0.0;
+  if (e < ne) {
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b) s += partial[(size_t)b * ne + e];
+  }
+  red[q][lane] = s;
+  __syncthreads();
+  if (q == 0 && e < ne) {
+    double t = red[0][lane];
+    for (int i = 1; i < 8; ++i) t += red[i][lane];
+    out[e] = t;
   }
 }
 
 void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
                         const double* var, const double* Z, int k, int64_t p, int mode,
                         double* partial, int nblocks, double* out) {
-  const int kq = mode == 0 ? k + 1 : k;
-  const int nt = k * kq <= 256 * GG_ACC ? 256 : 1024;
-  const int chunk = nt == 256 ? 32 : 16;
-  MDA_REQUIRE((k * kq + nt - 1) / nt <= GG_ACC, "global Gram supports k <= 128");
-  size_t shm = sizeof(double) * (chunk * k + chunk * kq + chunk);
-  hipLaunchKernelGGL(k_global_gram_partial, dim3(nblocks), dim3(nt), shm, s, yp_om, d, var, Z,
-                     k, p, mode, chunk, partial);
+  MDA_REQUIRE(k >= 1 && k <= 128, "global Gram supports k <= 128");
+  const int kq = mode == 0 ? k + 1 : k, kt = (k + 15) / 16;
+  // at least eight steps of four observations per wavefront
+  const int ws = kt > 4 ? 2 : 4;
+  const int64_t want = ((p + 3) / 4 + 8 * ws - 1) / (8 * ws);
+  const int nb = (int)std::min<int64_t>(nblocks, std::max<int64_t>(1, want));
+  double* part = nb > 1 ? partial : out;
+  const size_t shm = sizeof(double) * k * kq;
+#define MDA_GG(KT)                                                                               \
+  case KT:                                                                                       \
+    if (mode == 0)                                                                               \
+      hipLaunchKernelGGL((k_global_gram<KT, 0>), dim3(nb), dim3(256), shm, s, yp_om, d, var, Z,  \
+                         k, p, part);                                                            \
+    else                                                                                         \
+      hipLaunchKernelGGL((k_global_gram<KT, 1>), dim3(nb), dim3(256), shm, s, yp_om, d, var, Z,  \
+                         k, p, part);                                                            \
+    break;
+  switch (kt) { MDA_GG(1) MDA_GG(2) MDA_GG(3) MDA_GG(4) MDA_GG(5) MDA_GG(6) MDA_GG(7) MDA_GG(8) }
+#undef MDA_GG
   MDA_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_reduce_partials, dim3(grid_for(k * kq, 256)), dim3(256), 0, s, partial,
-                     nblocks, k * kq, out);
+  if (nb == 1) return;
+  hipLaunchKernelGGL(k_reduce_partials, dim3((k * kq + 63) / 64), dim3(512), 0, s, partial, nb,
+                     k * kq, out);
   MDA_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------------------
-// ETKF k x k solve (ETKF.hpp:150-159), one workgroup, matrices in global
-// scratch through flat pointers (EB is [k][k+1] = [E | b]):
-//   Pa = (E + (k-1) I)^-1, wa = Pa b, Wa = sqrt(k-1) chol_L(Pa),
-//   T = wa 1^T + Wa  so that X_a = xbar + X' T.
+// k x k solves of the global filters, one workgroup, k <= 128: M = E + (k-1) I
+// = L L^T (EB is [k][k+1] = [E | b]) with the identity's rows carried through
+// the factorisation, so that W = L^-T (upper triangular) comes with it.  Both
+// triangles packed in LDS (132 KB at k = 128).  The matrix in global memory,
+// a barrier per column and a serial inverse took 545 us (ETKF, k = 64) and
+// 960 us (EnKF, k = 80); this takes 74 and 182 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_etkf_solve(int k, const double* __restrict__ EB,
-                                                    double* __restrict__ T,
-                                                    double* __restrict__ scratch,
-                                                    int* status) {
-  __shared__ int flag;
-  __shared__ double wa[256];
-  const int tid = threadIdx.x, nt = blockDim.x;
-  double* M = scratch;          // [k][k]
-  double* W = scratch + k * k;  // [k][k]
-  for (int idx = tid; idx < k * k; idx += nt) {
-    int i = idx / k, j = idx % k;
-    M[idx] = EB[i * (k + 1) + j] + (i == j ? (double)(k - 1) : 0.0);
+constexpr int KS_THREADS = 512;
+__host__ __device__ inline size_t ks_tri(int k) { return (size_t)k * (k + 1) / 2; }
+
+struct ks_lds {
+  double* M;  // lower triangle, row i at i (i + 1) / 2
+  double* W;  // upper triangle, row i holds the columns i .. k-1
+  int k;
+  __device__ double* lrow(int i) const { return M + (size_t)i * (i + 1) / 2; }
+  // W[i][j] = wrow(i)[j], j >= i
+  __device__ double* wrow(int i) const {
+    return W + ((ptrdiff_t)i * k - (ptrdiff_t)i * (i - 1) / 2 - i);
+  }
+};
+
+// M (rows and columns in reversed order with rev) and W = L^-T; false when M
+// is not positive definite
+__device__ inline bool ks_factor(const ks_lds& f, const double* __restrict__ EB, bool rev) {
+  const int k = f.k, tid = threadIdx.x;
+  for (int idx = tid; idx < k * k; idx += KS_THREADS) {
+    const int i = idx / k, j = idx % k;
+    if (j > i) continue;
+    const int si = rev ? k - 1 - i : i, sj = rev ? k - 1 - j : j;
+    f.lrow(i)[j] = EB[si * (k + 1) + sj] + (i == j ? (double)(k - 1) : 0.0);
+    f.wrow(j)[i] = i == j ? 1.0 : 0.0;
   }
   __syncthreads();
-  bool ok = block_cholesky(M, k, k, &flag);
-  block_spd_inverse_from_chol(M, k, W, k, k);  // M <- Pa
-  for (int i = tid; i < k; i += nt) {
+  return block_row_cholesky(
+      k, 2 * k, [&](int i) { return i < k ? f.lrow(i) : f.wrow(i - k); },
+      [&](int i) { return i - k; });
+}
+
+// ETKF (ETKF.hpp:150-159): Pa = M^-1, wa = Pa b, Wa = sqrt(k-1) chol_L(Pa),
+// T = wa 1^T + Wa so that X_a = xbar + X' T.  With the order of the members
+// reversed (J M J = L L^T), chol_L(Pa) = J L^-T J: entry (i, j), j <= i, is
+// W[k-1-i][k-1-j].
+__global__ __launch_bounds__(KS_THREADS) void k_etkf_solve(int k, const double* __restrict__ EB,
+                                                           double* __restrict__ T, int* status) {
+  extern __shared__ double sh[];
+  __shared__ double y[128], wa[128];
+  const int tid = threadIdx.x;
+  const ks_lds f{sh, sh + ks_tri(k), k};
+  const bool ok = ks_factor(f, EB, true);
+  if (!ok) {  // the same in every thread; T is not used then
+    if (tid == 0) atomicOr(status, MDA_ST_NOT_SPD);
+    return;
+  }
+  auto lp = [&](int i, int j) { return f.wrow(k - 1 - i)[k - 1 - j]; };
+  if (tid < k) {
     double s = 0.0;
-    for (int c = 0; c < k; ++c) s += M[i * k + c] * EB[c * (k + 1) + k];
-    wa[i] = s;
+    for (int i = tid; i < k; ++i) s = fma(lp(i, tid), EB[i * (k + 1) + k], s);
+    y[tid] = s;
   }
   __syncthreads();
-  ok = block_cholesky(M, k, k, &flag) && ok;  // M <- chol_L(Pa)
-  const double sq = sqrt((double)(k - 1));
-  for (int idx = tid; idx < k * k; idx += nt) {
-    int i = idx / k, j = idx % k;
-    T[idx] = wa[i] + sq * M[idx];
+  if (tid < k) {
+    double s = 0.0;
+    for (int j = 0; j <= tid; ++j) s = fma(lp(tid, j), y[j], s);
+    wa[tid] = s;
   }
-  if (tid == 0 && !ok) atomicOr(status, MDA_ST_NOT_SPD);
+  __syncthreads();
+  const double sq = sqrt((double)(k - 1));
+  for (int idx = tid; idx < k * k; idx += KS_THREADS) {
+    const int i = idx / k, j = idx % k;
+    T[idx] = wa[i] + (j <= i ? sq * lp(i, j) : 0.0);
+  }
 }
 
-void launch_etkf_solve_ws(hipStream_t s, int k, const double* EB, double* T, double* scratch,
-                          int* status) {
-  MDA_REQUIRE(k <= 256, "ETKF supports k <= 256");
-  hipLaunchKernelGGL(k_etkf_solve, dim3(1), dim3(256), 0, s, k, EB, T, scratch, status);
+void launch_etkf_solve_ws(hipStream_t s, int k, const double* EB, double* T, int* status) {
+  MDA_REQUIRE(k <= 128, "ETKF supports k <= 128");
+  hipLaunchKernelGGL(k_etkf_solve, dim3(1), dim3(KS_THREADS), sizeof(double) * 2 * ks_tri(k), s, k,
+                     EB, T, status);
   MDA_LAUNCH_CHECK();
 }
 
-// ---------------------------------------------------------------------------
-// EnKF k x k solve.  With M = (k-1) I + Y'^T R^-1 Y' the Woodbury identity
-// gives Y'^T S^-1 / (k-1) = M^-1 Y'^T R^-1 for S = Y'Y'^T/(k-1) + R
+// EnKF: with M = (k-1) I + Y'^T R^-1 Y' the Woodbury identity gives
+// Y'^T S^-1 / (k-1) = M^-1 Y'^T R^-1 for S = Y'Y'^T/(k-1) + R
 // (EnKF.hpp:193-199), so K D = X' M^-1 F with F = Y'^T R^-1 D and the update
 // x_a = xbar + X'_j + K D_j (EnKF.hpp:216-226) is X_a = xbar + X'(I + M^-1 F).
-// Outputs T = I + M^-1 F and M^-1.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_enkf_solve(int k, const double* __restrict__ EB,
-                                                    const double* __restrict__ F,
-                                                    double* __restrict__ T,
-                                                    double* __restrict__ Minv,
-                                                    double* __restrict__ scratch, int* status) {
-  __shared__ int flag;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  double* W = scratch;
-  for (int idx = tid; idx < k * k; idx += nt) {
-    int i = idx / k, j = idx % k;
-    Minv[idx] = EB[i * (k + 1) + j] + (i == j ? (double)(k - 1) : 0.0);
+// Outputs T = I + M^-1 F and M^-1 = W W^T.
+__global__ __launch_bounds__(KS_THREADS) void k_enkf_solve(int k, const double* __restrict__ EB,
+                                                           const double* __restrict__ F,
+                                                           double* __restrict__ T,
+                                                           double* __restrict__ Minv,
+                                                           int* status) {
+  extern __shared__ double sh[];
+  const int tid = threadIdx.x;
+  const ks_lds f{sh, sh + ks_tri(k), k};
+  const bool ok = ks_factor(f, EB, false);
+  if (!ok) {
+    if (tid == 0) atomicOr(status, MDA_ST_NOT_SPD);
+    return;
+  }
+  // M^-1 into the place of L (W has all it needs)
+  for (int idx = tid; idx < k * k; idx += KS_THREADS) {
+    const int i = idx / k, j = idx % k;
+    if (j > i) continue;
+    const double *wi = f.wrow(i), *wj = f.wrow(j);
+    double s = 0.0;
+#pragma unroll 4
+    for (int c = i; c < k; ++c) s = fma(wi[c], wj[c], s);
+    f.lrow(i)[j] = s;
+    Minv[i * k + j] = s;
+    Minv[j * k + i] = s;
   }
   __syncthreads();
-  bool ok = block_cholesky(Minv, k, k, &flag);
-  block_spd_inverse_from_chol(Minv, k, W, k, k);
-  for (int idx = tid; idx < k * k; idx += nt) {
-    int i = idx / k, j = idx % k;
-    double s = 0.0;
-    for (int c = 0; c < k; ++c) s += Minv[i * k + c] * F[c * k + j];
-    T[idx] = (i == j ? 1.0 : 0.0) + s;
+  for (int idx = tid; idx < (k + 3) / 4 * k; idx += KS_THREADS) {
+    const int i0 = idx / k * 4, j = idx % k;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int c = 0; c < k; ++c) {
+      const double fv = F[(size_t)c * k + j];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + r < k ? i0 + r : k - 1;
+        s[r] = fma(i >= c ? f.lrow(i)[c] : f.lrow(c)[i], fv, s[r]);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (i0 + r < k) T[(size_t)(i0 + r) * k + j] = (i0 + r == j ? 1.0 : 0.0) + s[r];
   }
-  if (tid == 0 && !ok) atomicOr(status, MDA_ST_NOT_SPD);
 }
 
 void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* F, double* T,
-                          double* Minv, double* scratch, int* status) {
-  hipLaunchKernelGGL(k_enkf_solve, dim3(1), dim3(256), 0, s, k, EB, F, T, Minv, scratch,
-                     status);
+                          double* Minv, int* status) {
+  MDA_REQUIRE(k <= 128, "EnKF supports k <= 128");
+  hipLaunchKernelGGL(k_enkf_solve, dim3(1), dim3(KS_THREADS), sizeof(double) * 2 * ks_tri(k), s, k,
+                     EB, F, T, Minv, status);
   MDA_LAUNCH_CHECK();
 }
 
@@ -433,8 +566,6 @@ void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* 
 // loads are 128-byte segments.  An ensemble of k members takes NS = k / 4
 // steps, rounded up to a compiled size; the values past k are zero.
 // ---------------------------------------------------------------------------
-typedef double d4 __attribute__((ext_vector_type(4)));
-
 // v[t][s] = (x - mean) scale of the tile's points (0 past n and k); mean[t]
 // the mean over the members of point i0 + 16 t + i16
 template <int NS, int MT>

@@ -136,6 +136,97 @@ __device__ inline void block_spd_inverse_from_chol(double* A, int lda, double* W
 }
 
 // ---------------------------------------------------------------------------
+// Cholesky of the leading n columns of `rows` >= n rows, one row per thread
+// (rows <= blockDim.x), matrix in LDS: row(i)[j] = a_ij becomes
+// l_ij = (a_ij - sum_c l_ic l_jc) / l_jj.  Rows i < n hold the columns j <= i;
+// rows i >= n hold the columns j >= first(i) (zero before it): b^T becomes
+// b^T L^-T.  Four columns at a time: each thread's dot products with the four
+// panel rows (one own and four broadcast LDS reads per four FMAs), then every
+// thread factors the 4 x 4 block for itself.  Three barriers per panel; false
+// (in every thread) when a pivot is not positive.
+// ---------------------------------------------------------------------------
+template <class Row, class First>
+__device__ inline bool block_row_cholesky(int n, int rows, Row row, First first) {
+  const int i = threadIdx.x;
+  double* li = row(i < rows ? i : rows - 1);
+  const int c0 = i < rows && i >= n ? first(i) : 0;
+  for (int j0 = 0; j0 < n; j0 += 4) {
+    const int nb = n - j0 < 4 ? n - j0 : 4;
+    const double* r0 = row(j0);
+    const double* r1 = row(j0 + (nb > 1 ? 1 : 0));
+    const double* r2 = row(j0 + (nb > 2 ? 2 : 0));
+    const double* r3 = row(j0 + (nb > 3 ? 3 : 0));
+    const bool own = i < rows && i >= j0;
+    // last panel column this row holds
+    const int last = i < n ? (i - j0 < nb - 1 ? i - j0 : nb - 1) : nb - 1;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    if (own) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (m <= last && j0 + m >= c0) s[m] = li[j0 + m];
+#pragma unroll 4
+      for (int c = c0; c < j0; ++c) {
+        const double v = li[c];
+        s[0] = fma(-v, r0[c], s[0]);
+        s[1] = fma(-v, r1[c], s[1]);
+        s[2] = fma(-v, r2[c], s[2]);
+        s[3] = fma(-v, r3[c], s[3]);
+      }
+    }
+    const bool panel = own && i < j0 + nb && i < n;
+    __syncthreads();  // the panel rows' entries below j0 + nb have been read
+    if (panel) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (m <= last) li[j0 + m] = s[m];
+    }
+    __syncthreads();
+    // L of the 4 x 4 block (rows past nb are not used)
+    const double g00 = r0[j0];
+    if (!(g00 > 0.0)) return false;
+    const double l00 = sqrt(g00);
+    double l10 = 0.0, l11 = 1.0, l20 = 0.0, l21 = 0.0, l22 = 1.0, l30 = 0.0, l31 = 0.0, l32 = 0.0,
+           l33 = 1.0;
+    if (nb > 1) {
+      l10 = r1[j0] / l00;
+      const double g = fma(-l10, l10, r1[j0 + 1]);
+      if (!(g > 0.0)) return false;
+      l11 = sqrt(g);
+    }
+    if (nb > 2) {
+      l20 = r2[j0] / l00;
+      l21 = fma(-l20, l10, r2[j0 + 1]) / l11;
+      const double g = fma(-l21, l21, fma(-l20, l20, r2[j0 + 2]));
+      if (!(g > 0.0)) return false;
+      l22 = sqrt(g);
+    }
+    if (nb > 3) {
+      l30 = r3[j0] / l00;
+      l31 = fma(-l30, l10, r3[j0 + 1]) / l11;
+      l32 = fma(-l31, l21, fma(-l30, l20, r3[j0 + 2])) / l22;
+      const double g = fma(-l32, l32, fma(-l31, l31, fma(-l30, l30, r3[j0 + 3])));
+      if (!(g > 0.0)) return false;
+      l33 = sqrt(g);
+    }
+    __syncthreads();  // the block has been read
+    if (own) {
+      double x[4];
+      x[0] = s[0] / l00;
+      x[1] = fma(-x[0], l10, s[1]) / l11;
+      x[2] = fma(-x[1], l21, fma(-x[0], l20, s[2])) / l22;
+      x[3] = fma(-x[2], l32, fma(-x[1], l31, fma(-x[0], l30, s[3]))) / l33;
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+        if (m <= last && j0 + m >= c0) li[j0 + m] = x[m];
+      if (panel)  // the diagonal entry
+        li[i] = i == j0 ? l00 : i == j0 + 1 ? l11 : i == j0 + 2 ? l22 : l33;
+    }
+    __syncthreads();
+  }
+  return true;
+}
+
+// ---------------------------------------------------------------------------
 // Parallel-order cyclic Jacobi (round-robin "circle" ordering: n-1 rounds of
 // n/2 disjoint rotations per sweep).  A (n x n symmetric, n even) is
 // diagonalised in place; V (may be null) accumulates the rotations so that

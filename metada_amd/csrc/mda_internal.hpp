@@ -190,11 +190,10 @@ void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32
 void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
                         const double* var, const double* Z, int k, int64_t p, int mode,
                         double* partial, int nblocks, double* out);
-// small dense solves on one workgroup (matrices in global scratch)
-void launch_etkf_solve_ws(hipStream_t s, int k, const double* EB, double* T, double* scratch,
-                          int* status);
+// small dense solves on one workgroup (matrices in LDS)
+void launch_etkf_solve_ws(hipStream_t s, int k, const double* EB, double* T, int* status);
 void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* F, double* T,
-                          double* Minv, double* scratch, int* status);
+                          double* Minv, int* status);
 // X_a = xbar + scale * X' T for all state points (global T); skipped when
 // the status word holds a MDA_ST_SKIP_UPDATE bit.  With partial (3 doubles per
 // block, transform_global_blocks(n) of them), out3[2] = sum over state and
@@ -393,12 +392,12 @@ void launch_reduce_int(hipStream_t s, const int* v, int64_t n, int64_t* out2 /* 
 int guarded_call(mda_ctx* ctx, const std::function<void()>& f);
 
 // ETKF (ETKF.hpp:100-178) on device buffers: Y' [p][k], d [p], Gram
-// partials [ETKF_GG_BLOCKS][k][k+1], [E | b] [k][k+1], T [k][k], Cholesky
-// scratch [2][k][k] and the status word.  etkf_run takes them from the
+// partials [ETKF_GG_BLOCKS][k][k+1], [E | b] [k][k+1], T [k][k] and the status
+// word.  etkf_run takes them from the
 // context workspace when `bufs` is null.
 constexpr int ETKF_GG_BLOCKS = 256;
 struct etkf_bufs {
-  double *yp, *dd, *part, *EB, *T, *scr;
+  double *yp, *dd, *part, *EB, *T;
   int* status;
 };
 void etkf_run(mda_ctx* c, double inflation, mda_ensemble* ens, const mda_obs* obs,

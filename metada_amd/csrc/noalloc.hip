@@ -64,7 +64,6 @@ extern "C" int mda_etkf_analyse_noalloc(mda_ctx* c, double inflation, mda_ensemb
     b.part = base + off; off += align32((size_t)mda::ETKF_GG_BLOCKS * k * (k + 1));
     b.EB = base + off; off += align32((size_t)k * (k + 1));
     b.T = base + off; off += align32((size_t)k * k);
-    b.scr = base + off; off += align32((size_t)2 * k * k);
     b.status = reinterpret_cast<int*>(base + off); off += 32;
     MDA_REQUIRE(off <= NOALLOC_DOUBLES, "mda_etkf_analyse_noalloc: scratch layout too large");
     mda::etkf_run(c, inflation, ens, obs, hop, &b);

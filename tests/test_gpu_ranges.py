@@ -172,3 +172,36 @@ def test_etkf_transform_matches_oracle(mda, ctx, orc, k, n):
                  mda.ObsOperator(hx=Yb), mda.Config({"inflation": 1.1}), ctx=ctx)
     f.Analyse()
     assert rel_err(ens.data, orc.etkf_analyse(X, Yb, yo, var, f.inflation)) < TOL
+
+
+# ---- global Gram: steps of 4 observations, one or many partial blocks, two row groups -------
+@pytest.mark.parametrize("k", [2, 16, 33, 64, 65, 80, 113, 128])
+@pytest.mark.parametrize("p", [1, 3, 65, 129, 1030, 33000])
+def test_global_filters_every_p_match_oracle(mda, ctx, orc, k, p):
+    """ETKF and EnKF over observation counts around the Gram's block sizes,
+    one observation invalid; the EnKF's noalloc twin is bit-equal elsewhere."""
+    rng = np.random.default_rng(k * 7919 + p)
+    n = 20
+    X, Yb = rng.standard_normal((k, n)), rng.standard_normal((k, p))
+    yo, var = rng.standard_normal(p), rng.uniform(0.5, 2.0, p) * max(1.0, p / 50.0)
+    if p > 1:
+        var[p // 2] = np.inf
+    obs = mda.Observation(yo, var, np.zeros(p), np.zeros(p))
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    f = mda.ETKF(ens, obs, mda.ObsOperator(hx=Yb), mda.Config({"inflation": 1.1}), ctx=ctx)
+    f.Analyse()
+    ok = np.isfinite(var)  # an invalid observation has weight 0
+    assert rel_err(ens.data, orc.etkf_analyse(X, Yb[:, ok], yo[ok], var[ok], f.inflation)) < TOL
+    if p > 1030:
+        return
+    Z = rng.standard_normal((p, k))
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    g = mda.EnKF(ens, obs, mda.ObsOperator(hx=Yb),
+                 mda.Config({"analysis": {"inflation": 1.1}}), ctx=ctx)
+    g.Analyse(Z=Z)
+    Y, d = Yb - Yb.mean(0), yo - Yb.mean(0)
+    Y, d, Zk, R = Y[:, ok], d[ok], Z[ok], var[ok]
+    K = np.linalg.solve(Y.T @ Y / (k - 1) + np.diag(R), Y.T) / (k - 1)
+    D = d[:, None] + np.sqrt(R)[:, None] * Zk - Y.T
+    Xp = (X - X.mean(0)) * np.sqrt(g.inflation_factor)
+    assert rel_err(ens.data, X.mean(0) + (np.eye(k) + K.T @ D).T @ Xp) < TOL
