@@ -440,24 +440,24 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
       const enkf_gain_shape gs = enkf_gain_plan(k, n, p);
       double* Gf = c->get<double>("enkf_G", gs.gf_doubles());
       double* mm = c->get<double>("enkf_mm", gs.partial_doubles());
-      double* out3 = c->get<double>("enkf_mm_out", 3);
-      launch_enkf_gain_minmax(s, de.X, k, n, scale, Minv, yp, o.var, p, gs, Gf, mm, out3);
-      double h3[3] = {0.0, 0.0, 0.0};
-      d2h(c, h3, out3, sizeof(h3));
-      dg.max_kalman_gain = h3[0];
-      dg.min_kalman_gain = h3[1];
-      dg.background_spread = std::sqrt(h3[2] / ((double)n * k));
+      double* out4 = c->get<double>("enkf_mm_out", 4);
+      launch_enkf_gain_minmax(s, de.X, k, n, scale, Minv, yp, o.var, p, gs, Gf, mm, out4);
+      double h4[4] = {0.0, 0.0, 0.0, 0.0};
+      d2h(c, h4, out4, sizeof(h4));
+      dg.max_kalman_gain = h4[0];
+      dg.min_kalman_gain = h4[1];
+      dg.background_spread = std::sqrt(h4[2] / ((double)n * k));
       // cond(S) = ratio of the extreme singular values of the SPD
       // S = Y'Y'^T/(k-1) + R (EnKF.hpp:205-209)
       dg.condition_number = enkf_condition_number(c, yp, o.var, k, p, EB);
     }
     if (diag) {
-      double* pa = c->get<double>("enkf_xa_part", (size_t)3 * transform_global_blocks(n));
-      double* out3 = c->get<double>("enkf_mm_out", 3);
-      launch_transform_global(s, de.X, k, n, scale, T, st, pa, out3);
-      double h3[3] = {0.0, 0.0, 0.0};
-      d2h(c, h3, out3, sizeof(h3));
-      dg.analysis_spread = std::sqrt(h3[2] / ((double)n * k));
+      double* pa = c->get<double>("enkf_xa_part", (size_t)4 * transform_global_blocks(n));
+      double* out4 = c->get<double>("enkf_mm_out", 4);
+      launch_transform_global(s, de.X, k, n, scale, T, st, pa, out4);
+      double h4[4] = {0.0, 0.0, 0.0, 0.0};
+      d2h(c, h4, out4, sizeof(h4));
+      dg.analysis_spread = std::sqrt(h4[3] / ((double)n * k));
     } else {
       launch_transform_global(s, de.X, k, n, scale, T, st);
     }
@@ -535,9 +535,6 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     launch_zero(s, st, 2 * sizeof(int));
     launch_check_obs(s, o, st);
     launch_lw_flag_inf(s, o.var, p, st + 1);
-    // forecast statistics (RecomputeMean / RecomputePerturbations, :215-229)
-    double* mean = c->get<double>("lw_mean", n);
-    launch_mean_pert(s, de.X, k, n, 1.0, mean, nullptr);
     double* ybar = c->get<double>("lw_ybar", p);
     double* yp = c->get<double>("lw_yp", (size_t)p * k);
     double* dd = c->get<double>("lw_d", p);
@@ -552,14 +549,10 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     // member weights (:413-430)
     std::vector<double> sumsq(k, 0.0), chi2(k, 0.0);
     if (prm->weighting == MDA_LW_W_ADAPTIVE || prm->weighting == MDA_LW_W_INVERSE_VAR) {
-      constexpr int NB = 64;
-      double* part = c->get<double>("lw_part", (size_t)NB * k);
-      launch_lw_member_sumsq(s, de.X, mean, k, n, part, NB);
-      std::vector<double> hp((size_t)NB * k);
-      d2h(c, hp.data(), part, sizeof(double) * NB * k);
-      MDA_HIP(hipStreamSynchronize(s));
-      for (int i = 0; i < k; ++i)
-        for (int b = 0; b < NB; ++b) sumsq[i] += hp[(size_t)i * NB + b];
+      double* part = c->get<double>("lw_part", (size_t)LW_SUMSQ_BLOCKS * k);
+      double* ss = c->get<double>("lw_sumsq", k);
+      launch_lw_member_sumsq(s, de.X, k, n, part, ss);
+      d2h(c, sumsq.data(), ss, sizeof(double) * k);
     } else if (prm->weighting == MDA_LW_W_LIKELIHOOD) {
       double* dchi = c->get<double>("lw_chi2", k);
       launch_lw_chi2(s, o.yo, ybar, yp, o.var, k, p, dchi);
@@ -591,8 +584,6 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     MDA_HIP(hipEventRecord(c->ev[1], s));
     double* part2 = c->get<double>("sumsq_part", 1024);
     if (diag) {
-      launch_dev_sumsq(s, de.X, k, n, scale, part2, 512);
-      dg.background_spread = std::sqrt(host_sum(c, part2, 512) / ((double)n * k));
       launch_sumsq(s, dd, p, part2, 512);
       dg.innovation_norm = std::sqrt(host_sum(c, part2, 512));
     }
@@ -600,26 +591,25 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     MDA_HIP(hipStreamSynchronize(s));
     if (hst[0] & MDA_ST_NOT_SPD)
       throw mda_error(MDA_E_NUMERIC, "LWEnKF: S = L o Pf + R is singular");
-    // gain and update, fused (:272-301)
-    const size_t nbu = lw_update_blocks(n);
-    double* mm = c->get<double>("lw_mm", 2 * nbu);
+    // gain and update, fused (:272-301), with the forecast mean and spreads
+    // (RecomputeMean / RecomputePerturbations, :215-229) formed in the same pass
+    const lw_update_shape us = lw_update_plan(k, n, p);
+    double* Gf = c->get<double>("lw_Gf", us.frag_doubles());
+    double* Df = c->get<double>("lw_Df", us.frag_doubles());
+    double* tap = c->get<double>("lw_tap", us.ntap);
+    double* mm = c->get<double>("lw_mm", 4 * us.nblk);
+    double* out4 = c->get<double>("lw_out", 4);
     MDA_HIP(hipEventRecord(c->ev[2], s));
-    launch_lw_update(s, de.X, mean, scale, yp, D, k, n, p, radius, prm->localization,
-                     prm->gc_form, mm);
+    launch_lw_update(s, de.X, scale, yp, D, k, n, p, radius, prm->localization, prm->gc_form, us,
+                     Gf, Df, tap, mm, out4);
     MDA_HIP(hipEventRecord(c->ev[3], s));
-    std::vector<double> hm(2 * nbu);
-    d2h(c, hm.data(), mm, sizeof(double) * 2 * nbu);
-    MDA_HIP(hipStreamSynchronize(s));
-    double mx = -std::numeric_limits<double>::infinity(), mn = -mx;
-    for (size_t b = 0; b < nbu; ++b) {
-      mx = std::max(mx, hm[2 * b]);
-      mn = std::min(mn, hm[2 * b + 1]);
-    }
+    double h4[4] = {0.0, 0.0, 0.0, 0.0};
+    d2h(c, h4, out4, sizeof(h4));
     if (diag) {
-      launch_dev_sumsq(s, de.X, k, n, 1.0, part2, 512);
-      dg.analysis_spread = std::sqrt(host_sum(c, part2, 512) / ((double)n * k));
-      dg.max_kalman_gain = mx;
-      dg.min_kalman_gain = mn;
+      dg.background_spread = std::sqrt(h4[2] / ((double)n * k));
+      dg.analysis_spread = std::sqrt(h4[3] / ((double)n * k));
+      dg.max_kalman_gain = h4[0];
+      dg.min_kalman_gain = h4[1];
       dg.localization_radius = radius;
       dg.max_weight = *std::max_element(w.begin(), w.end());
       dg.min_weight = *std::min_element(w.begin(), w.end());

@@ -19,8 +19,6 @@
 
 namespace mda {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
 // S[a][b] = (sum_j Y'[a][j] Y'[b][j]) / (k-1) + (a == b ? var[a] : 0), Y'
 // obs-major [p][k]; the member sum runs in member order (as EnKF.hpp:193).
 __global__ void k_form_enkf_S(const double* __restrict__ yp, const double* __restrict__ var,

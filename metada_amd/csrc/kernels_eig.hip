@@ -28,8 +28,6 @@
 
 namespace mda {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
 constexpr int EIG_N = 64;  // largest ensemble size handled by this path
 
 __device__ inline void wave_lds_sync() {

@@ -65,33 +65,6 @@ void launch_sumsq(hipStream_t s, const double* X, int64_t count, double* partial
   MDA_LAUNCH_CHECK();
 }
 
-// sum over members and state of ((x - mean) * scale)^2, per-block partials
-// (EnKF.hpp:334 background spread, :246-253 analysis spread)
-__global__ void k_dev_sumsq(const double* __restrict__ X, int k, int64_t n, double scale,
-                            double* partial) {
-  __shared__ double red[256];
-  const double rk = 1.0 / (double)k;
-  double acc = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    double s = 0.0;
-    for (int j = 0; j < k; ++j) s += X[(size_t)j * n + i];
-    double m = s * rk;
-    for (int j = 0; j < k; ++j) {
-      double v = (X[(size_t)j * n + i] - m) * scale;
-      acc += v * v;
-    }
-  }
-  acc = block_sum(acc, red);
-  if (threadIdx.x == 0) partial[blockIdx.x] = acc;
-}
-
-void launch_dev_sumsq(hipStream_t s, const double* X, int k, int64_t n, double scale,
-                      double* partial, int nblocks) {
-  hipLaunchKernelGGL(k_dev_sumsq, dim3(nblocks), dim3(256), 0, s, X, k, n, scale, partial);
-  MDA_LAUNCH_CHECK();
-}
-
 // ---------------------------------------------------------------------------
 // Observation space (EnKF.hpp:168-184, LETKF.hpp:197-211): hx_j = H x_j for
 // every member (CSR stencil gather, or a caller-supplied member-major H(x)),
@@ -264,8 +237,6 @@ void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32
   MDA_LAUNCH_CHECK();
 }
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
 // ---------------------------------------------------------------------------
 // Global Gram over all observations (ETKF.hpp:150-155; EnKF via Woodbury):
 //   mode 0: G[a][c] = sum_o Y'[o][a] Y'[o][c] / var_o (c < k), and
@@ -392,6 +363,13 @@ __global__ __launch_bounds__(512) void k_reduce_partials(const double* __restric
   }
 }
 
+void launch_reduce_partials(hipStream_t s, const double* partial, int nblocks, int ne,
+                            double* out) {
+  hipLaunchKernelGGL(k_reduce_partials, dim3((ne + 63) / 64), dim3(512), 0, s, partial, nblocks,
+                     ne, out);
+  MDA_LAUNCH_CHECK();
+}
+
 void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
                         const double* var, const double* Z, int k, int64_t p, int mode,
                         double* partial, int nblocks, double* out) {
@@ -416,9 +394,7 @@ void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
 #undef MDA_GG
   MDA_LAUNCH_CHECK();
   if (nb == 1) return;
-  hipLaunchKernelGGL(k_reduce_partials, dim3((k * kq + 63) / 64), dim3(512), 0, s, partial, nb,
-                     k * kq, out);
-  MDA_LAUNCH_CHECK();
+  launch_reduce_partials(s, partial, nb, k * kq, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -559,75 +535,36 @@ void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* 
   MDA_LAUNCH_CHECK();
 }
 
-// ---------------------------------------------------------------------------
-// FP64 MFMA over state points (v_mfma_f64_16x16x4f64, one wavefront per
-// 16 MT points): lane (i16, kk) holds members 4s + kk of point i16 of each
-// tile, the layout of either operand (A[l%16][l/16], B[l/16][l%16]).  Member
-// loads are 128-byte segments.  An ensemble of k members takes NS = k / 4
-// steps, rounded up to a compiled size; the values past k are zero.
-// ---------------------------------------------------------------------------
-// v[t][s] = (x - mean) scale of the tile's points (0 past n and k); mean[t]
-// the mean over the members of point i0 + 16 t + i16
-template <int NS, int MT>
-__device__ __forceinline__ void load_pert(const double* __restrict__ X, int k, int64_t n,
-                                          double scale, int64_t i0, double (&v)[MT][NS],
-                                          double (&mean)[MT]) {
-  const int lane = threadIdx.x & 63, i16 = lane & 15, kk = lane >> 4;
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int64_t i = i0 + 16 * t + i16;
-    double sum = 0.0;
-#pragma unroll
-    for (int s = 0; s < NS; ++s) {
-      const int m = 4 * s + kk;
-      v[t][s] = m < k && i < n ? X[(size_t)m * n + i] : 0.0;
-    }
-#pragma unroll
-    for (int s = 0; s < NS; ++s) sum += v[t][s];
-    sum += __shfl_xor(sum, 16);
-    sum += __shfl_xor(sum, 32);
-    mean[t] = sum * (1.0 / (double)k);
-#pragma unroll
-    for (int s = 0; s < NS; ++s)
-      v[t][s] = 4 * s + kk < k && i < n ? (v[t][s] - mean[t]) * scale : 0.0;
-  }
-}
-
-// the compiled step counts: k <= 16, 32, ..., 128
-#define MDA_MEMBER_STEPS(k, CALL)        \
-  switch (((k) + 15) / 16) {             \
-    case 1: { CALL(4); } break;          \
-    case 2: { CALL(8); } break;          \
-    case 3: { CALL(12); } break;         \
-    case 4: { CALL(16); } break;         \
-    case 5: { CALL(20); } break;         \
-    case 6: { CALL(24); } break;         \
-    case 7: { CALL(28); } break;         \
-    default: { CALL(32); } break;        \
-  }
-
-// [max, min, sum] of nb partial triples, one block, in a fixed order
-__global__ __launch_bounds__(256) void k_fold_minmaxsum(const double* __restrict__ partial,
-                                                        int64_t nb, double* __restrict__ out) {
-  __shared__ double r0[256], r1[256], r2[256];
+// [max, min, sum, sum] of nb partial quadruples, one block, in a fixed order
+__global__ __launch_bounds__(256) void k_fold_extremes(const double* __restrict__ partial,
+                                                       int64_t nb, double* __restrict__ out) {
+  __shared__ double r0[256], r1[256], r2[256], r3[256];
   const int tid = threadIdx.x;
-  double mx = -1.0e308, mn = 1.0e308, ss = 0.0;
+  double mx = -1.0e308, mn = 1.0e308, s2 = 0.0, s3 = 0.0;
+#pragma unroll 4
   for (int64_t b = tid; b < nb; b += 256) {
-    mx = fmax(mx, partial[3 * b]);
-    mn = fmin(mn, partial[3 * b + 1]);
-    ss += partial[3 * b + 2];
+    mx = fmax(mx, partial[4 * b]);
+    mn = fmin(mn, partial[4 * b + 1]);
+    s2 += partial[4 * b + 2];
+    s3 += partial[4 * b + 3];
   }
-  r0[tid] = mx; r1[tid] = mn; r2[tid] = ss;
+  r0[tid] = mx; r1[tid] = mn; r2[tid] = s2; r3[tid] = s3;
   __syncthreads();
   for (int st = 128; st > 0; st >>= 1) {
     if (tid < st) {
       r0[tid] = fmax(r0[tid], r0[tid + st]);
       r1[tid] = fmin(r1[tid], r1[tid + st]);
       r2[tid] += r2[tid + st];
+      r3[tid] += r3[tid + st];
     }
     __syncthreads();
   }
-  if (tid == 0) { out[0] = r0[0]; out[1] = r1[0]; out[2] = r2[0]; }
+  if (tid == 0) { out[0] = r0[0]; out[1] = r1[0]; out[2] = r2[0]; out[3] = r3[0]; }
+}
+
+void launch_fold_extremes(hipStream_t s, const double* partial, int64_t nb, double* out4) {
+  hipLaunchKernelGGL(k_fold_extremes, dim3(1), dim3(256), 0, s, partial, nb, out4);
+  MDA_LAUNCH_CHECK();
 }
 
 // ---------------------------------------------------------------------------
@@ -642,7 +579,7 @@ __global__ __launch_bounds__(256) void k_fold_minmaxsum(const double* __restrict
 // MDA_ST_SKIP_UPDATE); a non-finite background value sets
 // MDA_ST_NONFINITE_STATE (the analysis at that index is then non-finite, as
 // the reference's arithmetic makes it).  With `partial`, each block leaves
-// [-1e308, 1e308, sum of (x_a - mean_a)^2] for the analysis spread
+// [-1e308, 1e308, 0, sum of (x_a - mean_a)^2] for the analysis spread
 // (EnKF.hpp:246-253): sums of the deviations from member 0's increment, which
 // are of the spread's own size.
 // ---------------------------------------------------------------------------
@@ -718,9 +655,11 @@ __global__ __launch_bounds__(TG_THREADS) void k_transform_global(
   if (tid == 0) {
     double t = 0.0;
     for (int w = 0; w < TG_THREADS / 64; ++w) t += red[w];
-    partial[3 * (size_t)blockIdx.x] = -1.0e308;
-    partial[3 * (size_t)blockIdx.x + 1] = 1.0e308;
-    partial[3 * (size_t)blockIdx.x + 2] = t;
+    double* out = partial + 4 * (size_t)blockIdx.x;
+    out[0] = -1.0e308;
+    out[1] = 1.0e308;
+    out[2] = 0.0;
+    out[3] = t;
   }
 }
 
@@ -729,7 +668,7 @@ unsigned transform_global_blocks(int64_t n) {
 }
 
 void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double scale,
-                             const double* T, int* status, double* partial, double* out3) {
+                             const double* T, int* status, double* partial, double* out4) {
   MDA_REQUIRE(k <= 128, "global transform supports k <= 128");
   const unsigned g = transform_global_blocks(n);
 #define MDA_TG(NS)                                                                           \
@@ -738,10 +677,7 @@ void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double 
   MDA_MEMBER_STEPS(k, MDA_TG)
 #undef MDA_TG
   MDA_LAUNCH_CHECK();
-  if (partial) {
-    hipLaunchKernelGGL(k_fold_minmaxsum, dim3(1), dim3(256), 0, s, partial, (int64_t)g, out3);
-    MDA_LAUNCH_CHECK();
-  }
+  if (partial) launch_fold_extremes(s, partial, g, out4);
 }
 
 // ---------------------------------------------------------------------------
@@ -836,10 +772,11 @@ __global__ __launch_bounds__(256) void k_enkf_gain_minmax(const double* __restri
   if (lane == 0) { red[0][wv] = mx; red[1][wv] = mn; red[2][wv] = ss; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    double* out = partial + 3 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x);
+    double* out = partial + 4 * ((size_t)blockIdx.y * gridDim.x + blockIdx.x);
     out[0] = fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3]));
     out[1] = fmin(fmin(red[1][0], red[1][1]), fmin(red[1][2], red[1][3]));
     out[2] = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);
+    out[3] = 0.0;
   }
 }
 
@@ -859,7 +796,7 @@ enkf_gain_shape enkf_gain_plan(int k, int64_t n, int64_t p) {
 void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, double scale,
                              const double* Minv, const double* yp_om, const double* var,
                              int64_t p, const enkf_gain_shape& g, double* Gf, double* partial,
-                             double* out3) {
+                             double* out4) {
   MDA_REQUIRE(k <= 128, "gain diagnostics support k <= 128");
   MDA_REQUIRE(g.nbx < (int64_t)1 << 31 && g.nby < 65536, "gain grid too large");
   hipLaunchKernelGGL(k_enkf_G, dim3(grid_for(g.ntile * g.ns * 64, 256, 4096)), dim3(256), 0, s,
@@ -871,8 +808,7 @@ void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, d
   MDA_MEMBER_STEPS(k, MDA_GAIN)
 #undef MDA_GAIN
   MDA_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_fold_minmaxsum, dim3(1), dim3(256), 0, s, partial, g.nbx * g.nby, out3);
-  MDA_LAUNCH_CHECK();
+  launch_fold_extremes(s, partial, g.nbx * g.nby, out4);
 }
 
 // ---------------------------------------------------------------------------

@@ -14,8 +14,6 @@
 
 namespace mda {
 
-typedef double d4 __attribute__((ext_vector_type(4)));
-
 // ---------------------------------------------------------------------------
 // 1. bucketing
 // ---------------------------------------------------------------------------

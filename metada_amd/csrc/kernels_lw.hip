@@ -17,6 +17,8 @@
 // request, Gaspari & Cohn (1999) eq. (4.10).  The taper and the weighted
 // covariance are evaluated without FMA contraction in the reference's
 // operation order, so S matches the reference's to the last bit up to exp().
+#include <algorithm>
+
 #include "mda_device.hpp"
 #include "mda_internal.hpp"
 
@@ -45,21 +47,31 @@ __device__ inline double lw_taper(double dist, double radius, int fn, int gc_for
   }
 }
 
-// sum over the state of (x_ji - mean_i)^2 per member j: partial[j][blk]
-__global__ __launch_bounds__(256) void k_lw_member_sumsq(const double* __restrict__ X,
-                                                         const double* __restrict__ mean,
+// partial[blk][j] = sum over the block's state points of (x_j - mean)^2, the
+// mean formed in the same pass over X (32 points a wavefront, their members in
+// registers); bound by reading X once.
+template <int NS>
+__global__ __launch_bounds__(256) void k_lw_member_sumsq(const double* __restrict__ X, int k,
                                                          int64_t n, double* __restrict__ partial) {
-  __shared__ double red[256];
-  const int j = blockIdx.y;
-  const double* xj = X + (size_t)j * n;
-  double acc = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    const double v = xj[i] - mean[i];
-    acc += v * v;
+  __shared__ double red[4][NS * 4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i16 = lane & 15, kk = lane >> 4;
+  double ss[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) ss[s] = 0.0;
+  for (int64_t i0 = ((int64_t)blockIdx.x * 4 + wv) * 32; i0 < n; i0 += (int64_t)gridDim.x * 128) {
+    double v[2][NS], mean[2];
+    load_pert<NS, 2>(X, k, n, 1.0, i0, v, mean);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) ss[s] = fma(v[0][s], v[0][s], fma(v[1][s], v[1][s], ss[s]));
   }
-  acc = block_sum(acc, red);
-  if (threadIdx.x == 0) partial[(size_t)j * gridDim.x + blockIdx.x] = acc;
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    for (int off = 1; off < 16; off <<= 1) ss[s] += __shfl_xor(ss[s], off);
+    if (i16 == 0) red[wv][4 * s + kk] = ss[s];
+  }
+  __syncthreads();
+  for (int j = threadIdx.x; j < k; j += 256)
+    partial[(size_t)blockIdx.x * k + j] = (red[0][j] + red[1][j]) + (red[2][j] + red[3][j]);
 }
 
 // chi2_j = sum_b (yo_b - Yb_bj) / r_b * (yo_b - Yb_bj), Yb = ybar + Y'  (:475-500)
@@ -128,235 +140,183 @@ __global__ void k_lw_innovations(const double* __restrict__ yo, const double* __
 }
 
 // ---------------------------------------------------------------------------
-// The gain and update, fused: a workgroup owns LW_TN state points of every
-// member.  Their inflated perturbations stay in LDS; the observations stream
-// through in chunks of LW_TB: the K tile (LW_TN x LW_TB) is formed from the
-// perturbations and G, tapered, folded into the gain extremes, and applied to
-// the chunk of D at once, so K never reaches HBM.  In place on X (every
-// workgroup reads its points before it writes them).
+// The gain and update, fused, on FP64 MFMA.  A wavefront owns 32 state points
+// with all their members in registers and takes 16 observations at a time:
+//   K^T tile  = G^T X'_rho   (rows = observations, columns = points; G
+//               fragments already divided by k - 1), times the taper,
+//   acc      += D^T K^T      (rows = members, columns = points).
+// Row kk + 4r of a product's result sits in register r of lane (i16, kk),
+// which is the right operand of the step over observations 4r .. 4r + 3, so
+// the tapered tile feeds the second product from its registers: K never
+// reaches LDS, and X is read and written once.  The result's members match
+// the fragments of X'_rho lane by lane as well.
+// The taper depends on |s - b| alone: a table of every index distance (one
+// evaluation each, instead of one per state point and observation) is read
+// in windows of p + 32 entries.  Fragments go through two LDS buffers shared
+// by the block's four wavefronts, and they and the tapers are fetched one tile
+// ahead (read where they are used, they left one wavefront per SIMD waiting on
+// L2 and HBM: 20.9 ms).
+// Bound by the FP64 matrix rate (4 n p k FLOP); 30.8 ms at n = 4,194,304,
+// p = 512, k = 64 with 4 x 4 register tiles out of LDS on the vector ALUs,
+// 10.8 ms here (51 TFLOP/s).
 // ---------------------------------------------------------------------------
-constexpr int LW_TN = 64, LW_TB = 32;
-
-template <int KQ>  // members per wave quarter: k <= 4 KQ
-__global__ __launch_bounds__(256) void k_lw_update(
-    double* __restrict__ X, const double* __restrict__ mean, double scale,
-    const double* __restrict__ Gt, const double* __restrict__ D, int k, int64_t n, int64_t p,
-    double radius, int fn, int gc_form, double* __restrict__ mm) {
-  extern __shared__ double sm[];
-  double* xs = sm;                      // [k][LW_TN]   X'_rho
-  double* gs = xs + (size_t)k * LW_TN;  // [k][LW_TB]   G chunk, member-major
-  double* ds = gs + (size_t)k * LW_TB;  // [LW_TB][k]   D chunk
-  double* ks = ds + (size_t)LW_TB * k;  // [LW_TB][LW_TN] K tile
-  __shared__ double red[256];
-  const int tid = threadIdx.x, a = tid & 63, q = tid >> 6;
-  const int64_t s0 = (int64_t)blockIdx.x * LW_TN;
-  const int64_t sa = s0 + a;
-  const bool live = sa < n;
-  const double md = live ? mean[sa] : 0.0;
-  for (int i = q; i < k; i += 4)
-    xs[i * LW_TN + a] = live ? (X[(size_t)i * n + sa] - md) * scale : 0.0;
+// Gf[tile][step][lane] = G[16 tile + i16][4 step + kk] / (k - 1),
+// Df[tile][r][tj][lane] = D[16 tile + 4r + kk][16 tj + i16] (ns = 4 nt steps),
+// tap[m] = taper at index distance m
+__global__ void k_lw_fragments(const double* __restrict__ Gt, const double* __restrict__ D, int k,
+                               int64_t p, int ns, int64_t ntile, int64_t n, int64_t ntap,
+                               double radius, int fn, int gc_form, double* __restrict__ Gf,
+                               double* __restrict__ Df, double* __restrict__ tap) {
+  const int64_t total = ntile * ns * 64;
+  const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x,
+                dt = (int64_t)gridDim.x * blockDim.x;
   const double kden = (double)(k - 1);
+  for (int64_t e = t0; e < total; e += dt) {
+    const int lane = (int)(e & 63), i16 = lane & 15, kk = lane >> 4;
+    const int64_t ot = (e >> 6) / ns;
+    const int st = (int)((e >> 6) % ns), nt = ns / 4;
+    const int64_t og = 16 * ot + i16, od = 16 * ot + 4 * (st / nt) + kk;
+    const int a = 4 * st + kk, m = 16 * (st % nt) + i16;
+    Gf[e] = og < p && a < k ? Gt[(size_t)og * k + a] / kden : 0.0;
+    Df[e] = od < p && m < k ? D[(size_t)od * k + m] : 0.0;
+  }
   const double gdim = (double)(n > p ? n : p);
-  double acc[KQ];
-#pragma unroll
-  for (int t = 0; t < KQ; ++t) acc[t] = 0.0;
-  double kmax = -INFINITY, kmin = INFINITY;
-  for (int64_t b0 = 0; b0 < p; b0 += LW_TB) {
-    const int nb = (int)(p - b0 < LW_TB ? p - b0 : LW_TB);
-    __syncthreads();  // the previous chunk is consumed
-    for (int e = tid; e < LW_TB * k; e += 256) {
-      const int bb = e / k, i = e % k;
-      const bool in = bb < nb;
-      gs[i * LW_TB + bb] = in ? Gt[(size_t)(b0 + bb) * k + i] : 0.0;
-      ds[bb * k + i] = in ? D[(size_t)(b0 + bb) * k + i] : 0.0;
-    }
-    __syncthreads();
-    // K tile: this thread's point a against observations q*8 .. q*8+7
-    double kv[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) kv[t] = 0.0;
-    for (int i = 0; i < k; ++i) {
-      const double xv = xs[i * LW_TN + a];
-      const double* g = gs + i * LW_TB + q * 8;
-#pragma unroll
-      for (int t = 0; t < 8; ++t) kv[t] = fma(xv, g[t], kv[t]);
-    }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-      const int bb = q * 8 + t;
-      double kk = 0.0;
-      if (live && bb < nb) {
-        const int64_t ob = b0 + bb;
-        const double dist = (double)(sa > ob ? sa - ob : ob - sa) / gdim;
-        kk = (kv[t] / kden) * lw_taper(dist, radius, fn, gc_form);
-        kmax = fmax(kmax, kk);
-        kmin = fmin(kmin, kk);
-      }
-      ks[bb * LW_TN + a] = kk;
-    }
-    __syncthreads();
-    // apply: acc[t] += sum_b K(a, b) D(b, q*KQ + t)
-    for (int bb = 0; bb < nb; ++bb) {
-      const double kk = ks[bb * LW_TN + a];
-      const double* dr = ds + bb * k + q * KQ;
-#pragma unroll
-      for (int t = 0; t < KQ; ++t)
-        if (q * KQ + t < k) acc[t] = fma(kk, dr[t], acc[t]);
-    }
-  }
-  if (live) {
-#pragma unroll
-    for (int t = 0; t < KQ; ++t) {
-      const int i = q * KQ + t;
-      if (i < k) X[(size_t)i * n + sa] = md + (xs[i * LW_TN + a] + acc[t]);
-    }
-  }
-  // gain extremes of this workgroup
-  red[tid] = kmax;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) red[tid] = fmax(red[tid], red[tid + s]);
-    __syncthreads();
-  }
-  if (tid == 0) mm[2 * blockIdx.x] = red[0];
-  __syncthreads();
-  red[tid] = kmin;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) red[tid] = fmin(red[tid], red[tid + s]);
-    __syncthreads();
-  }
-  if (tid == 0) mm[2 * blockIdx.x + 1] = red[0];
+  for (int64_t e = t0; e < ntap; e += dt) tap[e] = lw_taper((double)e / gdim, radius, fn, gc_form);
 }
 
-// ---------------------------------------------------------------------------
-// The same gain and update for k <= 64 with register blocking: the two
-// products are K_tile = X'_rho^T G (64 points x 32 observations) and
-// acc += K_tile D (64 points x 64 members), one after the other per chunk of
-// observations, with the taper in between.  Each thread holds a 4 x 2 tile of
-// K and a 4 x 4 tile of the accumulator, so every LDS value it reads feeds
-// two to four FMAs (the one-value-per-FMA LDS broadcast is what bounds the
-// unblocked form).  Members are padded to 64 with zeros.
-//   phase 1: thread (ty, tx) = (tid / 16, tid % 16): points ty + 16 r,
-//            observations tx + 16 t
-//   phase 2: points tx + 16 r, members ty + 16 t (stores coalesce along points)
-// ---------------------------------------------------------------------------
-constexpr int LB_TN = 64, LB_TB = 32, LB_KP = 64;
-
-// K tile entry (observation bb, point a) of the tile buffer: XOR-swizzled
-// within 16-point groups, so the phase-1 stores (16 observations at one
-// point per half-wave) and the phase-2 loads (16 points at one observation)
-// both fall in distinct banks.  80 KB of LDS in all: two workgroups per CU.
-__device__ inline int lb_ps(int bb, int a) { return bb * LB_TN + (a ^ (bb & 15)); }
-
-__global__ __launch_bounds__(256) void k_lw_update_blk(
-    double* __restrict__ X, const double* __restrict__ mean, double scale,
-    const double* __restrict__ Gt, const double* __restrict__ D, int k, int64_t n, int64_t p,
-    double radius, int fn, int gc_form, double* __restrict__ mm) {
-  extern __shared__ double sm[];
-  double* Qs = sm;                          // [LB_KP][LB_TN]  X'_rho, member-major
-  double* Gs = Qs + LB_KP * LB_TN;          // [LB_KP][LB_TB]  G chunk, member-major
-  double* Ds = Gs + LB_KP * LB_TB;          // [LB_TB][LB_KP]  D chunk
-  double* Ps = Ds + LB_TB * LB_KP;          // [LB_TB][LB_TN]  tapered K tile (lb_ps)
-  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  const int64_t s0 = (int64_t)blockIdx.x * LB_TN;
-  for (int e = tid; e < LB_KP * LB_TN; e += 256) {
-    const int i = e / LB_TN, a = e % LB_TN;
-    const int64_t sa = s0 + a;
-    Qs[e] = (i < k && sa < n) ? (X[(size_t)i * n + sa] - mean[sa]) * scale : 0.0;
-  }
-  const double kden = (double)(k - 1);
-  const double gdim = (double)(n > p ? n : p);
-  double acc[4][4];
+template <int NS>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 16 ? 2 : 1)))
+void k_lw_update(double* __restrict__ X, int k, int64_t n, double scale,
+                 const double* __restrict__ Gf, const double* __restrict__ Df,
+                 const double* __restrict__ tap, int64_t p, int64_t ntile,
+                 double* __restrict__ partial) {
+  constexpr int NT = NS / 4;
+  extern __shared__ double sh[];     // two tiles of [Gf | Df]
+  __shared__ double red[4][4];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i16 = lane & 15, kk = lane >> 4;
+  const int64_t i0 = ((int64_t)blockIdx.x * 4 + wv) * 32;
+  double mx = -INFINITY, mn = INFINITY, sb = 0.0, sa = 0.0;
+  double v[2][NS], mean[2];
+  load_pert<NS, 2>(X, k, n, scale, i0, v, mean);
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int t = 0; t < 4; ++t) acc[r][t] = 0.0;
-  double kmax = -INFINITY, kmin = INFINITY;
-  for (int64_t b0 = 0; b0 < p; b0 += LB_TB) {
-    const int nb = (int)(p - b0 < LB_TB ? p - b0 : LB_TB);
-    __syncthreads();  // the previous chunk is consumed (and Qs is complete)
-    for (int e = tid; e < LB_TB * LB_KP; e += 256) {
-      const int bb = e / LB_KP, i = e % LB_KP;
-      const bool in = bb < nb && i < k;
-      const size_t at = (size_t)(b0 + bb) * k + i;
-      Gs[i * LB_TB + bb] = in ? Gt[at] : 0.0;
-      Ds[bb * LB_KP + i] = in ? D[at] : 0.0;
+    for (int s = 0; s < NS; ++s) sb = fma(v[t][s], v[t][s], sb);
+  d4 acc[NT][2];
+#pragma unroll
+  for (int tj = 0; tj < NT; ++tj) acc[tj][0] = acc[tj][1] = d4{0.0, 0.0, 0.0, 0.0};
+  // the next tile's fragments (this thread's share) and tapers, on their way
+  // while a tile is computed
+  double gn[NT], dn[NT];
+  double tn[2][4];
+  auto fetch = [&](int64_t ot) {
+    const double* g = Gf + (size_t)ot * NS * 64 + threadIdx.x;
+    const double* d = Df + (size_t)ot * NS * 64 + threadIdx.x;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      gn[q] = g[256 * q];
+      dn[q] = d[256 * q];
     }
-    __syncthreads();
-    // phase 1: K for points ty + 16 r and observations tx + 16 t
-    double kt[4][2];
+    const int64_t d0 = i0 + i16 - 16 * ot - kk;  // s - b of register 0, tile 0
 #pragma unroll
-    for (int r = 0; r < 4; ++r) kt[r][0] = kt[r][1] = 0.0;
-    for (int i = 0; i < k; ++i) {
-      double q[4], g[2];
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) q[r] = Qs[i * LB_TN + ty + 16 * r];
+      for (int r = 0; r < 4; ++r) {
+        const int64_t m = d0 + 16 * t - 4 * r;
+        tn[t][r] = tap[m < 0 ? -m : m];
+      }
+  };
+  auto stage = [&](int b) {
+    double* g = sh + (size_t)b * 2 * NS * 64 + threadIdx.x;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) g[t] = Gs[i * LB_TB + tx + 16 * t];
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int t = 0; t < 2; ++t) kt[r][t] = fma(q[r], g[t], kt[r][t]);
+    for (int q = 0; q < NT; ++q) {
+      g[256 * q] = gn[q];
+      g[NS * 64 + 256 * q] = dn[q];
     }
+  };
+  fetch(0);
+  stage(0);
+  for (int64_t ot = 0; ot < ntile; ++ot) {
+    const int b = (int)(ot & 1);
+    double tp[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tp[t][r] = tn[t][r];
+    __syncthreads();  // tile ot is in LDS, tile ot - 1 has been read
+    if (ot + 1 < ntile) fetch(ot + 1);
+    const double* gf = sh + (size_t)b * 2 * NS * 64 + lane;
+    const double* df = gf + NS * 64;
+    d4 kt[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const double a = gf[64 * s];
+      kt[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v[0][s], kt[0], 0, 0, 0);
+      kt[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v[1][s], kt[1], 0, 0, 0);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const double kv = kt[t][r] * tp[t][r];
+        kt[t][r] = kv;
+        if (16 * ot + kk + 4 * r < p && i0 + 16 * t + i16 < n) {
+          mx = fmax(mx, kv);
+          mn = fmin(mn, kv);
+        }
+      }
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int a = ty + 16 * r, bb = tx + 16 * t;
-        const int64_t sa = s0 + a, ob = b0 + bb;
-        double kk = 0.0;
-        if (sa < n && bb < nb) {
-          const double dist = (double)(sa > ob ? sa - ob : ob - sa) / gdim;
-          kk = (kt[r][t] / kden) * lw_taper(dist, radius, fn, gc_form);
-          kmax = fmax(kmax, kk);
-          kmin = fmin(kmin, kk);
-        }
-        Ps[lb_ps(bb, a)] = kk;
+      for (int tj = 0; tj < NT; ++tj) {
+        const double a = df[64 * (r * NT + tj)];
+        acc[tj][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, kt[0][r], acc[tj][0], 0, 0, 0);
+        acc[tj][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, kt[1][r], acc[tj][1], 0, 0, 0);
       }
-    __syncthreads();
-    // phase 2: acc += K D for points tx + 16 r and members ty + 16 t
-    for (int bb = 0; bb < nb; ++bb) {
-      double pk[4], dv[4];
+    if (ot + 1 < ntile) stage(b ^ 1);
+  }
+  {
+    // x_a = mean + (x'_rho + K D); the spread from the deviations' distance to
+    // member 0's
 #pragma unroll
-      for (int r = 0; r < 4; ++r) pk[r] = Ps[lb_ps(bb, tx + 16 * r)];
+    for (int t = 0; t < 2; ++t) {
+      const int64_t i = i0 + 16 * t + i16;
+      const double sh = __shfl(v[t][0] + acc[0][t][0], i16);
+      double s1 = 0.0, s2 = 0.0;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) dv[t] = Ds[bb * LB_KP + ty + 16 * t];
+      for (int tj = 0; tj < NT; ++tj)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int t = 0; t < 4; ++t) acc[r][t] = fma(pk[r], dv[t], acc[r][t]);
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * tj + kk + 4 * r;
+          const double dv = v[t][4 * tj + r] + acc[tj][t][r];
+          if (j < k && i < n) {
+            X[(size_t)j * n + i] = mean[t] + dv;
+            s1 += dv - sh;
+            s2 = fma(dv - sh, dv - sh, s2);
+          }
+        }
+      for (int off = 16; off < 64; off <<= 1) {
+        s1 += __shfl_xor(s1, off);
+        s2 += __shfl_xor(s2, off);
+      }
+      if (kk == 0) sa += s2 - s1 * s1 / (double)k;
     }
   }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int a = tx + 16 * r;
-    const int64_t sa = s0 + a;
-    if (sa >= n) continue;
-    const double md = mean[sa];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int m = ty + 16 * t;
-      if (m < k) X[(size_t)m * n + sa] = md + (Qs[m * LB_TN + a] + acc[r][t]);
-    }
+  for (int off = 32; off > 0; off >>= 1) {
+    mx = fmax(mx, __shfl_xor(mx, off));
+    mn = fmin(mn, __shfl_xor(mn, off));
+    sb += __shfl_xor(sb, off);
+    sa += __shfl_xor(sa, off);
   }
-  double* red = Ps;  // the tile buffer is free after the last chunk
+  if (lane == 0) { red[0][wv] = mx; red[1][wv] = mn; red[2][wv] = sb; red[3][wv] = sa; }
   __syncthreads();
-  red[tid] = kmax;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) red[tid] = fmax(red[tid], red[tid + st]);
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    double* out = partial + 4 * (size_t)blockIdx.x;
+    out[0] = fmax(fmax(red[0][0], red[0][1]), fmax(red[0][2], red[0][3]));
+    out[1] = fmin(fmin(red[1][0], red[1][1]), fmin(red[1][2], red[1][3]));
+    out[2] = (red[2][0] + red[2][1]) + (red[2][2] + red[2][3]);
+    out[3] = (red[3][0] + red[3][1]) + (red[3][2] + red[3][3]);
   }
-  if (tid == 0) mm[2 * blockIdx.x] = red[0];
-  __syncthreads();
-  red[tid] = kmin;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (tid < st) red[tid] = fmin(red[tid], red[tid + st]);
-    __syncthreads();
-  }
-  if (tid == 0) mm[2 * blockIdx.x + 1] = red[0];
 }
 
 // any +inf variance (an invalid observation) -> *flag = 1
@@ -369,10 +329,15 @@ __global__ void k_lw_flag_inf(const double* __restrict__ var, int64_t p, int* __
 }
 
 // ---------------------------------------------------------------------------
-void launch_lw_member_sumsq(hipStream_t s, const double* X, const double* mean, int k, int64_t n,
-                            double* partial, int nblocks) {
-  hipLaunchKernelGGL(k_lw_member_sumsq, dim3(nblocks, k), dim3(256), 0, s, X, mean, n, partial);
+void launch_lw_member_sumsq(hipStream_t s, const double* X, int k, int64_t n, double* part,
+                            double* sumsq) {
+  const unsigned nb = grid_for(n, 128, LW_SUMSQ_BLOCKS);
+#define MDA_SS(NS) \
+  hipLaunchKernelGGL(k_lw_member_sumsq<NS>, dim3(nb), dim3(256), 0, s, X, k, n, part)
+  MDA_MEMBER_STEPS(k, MDA_SS)
+#undef MDA_SS
   MDA_LAUNCH_CHECK();
+  launch_reduce_partials(s, part, (int)nb, k, sumsq);
 }
 
 void launch_lw_chi2(hipStream_t s, const double* yo, const double* ybar, const double* yp_om,
@@ -399,35 +364,33 @@ void launch_lw_innovations(hipStream_t s, const double* yo, const double* ybar,
   MDA_LAUNCH_CHECK();
 }
 
-static_assert(LB_TN == LW_TN, "both update forms cover the same points per block");
-size_t lw_update_blocks(int64_t n) { return (size_t)((n + LW_TN - 1) / LW_TN); }
+lw_update_shape lw_update_plan(int k, int64_t n, int64_t p) {
+  lw_update_shape g;
+  g.ns = (k + 15) / 16 * 4;
+  g.ntile = (p + 15) / 16;
+  g.nblk = (n + 127) / 128;
+  g.ntap = (n > p ? n : p) + 64;  // padded points and observations look past the ends
+  return g;
+}
 
-void launch_lw_update(hipStream_t s, double* X, const double* mean, double scale,
-                      const double* Gt, const double* D, int k, int64_t n, int64_t p,
-                      double radius, int fn, int gc_form, double* mm) {
+void launch_lw_update(hipStream_t s, double* X, double scale, const double* Gt, const double* D,
+                      int k, int64_t n, int64_t p, double radius, int fn, int gc_form,
+                      const lw_update_shape& g, double* Gf, double* Df, double* tap,
+                      double* partial, double* out4) {
   MDA_REQUIRE(k >= 2 && k <= 128, "LWEnKF supports 2 <= k <= 128");
-  const unsigned nb = (unsigned)lw_update_blocks(n);
-  if (k <= LB_KP) {
-    const size_t shb = sizeof(double) * ((size_t)LB_KP * LB_TN + (size_t)LB_KP * LB_TB +
-                                         (size_t)LB_TB * LB_KP + (size_t)LB_TB * LB_TN);
-    hipLaunchKernelGGL(k_lw_update_blk, dim3(nb), dim3(256), shb, s, X, mean, scale, Gt, D, k, n,
-                       p, radius, fn, gc_form, mm);
-    MDA_LAUNCH_CHECK();
-    return;
-  }
-  const size_t shm = sizeof(double) * ((size_t)k * LW_TN + (size_t)k * LW_TB +
-                                       (size_t)LW_TB * k + (size_t)LW_TB * LW_TN);
-  if (k <= 32) {
-    hipLaunchKernelGGL(k_lw_update<8>, dim3(nb), dim3(256), shm, s, X, mean, scale, Gt, D, k, n,
-                       p, radius, fn, gc_form, mm);
-  } else if (k <= 64) {
-    hipLaunchKernelGGL(k_lw_update<16>, dim3(nb), dim3(256), shm, s, X, mean, scale, Gt, D, k, n,
-                       p, radius, fn, gc_form, mm);
-  } else {
-    hipLaunchKernelGGL(k_lw_update<32>, dim3(nb), dim3(256), shm, s, X, mean, scale, Gt, D, k, n,
-                       p, radius, fn, gc_form, mm);
-  }
+  MDA_REQUIRE(g.nblk < (int64_t)1 << 31, "LWEnKF state too large");
+  hipLaunchKernelGGL(k_lw_fragments, dim3(grid_for(std::max(g.frag_doubles(), g.ntap), 256, 4096)),
+                     dim3(256), 0, s, Gt, D, k, p, g.ns, g.ntile, n, g.ntap, radius, fn, gc_form,
+                     Gf, Df, tap);
   MDA_LAUNCH_CHECK();
+#define MDA_LU(NS)                                                                            \
+  hipLaunchKernelGGL(k_lw_update<NS>, dim3((unsigned)g.nblk), dim3(256),                     \
+                     sizeof(double) * 4 * NS * 64, s, X, k, n, scale, Gf, Df, tap, p, g.ntile, \
+                     partial)
+  MDA_MEMBER_STEPS(k, MDA_LU)
+#undef MDA_LU
+  MDA_LAUNCH_CHECK();
+  launch_fold_extremes(s, partial, g.nblk, out4);
 }
 
 void launch_lw_flag_inf(hipStream_t s, const double* var, int64_t p, int* flag) {

@@ -61,6 +61,55 @@ __device__ inline float gaspari_cohn_f32(float z) {
          2.f / (3.f * z);
 }
 
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+// ---------------------------------------------------------------------------
+// FP64 MFMA over state points (v_mfma_f64_16x16x4f64, one wavefront per
+// 16 MT points): lane (i16, kk) holds members 4s + kk of point i16 of each
+// tile, the layout of either operand (A[l%16][l/16], B[l/16][l%16]).  Member
+// loads are 128-byte segments.  An ensemble of k members takes NS = k / 4
+// steps, rounded up to a compiled size; the values past k are zero.
+// ---------------------------------------------------------------------------
+// v[t][s] = (x - mean) scale of the tile's points (0 past n and k); mean[t]
+// the mean over the members of point i0 + 16 t + i16
+template <int NS, int MT>
+__device__ __forceinline__ void load_pert(const double* __restrict__ X, int k, int64_t n,
+                                          double scale, int64_t i0, double (&v)[MT][NS],
+                                          double (&mean)[MT]) {
+  const int lane = threadIdx.x & 63, i16 = lane & 15, kk = lane >> 4;
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    const int64_t i = i0 + 16 * t + i16;
+    double sum = 0.0;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int m = 4 * s + kk;
+      v[t][s] = m < k && i < n ? X[(size_t)m * n + i] : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < NS; ++s) sum += v[t][s];
+    sum += __shfl_xor(sum, 16);
+    sum += __shfl_xor(sum, 32);
+    mean[t] = sum * (1.0 / (double)k);
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      v[t][s] = 4 * s + kk < k && i < n ? (v[t][s] - mean[t]) * scale : 0.0;
+  }
+}
+
+// the compiled step counts: k <= 16, 32, ..., 128
+#define MDA_MEMBER_STEPS(k, CALL)        \
+  switch (((k) + 15) / 16) {             \
+    case 1: { CALL(4); } break;          \
+    case 2: { CALL(8); } break;          \
+    case 3: { CALL(12); } break;         \
+    case 4: { CALL(16); } break;         \
+    case 5: { CALL(20); } break;         \
+    case 6: { CALL(24); } break;         \
+    case 7: { CALL(28); } break;         \
+    default: { CALL(32); } break;        \
+  }
+
 // ---------------------------------------------------------------------------
 // workgroup reductions
 // ---------------------------------------------------------------------------

@@ -167,8 +167,6 @@ void launch_mean_pert(hipStream_t s, const double* X, int k, int64_t n, double s
                       double* mean, double* pert);
 void launch_sumsq(hipStream_t s, const double* X, int64_t count, double* partial,
                   int nblocks);
-void launch_dev_sumsq(hipStream_t s, const double* X, int k, int64_t n, double scale,
-                      double* partial, int nblocks);
 // observation space: Y' obs-major [p][k], ybar, d; optional member-major Y'.
 // With `order`, observations are processed in the order order[0], order[1],
 // ...; observation order[t] is written at position t, or at opos[order[t]]
@@ -190,32 +188,37 @@ void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32
 void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
                         const double* var, const double* Z, int k, int64_t p, int mode,
                         double* partial, int nblocks, double* out);
+// out[e] = sum over blocks of partial[block][e], e < ne
+void launch_reduce_partials(hipStream_t s, const double* partial, int nblocks, int ne,
+                            double* out);
+// [max, min, sum, sum] over nb quadruples
+void launch_fold_extremes(hipStream_t s, const double* partial, int64_t nb, double* out4);
 // small dense solves on one workgroup (matrices in LDS)
 void launch_etkf_solve_ws(hipStream_t s, int k, const double* EB, double* T, int* status);
 void launch_enkf_solve_ws(hipStream_t s, int k, const double* EB, const double* F, double* T,
                           double* Minv, int* status);
 // X_a = xbar + scale * X' T for all state points (global T); skipped when
-// the status word holds a MDA_ST_SKIP_UPDATE bit.  With partial (3 doubles per
-// block, transform_global_blocks(n) of them), out3[2] = sum over state and
+// the status word holds a MDA_ST_SKIP_UPDATE bit.  With partial (4 doubles per
+// block, transform_global_blocks(n) of them), out4[3] = sum over state and
 // members of (x_a - mean_a)^2
 unsigned transform_global_blocks(int64_t n);
 void launch_transform_global(hipStream_t s, double* X, int k, int64_t n, double scale,
                              const double* T, int* status, double* partial = nullptr,
-                             double* out3 = nullptr);
+                             double* out4 = nullptr);
 // EnKF diagnostics
 struct enkf_gain_shape {
   int ns;              // MFMA steps over the members
   int64_t ntile, per;  // tiles of 16 observations, tiles per block
   int64_t nbx, nby;    // blocks over state points and over observation tiles
   int64_t gf_doubles() const { return ntile * ns * 64; }
-  int64_t partial_doubles() const { return 3 * nbx * nby; }
+  int64_t partial_doubles() const { return 4 * nbx * nby; }
 };
 enkf_gain_shape enkf_gain_plan(int k, int64_t n, int64_t p);
-// out3 = [max K, min K, sum over state and members of ((x - mean) scale)^2]
+// out4 = [max K, min K, sum over state and members of ((x - mean) scale)^2, 0]
 void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, double scale,
                              const double* Minv, const double* yp_om, const double* var,
                              int64_t p, const enkf_gain_shape& g, double* Gf, double* partial,
-                             double* out3);
+                             double* out4);
 void launch_metrics(hipStream_t s, const double* X, int k, int64_t n, const double* truth,
                     double* partial, int nblocks);
 
@@ -434,8 +437,10 @@ void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* 
                         int64_t* piv, double* pval, int* status);
 
 // LWEnKF (kernels_lw.hip)
-void launch_lw_member_sumsq(hipStream_t s, const double* X, const double* mean, int k, int64_t n,
-                            double* partial, int nblocks);
+// sumsq[j] = sum over the state of (x_j - mean)^2; part: LW_SUMSQ_BLOCKS * k
+constexpr int LW_SUMSQ_BLOCKS = 1024;
+void launch_lw_member_sumsq(hipStream_t s, const double* X, int k, int64_t n, double* part,
+                            double* sumsq);
 void launch_lw_chi2(hipStream_t s, const double* yo, const double* ybar, const double* yp_om,
                     const double* var, int k, int64_t p, double* chi2);
 void launch_lw_form_S(hipStream_t s, const double* yp_om, const double* w, const double* var,
@@ -444,10 +449,20 @@ void launch_lw_form_S(hipStream_t s, const double* yp_om, const double* w, const
 void launch_lw_innovations(hipStream_t s, const double* yo, const double* ybar,
                            const double* yp_om, const double* var, const double* Z, int k,
                            int64_t p, double* D);
-size_t lw_update_blocks(int64_t n);
-void launch_lw_update(hipStream_t s, double* X, const double* mean, double scale,
-                      const double* Gt, const double* D, int k, int64_t n, int64_t p,
-                      double radius, int fn, int gc_form, double* mm);
+// workspace of the fused gain and update: fragments of G and D, the taper of
+// every index distance, per-block partials
+struct lw_update_shape {
+  int ns;                 // MFMA steps over the members
+  int64_t ntile, nblk;    // tiles of 16 observations, blocks of 128 state points
+  int64_t ntap;           // taper table entries
+  int64_t frag_doubles() const { return ntile * ns * 64; }
+};
+lw_update_shape lw_update_plan(int k, int64_t n, int64_t p);
+// out4 = [max K, min K, sum of squares of X'_rho, sum of (x_a - mean_a)^2]
+void launch_lw_update(hipStream_t s, double* X, double scale, const double* Gt, const double* D,
+                      int k, int64_t n, int64_t p, double radius, int fn, int gc_form,
+                      const lw_update_shape& g, double* Gf, double* Df, double* tap,
+                      double* partial, double* out4);
 void launch_lw_flag_inf(hipStream_t s, const double* var, int64_t p, int* flag);
 
 }  // namespace mda

@@ -205,3 +205,31 @@ def test_global_filters_every_p_match_oracle(mda, ctx, orc, k, p):
     D = d[:, None] + np.sqrt(R)[:, None] * Zk - Y.T
     Xp = (X - X.mean(0)) * np.sqrt(g.inflation_factor)
     assert rel_err(ens.data, X.mean(0) + (np.eye(k) + K.T @ D).T @ Xp) < TOL
+
+
+# ---- LWEnKF update: 32 points a wavefront, tiles of 16 observations, members in steps of 16 --
+@pytest.mark.parametrize("k,n,p,fn", [
+    (2, 5, 3, "gaussian"), (16, 31, 16, "cutoff"), (17, 32, 17, "exponential"),
+    (33, 129, 33, "gaussian"), (48, 20, 150, "gaspari_cohn"), (64, 100, 15, "gaussian"),
+    (65, 40, 100, "exponential"), (100, 257, 47, "gaussian"), (128, 33, 65, "gaspari_cohn")])
+def test_lwenkf_update_matches_oracle(mda, ctx, orc, k, n, p, fn):
+    rng = np.random.default_rng(31 * k + n)
+    X, Yb = 2.0 + rng.standard_normal((k, n)), rng.standard_normal((k, p))
+    yo, var = rng.standard_normal(p), rng.uniform(0.5, 2.0, p)
+    Z = rng.standard_normal((p, k))
+    cfg = mda.Config({"analysis": {"inflation": 1.1, "localization_radius": 0.3,
+                                   "localization_function": fn, "weighting_scheme": "adaptive"}})
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    f = mda.LWEnKF(ens, mda.Observation(yo, var, np.zeros(p), np.zeros(p)),
+                   mda.ObsOperator(hx=Yb), cfg, ctx=ctx, gc_form="standard")
+    f.Analyse(Z=Z)
+    Xo, w, d, _ = orc.lwenkf_analyse(X, Yb, yo, var, Z, f.inflation_factor,
+                                     f.localization_radius, fn, "adaptive", gc_standard=True)
+    assert rel_err(ens.data, Xo) < TOL
+    np.testing.assert_allclose(f.weights, w, rtol=1e-12)
+    r = f.getAnalysisResults()
+    for key in ("background_spread", "analysis_spread", "max_kalman_gain", "min_kalman_gain",
+                "innovation_norm", "condition_number"):
+        scale = max(abs(d["max_kalman_gain"]), abs(d["min_kalman_gain"])) \
+            if "gain" in key else abs(d[key])
+        assert abs(r[key] - d[key]) <= 1e-9 * scale, (key, r[key], d[key])
