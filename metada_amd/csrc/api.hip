@@ -876,14 +876,12 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   sa.flag = c->get<int>(pre + "eig_flag", ncol);
   sa.wlist = c->get<int>(pre + "solve_list", ncol);
   sa.wcount = c->get<unsigned>(pre + "solve_count", 1);
-  // Jacobi (fallback, or the Jacobi-only method) beyond the LDS capacity runs
-  // in a global per-block scratch
-  {
-    const int64_t kp = (k + 1) & ~1;
-    if (sizeof(double) * 2 * kp * (kp + 1) > 96 * 1024) {
-      sa.jblocks = 1024;
-      sa.jscratch = c->get<double>(pre + "jac_scratch", (size_t)sa.jblocks * 2 * kp * (kp + 1));
-    }
+  // the Jacobi solve (fallback, or the Jacobi-only method) beyond the LDS
+  // capacity keeps its eigenvectors in a global per-block scratch
+  if (letkf_solve_v_global(k)) {
+    sa.jblocks = 1024;
+    sa.jscratch = c->get<double>(pre + "jac_scratch",
+                                 sa.jblocks * letkf_solve_matrix_bytes(k) / sizeof(double));
   }
   sa.method = P.eig_path ? MDA_EIG_AUTO : MDA_EIG_JACOBI;
   // eigenvalue noise of the Gram relative to ||A||: FP32 products with FP32

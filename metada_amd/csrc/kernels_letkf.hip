@@ -1493,16 +1493,21 @@ __global__ void k_solve_worklist(int64_t ncol, const int* __restrict__ only,
   }
 }
 
-__global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double* gscratch,
-                                                     int use_lds, const int* only,
-                                                     const int* list, const unsigned* cnt) {
+// A and V in LDS while both fit (k <= 96), else A in LDS and V in a global
+// per-block scratch (VG).  NT = 512 threads where a CU holds one block only.
+// At 1,800 columns by Jacobi, against both matrices in global memory beyond
+// k = 76: k = 80 101.7 -> 19.2 ms, k = 100 205.7 -> 132 ms.
+template <int NT, bool VG>
+__global__ __launch_bounds__(NT) void k_letkf_solve(letkf_solve_args a, double* vscratch,
+                                                    const int* only, const int* list,
+                                                    const unsigned* cnt) {
   extern __shared__ double sh[];
-  __shared__ double rc[64], rs[64], red[256], bv[128], yv[128], wb[128];
+  __shared__ double rc[64], rs[64], red[NT], bv[128], yv[128], wb[128];
   __shared__ int rp[64], rq[64], flag;
   const int k = a.k, tid = threadIdx.x, nt = blockDim.x;
   const int kp = (k + 1) & ~1, ld = kp + 1, ks = a.ks;
-  double* A = use_lds ? sh : gscratch + (size_t)blockIdx.x * 2 * kp * ld;
-  double* V = A + kp * ld;
+  double* A = sh;
+  double* V = VG ? vscratch + (size_t)blockIdx.x * kp * ld : sh + kp * ld;
   // fallback mode: the listed columns (flagged, or empty: sqrt(rho) I);
   // otherwise every column
   const int64_t nwork = list ? (int64_t)*cnt : a.ncol;
@@ -1616,17 +1621,23 @@ __global__ __launch_bounds__(256) void k_letkf_solve(letkf_solve_args a, double*
   }
 }
 
+// one matrix of the solve, padded to an even size with an odd row stride
+size_t letkf_solve_matrix_bytes(int k) {
+  const size_t kp = (k + 1) & ~1;
+  return sizeof(double) * kp * (kp + 1);
+}
+// two matrices and the kernel's static arrays within 160 KB: k <= 96
+bool letkf_solve_v_global(int k) { return 2 * letkf_solve_matrix_bytes(k) > 150 * 1024; }
+
 void launch_letkf_solve(hipStream_t s, const letkf_solve_args& a) {
   MDA_REQUIRE(a.k >= 2 && a.k <= 128, "LETKF solve supports 2 <= k <= 128");
-  const int kp = (a.k + 1) & ~1, ld = kp + 1;
-  size_t shm = sizeof(double) * 2 * kp * ld;
-  int use_lds = shm <= 96 * 1024;
+  const size_t mat = letkf_solve_matrix_bytes(a.k);
+  const bool v_global = letkf_solve_v_global(a.k);
+  const size_t shm = v_global ? mat : 2 * mat;
   unsigned nb = (unsigned)(a.ncol < 65536 ? a.ncol : 65536);
   if (nb < 1) nb = 1;
-  double* gscratch = nullptr;
-  if (!use_lds) {  // A and V in a global per-block scratch
+  if (v_global) {
     MDA_REQUIRE(a.jscratch && a.jblocks > 0, "Jacobi scratch missing");
-    gscratch = a.jscratch;
     if (nb > (unsigned)a.jblocks) nb = (unsigned)a.jblocks;
   }
   const int* only = nullptr;
@@ -1648,8 +1659,16 @@ void launch_letkf_solve(hipStream_t s, const letkf_solve_args& a) {
       cnt = a.wcount;
     }
   }
-  hipLaunchKernelGGL(k_letkf_solve, dim3(nb), dim3(256), use_lds ? shm : 0, s, a, gscratch,
-                     use_lds, only, list, cnt);
+  // more than half of a CU's LDS: one block per CU, of 512 threads
+  if (v_global)
+    hipLaunchKernelGGL((k_letkf_solve<512, true>), dim3(nb), dim3(512), shm, s, a, a.jscratch,
+                       only, list, cnt);
+  else if (shm > 72 * 1024)
+    hipLaunchKernelGGL((k_letkf_solve<512, false>), dim3(nb), dim3(512), shm, s, a, nullptr, only,
+                       list, cnt);
+  else
+    hipLaunchKernelGGL((k_letkf_solve<256, false>), dim3(nb), dim3(256), shm, s, a, nullptr, only,
+                       list, cnt);
   MDA_LAUNCH_CHECK();
 }
 

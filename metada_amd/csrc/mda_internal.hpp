@@ -342,8 +342,8 @@ struct letkf_solve_args {
   double* lam;   // [ncol][ks]
   double* U;     // [ncol][ks][ks] Householder reflectors
   int* flag;     // [ncol] columns re-solved by the Jacobi fallback
-  // Jacobi in global memory (k too large for LDS): per-block scratch of
-  // 2 kp (kp + 1) doubles for jblocks blocks
+  // Jacobi whose two matrices exceed the LDS (letkf_solve_v_global): one in a
+  // global scratch of letkf_solve_matrix_bytes(k) for each of jblocks blocks
   double* jscratch;
   int jblocks;
   // fallback work list [ncol] and its length (set: only the flagged and empty
@@ -371,6 +371,8 @@ struct letkf_solve_args {
 // true when the tridiagonal eigensolver of block size ks can apply the
 // transform itself
 bool letkf_eig_fusable(int ks);
+size_t letkf_solve_matrix_bytes(int k);
+bool letkf_solve_v_global(int k);
 void launch_letkf_solve(hipStream_t s, const letkf_solve_args& a);
 // block size of the tridiagonal eigensolver for k members: the smallest
 // compiled size >= k
