@@ -1428,15 +1428,11 @@ int mda_ensemble_metrics(mda_ctx* c, const mda_ensemble* ens, const double* trut
     MDA_REQUIRE(truth && out, "truth and out are required");
     dev_ensemble de = stage_ensemble(c, ens);
     const double* t = to_device(c, "truth", truth, de.n, truth_on_device != 0);
-    const int nb = 512;
-    double* part = c->get<double>("metrics_part", (size_t)nb * 9);
-    launch_metrics(c->stream, de.X, de.k, de.n, t, part, nb);
-    std::vector<double> h((size_t)nb * 9);
-    d2h(c, h.data(), part, sizeof(double) * nb * 9);
-    MDA_HIP(hipStreamSynchronize(c->stream));
+    double* part = c->get<double>("metrics_part", (size_t)METRICS_BLOCKS * 9);
+    double* out9 = c->get<double>("metrics_out", 9);
+    launch_metrics(c->stream, de.X, de.k, de.n, t, part, out9);
     double a[9] = {0};
-    for (int b = 0; b < nb; ++b)
-      for (int q = 0; q < 9; ++q) a[q] += h[(size_t)b * 9 + q];
+    d2h(c, a, out9, sizeof(a));
     const double nn = (double)de.n;
     out->rmse = std::sqrt(a[0] / nn);
     out->bias = a[1] / nn;

@@ -219,8 +219,10 @@ void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, d
                              const double* Minv, const double* yp_om, const double* var,
                              int64_t p, const enkf_gain_shape& g, double* Gf, double* partial,
                              double* out4);
+// the nine sums of Metrics::CalculateAll; partial: 9 METRICS_BLOCKS doubles
+constexpr int METRICS_BLOCKS = 2048;
 void launch_metrics(hipStream_t s, const double* X, int k, int64_t n, const double* truth,
-                    double* partial, int nblocks);
+                    double* partial, double* out9);
 
 // LETKF
 struct bucket_grid {

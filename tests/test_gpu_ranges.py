@@ -233,3 +233,19 @@ def test_lwenkf_update_matches_oracle(mda, ctx, orc, k, n, p, fn):
         scale = max(abs(d["max_kalman_gain"]), abs(d["min_kalman_gain"])) \
             if "gain" in key else abs(d[key])
         assert abs(r[key] - d[key]) <= 1e-9 * scale, (key, r[key], d[key])
+
+
+# ---- verification scores: members held in registers, and the general form beyond 128 --------
+@pytest.mark.parametrize("k,n", [(2, 1), (7, 300), (8, 255), (9, 257), (40, 1000), (41, 64),
+                                 (63, 500), (65, 33), (97, 100), (128, 270), (129, 50)])
+def test_metrics_every_k(mda, ctx, k, n):
+    rng = np.random.default_rng(k + n)
+    X, t = 280.0 + rng.standard_normal((k, n)), 280.0 + rng.standard_normal(n)
+    m = mda.metrics(mda.Ensemble(X, n, 1, 1), t, ctx=ctx)
+    mean = X.mean(0)
+    crps = (np.abs(X - t).mean(0) -
+            np.abs(X[:, None] - X[None]).sum((0, 1)) / (2.0 * k * k)).mean()
+    # values near 280 with unit spread: 280 eps per difference, k terms
+    for key, want in (("crps", crps), ("avg_spread", X.std(0, ddof=1).mean()),
+                      ("bias", (mean - t).mean()), ("rmse", np.sqrt(((mean - t) ** 2).mean()))):
+        assert abs(m[key] - want) < 1e-12 * max(1.0, k / 8), key
