@@ -249,3 +249,26 @@ def test_metrics_every_k(mda, ctx, k, n):
     for key, want in (("crps", crps), ("avg_spread", X.std(0, ddof=1).mean()),
                       ("bias", (mean - t).mean()), ("rmse", np.sqrt(((mean - t) ** 2).mean()))):
         assert abs(m[key] - want) < 1e-12 * max(1.0, k / 8), key
+
+
+# ---- MLP: 16 samples a wavefront step, 64 a block, up to 256 (gradient) / 1024 blocks -------
+@pytest.mark.parametrize("m", [1, 15, 17, 63, 64, 65, 1023, 16385, 70001])
+def test_mlp_every_m_matches_oracle(mda, ctx, orc, m):
+    import ctypes as C
+    rng = np.random.default_rng(m)
+    p = np.concatenate([rng.standard_normal(512) * 0.35, rng.standard_normal(64) * 0.1,
+                        rng.standard_normal(4096) * 0.12, rng.standard_normal(64) * 0.1,
+                        rng.standard_normal(64) * 0.2, [-1.0]]).astype(np.float32)
+    feat = rng.standard_normal((m, 8)).astype(np.float32)
+    target = (1.0 + rng.random(m)).astype(np.float32)
+    rho, grad, loss = np.empty(m, np.float32), np.empty_like(p), C.c_double()
+    ctx.check(ctx.lib.mda_mlp_forward(ctx.h, p.ctypes.data, feat.ctypes.data, m,
+                                      rho.ctypes.data, 0))
+    ctx.check(ctx.lib.mda_mlp_loss_grad(ctx.h, p.ctypes.data, feat.ctypes.data,
+                                        target.ctypes.data, m, C.byref(loss), grad.ctypes.data, 0))
+    p64, f64 = p.astype(np.float64), feat.astype(np.float64)
+    # FP32 sums of 64 terms, twice: 64 eps at most on values of order one
+    np.testing.assert_allclose(rho, orc.mlp_forward(p64, f64), rtol=64 * 6e-8)
+    lo, go = orc.mlp_loss_grad(p64, f64, target.astype(np.float64))
+    assert abs(loss.value - lo) <= 128 * 6e-8 * max(lo, 1e-3)
+    assert np.linalg.norm(grad - go) <= 128 * 6e-8 * np.linalg.norm(go)
