@@ -706,6 +706,8 @@ struct letkf_plan {
   int64_t chist_cap = 0;
 };
 
+static int64_t n_passes(const letkf_plan& P) { return (P.ncol + P.chunk - 1) / P.chunk; }
+
 static void check_letkf_params(const mda_letkf_params* prm, const mda_geometry* geom) {
   MDA_REQUIRE(prm && geom, "params and geometry are required");
   MDA_REQUIRE(std::isfinite(prm->inflation) && prm->inflation > 0.0, "inflation must be > 0");
@@ -849,7 +851,7 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   if (geom->coord == MDA_COORD_GEOGRAPHIC) {
     ga.shell_cap = std::max<int64_t>(65536, 4 * nck);
     ga.shell = c->get<int4>(pre + "shell_list", (size_t)ga.shell_cap);
-    ga.shell_count = c->get<uint32_t>(pre + "shell_count", 1);
+    ga.shell_count = c->get<uint32_t>(pre + "shell_count", (ncol + nck - 1) / nck);
   }
   P.queue = queue;
   if (queue) {
@@ -875,7 +877,7 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   sa.U = P.eig_path ? c->get<double>(pre + "eig_U", (size_t)nck * ks * ks) : nullptr;
   sa.flag = c->get<int>(pre + "eig_flag", ncol);
   sa.wlist = c->get<int>(pre + "solve_list", ncol);
-  sa.wcount = c->get<unsigned>(pre + "solve_count", 1);
+  sa.wcount = c->get<unsigned>(pre + "solve_count", (ncol + nck - 1) / nck);
   // the Jacobi solve (fallback, or the Jacobi-only method) beyond the LDS
   // capacity keeps its eigenvectors in a global per-block scratch
   if (letkf_solve_v_global(k)) {
@@ -915,18 +917,35 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
 // its rows are moved into bucket order afterwards.  Both idempotent.
 static void enqueue_buckets(hipStream_t s, letkf_plan& P) {
   letkf_gram_args& ga = P.ga;
-  // the analysis's status word, then the observations' validity
-  launch_zero(s, P.sa.status, sizeof(int));
-  launch_check_obs(s, P.o, P.sa.status);
+  letkf_begin_args b{};
+  b.ncol = P.ncol; b.npass = n_passes(P);
+  b.status = P.sa.status; b.sweeps = P.sweeps; b.flag = P.sa.flag;
+  b.nloc = P.p == 0 ? ga.nloc : nullptr;
+  b.stats = P.stats; b.wcount = P.sa.wcount; b.shell_count = ga.shell_count;
+  launch_letkf_begin(s, b);
   if (P.p == 0) return;  // every column takes the empty-column branch
-  launch_bucket_keys(s, P.rcoord, P.ccoord, P.p, P.bg, P.keys, P.vals);
-  radix_sort_pairs(s, P.keys, P.vals, P.keys2, P.vals2, P.p, P.key_bits, P.hist, P.hist_cap);
+  obs_prepare_args q{};
+  q.p = P.p; q.nxy = P.nx * P.ny;
+  q.yo = P.o.yo; q.var = P.o.var; q.rcoord = P.rcoord; q.ccoord = P.ccoord;
+  q.grid = P.bg; q.keys = P.keys; q.vals = P.vals;
+  q.row_ptr = P.h.row_ptr; q.col = P.h.col; q.tkeys = P.tkeys; q.tvals = P.tvals;
+  q.status = P.sa.status;
+  launch_obs_prepare(s, q);
+  if (P.p <= SORT_SMALL) {
+    const sort_job jobs[2] = {{P.keys, P.vals, P.key_bits}, {P.tkeys, P.tvals, P.tap_bits}};
+    launch_sort_small(s, jobs, P.tkeys ? 2 : 1, P.p);
+  } else {
+    radix_sort_pairs(s, P.keys, P.vals, P.keys2, P.vals2, P.p, P.key_bits, P.hist, P.hist_cap);
+    if (P.tkeys)
+      radix_sort_pairs(s, P.tkeys, P.tvals, P.keys2, P.vals2, P.p, P.tap_bits, P.hist,
+                       P.hist_cap);
+  }
   launch_bucket_ranges(s, P.keys, P.p, P.nbuckets, P.bstart);
   launch_gather_obs(s, P.vals, P.p, P.o.var, P.o.a, P.o.b, P.o.c, P.prm->rweight,
                     const_cast<double*>(ga.rinv), const_cast<double*>(ga.oa),
                     const_cast<double*>(ga.ob), const_cast<double*>(ga.oc),
                     const_cast<double*>(ga.ux), const_cast<double*>(ga.uy),
-                    const_cast<double*>(ga.uz));
+                    const_cast<double*>(ga.uz), P.ipos);
   // window geometry of every column for the Gram
   launch_column_setup(s, ga);
 }
@@ -944,10 +963,6 @@ static void enqueue_local(hipStream_t s, letkf_plan& P) {
   } else if (P.tkeys) {
     // in the order of the first stencil tap (neighbouring state gathers),
     // each observation's rows written at its bucket position
-    launch_tap_keys(s, P.h.row_ptr, P.h.col, P.p, P.nx * P.ny, P.tkeys, P.tvals);
-    radix_sort_pairs(s, P.tkeys, P.tvals, P.keys2, P.vals2, P.p, P.tap_bits, P.hist,
-                     P.hist_cap);
-    launch_invert_order(s, P.vals, P.p, P.ipos);
     launch_obs_stats(s, P.de.X, P.k, P.n, P.p, P.h.row_ptr, P.h.col, P.h.w, nullptr, P.o.yo,
                      nullptr, const_cast<double*>(ga.yp), const_cast<double*>(ga.d), nullptr,
                      P.tvals, y32, P.ipos, st);
@@ -985,6 +1000,7 @@ static letkf_solve_args solve_pass(const letkf_plan& P, int64_t c0, int64_t nc) 
   sa.lam += c0 * P.ks;
   if (sa.eig_nloc) sa.eig_nloc += c0;
   sa.flag += c0;
+  sa.wcount += c0 / P.chunk;
   sa.X = P.de.X;
   sa.x_ncol = P.ncol;
   sa.x_nlev = P.nlev;
@@ -1006,7 +1022,7 @@ static void enqueue_gram(hipStream_t s, letkf_plan& P, int64_t c0, int64_t nc, i
     ga.order = P.ccols;  // the sort leaves the ordered pairs in the first arrays
     ga.queue = P.qcount;
   }
-  if (ga.shell_count) launch_zero(s, ga.shell_count, sizeof(uint32_t));
+  if (ga.shell_count) ga.shell_count += c0 / P.chunk;  // cleared by enqueue_buckets
   launch_letkf_gram(s, ga);
   launch_letkf_shell_fixup(s, ga, P.sa.status);
 }
@@ -1021,8 +1037,6 @@ struct pass_marks {
 // receives one set of events per pass.
 static void enqueue_columns(hipStream_t s, letkf_plan& P, std::pair<int, int> cfg,
                             const std::vector<pass_marks>* marks) {
-  launch_zero(s, P.sweeps, sizeof(int) * P.ncol);
-  if (P.p == 0) launch_zero(s, P.ga.nloc, sizeof(int) * P.ncol);
   int pass = 0;
   for (int64_t c0 = 0; c0 < P.ncol; c0 += P.chunk, ++pass) {
     const int64_t nc = std::min(P.chunk, P.ncol - c0);
@@ -1041,13 +1055,8 @@ static void enqueue_columns(hipStream_t s, letkf_plan& P, std::pair<int, int> cf
   }
 }
 
-static int64_t n_passes(const letkf_plan& P) { return (P.ncol + P.chunk - 1) / P.chunk; }
-
 static void enqueue_stats(hipStream_t s, letkf_plan& P) {
-  launch_zero(s, P.stats, sizeof(int64_t) * 9);
-  launch_reduce_int(s, P.ga.nloc, P.ncol, P.stats, nullptr);
-  launch_reduce_int(s, P.sweeps, P.ncol, P.stats + 3, nullptr);
-  if (P.eig_path) launch_reduce_int(s, P.sa.flag, P.ncol, P.stats + 6, nullptr);
+  launch_reduce_int(s, P.ga.nloc, P.sweeps, P.eig_path ? P.sa.flag : nullptr, P.ncol, P.stats);
 }
 
 static void finish_letkf(mda_ctx* c, letkf_plan& P, mda_letkf_diag* diag) {
@@ -1151,8 +1160,11 @@ static std::pair<int, int> autotune_gram(mda_ctx* c, letkf_plan& P, bool allow_q
       // timed on the first pass of columns
       const int64_t nc = std::min(P.chunk, P.ncol);
       enqueue_gram(s, P, 0, nc, nb, q != 0);  // warm
+      // each Gram appends to the boundary list of its pass
+      if (P.ga.shell_count) launch_zero(s, P.ga.shell_count, sizeof(uint32_t));
       MDA_HIP(hipEventRecord(c->ev[10], s));
       enqueue_gram(s, P, 0, nc, nb, q != 0);
+      if (P.ga.shell_count) launch_zero(s, P.ga.shell_count, sizeof(uint32_t));
       MDA_HIP(hipEventRecord(c->ev[11], s));
       MDA_HIP(hipEventSynchronize(c->ev[11]));
       const float ms = elapsed(c->ev[10], c->ev[11]);

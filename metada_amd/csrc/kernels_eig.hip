@@ -1782,9 +1782,7 @@ void launch_letkf_eig(hipStream_t s, const letkf_solve_args& a, double* de, doub
     hipLaunchKernelGGL(k_eig_select, dim3(grid_for(a.ncol, 256, 4096)), dim3(256), 0, s, a.ncol,
                        a.k, a.nloc, a.eig_nloc, flag);
     MDA_LAUNCH_CHECK();
-  } else {
-    launch_zero(s, flag, sizeof(int) * a.ncol);
-  }
+  }  // otherwise the flags are clear (letkf_begin_args)
   switch (a.ks) {
     case 8: launch_eig_n<8>(s, a, de, lam, flag); break;
     case 16: launch_eig_n<16>(s, a, de, lam, flag); break;

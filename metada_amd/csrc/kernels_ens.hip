@@ -195,48 +195,6 @@ void launch_obs_stats(hipStream_t s, const double* X, int k, int64_t n, int64_t 
   MDA_LAUNCH_CHECK();
 }
 
-// Processing order of the observation statistics: key = grid index of the
-// first stencil tap (0 for an empty stencil), value = observation index.
-__global__ void k_tap_keys(const int64_t* __restrict__ row_ptr, const int64_t* __restrict__ col,
-                           int64_t p, int64_t nxy, uint32_t* __restrict__ keys,
-                           uint32_t* __restrict__ vals) {
-  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < p;
-       o += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t t0 = row_ptr[o];
-    const int64_t c = t0 < row_ptr[o + 1] ? col[t0] : 0;
-    // groups of four levels share one key range: the observations of those
-    // levels in one grid row sort together, and a stencil's upper level is
-    // the next observation's lower one (measured: groups of 1, 2, 4, 8
-    // levels take 3.9, 3.5, 3.3, 3.4 ms at 1e6 observations, k = 64)
-    const int64_t lev = c / nxy;
-    keys[o] = (uint32_t)((lev >> 2) * nxy + (c - lev * nxy));
-    vals[o] = (uint32_t)o;
-  }
-}
-
-void launch_tap_keys(hipStream_t s, const int64_t* row_ptr, const int64_t* col, int64_t p,
-                     int64_t nxy, uint32_t* keys, uint32_t* vals) {
-  if (p <= 0) return;
-  hipLaunchKernelGGL(k_tap_keys, dim3(grid_for(p, 256, 65536)), dim3(256), 0, s, row_ptr, col,
-                     p, nxy, keys, vals);
-  MDA_LAUNCH_CHECK();
-}
-
-// ipos[order[t]] = t
-__global__ void k_invert_order(const uint32_t* __restrict__ order, int64_t p,
-                               uint32_t* __restrict__ ipos) {
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < p;
-       t += (int64_t)gridDim.x * blockDim.x)
-    ipos[order[t]] = (uint32_t)t;
-}
-
-void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32_t* ipos) {
-  if (p <= 0) return;
-  hipLaunchKernelGGL(k_invert_order, dim3(grid_for(p, 256, 65536)), dim3(256), 0, s, order, p,
-                     ipos);
-  MDA_LAUNCH_CHECK();
-}
-
 // ---------------------------------------------------------------------------
 // Global Gram over all observations (ETKF.hpp:150-155; EnKF via Woodbury):
 //   mode 0: G[a][c] = sum_o Y'[o][a] Y'[o][c] / var_o (c < k), and

@@ -7,6 +7,8 @@
 //   3. per-column k x k solve: parallel Jacobi (symmetric square root) or
 //      Cholesky (reference square root) -> transform T_g;
 //   4. X_a = xbar + X' T_g for every level of the column.
+#include <algorithm>
+
 #include "mda_crmath.hpp"
 #include "mda_device.hpp"
 #include "mda_internal.hpp"
@@ -31,43 +33,171 @@ __device__ inline uint32_t bucket_of(const bucket_grid& g, double r, double c) {
   return (uint32_t)row * (uint32_t)g.ncolb + (uint32_t)col;
 }
 
-// rcoord: latitude (GEOGRAPHIC) or y; ccoord: longitude or x
-__global__ void k_bucket_keys(const double* __restrict__ rcoord,
-                              const double* __restrict__ ccoord, int64_t p, bucket_grid g,
-                              uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < p;
+// Clears what an analysis accumulates into: one launch instead of one per
+// array (a small analysis is bound by its launches).
+__global__ void k_letkf_begin(letkf_begin_args a) {
+  const int64_t t0 = blockIdx.x * (int64_t)blockDim.x + threadIdx.x,
+                dt = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t g = t0; g < a.ncol; g += dt) {
+    a.sweeps[g] = 0;
+    a.flag[g] = 0;
+    if (a.nloc) a.nloc[g] = 0;
+  }
+  for (int64_t i = t0; i < a.npass; i += dt) {
+    a.wcount[i] = 0u;
+    if (a.shell_count) a.shell_count[i] = 0u;
+  }
+  if (t0 < 9) a.stats[t0] = 0;
+  if (t0 == 0) *a.status = 0;
+}
+
+void launch_letkf_begin(hipStream_t s, const letkf_begin_args& a) {
+  hipLaunchKernelGGL(k_letkf_begin, dim3(grid_for(std::max(a.ncol, a.npass), 256, 4096)),
+                     dim3(256), 0, s, a);
+  MDA_LAUNCH_CHECK();
+}
+
+// One pass over the observations before they are sorted: validity (values
+// finite, variances > 0 with +inf marking an invalid observation,
+// GridObservation.hpp:239-252; a violation sets MDA_ST_NONFINITE_OBS), bucket
+// key, and with a stencil H (tkeys) the key of its first tap for the
+// processing order of the observation statistics (0 for an empty stencil).
+__global__ void k_obs_prepare(obs_prepare_args a) {
+  bool bad = false;
+  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < a.p;
        o += (int64_t)gridDim.x * blockDim.x) {
-    keys[o] = bucket_of(g, rcoord[o], ccoord[o]);
-    vals[o] = (uint32_t)o;
+    bad = bad || !isfinite(a.yo[o]) || !(a.var[o] > 0.0);
+    a.keys[o] = bucket_of(a.grid, a.rcoord[o], a.ccoord[o]);
+    a.vals[o] = (uint32_t)o;
+    if (a.tkeys) {
+      const int64_t t0 = a.row_ptr[o];
+      const int64_t c = t0 < a.row_ptr[o + 1] ? a.col[t0] : 0;
+      // groups of four levels share one key range: the observations of those
+      // levels in one grid row sort together, and a stencil's upper level is
+      // the next observation's lower one (measured: groups of 1, 2, 4, 8
+      // levels take 3.9, 3.5, 3.3, 3.4 ms at 1e6 observations, k = 64)
+      const int64_t lev = c / a.nxy;
+      a.tkeys[o] = (uint32_t)((lev >> 2) * a.nxy + (c - lev * a.nxy));
+      a.tvals[o] = (uint32_t)o;
+    }
+  }
+  if (__ballot(bad) != 0ull && (threadIdx.x & 63) == 0) atomicOr(a.status, MDA_ST_NONFINITE_OBS);
+}
+
+void launch_obs_prepare(hipStream_t s, const obs_prepare_args& a) {
+  if (a.p <= 0) return;
+  hipLaunchKernelGGL(k_obs_prepare, dim3(grid_for(a.p, 256, 8192)), dim3(256), 0, s, a);
+  MDA_LAUNCH_CHECK();
+}
+
+// The sort below for up to SORT_SMALL pairs in one launch: a workgroup per
+// job keeps keys and values in LDS through all passes.  The three launches of
+// each pass of the large form cost more than their work here: a Lorenz-96
+// cycle of 2,000 observations spent 77 us of kernel time and fifteen launches
+// on its two sorts.
+__global__ __launch_bounds__(1024) void k_sort_small(sort_job j0, sort_job j1, int p) {
+  extern __shared__ uint32_t buf[];  // keys, values, twice [SORT_SMALL]
+  __shared__ uint32_t wcnt[16][256];
+  __shared__ uint32_t run[256], wtot[4];
+  const sort_job job = blockIdx.x ? j1 : j0;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  uint32_t *k0 = buf, *v0 = buf + SORT_SMALL, *k1 = buf + 2 * SORT_SMALL,
+           *v1 = buf + 3 * SORT_SMALL;
+  for (int i = tid; i < p; i += 1024) {
+    k0[i] = job.keys[i];
+    v0[i] = job.vals[i];
+  }
+  const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
+  for (int shift = 0; shift < job.bits; shift += 8) {
+    if (tid < 256) run[tid] = 0u;
+    __syncthreads();
+    for (int i = tid; i < p; i += 1024) atomicAdd(&run[(k0[i] >> shift) & 255u], 1u);
+    __syncthreads();
+    // exclusive scan of the 256 digit counts
+    uint32_t c = 0u, sc = 0u;
+    if (tid < 256) {
+      c = run[tid];
+      sc = c;
+      for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t u = __shfl_up(sc, off);
+        if (lane >= off) sc += u;
+      }
+      if (lane == 63) wtot[wv] = sc;
+    }
+    __syncthreads();
+    if (tid < 256) {
+      uint32_t b = 0u;
+      for (int w = 0; w < wv; ++w) b += wtot[w];
+      run[tid] = b + sc - c;
+    }
+    for (int s0 = 0; s0 < p; s0 += 1024) {
+      for (int e = tid; e < 16 * 256; e += 1024) (&wcnt[0][0])[e] = 0u;
+      __syncthreads();
+      const int i = s0 + tid;
+      const bool valid = i < p;
+      const uint32_t key = valid ? k0[i] : 0u, val = valid ? v0[i] : 0u;
+      const uint32_t dig = (key >> shift) & 255u;
+      uint64_t match = __ballot(valid);
+      for (int b = 0; b < 8; ++b) {
+        const uint64_t m = __ballot(valid && ((dig >> b) & 1u));
+        match &= ((dig >> b) & 1u) ? m : ~m;
+      }
+      const uint32_t rank = (uint32_t)__popcll(match & below);
+      if (valid && rank == 0) wcnt[wv][dig] = (uint32_t)__popcll(match);
+      __syncthreads();
+      if (tid < 256) {  // running positions per digit, wavefront by wavefront
+        uint32_t r = run[tid];
+        for (int w = 0; w < 16; ++w) {
+          const uint32_t n = wcnt[w][tid];
+          wcnt[w][tid] = r;
+          r += n;
+        }
+        run[tid] = r;
+      }
+      __syncthreads();
+      if (valid) {
+        const uint32_t dst = wcnt[wv][dig] + rank;
+        k1[dst] = key;
+        v1[dst] = val;
+      }
+      __syncthreads();
+    }
+    uint32_t* t = k0; k0 = k1; k1 = t;
+    t = v0; v0 = v1; v1 = t;
+  }
+  for (int i = tid; i < p; i += 1024) {
+    job.keys[i] = k0[i];
+    job.vals[i] = v0[i];
   }
 }
 
-void launch_bucket_keys(hipStream_t s, const double* rcoord, const double* ccoord, int64_t p,
-                        bucket_grid g, uint32_t* keys, uint32_t* vals) {
-  hipLaunchKernelGGL(k_bucket_keys, dim3(grid_for(p, 256, 8192)), dim3(256), 0, s, rcoord,
-                     ccoord, p, g, keys, vals);
+void launch_sort_small(hipStream_t s, const sort_job* jobs, int njobs, int64_t p) {
+  MDA_REQUIRE(njobs >= 1 && njobs <= 2 && p <= SORT_SMALL, "small sort size out of range");
+  if (p <= 0) return;
+  hipLaunchKernelGGL(k_sort_small, dim3(njobs), dim3(1024), sizeof(uint32_t) * 4 * SORT_SMALL, s,
+                     jobs[0], jobs[njobs - 1], (int)p);
   MDA_LAUNCH_CHECK();
 }
 
 // Stable LSD radix sort of (key, value) pairs, 8-bit digits.  A block owns
-// RS_TILE consecutive keys (RS_KPT sub-tiles of RS_BLOCK).  Per pass: block
+// kpt sub-tiles of RS_BLOCK consecutive keys: 16, or 4 below 262,144 keys, where
+// 16 would leave most CUs without a block (40,000 keys: 23 us a pass with ten
+// blocks) and the scan stays short.  Per pass: block
 // digit histograms (digit-major), one exclusive scan, stable scatter with
 // in-wave ranks from ballots and per-digit running counts across the
 // block's sub-tiles.  Deterministic.
 constexpr int RS_BLOCK = 256;
-constexpr int RS_KPT = 16;
-constexpr int RS_TILE = RS_BLOCK * RS_KPT;
 
 __global__ __launch_bounds__(RS_BLOCK) void k_rs_hist(const uint32_t* __restrict__ keys,
-                                                      int64_t p, int shift,
+                                                      int64_t p, int shift, int kpt,
                                                       uint32_t* __restrict__ hist,
                                                       int64_t nblocks) {
   __shared__ uint32_t cnt[256];
   cnt[threadIdx.x] = 0;
   __syncthreads();
-  const int64_t base = blockIdx.x * (int64_t)RS_TILE + threadIdx.x;
-#pragma unroll
-  for (int st = 0; st < RS_KPT; ++st) {
+  const int64_t base = blockIdx.x * (int64_t)(RS_BLOCK * kpt) + threadIdx.x;
+#pragma unroll 4
+  for (int st = 0; st < kpt; ++st) {
     const int64_t i = base + (int64_t)st * RS_BLOCK;
     if (i < p) atomicAdd(&cnt[(keys[i] >> shift) & 255u], 1u);
   }
@@ -76,44 +206,63 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_hist(const uint32_t* __restrict
 }
 
 // exclusive scan of `total` uint32 in place, one workgroup of 1024 threads
-// walking the array in coalesced tiles of 4096 (4 consecutive values per
-// thread), carrying the running total between tiles
+// walking the array in coalesced tiles of 8192 (8 consecutive values per
+// thread; wavefront scans by shuffles, one barrier a tile), carrying the
+// running total between tiles
 __global__ __launch_bounds__(1024) void k_rs_scan(uint32_t* __restrict__ h, int64_t total) {
-  __shared__ uint32_t part[1024];
-  __shared__ uint32_t carry_s;
-  const int tid = threadIdx.x;
-  if (tid == 0) carry_s = 0;
-  __syncthreads();
-  for (int64_t t0 = 0; t0 < total; t0 += 4096) {
-    const int64_t i0 = t0 + 4 * (int64_t)tid;
-    uint32_t v[4];
+  __shared__ uint32_t wsum[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  uint32_t carry = 0u;
+  int par = 0;
+  for (int64_t t0 = 0; t0 < total; t0 += 8192, par ^= 1) {
+    const int64_t i0 = t0 + 8 * (int64_t)tid;
+    uint32_t v[8], s = 0u;
+    const bool whole = i0 + 8 <= total;
+    if (whole) {
+      const uint4 a = *(const uint4*)(h + i0), b = *(const uint4*)(h + i0 + 4);
+      v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+      v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+    } else {
 #pragma unroll
-    for (int q = 0; q < 4; ++q) v[q] = i0 + q < total ? h[i0 + q] : 0u;
-    const uint32_t s = v[0] + v[1] + v[2] + v[3];
-    part[tid] = s;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const uint32_t u = tid >= off ? part[tid - off] : 0u;
-      __syncthreads();
-      part[tid] += u;
-      __syncthreads();
+      for (int q = 0; q < 8; ++q) v[q] = i0 + q < total ? h[i0 + q] : 0u;
     }
-    const uint32_t carry = carry_s;
-    uint32_t run = carry + part[tid] - s;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (i0 + q < total) h[i0 + q] = run;
-      run += v[q];
+    for (int q = 0; q < 8; ++q) s += v[q];
+    uint32_t inc = s;
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t u = __shfl_up(inc, off);
+      if (lane >= off) inc += u;
     }
-    __syncthreads();
-    if (tid == 1023) carry_s = carry + part[1023];
-    __syncthreads();
+    if (lane == 63) wsum[par][wv] = inc;
+    __syncthreads();  // wsum alternates, so one barrier a tile suffices
+    uint32_t before = 0u, all = 0u;
+    for (int w = 0; w < 16; ++w) {
+      const uint32_t u = wsum[par][w];
+      before += w < wv ? u : 0u;
+      all += u;
+    }
+    uint32_t run = carry + before + inc - s;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const uint32_t n = v[q];
+      v[q] = run;
+      run += n;
+    }
+    if (whole) {
+      *(uint4*)(h + i0) = make_uint4(v[0], v[1], v[2], v[3]);
+      *(uint4*)(h + i0 + 4) = make_uint4(v[4], v[5], v[6], v[7]);
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; ++q)
+        if (i0 + q < total) h[i0 + q] = v[q];
+    }
+    carry += all;
   }
 }
 
 __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(
     const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-    uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int64_t p, int shift,
+    uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int64_t p, int shift, int kpt,
     const uint32_t* __restrict__ hist, int64_t nblocks) {
   __shared__ uint32_t wcnt[RS_BLOCK / 64][256];
   __shared__ uint32_t run[256];  // keys of each digit in the block's earlier sub-tiles
@@ -122,9 +271,9 @@ __global__ __launch_bounds__(RS_BLOCK) void k_rs_scatter(
   run[tid] = hist[(size_t)tid * nblocks + blockIdx.x];
   __syncthreads();
   const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
-  for (int st = 0; st < RS_KPT; ++st) {
-    const int64_t i = blockIdx.x * (int64_t)RS_TILE + (int64_t)st * RS_BLOCK + tid;
-    if (blockIdx.x * (int64_t)RS_TILE + (int64_t)st * RS_BLOCK >= p) break;  // block-uniform
+  for (int st = 0; st < kpt; ++st) {
+    const int64_t i = (blockIdx.x * (int64_t)kpt + st) * RS_BLOCK + tid;
+    if ((blockIdx.x * (int64_t)kpt + st) * RS_BLOCK >= p) break;  // block-uniform
     const bool valid = i < p;
     const uint32_t key = valid ? kin[i] : 0u, val = valid ? vin[i] : 0u;
     const uint32_t dig = (key >> shift) & 255u;
@@ -159,18 +308,24 @@ void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* k
                       uint32_t* vals_tmp, int64_t p, int key_bits, uint32_t* hist,
                       int64_t hist_cap) {
   if (p <= 0) return;
-  int64_t nblocks = (p + RS_TILE - 1) / RS_TILE;
+  if (p <= SORT_SMALL) {
+    const sort_job job = {keys, vals, key_bits};
+    launch_sort_small(s, &job, 1, p);
+    return;
+  }
+  const int kpt = p < 262144 ? 4 : 16;
+  const int64_t nblocks = (p + RS_BLOCK * kpt - 1) / (RS_BLOCK * kpt);
   MDA_REQUIRE(nblocks * 256 <= hist_cap, "radix histogram workspace too small");
   uint32_t *ki = keys, *vi = vals, *ko = keys_tmp, *vo = vals_tmp;
   int passes = 0;
   for (int shift = 0; shift < key_bits; shift += 8) {
     hipLaunchKernelGGL(k_rs_hist, dim3((unsigned)nblocks), dim3(RS_BLOCK), 0, s, ki, p, shift,
-                       hist, nblocks);
+                       kpt, hist, nblocks);
     MDA_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_rs_scan, dim3(1), dim3(1024), 0, s, hist, nblocks * 256);
     MDA_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_rs_scatter, dim3((unsigned)nblocks), dim3(RS_BLOCK), 0, s, ki, vi, ko,
-                       vo, p, shift, hist, nblocks);
+                       vo, p, shift, kpt, hist, nblocks);
     MDA_LAUNCH_CHECK();
     uint32_t* t = ki; ki = ko; ko = t;
     t = vi; vi = vo; vo = t;
@@ -248,17 +403,19 @@ void launch_bucket_ranges(hipStream_t s, const uint32_t* sorted_keys, int64_t p,
 
 // Per-observation data in bucket order: 1/var (or 1), the coordinates, and
 // for the FP32 / BF16x3 contractions of GEOGRAPHIC problems the unit vector
-// of each location (ux, uy, uz may be null).
+// of each location (ux, uy, uz may be null); ipos[order[t]] = t when ipos is
+// not null.
 __global__ void k_gather_obs(const uint32_t* __restrict__ order, int64_t p,
                              const double* __restrict__ var, const double* __restrict__ oa,
                              const double* __restrict__ ob, const double* __restrict__ oc,
                              int rweight, double* __restrict__ s_rinv, double* __restrict__ s_a,
                              double* __restrict__ s_b, double* __restrict__ s_c,
                              double* __restrict__ ux, double* __restrict__ uy,
-                             double* __restrict__ uz) {
+                             double* __restrict__ uz, uint32_t* __restrict__ ipos) {
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < p;
        t += (int64_t)gridDim.x * blockDim.x) {
     const uint32_t o = order[t];
+    if (ipos) ipos[o] = (uint32_t)t;
     const double a = oa[o], b = ob[o];
     s_rinv[t] = rweight == MDA_RW_IDENTITY ? 1.0 : 1.0 / var[o];
     s_a[t] = a;
@@ -274,10 +431,10 @@ __global__ void k_gather_obs(const uint32_t* __restrict__ order, int64_t p,
 void launch_gather_obs(hipStream_t s, const uint32_t* order, int64_t p, const double* var,
                        const double* oa, const double* ob, const double* oc, int rweight,
                        double* s_rinv, double* s_a, double* s_b, double* s_c, double* ux,
-                       double* uy, double* uz) {
+                       double* uy, double* uz, uint32_t* ipos) {
   if (p <= 0) return;
   hipLaunchKernelGGL(k_gather_obs, dim3(grid_for(p, 256, 65536)), dim3(256), 0, s, order, p,
-                     var, oa, ob, oc, rweight, s_rinv, s_a, s_b, s_c, ux, uy, uz);
+                     var, oa, ob, oc, rweight, s_rinv, s_a, s_b, s_c, ux, uy, uz, ipos);
   MDA_LAUNCH_CHECK();
 }
 
@@ -1473,8 +1630,6 @@ void launch_letkf_gram(hipStream_t s, const letkf_gram_args& a) {
 // local observations), compacted into a list with wave-aggregated atomics.
 // The list's order varies from run to run; every column is solved on its own,
 // so the results do not.
-__global__ void k_solve_count_zero(unsigned* cnt) { *cnt = 0u; }
-
 __global__ void k_solve_worklist(int64_t ncol, const int* __restrict__ only,
                                  const int* __restrict__ nloc, int* __restrict__ list,
                                  unsigned* __restrict__ cnt) {
@@ -1650,8 +1805,6 @@ void launch_letkf_solve(hipStream_t s, const letkf_solve_args& a) {
     if (a.wlist && a.wcount) {
       // the columns to solve, listed, so that an analysis without fallback
       // columns costs a scan instead of a pass over every column
-      hipLaunchKernelGGL(k_solve_count_zero, dim3(1), dim3(1), 0, s, a.wcount);
-      MDA_LAUNCH_CHECK();
       hipLaunchKernelGGL(k_solve_worklist, dim3(grid_for(a.ncol, 256, 4096)), dim3(256), 0, s,
                          a.ncol, a.flag, a.nloc, a.wlist, a.wcount);
       MDA_LAUNCH_CHECK();
@@ -2216,8 +2369,12 @@ void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t nco
   MDA_LAUNCH_CHECK();
 }
 
-// nloc statistics: out[0] = sum, out[1] = max, out[2] = #zeros
-__global__ void k_reduce_int(const int* __restrict__ v, int64_t n, int64_t* out) {
+// per-column statistics of up to three arrays (gridDim.y): out[3y] = sum,
+// out[3y + 1] = max, out[3y + 2] = #zeros
+__global__ void k_reduce_int(const int* __restrict__ v0, const int* __restrict__ v1,
+                             const int* __restrict__ v2, int64_t n, int64_t* out) {
+  const int* v = blockIdx.y == 0 ? v0 : blockIdx.y == 1 ? v1 : v2;
+  out += 3 * blockIdx.y;
   __shared__ long long s_sum[256], s_max[256], s_zero[256];
   long long su = 0, mx = 0, ze = 0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
@@ -2243,9 +2400,10 @@ __global__ void k_reduce_int(const int* __restrict__ v, int64_t n, int64_t* out)
   }
 }
 
-void launch_reduce_int(hipStream_t s, const int* v, int64_t n, int64_t* out3,
-                       int64_t* /*unused*/) {
-  hipLaunchKernelGGL(k_reduce_int, dim3(grid_for(n, 256, 1024)), dim3(256), 0, s, v, n, out3);
+void launch_reduce_int(hipStream_t s, const int* v0, const int* v1, const int* v2, int64_t n,
+                       int64_t* out9) {
+  hipLaunchKernelGGL(k_reduce_int, dim3(grid_for(n, 256, 256), v2 ? 3 : 2), dim3(256), 0, s, v0,
+                     v1, v2, n, out9);
   MDA_LAUNCH_CHECK();
 }
 

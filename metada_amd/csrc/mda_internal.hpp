@@ -177,12 +177,6 @@ void launch_obs_stats(hipStream_t s, const double* X, int k, int64_t n, int64_t 
                       double* d, double* yp_mm, const uint32_t* order = nullptr,
                       float* y32 = nullptr, const uint32_t* opos = nullptr,
                       int* status = nullptr);
-// keys = grid position of each observation's first stencil tap (groups of
-// four levels share a key range; nxy = points per level), vals = 0..p-1
-void launch_tap_keys(hipStream_t s, const int64_t* row_ptr, const int64_t* col, int64_t p,
-                     int64_t nxy, uint32_t* keys, uint32_t* vals);
-// ipos[order[t]] = t
-void launch_invert_order(hipStream_t s, const uint32_t* order, int64_t p, uint32_t* ipos);
 // global (all-observation) Gram: G[a][c] = sum_o r_o Y'[o][a] Q[o][c] with Q =
 // [Y' | d] (mode 0) or D = d + sigma Z - Y' (mode 1, EnKF); partials reduced.
 void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
@@ -232,19 +226,46 @@ struct bucket_grid {
   double da, db;         // bucket sizes
   int wrap;              // longitude wrap-around
 };
-void launch_bucket_keys(hipStream_t s, const double* oa, const double* ob, int64_t p,
-                        bucket_grid g, uint32_t* keys, uint32_t* vals);
+// clears status, stats [9], and per column sweeps, flag and (when set) nloc,
+// and per pass the fallback and boundary-list counts
+struct letkf_begin_args {
+  int64_t ncol, npass;
+  int *status, *sweeps, *flag, *nloc;
+  int64_t* stats;
+  unsigned* wcount;
+  uint32_t* shell_count;
+};
+void launch_letkf_begin(hipStream_t s, const letkf_begin_args& a);
+// validity, bucket keys and (tkeys set) keys of the first stencil tap, nxy
+// points per level; rcoord: latitude (GEOGRAPHIC) or y, ccoord: longitude or x
+struct obs_prepare_args {
+  int64_t p, nxy;
+  const double *yo, *var, *rcoord, *ccoord;
+  bucket_grid grid;
+  uint32_t *keys, *vals;
+  const int64_t *row_ptr, *col;
+  uint32_t *tkeys, *tvals;
+  int* status;
+};
+void launch_obs_prepare(hipStream_t s, const obs_prepare_args& a);
+// stable sort of up to two sets of p <= SORT_SMALL (key, value) pairs, in place
+constexpr int SORT_SMALL = 4096;
+struct sort_job {
+  uint32_t *keys, *vals;
+  int bits;  // of the keys
+};
+void launch_sort_small(hipStream_t s, const sort_job* jobs, int njobs, int64_t p);
 void radix_sort_pairs(hipStream_t s, uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp,
                       uint32_t* vals_tmp, int64_t p, int key_bits, uint32_t* hist,
                       int64_t hist_cap);
 void launch_bucket_ranges(hipStream_t s, const uint32_t* sorted_keys, int64_t p,
                           int nbuckets, int* start);
 // per-observation data in bucket order (1/var, coordinates; unit vectors of
-// GEOGRAPHIC locations when ux is not null)
+// GEOGRAPHIC locations when ux is not null; ipos[order[t]] = t when set)
 void launch_gather_obs(hipStream_t s, const uint32_t* order, int64_t p, const double* var,
                        const double* oa, const double* ob, const double* oc, int rweight,
                        double* s_rinv, double* s_a, double* s_b, double* s_c, double* ux,
-                       double* uy, double* uz);
+                       double* uy, double* uz, uint32_t* ipos);
 // Y' rows and d in bucket order, plus the FP32 copy of Y' when y32 is not null
 void launch_gather_rows(hipStream_t s, const uint32_t* order, int64_t p, int k,
                         const double* yp_om, const double* d, double* s_yp, double* s_d,
@@ -391,8 +412,9 @@ void launch_letkf_eig(hipStream_t s, const letkf_solve_args& a, double* de, doub
 void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t ncol,
                             int64_t nlev, const double* T, int* status, int64_t col0 = 0, int64_t nc = -1,
                             int precision = MDA_PREC_FP64, const int* only = nullptr);
-void launch_reduce_int(hipStream_t s, const int* v, int64_t n, int64_t* out2 /* sum,max */,
-                       int64_t* out_empty);
+// [sum, max, #zeros] of each array (v2 may be null), added into out9
+void launch_reduce_int(hipStream_t s, const int* v0, const int* v1, const int* v2, int64_t n,
+                       int64_t* out9);
 
 // runs f with the context's device current and converts its exceptions into
 // MDA_E_* codes (message in ctx->err)

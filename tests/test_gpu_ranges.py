@@ -272,3 +272,29 @@ def test_mlp_every_m_matches_oracle(mda, ctx, orc, m):
     lo, go = orc.mlp_loss_grad(p64, f64, target.astype(np.float64))
     assert abs(loss.value - lo) <= 128 * 6e-8 * max(lo, 1e-3)
     assert np.linalg.norm(grad - go) <= 128 * 6e-8 * np.linalg.norm(go)
+
+
+# ---- observation sorts: one workgroup up to 4096, 1024 or 4096 keys a block beyond ----------
+@pytest.mark.parametrize("p", [3, 1023, 1025, 4095, 4096, 4097, 30000, 262143, 262150])
+def test_observation_order_matches_oracle(mda, ctx, orc, p):
+    """Local sets and the analysis through both sorts (buckets and first
+    stencil taps) and a multi-level state."""
+    rng = np.random.default_rng(p)
+    nlon, nlat, nlev, k = 24, 12, 9, 8
+    lonc, latc = (np.arange(nlon) + 0.5) * 15.0, -90 + (np.arange(nlat) + 0.5) * 15.0
+    col_lon, col_lat = (v.ravel().copy() for v in np.meshgrid(lonc, latc))
+    lat, lon = np.degrees(np.arcsin(rng.uniform(-1, 1, p))), rng.uniform(0, 360, p)
+    H = mda.ObsOperator.trilinear_latlon(lat, lon, rng.uniform(0, nlev - 1, p), nlon, nlat, nlev)
+    X = rng.standard_normal((k, nlon * nlat * nlev))
+    yo, var = rng.standard_normal(p), rng.uniform(1, 2, p) * max(1.0, p / 500.0)
+    ens = mda.Ensemble(X.copy(), nlon, nlat, nlev)
+    f = mda.LETKF(ens, mda.Observation(yo, var, lat, lon, coord=mda._lib.COORD_GEOGRAPHIC), H,
+                  mda.Config({"inflation": 1.05, "localization_radius": 900.0}),
+                  geometry=mda.ColumnGeometry(mda._lib.COORD_GEOGRAPHIC, col_lat, col_lon),
+                  ctx=ctx)
+    f.Analyse()
+    prob = orc.Problem(k, nlon, nlat, nlev, orc.COORD_GEOGRAPHIC, col_lat, col_lon, lat, lon, yo,
+                       var, f.inflation, f.localization_radius)
+    Xo, _, nloc = orc.letkf_standard(prob, X, H.apply_host(X))
+    np.testing.assert_array_equal(f.local_counts(), nloc)
+    assert rel_err(ens.data, Xo) < TOL
