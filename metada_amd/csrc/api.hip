@@ -15,8 +15,15 @@ namespace {
 template <class F>
 int guarded(mda_ctx* ctx, F&& f) {
   if (!ctx) return MDA_E_ARG;
+  struct nesting {
+    int& d;
+    explicit nesting(int& v) : d(v) { ++d; }
+    ~nesting() { --d; }
+  };
   try {
     device_guard dg(ctx->device);
+    nesting nest(ctx->depth);
+    if (ctx->depth == 1) ctx->begin_call();
     f();
     ctx->err.clear();
     return MDA_OK;
@@ -48,8 +55,24 @@ dev_ensemble stage_ensemble(mda_ctx* c, const mda_ensemble* e) {
     d.X = e->data;
     return d;
   }
-  d.X = c->get<double>("ens", (size_t)d.k * d.n);
   d.staged = true;
+  // a small ensemble lives in the staging buffer, members packed
+  const size_t bytes = sizeof(double) * d.k * d.n, at = c->stage_place(bytes);
+  if (at != SIZE_MAX) {
+    char* h = c->stage_host + at;
+    if (e->data) {
+      std::memcpy(h, e->data, bytes);
+    } else {
+      MDA_REQUIRE(e->members != nullptr, "ensemble needs data or members");
+      for (int j = 0; j < d.k; ++j) {
+        MDA_REQUIRE(e->members[j] != nullptr, "member pointer is null");
+        std::memcpy(h + sizeof(double) * j * d.n, e->members[j], sizeof(double) * d.n);
+      }
+    }
+    d.X = reinterpret_cast<double*>(c->stage_dev + at);
+    return d;
+  }
+  d.X = c->get<double>("ens", (size_t)d.k * d.n);
   if (e->data) {
     h2d(c, d.X, e->data, sizeof(double) * d.k * d.n);
   } else {
@@ -64,13 +87,18 @@ dev_ensemble stage_ensemble(mda_ctx* c, const mda_ensemble* e) {
 
 void unstage_ensemble(mda_ctx* c, const mda_ensemble* e, const dev_ensemble& d) {
   if (!d.staged) return;
+  const size_t bytes = sizeof(double) * d.k * d.n;
   if (e->data) {
-    d2h(c, e->data, d.X, sizeof(double) * d.k * d.n);
+    d2h(c, e->data, d.X, bytes);
+  } else if (bytes <= mda_ctx::RESULT_BYTES) {
+    std::vector<double> all((size_t)d.k * d.n);
+    d2h(c, all.data(), d.X, bytes);
+    for (int j = 0; j < d.k; ++j)
+      std::memcpy(e->members[j], all.data() + (size_t)j * d.n, sizeof(double) * d.n);
   } else {
     for (int j = 0; j < d.k; ++j)
       d2h(c, e->members[j], d.X + (size_t)j * d.n, sizeof(double) * d.n);
   }
-  MDA_HIP(hipStreamSynchronize(c->stream));
 }
 
 struct dev_obs {
@@ -134,13 +162,12 @@ dev_hop stage_hop(mda_ctx* c, const mda_hop* h, int k, int64_t p, int64_t n) {
   return d;
 }
 
-double host_sum(mda_ctx* c, const double* dev, int n) {
-  std::vector<double> h(n);
-  d2h(c, h.data(), dev, sizeof(double) * n);
-  MDA_HIP(hipStreamSynchronize(c->stream));
-  double s = 0.0;
-  for (double v : h) s += v;
-  return s;
+// sum of squares of d [p] into *out (device)
+void enqueue_sumsq(mda_ctx* c, const double* d, int64_t p, double* out) {
+  const int nb = (int)grid_for(p, 256, 512);
+  double* part = c->get<double>("sumsq_part", 512);
+  launch_sumsq(c->stream, d, p, part, nb);
+  launch_reduce_partials(c->stream, part, nb, 1, out);
 }
 
 float elapsed(hipEvent_t a, hipEvent_t b) {
@@ -218,6 +245,13 @@ int mda_ctx_create(int device, mda_ctx** out) {
       return MDA_E_DEVICE;
     }
   }
+  try {
+    c->create_staging();
+  } catch (const mda_error& e) {
+    c->destroy_staging();
+    delete c;
+    return e.code;
+  }
   (void)hipSetDevice(prev);
   *out = c;
   return MDA_OK;
@@ -229,6 +263,7 @@ int mda_ctx_destroy(mda_ctx* c) {
   (void)hipGetDevice(&prev);
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
+  c->destroy_staging();
   for (auto& kv : c->ws)
     if (kv.second.ptr) (void)hipFree(kv.second.ptr);
   for (auto& e : c->ev)
@@ -271,6 +306,7 @@ int mda_ensemble_mean_perturbations(mda_ctx* c, const mda_ensemble* ens, double 
     dev_ensemble d = stage_ensemble(c, ens);
     double* dm = mean ? (out_on_device ? mean : c->get<double>("out_mean", d.n)) : nullptr;
     double* dp = pert ? (out_on_device ? pert : c->get<double>("out_pert", d.k * d.n)) : nullptr;
+    c->send_staged();
     launch_mean_pert(c->stream, d.X, d.k, d.n, scale, dm, dp);
     if (!out_on_device) {
       if (mean) d2h(c, mean, dm, sizeof(double) * d.n);
@@ -292,6 +328,7 @@ int mda_obs_innovations(mda_ctx* c, const mda_ensemble* ens, const mda_obs* obs,
     double* dyb = ybar ? (out_on_device ? ybar : c->get<double>("out_ybar", p)) : nullptr;
     double* dyp = yp ? (out_on_device ? yp : c->get<double>("out_yp", de.k * p)) : nullptr;
     double* dd = d ? (out_on_device ? d : c->get<double>("out_d", p)) : nullptr;
+    c->send_staged();
     launch_obs_stats(c->stream, de.X, de.k, de.n, p, h.row_ptr, h.col, h.w, h.hx, o.yo, dyb,
                      nullptr, dd, dyp);
     if (!out_on_device) {
@@ -313,24 +350,39 @@ int mda_obs_innovations(mda_ctx* c, const mda_ensemble* ens, const mda_obs* obs,
 //                             eigenvalue of E = Y'^T R^-1 Y' (from [E | b]);
 //   otherwise                 both extremes by multisection on k x k
 //                             factorisations (p <= MDA_DENSE_MAX, NaN beyond).
-static double enkf_condition_number(mda_ctx* c, const double* yp, const double* var, int k,
-                                    int64_t p, double* EB) {
-  hipStream_t s = c->stream;
-  std::vector<double> hv(p);
-  d2h(c, hv.data(), var, sizeof(double) * p);
+// Enqueues what the device computes of it into res [4]; the value follows from
+// enkf_condition_value.
+enum { COND_NONE, COND_INF, COND_DENSE, COND_CONSTANT, COND_LOWRANK };
+
+static int enqueue_enkf_condition(mda_ctx* c, const double* yp, const double* var,
+                                  const double* hv, int k, int64_t p, double* EB, double* res) {
+  // invalid variances end the analysis with an error (status word)
+  if (std::any_of(hv, hv + p, [](double v) { return !(v > 0.0); })) return COND_NONE;
   // an invalid observation (var = +inf) is an infinite singular value of S
-  if (std::any_of(hv.begin(), hv.end(), [](double v) { return std::isinf(v); }))
-    return std::numeric_limits<double>::infinity();
+  if (std::any_of(hv, hv + p, [](double v) { return std::isinf(v); })) return COND_INF;
   if (p <= 128) {
     double* S = c->get<double>("enkf_S", (size_t)128 * 128);
-    launch_form_enkf_S(s, yp, var, k, p, S);
-    const dense_extremes x = dense_sym_extremes(c, S, p);
-    return x.absmax / x.absmin;
+    launch_form_enkf_S(c->stream, yp, var, k, p, S);
+    dense_sym_extremes(c, S, p, 0, res);
+    return COND_DENSE;
   }
-  const bool constant = std::all_of(hv.begin(), hv.end(), [&](double v) { return v == hv[0]; });
-  if (constant) return 1.0 + dense_sym_extremes(c, EB, k, k + 1).lmax / (double)(k - 1);
-  if (p > MDA_DENSE_MAX) return std::numeric_limits<double>::quiet_NaN();
-  return lowrank_spd_condition(c, yp, var, hv, k, p);
+  if (std::all_of(hv, hv + p, [&](double v) { return v == hv[0]; })) {
+    dense_sym_extremes(c, EB, k, k + 1, res);
+    return COND_CONSTANT;
+  }
+  if (p > MDA_DENSE_MAX) return COND_NONE;
+  lowrank_spd_extremes(c, yp, var, hv, k, p, res);
+  return COND_LOWRANK;
+}
+
+static double enkf_condition_value(int how, const double* res, int k) {
+  switch (how) {
+    case COND_INF: return std::numeric_limits<double>::infinity();
+    case COND_DENSE: return res[3] / res[2];
+    case COND_CONSTANT: return 1.0 + res[1] / (double)(k - 1);
+    case COND_LOWRANK: return res[0] / res[1];
+    default: return std::numeric_limits<double>::quiet_NaN();
+  }
 }
 
 }  // extern "C"
@@ -363,6 +415,7 @@ void etkf_run(mda_ctx* c, double inflation, mda_ensemble* ens, const mda_obs* ob
     b.status = c->get<int>("g_status", 1);
   }
   hipStream_t s = c->stream;
+  c->send_staged();
   launch_zero(s, b.status, sizeof(int));
   launch_check_obs(s, o, b.status);
   launch_obs_stats(s, de.X, k, de.n, p, h.row_ptr, h.col, h.w, h.hx, o.yo, nullptr, b.yp, b.dd,
@@ -371,8 +424,7 @@ void etkf_run(mda_ctx* c, double inflation, mda_ensemble* ens, const mda_obs* ob
   launch_etkf_solve_ws(s, k, b.EB, b.T, b.status);
   launch_transform_global(s, de.X, k, de.n, inflation, b.T, b.status);
   int hs = 0;
-  MDA_HIP(hipMemcpyAsync(&hs, b.status, sizeof(int), hipMemcpyDeviceToHost, s));
-  MDA_HIP(hipStreamSynchronize(s));
+  d2h(c, &hs, b.status, sizeof(int));
   throw_status(hs, "ETKF");
   unstage_ensemble(c, ens, de);
 }
@@ -402,10 +454,23 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
     const double* dZ = to_device(c, "enkf_Z", Z, (size_t)p * k, z_on_device != 0);
     // all inflation methods are multiplicative sqrt(rho) (EnKF.hpp:316-331)
     const double scale = std::sqrt(inflation);
+    // variances on the host (condition number)
+    std::vector<double> hvar;
+    const double* hv = obs->variance;
+    c->send_staged();
+    if (diag && obs->on_device) {
+      hvar.resize(p);
+      d2h(c, hvar.data(), o.var, sizeof(double) * p);
+      hv = hvar.data();
+    }
     double* yp = c->get<double>("yp_om", (size_t)p * k);
     double* dd = c->get<double>("d", p);
-    int* st = c->get<int>("g_status", 1);
-    launch_zero(s, st, sizeof(int));
+    // everything the host reads back, in one block: [0, 4) gain extremes and
+    // background sum of squares, [4, 8) analysis sum of squares, [8, 12)
+    // condition number, [12] innovation norm^2, [13] the status word
+    double* res = c->get<double>("enkf_res", 14);
+    int* st = reinterpret_cast<int*>(res + 13);
+    launch_zero(s, res, sizeof(double) * 14);
     launch_check_obs(s, o, st);
     launch_obs_stats(s, de.X, k, n, p, h.row_ptr, h.col, h.w, h.hx, o.yo, nullptr, yp, dd,
                      nullptr, nullptr, nullptr, nullptr, st);
@@ -418,54 +483,46 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
     double* T = c->get<double>("gT", (size_t)k * k);
     double* Minv = c->get<double>("gMinv", (size_t)k * k);
     launch_enkf_solve_ws(s, k, EB, F, T, Minv, st);
-    {
-      // a failed factorisation or non-finite input ends the call before any
-      // diagnostics or update
-      int hs0 = 0;
-      d2h(c, &hs0, st, sizeof(int));
-      throw_status(hs0 & MDA_ST_SKIP_UPDATE, "EnKF");
-    }
-    mda_enkf_diag dg{};
-    dg.ensemble_size = k;
-    dg.observation_count = p;
-    dg.inflation_method = method;
-    dg.inflation_factor = inflation;
-    dg.analysis_increment_norm = 0.0;
-    double* part2 = c->get<double>("sumsq_part", 1024);
+    int cond = COND_NONE;
     if (diag) {
-      launch_sumsq(s, dd, p, part2, 512);
-      dg.innovation_norm = std::sqrt(host_sum(c, part2, 512));
+      enqueue_sumsq(c, dd, p, res + 12);
       // max / min Kalman gain over the n x p entries of K (EnKF.hpp:202-203;
       // O(n p k) work, as in the reference) and the background spread
       const enkf_gain_shape gs = enkf_gain_plan(k, n, p);
       double* Gf = c->get<double>("enkf_G", gs.gf_doubles());
       double* mm = c->get<double>("enkf_mm", gs.partial_doubles());
-      double* out4 = c->get<double>("enkf_mm_out", 4);
-      launch_enkf_gain_minmax(s, de.X, k, n, scale, Minv, yp, o.var, p, gs, Gf, mm, out4);
-      double h4[4] = {0.0, 0.0, 0.0, 0.0};
-      d2h(c, h4, out4, sizeof(h4));
-      dg.max_kalman_gain = h4[0];
-      dg.min_kalman_gain = h4[1];
-      dg.background_spread = std::sqrt(h4[2] / ((double)n * k));
+      launch_enkf_gain_minmax(s, de.X, k, n, scale, Minv, yp, o.var, p, gs, Gf, mm, res);
       // cond(S) = ratio of the extreme singular values of the SPD
       // S = Y'Y'^T/(k-1) + R (EnKF.hpp:205-209)
-      dg.condition_number = enkf_condition_number(c, yp, o.var, k, p, EB);
-    }
-    if (diag) {
+      cond = enqueue_enkf_condition(c, yp, o.var, hv, k, p, EB, res + 8);
       double* pa = c->get<double>("enkf_xa_part", (size_t)4 * transform_global_blocks(n));
-      double* out4 = c->get<double>("enkf_mm_out", 4);
-      launch_transform_global(s, de.X, k, n, scale, T, st, pa, out4);
-      double h4[4] = {0.0, 0.0, 0.0, 0.0};
-      d2h(c, h4, out4, sizeof(h4));
-      dg.analysis_spread = std::sqrt(h4[3] / ((double)n * k));
+      launch_transform_global(s, de.X, k, n, scale, T, st, pa, res + 4);
     } else {
       launch_transform_global(s, de.X, k, n, scale, T, st);
     }
+    double hr[14];
+    d2h(c, hr, res, sizeof(hr));
     int hs = 0;
-    d2h(c, &hs, st, sizeof(int));
-    MDA_HIP(hipStreamSynchronize(s));
+    std::memcpy(&hs, hr + 13, sizeof(int));
+    // a failed factorisation or non-finite input: the transform has left the
+    // ensemble alone
+    throw_status(hs & MDA_ST_SKIP_UPDATE, "EnKF");
     unstage_ensemble(c, ens, de);
-    if (diag) *diag = dg;
+    if (diag) {
+      mda_enkf_diag dg{};
+      dg.ensemble_size = k;
+      dg.observation_count = p;
+      dg.inflation_method = method;
+      dg.inflation_factor = inflation;
+      dg.analysis_increment_norm = 0.0;
+      dg.innovation_norm = std::sqrt(hr[12]);
+      dg.background_spread = std::sqrt(hr[2] / ((double)n * k));
+      dg.analysis_spread = std::sqrt(hr[7] / ((double)n * k));
+      dg.max_kalman_gain = hr[0];
+      dg.min_kalman_gain = hr[1];
+      dg.condition_number = enkf_condition_value(cond, hr + 8, k);
+      *diag = dg;
+    }
     throw_status(hs, "EnKF");
   });
 }
@@ -531,8 +588,15 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     const double* dZ = to_device(c, "lw_Z", Z, (size_t)p * k, z_on_device != 0);
     const double scale = std::sqrt(prm->inflation);
     const double radius = prm->localization_radius;
-    int* st = c->get<int>("lw_status", 2);  // [0] status word, [1] invalid-observation flag
-    launch_zero(s, st, 2 * sizeof(int));
+    c->send_staged();
+    // what the host reads back, in one block: [0, 4) gain extremes and sums of
+    // squares, [4, 8) extreme eigenvalues of S, [8] innovation norm^2, [9] the
+    // status word and the invalid-observation flag, [10, 10 + k) member norms or
+    // chi^2
+    double* res = c->get<double>("lw_res", 10 + k);
+    int* st = reinterpret_cast<int*>(res + 9);
+    double* mem = res + 10;
+    launch_zero(s, res, sizeof(double) * (10 + k));
     launch_check_obs(s, o, st);
     launch_lw_flag_inf(s, o.var, p, st + 1);
     double* ybar = c->get<double>("lw_ybar", p);
@@ -540,25 +604,23 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     double* dd = c->get<double>("lw_d", p);
     launch_obs_stats(s, de.X, k, n, p, h.row_ptr, h.col, h.w, h.hx, o.yo, ybar, yp, dd, nullptr,
                      nullptr, nullptr, nullptr, st);
+    // member weights (:413-430)
+    std::vector<double> sumsq(k, 0.0), chi2(k, 0.0), hres(10 + k);
+    const bool norms =
+        prm->weighting == MDA_LW_W_ADAPTIVE || prm->weighting == MDA_LW_W_INVERSE_VAR;
+    if (norms) {
+      double* part = c->get<double>("lw_part", (size_t)LW_SUMSQ_BLOCKS * k);
+      launch_lw_member_sumsq(s, de.X, k, n, part, mem);
+    } else if (prm->weighting == MDA_LW_W_LIKELIHOOD) {
+      launch_lw_chi2(s, o.yo, ybar, yp, o.var, k, p, mem);
+    }
+    d2h(c, hres.data(), res, sizeof(double) * (10 + k));
     int hst[2] = {0, 0};
-    d2h(c, hst, st, sizeof(hst));
-    MDA_HIP(hipStreamSynchronize(s));
+    std::memcpy(hst, &hres[9], sizeof(hst));
     if (hst[1])
       throw mda_error(MDA_E_ARG, "LWEnKF: invalid observations (+inf variance) are not supported");
     throw_status(hst[0] & MDA_ST_SKIP_UPDATE, "LWEnKF");
-    // member weights (:413-430)
-    std::vector<double> sumsq(k, 0.0), chi2(k, 0.0);
-    if (prm->weighting == MDA_LW_W_ADAPTIVE || prm->weighting == MDA_LW_W_INVERSE_VAR) {
-      double* part = c->get<double>("lw_part", (size_t)LW_SUMSQ_BLOCKS * k);
-      double* ss = c->get<double>("lw_sumsq", k);
-      launch_lw_member_sumsq(s, de.X, k, n, part, ss);
-      d2h(c, sumsq.data(), ss, sizeof(double) * k);
-    } else if (prm->weighting == MDA_LW_W_LIKELIHOOD) {
-      double* dchi = c->get<double>("lw_chi2", k);
-      launch_lw_chi2(s, o.yo, ybar, yp, o.var, k, p, dchi);
-      d2h(c, chi2.data(), dchi, sizeof(double) * k);
-      MDA_HIP(hipStreamSynchronize(s));
-    }
+    std::copy(hres.begin() + 10, hres.end(), norms ? sumsq.begin() : chi2.begin());
     const std::vector<double> w = lw_weights(prm->weighting, sumsq, chi2, k);
     double* dw = c->get<double>("lw_w", k);
     h2d(c, dw, w.data(), sizeof(double) * k);
@@ -573,8 +635,8 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     if (diag) {
       // cond(S) = sigma_max / sigma_min (:280-284); S is symmetric, so its
       // singular values are the |eigenvalues|
-      const dense_extremes x = dense_sym_extremes(c, S, p);
-      dg.condition_number = x.absmax / x.absmin;
+      dense_sym_extremes(c, S, p, 0, res + 4);
+      enqueue_sumsq(c, dd, p, res + 8);
     }
     // G^T = S^-T Y' (p x k), in place of Y'
     int64_t* piv = c->get<int64_t>("lw_piv", 1);
@@ -582,15 +644,6 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     MDA_HIP(hipEventRecord(c->ev[0], s));
     dense_gauss_jordan(s, p, k, St, yp, piv, pval, st);
     MDA_HIP(hipEventRecord(c->ev[1], s));
-    double* part2 = c->get<double>("sumsq_part", 1024);
-    if (diag) {
-      launch_sumsq(s, dd, p, part2, 512);
-      dg.innovation_norm = std::sqrt(host_sum(c, part2, 512));
-    }
-    d2h(c, hst, st, sizeof(int));
-    MDA_HIP(hipStreamSynchronize(s));
-    if (hst[0] & MDA_ST_NOT_SPD)
-      throw mda_error(MDA_E_NUMERIC, "LWEnKF: S = L o Pf + R is singular");
     // gain and update, fused (:272-301), with the forecast mean and spreads
     // (RecomputeMean / RecomputePerturbations, :215-229) formed in the same pass
     const lw_update_shape us = lw_update_plan(k, n, p);
@@ -598,18 +651,21 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     double* Df = c->get<double>("lw_Df", us.frag_doubles());
     double* tap = c->get<double>("lw_tap", us.ntap);
     double* mm = c->get<double>("lw_mm", 4 * us.nblk);
-    double* out4 = c->get<double>("lw_out", 4);
     MDA_HIP(hipEventRecord(c->ev[2], s));
     launch_lw_update(s, de.X, scale, yp, D, k, n, p, radius, prm->localization, prm->gc_form, us,
-                     Gf, Df, tap, mm, out4);
+                     Gf, Df, tap, mm, res, st);
     MDA_HIP(hipEventRecord(c->ev[3], s));
-    double h4[4] = {0.0, 0.0, 0.0, 0.0};
-    d2h(c, h4, out4, sizeof(h4));
+    d2h(c, hres.data(), res, sizeof(double) * 10);
+    std::memcpy(hst, &hres[9], sizeof(hst));
+    if (hst[0] & MDA_ST_NOT_SPD)  // the update has left the ensemble alone
+      throw mda_error(MDA_E_NUMERIC, "LWEnKF: S = L o Pf + R is singular");
     if (diag) {
-      dg.background_spread = std::sqrt(h4[2] / ((double)n * k));
-      dg.analysis_spread = std::sqrt(h4[3] / ((double)n * k));
-      dg.max_kalman_gain = h4[0];
-      dg.min_kalman_gain = h4[1];
+      dg.innovation_norm = std::sqrt(hres[8]);
+      dg.condition_number = hres[7] / hres[6];
+      dg.background_spread = std::sqrt(hres[2] / ((double)n * k));
+      dg.analysis_spread = std::sqrt(hres[3] / ((double)n * k));
+      dg.max_kalman_gain = hres[0];
+      dg.min_kalman_gain = hres[1];
       dg.localization_radius = radius;
       dg.max_weight = *std::max_element(w.begin(), w.end());
       dg.min_weight = *std::min_element(w.begin(), w.end());
@@ -773,11 +829,19 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   } else {
     double xmin = 0, xmax = (double)(P.nx - 1), ymin = 0, ymax = (double)(P.ny - 1);
     if (geom->col_a) {
-      std::vector<double> hx(ncol), hy(ncol);
-      d2h(c, hx.data(), ca, sizeof(double) * ncol);
-      d2h(c, hy.data(), cb, sizeof(double) * ncol);
-      auto mx = std::minmax_element(hx.begin(), hx.end());
-      auto my = std::minmax_element(hy.begin(), hy.end());
+      std::vector<double> hx, hy;
+      const double *px = geom->col_a, *py = geom->col_b;
+      if (gd) {
+        c->send_staged();
+        hx.resize(ncol);
+        hy.resize(ncol);
+        d2h(c, hx.data(), ca, sizeof(double) * ncol);
+        d2h(c, hy.data(), cb, sizeof(double) * ncol);
+        px = hx.data();
+        py = hy.data();
+      }
+      auto mx = std::minmax_element(px, px + ncol);
+      auto my = std::minmax_element(py, py + ncol);
       xmin = *mx.first; xmax = *mx.second; ymin = *my.first; ymax = *my.second;
     }
     double r = std::min(prm->radius, 1e15);
@@ -871,7 +935,9 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   sa.combine = prm->combine;
   sa.T = c->get<double>(pre + "col_T", (size_t)nck * ks * ks);
   P.sweeps = sa.sweeps = c->get<int>(pre + "col_sweeps", ncol);
-  sa.status = c->get<int>(pre + "col_status", 1);
+  // statistics [9] and the status word behind them: read back in one copy
+  P.stats = c->get<int64_t>(pre + "col_stats", 10);
+  sa.status = reinterpret_cast<int*>(P.stats + 9);
   sa.de = c->get<double>(pre + "eig_de", (size_t)ncol * 2 * ks);
   sa.lam = c->get<double>(pre + "eig_lam", (size_t)ncol * ks);
   sa.U = P.eig_path ? c->get<double>(pre + "eig_U", (size_t)nck * ks * ks) : nullptr;
@@ -904,7 +970,7 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   // E3 applies the transform itself unless T is to be kept
   sa.fuse = P.eig_path && !sa.eig_nloc && letkf_eig_fusable(ks) && prm->combine == MDA_COMBINE_MATRIX &&
             prm->transform_precision == MDA_PREC_FP64 && !prm->keep_transforms;
-  P.stats = c->get<int64_t>(pre + "col_stats", 9);
+  c->send_staged();
   return P;
 }
 
@@ -1060,10 +1126,10 @@ static void enqueue_stats(hipStream_t s, letkf_plan& P) {
 }
 
 static void finish_letkf(mda_ctx* c, letkf_plan& P, mda_letkf_diag* diag) {
-  int64_t hs[9] = {0};
+  int64_t hs[10] = {0};
   int hstat = 0;
   d2h(c, hs, P.stats, sizeof(hs));
-  d2h(c, &hstat, P.sa.status, sizeof(int));
+  std::memcpy(&hstat, hs + 9, sizeof(int));
   // the transforms stay readable only when one pass covered every column
   c->last_T = P.chunk == P.ncol && !P.sa.fuse ? P.sa.T : nullptr;
   c->last_k = P.k; c->last_ks = P.ks; c->last_ncol = P.ncol; c->last_nloc = P.ga.nloc;
@@ -1348,6 +1414,7 @@ int mda_hop_idw4_build(mda_ctx* c, const mda_obs* obs, int32_t obs_coord,
       clon = to_device(c, "hop_clon", geom->col_b, ncol, geom->on_device != 0);
       vc = to_device(c, "hop_vcoord", vcoord, nlev, geom->on_device != 0);
     }
+    c->send_staged();
     // rows of 4 taps, none for an invalid observation (variance +inf)
     std::vector<double> hv(p);
     d2h(c, hv.data(), o.var, sizeof(double) * p);
@@ -1376,6 +1443,7 @@ int mda_ensemble_save(mda_ctx* c, const mda_ensemble* ens, const char* base, con
     dev_ensemble d = stage_ensemble(c, ens);
     // Ensemble::RecomputeMean order (Ensemble.hpp:105-114) on the device
     double* dm = c->get<double>("save_mean", d.n);
+    c->send_staged();
     launch_mean_pert(c->stream, d.X, d.k, d.n, 1.0, dm, nullptr);
     std::vector<double> host(d.n);
     const int64_t nrows = ens->ny * ens->nlev;
@@ -1440,6 +1508,7 @@ int mda_ensemble_metrics(mda_ctx* c, const mda_ensemble* ens, const double* trut
     MDA_REQUIRE(truth && out, "truth and out are required");
     dev_ensemble de = stage_ensemble(c, ens);
     const double* t = to_device(c, "truth", truth, de.n, truth_on_device != 0);
+    c->send_staged();
     double* part = c->get<double>("metrics_part", (size_t)METRICS_BLOCKS * 9);
     double* out9 = c->get<double>("metrics_out", 9);
     launch_metrics(c->stream, de.X, de.k, de.n, t, part, out9);
@@ -1501,6 +1570,7 @@ int mda_letkf_inflation_features(mda_ctx* c, const mda_letkf_params* prm,
     double* sp = c->get<double>("feat_sp", o.p);
     launch_obs_spread(s, ga.yp, o.p, de.k, sp);
     const double* rp = to_device(c, "feat_rho_prev", rho_prev, ncol, prm->rho_on_device != 0);
+    c->send_staged();
     float* f = features_on_device ? features : c->get<float>("feat_out", (size_t)ncol * 8);
     launch_letkf_features(s, ga, sp, de.X, ens->nlev, rp, f);
     if (!features_on_device) d2h(c, features, f, sizeof(float) * ncol * 8);
@@ -1517,6 +1587,7 @@ int mda_mlp_forward(mda_ctx* c, const float* params, const float* features, int6
     const float* P = to_device(c, "mlp_params_in", params, MDA_MLP_NPARAM, od);
     const float* F = to_device(c, "mlp_feat_in", features, (size_t)m * MDA_MLP_NIN, od);
     float* R = od ? rho : c->get<float>("mlp_rho_out", m);
+    c->send_staged();
     launch_mlp_forward(c->stream, P, F, m, R);
     if (!od) d2h(c, rho, R, sizeof(float) * m);
     MDA_HIP(hipStreamSynchronize(c->stream));
@@ -1535,6 +1606,7 @@ int mda_mlp_loss_grad(mda_ctx* c, const float* params, const float* features,
     const float* T = to_device(c, "mlp_target_in", target, m, od);
     float* G = od ? grad : c->get<float>("mlp_grad_out", MDA_MLP_NPARAM);
     double* Ld = c->get<double>("mlp_loss", 1);
+    c->send_staged();
     launch_mlp_loss_grad(c, c->stream, P, F, T, m, G, Ld);
     d2h(c, loss, Ld, sizeof(double));
     if (!od) d2h(c, grad, G, sizeof(float) * MDA_MLP_NPARAM);

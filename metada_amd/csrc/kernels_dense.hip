@@ -328,7 +328,7 @@ __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restri
   }
 }
 
-dense_extremes dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda) {
+void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* out) {
   hipStream_t s = c->stream;
   if (lda == 0) lda = p;
   double* d = c->get<double>("dense_d", p);
@@ -346,18 +346,9 @@ dense_extremes dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda)
     double* sc = c->get<double>("dense_sc", 4);
     dense_tridiagonalise(s, p, A, d, e, u, pv, w, sc);
   }
-  double* out = c->get<double>("dense_ext", 4);
   hipLaunchKernelGGL(k_tridiag_extremes, dim3(1), dim3(512), sizeof(double) * 2 * p, s, d, e,
                      (int)p, out);
   MDA_LAUNCH_CHECK();
-  double h[4];
-  d2h(c, h, out, sizeof(h));
-  dense_extremes r;
-  r.lmin = h[0];
-  r.lmax = h[1];
-  r.absmin = h[2];
-  r.absmax = h[3];
-  return r;
 }
 
 // ---------------------------------------------------------------------------
@@ -570,8 +561,8 @@ __global__ __launch_bounds__(256) void k_ce_final(const double* __restrict__ rs,
   }
 }
 
-double lowrank_spd_condition(mda_ctx* c, const double* yp, const double* var,
-                             const std::vector<double>& hvar, int k, int64_t p) {
+void lowrank_spd_extremes(mda_ctx* c, const double* yp, const double* var, const double* hvar,
+                          int k, int64_t p, double* out) {
   MDA_REQUIRE(k >= 2 && k <= 128 && p >= 1, "condition number: size out of range");
   hipStream_t s = c->stream;
   std::vector<uint32_t> order(p);
@@ -586,7 +577,6 @@ double lowrank_spd_condition(mda_ctx* c, const double* yp, const double* var,
   double* rs = c->get<double>("ce_r", 4 * nstep);
   double* ss = c->get<double>("ce_s", 4 * nstep);
   int* flags = c->get<int>("ce_flags", 2 * CE_PTS * CE_ROUNDS);
-  double* out = c->get<double>("ce_out", 2);
   // W in LDS up to qcap rows (144 KB with the triangle; all k rows for
   // k <= 110), else in a global scratch
   const size_t tri = (size_t)k * (k + 1) / 2, wld = k | 1, cap = 18432;
@@ -608,9 +598,6 @@ double lowrank_spd_condition(mda_ctx* c, const double* yp, const double* var,
   }
   hipLaunchKernelGGL(k_ce_final, dim3(1), dim3(256), 0, s, rs, ss, k, p, flags, out);
   MDA_LAUNCH_CHECK();
-  double h[2];
-  d2h(c, h, out, sizeof(h));
-  return h[0] / h[1];
 }
 
 // ---------------------------------------------------------------------------

@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS <= 16 ? 
 void k_lw_update(double* __restrict__ X, int k, int64_t n, double scale,
                  const double* __restrict__ Gf, const double* __restrict__ Df,
                  const double* __restrict__ tap, int64_t p, int64_t ntile,
-                 double* __restrict__ partial) {
+                 double* __restrict__ partial, const int* __restrict__ status) {
   constexpr int NT = NS / 4;
   extern __shared__ double sh[];     // two tiles of [Gf | Df]
   __shared__ double red[4][4];
@@ -276,6 +276,7 @@ void k_lw_update(double* __restrict__ X, int k, int64_t n, double scale,
     if (ot + 1 < ntile) stage(b ^ 1);
   }
   {
+    const bool update = (*status & MDA_ST_SKIP_UPDATE) == 0;
     // x_a = mean + (x'_rho + K D); the spread from the deviations' distance to
     // member 0's
 #pragma unroll
@@ -290,7 +291,7 @@ void k_lw_update(double* __restrict__ X, int k, int64_t n, double scale,
           const int j = 16 * tj + kk + 4 * r;
           const double dv = v[t][4 * tj + r] + acc[tj][t][r];
           if (j < k && i < n) {
-            X[(size_t)j * n + i] = mean[t] + dv;
+            if (update) X[(size_t)j * n + i] = mean[t] + dv;
             s1 += dv - sh;
             s2 = fma(dv - sh, dv - sh, s2);
           }
@@ -376,7 +377,7 @@ lw_update_shape lw_update_plan(int k, int64_t n, int64_t p) {
 void launch_lw_update(hipStream_t s, double* X, double scale, const double* Gt, const double* D,
                       int k, int64_t n, int64_t p, double radius, int fn, int gc_form,
                       const lw_update_shape& g, double* Gf, double* Df, double* tap,
-                      double* partial, double* out4) {
+                      double* partial, double* out4, const int* status) {
   MDA_REQUIRE(k >= 2 && k <= 128, "LWEnKF supports 2 <= k <= 128");
   MDA_REQUIRE(g.nblk < (int64_t)1 << 31, "LWEnKF state too large");
   hipLaunchKernelGGL(k_lw_fragments, dim3(grid_for(std::max(g.frag_doubles(), g.ntap), 256, 4096)),
@@ -386,7 +387,7 @@ void launch_lw_update(hipStream_t s, double* X, double scale, const double* Gt, 
 #define MDA_LU(NS)                                                                            \
   hipLaunchKernelGGL(k_lw_update<NS>, dim3((unsigned)g.nblk), dim3(256),                     \
                      sizeof(double) * 4 * NS * 64, s, X, k, n, scale, Gf, Df, tap, p, g.ntile, \
-                     partial)
+                     partial, status)
   MDA_MEMBER_STEPS(k, MDA_LU)
 #undef MDA_LU
   MDA_LAUNCH_CHECK();

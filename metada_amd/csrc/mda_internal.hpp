@@ -84,6 +84,47 @@ struct mda_ctx {
   int* last_nloc = nullptr;  // device, [ncol]
   int* last_flag = nullptr;  // device, [ncol] (tridiagonal path only)
 
+  // Staging of small host arrays (create_staging): a pinned buffer with a
+  // device buffer of the same layout.  stage() copies an array into the pinned
+  // one and returns its device address; one asynchronous copy (send_staged)
+  // carries everything staged since the last, before the first kernel that
+  // reads it.  Offsets start again with every entry point, once the stream has
+  // drained.  `result` is the pinned end of small copies back.
+  static constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MAX = 512u << 10, RESULT_BYTES = 1u << 20;
+  char *stage_host = nullptr, *stage_dev = nullptr, *result = nullptr;
+  size_t stage_off = 0, stage_sent = 0;
+  int depth = 0;  // nested entry points
+
+  void create_staging() {
+    MDA_HIP(hipHostMalloc((void**)&stage_host, STAGE_BYTES));
+    MDA_HIP(hipHostMalloc((void**)&result, RESULT_BYTES));
+    MDA_HIP(hipMalloc((void**)&stage_dev, STAGE_BYTES));
+  }
+  void destroy_staging() {
+    if (stage_host) (void)hipHostFree(stage_host);
+    if (result) (void)hipHostFree(result);
+    if (stage_dev) (void)hipFree(stage_dev);
+  }
+  // place for `bytes` in both buffers (offset), or SIZE_MAX when the array is
+  // too large or the buffers are full
+  size_t stage_place(size_t bytes) {
+    if (bytes > STAGE_MAX || stage_off + bytes > STAGE_BYTES) return SIZE_MAX;
+    const size_t at = stage_off;
+    stage_off = (stage_off + bytes + 255) & ~(size_t)255;
+    return at;
+  }
+  void send_staged() {
+    if (stage_sent == stage_off) return;
+    MDA_HIP(hipMemcpyAsync(stage_dev + stage_sent, stage_host + stage_sent,
+                           stage_off - stage_sent, hipMemcpyHostToDevice, stream));
+    stage_sent = stage_off;
+  }
+  void begin_call() {
+    if (stage_off == 0) return;
+    MDA_HIP(hipStreamSynchronize(stream));  // no copy or kernel of the last call is left
+    stage_off = stage_sent = 0;
+  }
+
   // returns a device buffer of at least `bytes`; contents are unspecified.
   // Each name has one meaning; a call fetches a name once, since growing a
   // buffer frees the previous allocation.
@@ -124,27 +165,58 @@ struct device_guard {
   ~device_guard() { (void)hipSetDevice(prev); }
 };
 
-// Host <-> device transfers.  Host buffers are ordinary pageable memory, so
-// the copy is synchronous: the context's stream is drained first (it is
-// non-blocking, so the copy would not otherwise wait for it) and the copy has
-// completed when the call returns.
+// Host <-> device transfers.  Small arrays go through the context's pinned
+// buffers: h2d enqueues its copy (the source may change when it returns), d2h
+// enqueues one, waits for the stream and copies out, so a call with a handful
+// of small inputs waits once instead of twice per array.  Large host buffers
+// are ordinary pageable memory, copied synchronously: the context's stream is
+// drained first (it is non-blocking, so the copy would not otherwise wait for
+// it).
 inline void h2d(mda_ctx* c, void* dst, const void* src, size_t bytes) {
-  MDA_HIP(hipStreamSynchronize(c->stream));
-  MDA_HIP(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+  if (bytes == 0) return;
+  const size_t at = c->stage_place(bytes);
+  if (at == SIZE_MAX) {
+    MDA_HIP(hipStreamSynchronize(c->stream));
+    MDA_HIP(hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice));
+    return;
+  }
+  std::memcpy(c->stage_host + at, src, bytes);
+  // what was staged before it goes out first; its own bytes go to dst only
+  if (c->stage_sent < at)
+    MDA_HIP(hipMemcpyAsync(c->stage_dev + c->stage_sent, c->stage_host + c->stage_sent,
+                           at - c->stage_sent, hipMemcpyHostToDevice, c->stream));
+  MDA_HIP(hipMemcpyAsync(dst, c->stage_host + at, bytes, hipMemcpyHostToDevice, c->stream));
+  c->stage_sent = c->stage_off;
 }
 inline void d2h(mda_ctx* c, void* dst, const void* src, size_t bytes) {
+  // kernels enqueued before this may have read staged inputs
+  if (c->stage_sent != c->stage_off)
+    throw mda_error(MDA_E_DEVICE, "internal: staged inputs were not sent to the device");
+  if (bytes == 0) return;
+  if (bytes <= mda_ctx::RESULT_BYTES) {
+    MDA_HIP(hipMemcpyAsync(c->result, src, bytes, hipMemcpyDeviceToHost, c->stream));
+    MDA_HIP(hipStreamSynchronize(c->stream));
+    std::memcpy(dst, c->result, bytes);
+    return;
+  }
   MDA_HIP(hipStreamSynchronize(c->stream));
   MDA_HIP(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
 }
 
-// Host data staged to the device (no-op when already on the device).
+// Host data staged to the device (no-op when already on the device).  A small
+// array is on its way only after send_staged().
 template <class T>
 const T* to_device(mda_ctx* c, const std::string& name, const T* src, size_t count,
                    bool on_device) {
   if (src == nullptr) return nullptr;
   if (on_device) return src;
+  const size_t bytes = count * sizeof(T), at = c->stage_place(bytes);
+  if (at != SIZE_MAX) {
+    std::memcpy(c->stage_host + at, src, bytes);
+    return reinterpret_cast<const T*>(c->stage_dev + at);
+  }
   T* d = c->get<T>(name, count);
-  h2d(c, d, src, count * sizeof(T));
+  h2d(c, d, src, bytes);
   return d;
 }
 
@@ -442,21 +514,19 @@ void launch_idw4_stencil(hipStream_t s, int64_t p, int coord, const double* oa, 
 
 // dense p x p algebra of the global filters (p <= MDA_DENSE_MAX)
 constexpr int64_t MDA_DENSE_MAX = 4096;
-struct dense_extremes {
-  double lmin, lmax;      // smallest and largest eigenvalue
-  double absmin, absmax;  // smallest and largest |eigenvalue| (singular values)
-};
 void launch_form_enkf_S(hipStream_t s, const double* yp, const double* var, int k, int64_t p,
                         double* S);
 void dense_tridiagonalise(hipStream_t s, int64_t p, double* A, double* d, double* e, double* u,
                           double* pv, double* w, double* sc);
-// extreme eigenvalues of the symmetric device matrix A (destroyed beyond 128
-// rows); lda: row stride, 0 = p (rows beyond 128 are contiguous)
-dense_extremes dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda = 0);
-// cond(S) of S = Y'Y'^T/(k-1) + diag(var) through k x k factorisations
-// (hvar: the finite variances on the host)
-double lowrank_spd_condition(mda_ctx* c, const double* yp, const double* var,
-                             const std::vector<double>& hvar, int k, int64_t p);
+// enqueues the extreme eigenvalues of the symmetric device matrix A (destroyed
+// beyond 128 rows) into out [4] = lmin, lmax, |l|min, |l|max (device); lda: row
+// stride, 0 = p (rows beyond 128 are contiguous)
+void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* out);
+// enqueues lambda_max and lambda_min of S = Y'Y'^T/(k-1) + diag(var), through
+// k x k factorisations, into out [2] (device); hvar: the variances on the host,
+// finite and > 0
+void lowrank_spd_extremes(mda_ctx* c, const double* yp, const double* var, const double* hvar,
+                          int k, int64_t p, double* out);
 // B <- A^-1 B by Gauss-Jordan with partial pivoting (A destroyed); a zero
 // pivot sets MDA_ST_NOT_SPD in *status
 void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* B,
@@ -484,11 +554,12 @@ struct lw_update_shape {
   int64_t frag_doubles() const { return ntile * ns * 64; }
 };
 lw_update_shape lw_update_plan(int k, int64_t n, int64_t p);
-// out4 = [max K, min K, sum of squares of X'_rho, sum of (x_a - mean_a)^2]
+// out4 = [max K, min K, sum of squares of X'_rho, sum of (x_a - mean_a)^2]; X is
+// left alone when the status word holds a MDA_ST_SKIP_UPDATE bit
 void launch_lw_update(hipStream_t s, double* X, double scale, const double* Gt, const double* D,
                       int k, int64_t n, int64_t p, double radius, int fn, int gc_form,
                       const lw_update_shape& g, double* Gf, double* Df, double* tap,
-                      double* partial, double* out4);
+                      double* partial, double* out4, const int* status);
 void launch_lw_flag_inf(hipStream_t s, const double* var, int64_t p, int* flag);
 
 }  // namespace mda

@@ -298,3 +298,36 @@ def test_observation_order_matches_oracle(mda, ctx, orc, p):
     Xo, _, nloc = orc.letkf_standard(prob, X, H.apply_host(X))
     np.testing.assert_array_equal(f.local_counts(), nloc)
     assert rel_err(ens.data, Xo) < TOL
+
+
+# ---- host arrays: staged together up to 512 KB each and 4 MB in all, copied singly beyond ----
+@pytest.mark.parametrize("nx,p", [(64, 10), (8192, 500), (8193, 500), (8192, 65536),
+                                  (8000, 65537), (9000, 130000)])
+def test_host_arrays_equal_device_arrays(mda, ctx, nx, p):
+    """The same analyses from host arrays and from device tensors, to the last
+    bit, one call right after the other on one context."""
+    import torch
+    rng = np.random.default_rng(nx + p)
+    k = 8
+    X, x = rng.standard_normal((k, nx)), rng.uniform(0, nx - 1, p)
+    i = np.minimum(x.astype(np.int64), nx - 2)
+    col, w = np.stack([i, i + 1], 1).ravel(), np.stack([i + 1 - x, x - i], 1).ravel()
+    rp = np.arange(0, 2 * p + 1, 2)
+    yo, var, Z = rng.standard_normal(p), rng.uniform(1, 2, p) * 50, rng.standard_normal((p, k))
+    out = {}
+    for where in ("host", "device", "host again"):
+        t = (lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()) if where == "device" \
+            else (lambda a: a.copy())
+        obs = mda.Observation(t(yo), t(var), t(x), t(np.zeros(p)))
+        H = mda.ObsOperator(t(rp), t(col), t(w))
+        a, b = (mda.Ensemble(t(X), nx, 1, 1) for _ in range(2))
+        torch.cuda.synchronize()
+        mda.LETKF(a, obs, H, mda.Config({"inflation": 1.05, "localization_radius": 12.0}),
+                  ctx=ctx).Analyse()
+        f = mda.EnKF(b, obs, H, mda.Config({"analysis": {"inflation": 1.1}}), ctx=ctx)
+        f.Analyse(Z=t(Z))
+        r = f.getAnalysisResults()
+        out[where] = (a.to_host(), b.to_host(), [r["max_kalman_gain"], r["analysis_spread"]])
+    for where in ("device", "host again"):
+        for u, v in zip(out["host"], out[where]):
+            np.testing.assert_array_equal(u, v)
