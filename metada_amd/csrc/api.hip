@@ -639,10 +639,9 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
       enqueue_sumsq(c, dd, p, res + 8);
     }
     // G^T = S^-T Y' (p x k), in place of Y'
-    int64_t* piv = c->get<int64_t>("lw_piv", 1);
-    double* pval = c->get<double>("lw_pval", 1);
+    double* gj = c->get<double>("lw_gj", dense_gauss_jordan_work(p));
     MDA_HIP(hipEventRecord(c->ev[0], s));
-    dense_gauss_jordan(s, p, k, St, yp, piv, pval, st);
+    dense_gauss_jordan(s, p, k, St, yp, gj, st);
     MDA_HIP(hipEventRecord(c->ev[1], s));
     // gain and update, fused (:272-301), with the forecast mean and spreads
     // (RecomputeMean / RecomputePerturbations, :215-229) formed in the same pass

@@ -7,9 +7,8 @@
 //     Sturm counts of the tridiagonal,
 //   - Gauss-Jordan elimination with partial pivoting, A^-1 B for p x m B (the
 //     S^-1 products of EnKF.hpp:199 and LWEnKF.hpp:273-276).
-// Each elimination step is a short sequence of launches over the trailing
-// matrix: O(p^3) work, as the reference's own dense algebra.  Sizes are
-// bounded by MDA_DENSE_MAX.
+// Each step is one or two launches over the trailing matrix: O(p^3) work, as
+// the reference's own dense algebra.  Sizes are bounded by MDA_DENSE_MAX.
 #include <algorithm>
 #include <cmath>
 #include <numeric>
@@ -43,120 +42,184 @@ void launch_form_enkf_S(hipStream_t s, const double* yp, const double* var, int 
   MDA_LAUNCH_CHECK();
 }
 
-// ---------------------------------------------------------------------------
-// Householder tridiagonalisation, step j (m = p - j - 1 trailing rows):
-//   x = A[j+1:, j], alpha = -sign(x_0) ||x||, u = x - alpha e_1,
-//   tau = 2 / u^T u, pv = tau A' u, w = pv - (tau/2)(pv^T u) u,
-//   A' <- A' - u w^T - w u^T;  d_j = A[j][j], e_j = alpha.
-// ---------------------------------------------------------------------------
-__device__ inline double block_reduce_sum(double v, double* red) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+// Lane shifts in the vector unit (DPP), a few cycles each where a shuffle
+// through LDS takes over a hundred; lanes without a source, and rows outside
+// ROWS, take `none`.
+template <int CTRL, int ROWS = 0xf>
+__device__ inline double dpp(double v, double none) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(none), __double2loint(v), CTRL, ROWS,
+                                             0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(none), __double2hiint(v), CTRL, ROWS,
+                                             0xf, false);
+  return __hiloint2double(hi, lo);
+}
+
+__device__ inline double read_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// row_shr 1, 2, 4, 8: lane 15 of a row of 16 holds the row's result; row_bcast
+// 15 and 31 carry it on, lane 63 holds the wavefront's
+__device__ inline double wave_sum(double v) {
+  v += dpp<0x111>(v, 0.0);
+  v += dpp<0x112>(v, 0.0);
+  v += dpp<0x114>(v, 0.0);
+  v += dpp<0x118>(v, 0.0);
+  v += dpp<0x142, 0xa>(v, 0.0);
+  v += dpp<0x143, 0xc>(v, 0.0);
+  return read_lane(v, 63);
+}
+
+__device__ inline double row_max(double v) {  // in lane 15 of each row
+  v = fmax(v, dpp<0x111>(v, v));
+  v = fmax(v, dpp<0x112>(v, v));
+  v = fmax(v, dpp<0x114>(v, v));
+  return fmax(v, dpp<0x118>(v, v));
+}
+
+__device__ inline double wave_max(double v) {
+  v = row_max(v);
+  v = fmax(v, dpp<0x142>(v, v));
+  v = fmax(v, dpp<0x143>(v, v));
+  return read_lane(v, 63);
+}
+
+// sum over the block's wavefronts (at most 16), in every thread
+__device__ inline double block_wave_sum(double v, double* red) {
+  v = wave_sum(v);
+  const int nw = blockDim.x >> 6;
   __syncthreads();
-  if (lane == 0) red[wv] = v;
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   double t = 0.0;
   for (int i = 0; i < nw; ++i) t += red[i];
   return t;
 }
 
-__global__ __launch_bounds__(1024) void k_hh_vec(int64_t p, int64_t j, const double* __restrict__ A,
-                                                 double* __restrict__ u, double* __restrict__ sc,
+// ---------------------------------------------------------------------------
+// Householder tridiagonalisation, step j (m = p - j - 1 trailing rows):
+//   x = A[j+1:, j], alpha = -sign(x_0) ||x||, u = x - alpha e_1,
+//   tau = 2 / u^T u, pv = tau A' u, w = pv - (tau/2)(pv^T u) u,
+//   A' <- A' - u w^T - w u^T;  d_j = A[j][j], e_j = alpha.
+// One launch per step.  A step's rank-2 update is applied by the next step's
+// launch: every block forms w of the step before and the new column j (row j,
+// which no block writes) for itself, O(p) work, and then takes its rows, each
+// updated, stored and multiplied by the new u in the same pass.  The vectors
+// of successive steps alternate between two buffers.  Bound by the latency of a
+// launch and its dependent reads up to p of about 1,000 (p = 512: 2.7 ms, 5.3 us
+// a step; 7.1 ms with four launches a step) and by the one read and write of the
+// trailing matrix beyond.
+// ---------------------------------------------------------------------------
+struct hh_vectors {  // of one step: u [p], pv [p], tau
+  double *u, *pv, *tau;
+};
+
+constexpr int HH_PF = 8;
+
+__global__ __launch_bounds__(256) void k_hh_step(int p, int j, double* __restrict__ A,
+                                                 hh_vectors prev, hh_vectors next,
                                                  double* __restrict__ d, double* __restrict__ e) {
-  __shared__ double red[16];
-  double s = 0.0;
-  for (int64_t r = j + 1 + threadIdx.x; r < p; r += blockDim.x) {
-    const double x = A[(size_t)r * p + j];
-    s += x * x;
+  extern __shared__ double sh[];  // u and w of the step before, u of this one
+  __shared__ double red[4];
+  double *up = sh, *wp = sh + p, *un = sh + 2 * p;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  // the first HH_PF entries a lane takes of its wavefront's first row, on
+  // their way while the vectors are formed
+  const int r0 = j + 1 + blockIdx.x * 4 + wv;
+  double pf[HH_PF];
+#pragma unroll
+  for (int q = 0; q < HH_PF; ++q) {
+    const int c = j + 1 + lane + 64 * q;
+    pf[q] = r0 < p && c < p ? A[(size_t)r0 * p + c] : 0.0;
   }
-  const double nrm2 = block_reduce_sum(s, red);
-  const double x0 = A[(size_t)(j + 1) * p + j];
+  double part = 0.0;
+  for (int c = j + tid; c < p; c += 256) {
+    const double a = j > 0 ? prev.u[c] : 0.0, b = j > 0 ? prev.pv[c] : 0.0;
+    up[c] = a;
+    wp[c] = b;
+    un[c] = A[(size_t)j * p + c];
+    part = fma(a, b, part);
+  }
+  const double K = j > 0 ? 0.5 * *prev.tau * block_wave_sum(part, red) : 0.0;
+  for (int c = j + tid; c < p; c += 256) wp[c] -= K * up[c];
+  __syncthreads();
+  const double upj = up[j], wpj = wp[j];
+  double s2 = 0.0;
+  for (int c = j + tid; c < p; c += 256) {
+    const double x = fma(-upj, wp[c], fma(-wpj, up[c], un[c]));
+    un[c] = x;
+    if (c > j) s2 = fma(x, x, s2);
+  }
+  const double nrm2 = block_wave_sum(s2, red);  // its barriers order un
+  const double x0 = un[j + 1], dj = un[j];
   const bool nz = nrm2 > 0.0;
   const double alpha = nz ? (x0 > 0.0 ? -1.0 : 1.0) * sqrt(nrm2) : 0.0;
   const double tau = nz ? 2.0 / (nrm2 - 2.0 * alpha * x0 + alpha * alpha) : 0.0;
-  for (int64_t r = threadIdx.x; r < p; r += blockDim.x) {
-    double v = 0.0;
-    if (r > j && nz) v = A[(size_t)r * p + j] - (r == j + 1 ? alpha : 0.0);
-    u[r] = v;
+  __syncthreads();  // every thread has read x0
+  for (int c = j + tid; c < p; c += 256) {
+    const double v = c == j || !nz ? 0.0 : un[c] - (c == j + 1 ? alpha : 0.0);
+    un[c] = v;
+    if (blockIdx.x == 0) next.u[c] = v;
   }
-  if (threadIdx.x == 0) {
-    sc[0] = tau;
-    d[j] = A[(size_t)j * p + j];
+  if (blockIdx.x == 0 && tid == 0) {
+    d[j] = dj;
     e[j] = alpha;
+    *next.tau = tau;
+  }
+  __syncthreads();
+  for (int r = r0; r < p; r += gridDim.x * 4) {
+    const double ur = up[r], wr = wp[r];
+    double* row = A + (size_t)r * p;
+    double acc = 0.0;
+    int c = j + 1 + lane;
+    if (r == r0) {
+#pragma unroll
+      for (int q = 0; q < HH_PF; ++q, c += 64)
+        if (c < p) {
+          const double a = fma(-ur, wp[c], fma(-wr, up[c], pf[q]));
+          row[c] = a;
+          acc = fma(a, un[c], acc);
+        }
+    }
+#pragma unroll 4
+    for (; c < p; c += 64) {
+      const double a = fma(-ur, wp[c], fma(-wr, up[c], row[c]));
+      row[c] = a;
+      acc = fma(a, un[c], acc);
+    }
+    acc = wave_sum(acc);
+    if (lane == 0) next.pv[r] = tau * acc;
   }
 }
 
-// pv[r] = tau sum_{c > j} A[r][c] u[c] for r > j: one wavefront per row
-__global__ __launch_bounds__(256) void k_hh_symv(int64_t p, int64_t j, const double* __restrict__ A,
-                                                 const double* __restrict__ u,
-                                                 const double* __restrict__ sc,
-                                                 double* __restrict__ pv) {
-  const int lane = threadIdx.x & 63;
-  const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
-  const double tau = sc[0];
-  for (int64_t r = j + 1 + blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < p;
-       r += nw) {
-    const double* row = A + (size_t)r * p;
-    double s = 0.0;
-    for (int64_t c = j + 1 + lane; c < p; c += 64) s += row[c] * u[c];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
-    if (lane == 0) pv[r] = tau * s;
-  }
-}
-
-// w = pv - (tau/2)(pv^T u) u (one block)
-__global__ __launch_bounds__(1024) void k_hh_w(int64_t p, int64_t j, const double* __restrict__ u,
-                                               const double* __restrict__ pv,
-                                               const double* __restrict__ sc,
-                                               double* __restrict__ w) {
-  __shared__ double red[16];
-  double s = 0.0;
-  for (int64_t r = j + 1 + threadIdx.x; r < p; r += blockDim.x) s += pv[r] * u[r];
-  const double K = 0.5 * sc[0] * block_reduce_sum(s, red);
-  for (int64_t r = j + 1 + threadIdx.x; r < p; r += blockDim.x) w[r] = pv[r] - K * u[r];
-}
-
-// A' <- A' - u w^T - w u^T on the trailing block (two FMAs per entry)
-__global__ __launch_bounds__(256) void k_hh_syr2(int64_t p, int64_t j, double* __restrict__ A,
-                                                 const double* __restrict__ u,
-                                                 const double* __restrict__ w) {
-  const int64_t m = p - j - 1;
-  const int64_t total = m * m;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = j + 1 + t / m, c = j + 1 + t % m;
-    double& a = A[(size_t)r * p + c];
-    a = fma(-u[r], w[c], fma(-w[r], u[c], a));
-  }
-}
-
-// last 2 x 2 block of the tridiagonal
-__global__ void k_hh_tail(int64_t p, const double* __restrict__ A, double* __restrict__ d,
-                          double* __restrict__ e) {
+// last 2 x 2 block, with the last step's update still to apply
+__global__ void k_hh_tail(int p, const double* __restrict__ A, hh_vectors prev,
+                          double* __restrict__ d, double* __restrict__ e) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (p >= 2) {
-    d[p - 2] = A[(size_t)(p - 2) * p + (p - 2)];
-    e[p - 2] = A[(size_t)(p - 1) * p + (p - 2)];
-  }
-  d[p - 1] = A[(size_t)(p - 1) * p + (p - 1)];
-  e[p - 1] = 0.0;
+  const int a = p - 2, b = p - 1;
+  const double ua = prev.u[a], ub = prev.u[b];
+  const double K = 0.5 * *prev.tau * fma(prev.pv[a], ua, prev.pv[b] * ub);
+  const double wa = prev.pv[a] - K * ua, wb = prev.pv[b] - K * ub;
+  d[a] = fma(-ua, wa, fma(-wa, ua, A[(size_t)a * p + a]));
+  e[a] = fma(-ub, wa, fma(-wb, ua, A[(size_t)b * p + a]));
+  d[b] = fma(-ub, wb, fma(-wb, ub, A[(size_t)b * p + b]));
+  e[b] = 0.0;
 }
 
-void dense_tridiagonalise(hipStream_t s, int64_t p, double* A, double* d, double* e, double* u,
-                          double* pv, double* w, double* sc) {
-  MDA_REQUIRE(p >= 1 && p <= MDA_DENSE_MAX, "dense matrix size out of range");
-  for (int64_t j = 0; j + 2 < p; ++j) {
-    const int64_t m = p - j - 1;
-    hipLaunchKernelGGL(k_hh_vec, dim3(1), dim3(1024), 0, s, p, j, A, u, sc, d, e);
-    MDA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_hh_symv, dim3(grid_for(m, 4, 2048)), dim3(256), 0, s, p, j, A, u, sc, pv);
-    MDA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_hh_w, dim3(1), dim3(1024), 0, s, p, j, u, pv, sc, w);
-    MDA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_hh_syr2, dim3(grid_for(m * m, 256, 8192)), dim3(256), 0, s, p, j, A, u, w);
+// p >= 3; work: 4 p + 2 doubles
+static void dense_tridiagonalise(hipStream_t s, int p, double* A, double* d, double* e,
+                                 double* work) {
+  MDA_REQUIRE(p >= 3 && p <= MDA_DENSE_MAX, "dense matrix size out of range");
+  hh_vectors v[2];
+  for (int i = 0; i < 2; ++i)
+    v[i] = {work + (size_t)i * 2 * p, work + (size_t)i * 2 * p + p, work + (size_t)4 * p + i};
+  for (int j = 0; j + 2 < p; ++j) {
+    hipLaunchKernelGGL(k_hh_step, dim3(grid_for(p - j - 1, 4, 1024)), dim3(256),
+                       sizeof(double) * 3 * p, s, p, j, A, v[(j + 1) & 1], v[j & 1], d, e);
     MDA_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL(k_hh_tail, dim3(1), dim3(64), 0, s, p, A, d, e);
+  hipLaunchKernelGGL(k_hh_tail, dim3(1), dim3(64), 0, s, p, A, v[(p - 3) & 1], d, e);
   MDA_LAUNCH_CHECK();
 }
 
@@ -170,11 +233,6 @@ void dense_tridiagonalise(hipStream_t s, int64_t p, double* A, double* d, double
 // one-workgroup Jacobi of the matrix in global memory.
 // ---------------------------------------------------------------------------
 constexpr int SYM_LDS_N = 128;
-
-__device__ inline double wave_sum_xor(double v) {
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-  return v;
-}
 
 __global__ __launch_bounds__(512) void k_sym_tridiag_lds(const double* __restrict__ A,
                                                          int64_t lda, int n, int ld,
@@ -194,7 +252,7 @@ __global__ __launch_bounds__(512) void k_sym_tridiag_lds(const double* __restric
     // x = A[j][j+1..] (row j equals column j): entries lane and lane + 64
     const double x0 = lane > j && lane < n ? a[j * ld + lane] : 0.0;
     const double x1 = lane + 64 > j && lane + 64 < n ? a[j * ld + lane + 64] : 0.0;
-    const double nrm2 = wave_sum_xor(fma(x0, x0, x1 * x1));
+    const double nrm2 = wave_sum(fma(x0, x0, x1 * x1));
     const double xh = a[j * ld + j + 1];
     const bool nz = nrm2 > 0.0;
     const double alpha = nz ? (xh > 0.0 ? -1.0 : 1.0) * sqrt(nrm2) : 0.0;
@@ -218,7 +276,7 @@ __global__ __launch_bounds__(512) void k_sym_tridiag_lds(const double* __restric
     __syncthreads();
     const double p0 = lane > j && lane < n ? pv[lane] : 0.0;
     const double p1 = lane + 64 > j && lane + 64 < n ? pv[lane + 64] : 0.0;
-    const double K = 0.5 * tau * wave_sum_xor(fma(p0, u0, p1 * u1));
+    const double K = 0.5 * tau * wave_sum(fma(p0, u0, p1 * u1));
     if (live) {
       const double ur = u[r], wr = pr - K * ur;
       for (int c = h; c < n; c += 4)
@@ -241,19 +299,37 @@ __global__ __launch_bounds__(512) void k_sym_tridiag_lds(const double* __restric
 
 // ---------------------------------------------------------------------------
 // Extreme eigenvalues of a symmetric tridiagonal (d, e), one workgroup:
-// multisection on Sturm counts, 128 threads (points) for each of the smallest,
-// the largest, the largest negative and the smallest non-negative eigenvalue,
-// 7 bits a round.  count(x) = number of eigenvalues < x from the pivots of
-// the LDL^T factorisation of T - x I.  out = [lmin, lmax, |l|min, |l|max].
+// multisection on Sturm counts, 128 points a round for each of the smallest,
+// the largest, the largest negative and the smallest non-negative eigenvalue.
+// count(x) = number of eigenvalues < x = sign changes of the leading
+// minors of T - x I, from their three-term recurrence: one fused multiply-add
+// deep per row, where the pivots' quotients are a division deep.  T is scaled by a
+// power of two to unit span, the pair of minors to unit size every 4 rows; a zero
+// minor counts as a pivot of -1e-40.  n = 512: 0.25 ms (0.5 ms by quotients).  out = [lmin, lmax, |l|min, |l|max].
 // ---------------------------------------------------------------------------
-__device__ inline int sturm_count(const double* d, const double* e2, int n, double x,
-                                  double pivmin) {
+typedef double d2 __attribute__((ext_vector_type(2)));
+
+// de[i] = (d_i, e_{i-1}^2), n rounded up to whole groups of 8 rows by rows (2, 0)
+__device__ inline int sturm_count(const d2* de, int n, double x) {
+  double m0 = 0.0, m1 = 1.0;  // the last two minors; e_{-1} = 0
   int cnt = 0;
-  double q = 1.0;
-  for (int i = 0; i < n; ++i) {
-    q = (d[i] - x) - (i > 0 ? e2[i - 1] / q : 0.0);
-    if (fabs(q) < pivmin) q = -pivmin;
-    cnt += q < 0.0;
+  for (int i0 = 0; i0 < n; i0 += 8) {
+    d2 r[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) r[q] = de[i0 + q];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      double m = fma(r[q][0] - x, m1, -r[q][1] * m0);
+      if (m == 0.0) m = -1e-40 * m1;
+      cnt += (int)((unsigned)(__double2hiint(m) ^ __double2hiint(m1)) >> 31);
+      m0 = m1;
+      m1 = m;
+      if (q == 3 || q == 7) {
+        const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(m0), fabs(m1)));
+        m0 = __builtin_amdgcn_ldexp(m0, ex);
+        m1 = __builtin_amdgcn_ldexp(m1, ex);
+      }
+    }
   }
   return cnt;
 }
@@ -261,39 +337,37 @@ __device__ inline int sturm_count(const double* d, const double* e2, int n, doub
 __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restrict__ dg,
                                                           const double* __restrict__ eg, int n,
                                                           double* __restrict__ out) {
-  extern __shared__ double sh[];  // d [n], e^2 [n]
-  __shared__ double red[3][8], slo[4], shi[4];
+  extern __shared__ d2 de[];
+  __shared__ double red[2][8], slo[4], shi[4];
   __shared__ uint64_t bal[8];
-  double* d = sh;
-  double* e2 = sh + n;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  double lo = INFINITY, hi = -INFINITY, em = 0.0;
+  double lo = INFINITY, hi = -INFINITY;
   for (int i = tid; i < n; i += 512) {
     const double di = dg[i], ei = i + 1 < n ? fabs(eg[i]) : 0.0;
     const double r = (i > 0 ? fabs(eg[i - 1]) : 0.0) + ei;
-    d[i] = di;
-    e2[i] = ei * ei;
     lo = fmin(lo, di - r);
     hi = fmax(hi, di + r);
-    em = fmax(em, ei);
   }
   for (int off = 32; off > 0; off >>= 1) {
     lo = fmin(lo, __shfl_xor(lo, off));
     hi = fmax(hi, __shfl_xor(hi, off));
-    em = fmax(em, __shfl_xor(em, off));
   }
-  if (lane == 0) { red[0][wv] = lo; red[1][wv] = hi; red[2][wv] = em; }
+  if (lane == 0) { red[0][wv] = lo; red[1][wv] = hi; }
   __syncthreads();
   for (int w = 0; w < 8; ++w) {
     lo = fmin(lo, red[0][w]);
     hi = fmax(hi, red[1][w]);
-    em = fmax(em, red[2][w]);
   }
   const double span = fmax(fabs(lo), fabs(hi));
-  lo -= 1e-14 * span + 1e-300;
-  hi += 1e-14 * span + 1e-300;
-  const double pivmin = fmax(1e-300, 1e-300 * em * em);
-  const int neg = sturm_count(d, e2, n, 0.0, pivmin);
+  const int sc = span > 0.0 && isfinite(span) ? -ilogb(span) - 1 : 0;
+  for (int i = tid; i < (n + 7) / 8 * 8; i += 512) {
+    const double ei = i > 0 && i < n ? ldexp(eg[i - 1], sc) : 0.0;
+    de[i] = d2{i < n ? ldexp(dg[i], sc) : 2.0, ei * ei};
+  }
+  __syncthreads();
+  lo = ldexp(lo, sc) - 1e-14;
+  hi = ldexp(hi, sc) + 1e-14;
+  const int neg = sturm_count(de, n, 0.0);
   const int tg = tid >> 7, t = tid & 127;
   const int idx = tg == 0 ? 0 : tg == 1 ? n - 1 : tg == 2 ? neg - 1 : neg;
   if (t == 0) {
@@ -303,14 +377,13 @@ __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restri
   __syncthreads();
   for (int round = 0; round < 10; ++round) {
     const double a = slo[tg], b = shi[tg], w = b - a;
-    const double x = a + w * ((double)(t + 1) / 129.0);
-    const bool above = idx >= 0 && idx < n && sturm_count(d, e2, n, x, pivmin) > idx;
-    const uint64_t m = __ballot(above);
-    if (lane == 0) bal[wv] = m;
+    const int cnt = sturm_count(de, n, a + w * ((double)(t + 1) / 129.0));
+    const uint64_t above = __ballot(idx >= 0 && idx < n && cnt > idx);
+    if (lane == 0) bal[wv] = above;
     __syncthreads();
-    if (t == 0) {
+    if (t == 0) {  // f: first point above the eigenvalue
       const uint64_t b0 = bal[2 * tg], b1 = bal[2 * tg + 1];
-      const int f = b0 ? __builtin_ctzll(b0) : b1 ? 64 + __builtin_ctzll(b1) : 128;
+      const int f = b0 ? __ffsll((long long)b0) - 1 : b1 ? 64 + __ffsll((long long)b1) - 1 : 128;
       if (f > 0) slo[tg] = a + w * ((double)f / 129.0);
       if (f < 128) shi[tg] = a + w * ((double)(f + 1) / 129.0);
     }
@@ -321,10 +394,10 @@ __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restri
     double am = INFINITY;
     if (neg > 0) am = fmin(am, fabs(0.5 * (slo[2] + shi[2])));
     if (neg < n) am = fmin(am, fabs(0.5 * (slo[3] + shi[3])));
-    out[0] = l0;
-    out[1] = l1;
-    out[2] = am;
-    out[3] = fmax(fabs(l0), fabs(l1));
+    out[0] = ldexp(l0, -sc);
+    out[1] = ldexp(l1, -sc);
+    out[2] = ldexp(am, -sc);
+    out[3] = ldexp(fmax(fabs(l0), fabs(l1)), -sc);
   }
 }
 
@@ -340,13 +413,9 @@ void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* o
     MDA_LAUNCH_CHECK();
   } else {
     MDA_REQUIRE(lda == p, "the large reduction takes contiguous rows");
-    double* u = c->get<double>("dense_u", p);
-    double* pv = c->get<double>("dense_pv", p);
-    double* w = c->get<double>("dense_w", p);
-    double* sc = c->get<double>("dense_sc", 4);
-    dense_tridiagonalise(s, p, A, d, e, u, pv, w, sc);
+    dense_tridiagonalise(s, (int)p, A, d, e, c->get<double>("dense_hh", 4 * p + 2));
   }
-  hipLaunchKernelGGL(k_tridiag_extremes, dim3(1), dim3(512), sizeof(double) * 2 * p, s, d, e,
+  hipLaunchKernelGGL(k_tridiag_extremes, dim3(1), dim3(512), sizeof(double) * 2 * (p + 7), s, d, e,
                      (int)p, out);
   MDA_LAUNCH_CHECK();
 }
@@ -366,7 +435,8 @@ void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* o
 // (256 workgroups, one per CU): the weighted Gram on FP64 MFMA, the rows of
 // Y_- carried through the factorisation of A, all in LDS.  Eight rounds narrow
 // each bracket by 129^8 = 8e16.  At p = 1,500, k = 80 the dense reduction of S
-// took 33 ms (four launches per column), this 1.8 ms.
+// took 33 ms (four launches per column, before
+// the steps above shared one), this 1.8 ms.
 // ---------------------------------------------------------------------------
 constexpr int CE_PTS = 128, CE_ROUNDS = 8;
 
@@ -410,7 +480,7 @@ __device__ inline void ce_bracket(int kind, int rounds, int k, int64_t p,
     tr += ss[t];
     mn = fmin(mn, fma(ss[t], rk1, rs[t]));
   }
-  tr = wave_sum_xor(tr);
+  tr = wave_sum(tr);
   for (int off = 32; off > 0; off >>= 1) mn = fmin(mn, __shfl_xor(mn, off));
   __syncthreads();
   if (lane == 0) { red[wv] = tr; red[4 + wv] = mn; }
@@ -602,98 +672,274 @@ void lowrank_spd_extremes(mda_ctx* c, const double* yp, const double* var, const
 
 // ---------------------------------------------------------------------------
 // Gauss-Jordan elimination with partial pivoting on [A | B] (A p x p, B p x m,
-// both row-major, destroyed): B <- A^-1 B.  Step j: the pivot row is the
-// first row r >= j with the largest |A[r][j]| (the choice of partial-pivot
-// LU); rows j and r swap; row j is divided by the pivot; every other row r
-// takes -A[r][j] times row j (columns > j of A, all of B).
+// both row-major, destroyed): B <- A^-1 B, in blocks of GJ_NB columns, two
+// launches each.
+//   panel   one workgroup, rows in registers (a thread owns positions tid,
+//           tid + NT, ...): LU with partial pivoting of the block's columns over
+//           the rows >= j0, the pivot of a column being the first row with the
+//           largest entry.  With A11 = L11 U11 the pivot rows and l_r the
+//           multipliers of any other row, W[r] = -l_r L11^-1, and W[j0 + t] =
+//           row t of A11^-1.
+//   strips  a workgroup per 32 columns right of the block or of B: the row
+//           exchanges, then every row r <- (r not a pivot row ? row r : 0) +
+//           W[r] (old pivot rows) on FP64 MFMA.
+// Bound by the panel's chain of pivots (p = 512, m = 64: 33 us a panel, 11 us a
+// strip launch, 1.4 ms in all; 5.1 ms column by column, three launches each).
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void k_gj_pivot(int64_t p, int64_t j, const double* __restrict__ A,
-                                                   int64_t* __restrict__ piv,
-                                                   double* __restrict__ pval,
-                                                   int* __restrict__ status) {
-  __shared__ double bv[1024];
-  __shared__ int64_t bi[1024];
-  double best = -1.0;
-  int64_t bidx = j;
-  for (int64_t r = j + threadIdx.x; r < p; r += blockDim.x) {
-    const double v = fabs(A[(size_t)r * p + j]);
-    if (v > best) { best = v; bidx = r; }
+constexpr int GJ_NB = 16, GJ_W = 32;
+
+struct gj_moves {      // of one block, applied to the columns outside it
+  int pivot[GJ_NB];    // row that becomes row j0 + t
+  int ndisp;           // rows displaced by them: to[i] receives row from[i]
+  int to[GJ_NB], from[GJ_NB];
+};
+
+template <int NT, int R, int NB>
+__global__ __launch_bounds__(NT) void k_gj_panel(int p, int j0, int nb, const double* __restrict__ A,
+                                                 double* __restrict__ W,
+                                                 gj_moves* __restrict__ moves,
+                                                 int* __restrict__ status) {
+  constexpr int NW = NT / 64;
+  // of a step, by its parity: each wavefront's candidate (value and row index
+  // in one key, its row, its row without the multipliers) and the row that the
+  // pivot row changes places with
+  __shared__ double key[2][NW], cand[2][NW][2][NB], xrow[2][NB], LU[NB][NB + 1];
+  __shared__ int piv[NB];
+  __shared__ gj_moves mv;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  double a[R][NB];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = tid + NT * i;
+#pragma unroll
+    for (int c = 0; c < NB; ++c) a[i][c] = r < p && c < nb ? A[(size_t)r * p + j0 + c] : 0.0;
   }
-  bv[threadIdx.x] = best;
-  bi[threadIdx.x] = bidx;
-  __syncthreads();
-  for (int s2 = blockDim.x / 2; s2 > 0; s2 >>= 1) {
-    if ((int)threadIdx.x < s2) {
-      const double v2 = bv[threadIdx.x + s2];
-      const int64_t i2 = bi[threadIdx.x + s2];
-      if (v2 > bv[threadIdx.x] || (v2 == bv[threadIdx.x] && i2 < bi[threadIdx.x])) {
-        bv[threadIdx.x] = v2;
-        bi[threadIdx.x] = i2;
+  // Every step ends by rotating the rows one column to the left, so that the
+  // step's column is a[.][0], the loop stays rolled and the columns are in order
+  // again after NB steps.
+#pragma unroll 1
+  for (int t = 0; t < NB; ++t) {
+    if (t < nb) {
+      // key: |value| with its last 12 bits replaced by 4095 - row, so that the
+      // first of the largest wins; a NaN is never taken
+      const int par = t & 1;
+      double kv = -1.0;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int r = tid + NT * i;
+        const double v = fabs(a[i][0]);
+        if (r >= j0 + t && r < p && v == v)
+          kv = fmax(kv, __hiloint2double(__double2hiint(v),
+                                         (__double2loint(v) & ~4095) | (4095 - r)));
+      }
+      kv = wave_max(kv);
+      const int rw = kv >= 0.0 ? 4095 - (__double2loint(kv) & 4095) : -1;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int r = tid + NT * i;
+        if (r == rw) {
+#pragma unroll
+          for (int c = 0; c < NB; ++c) {
+            cand[par][wv][0][c] = a[i][c];
+            cand[par][wv][1][c] = c + t < NB ? a[i][c] : 0.0;
+          }
+        }
+        if (r == j0 + t) {
+#pragma unroll
+          for (int c = 0; c < NB; ++c) xrow[par][c] = a[i][c];
+        }
+      }
+      if (lane == 0) key[par][wv] = kv;
+      __syncthreads();
+      const double best = read_lane(row_max(key[par][lane % NW]), 15);
+      // no comparable entry (NaN): no exchange, and no finite pivot
+      const int bi = best >= 0.0 ? 4095 - (__double2loint(best) & 4095) : j0 + t;
+      const int bw = (bi % NT) >> 6;
+      const double(&prow)[NB] = cand[par][bw][0];
+      const double(&urow)[NB] = cand[par][bw][1];
+      const double pvt = best >= 0.0 ? prow[0] : __builtin_nan("");
+      if (tid == 0) {
+        piv[t] = bi;
+        if (!(pvt != 0.0) || !isfinite(pvt)) atomicOr(status, MDA_ST_NOT_SPD);
+      }
+      const double inv = 1.0 / pvt;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        const int r = tid + NT * i;
+        if (r == j0 + t) {
+#pragma unroll
+          for (int c = 0; c < NB; ++c) a[i][c] = prow[c];
+        } else {
+          if (r == bi) {
+#pragma unroll
+            for (int c = 0; c < NB; ++c) a[i][c] = xrow[par][c];
+          }
+          if (r < j0 || r > j0 + t) {  // not a pivot row
+            const double l = a[i][0] * inv;
+            a[i][0] = l;
+#pragma unroll
+            for (int c = 1; c < NB; ++c) a[i][c] = fma(-l, urow[c], a[i][c]);
+          }
+        }
       }
     }
-    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const double a0 = a[i][0];
+#pragma unroll
+      for (int c = 1; c < NB; ++c) a[i][c - 1] = a[i][c];
+      a[i][NB - 1] = a0;
+    }
   }
-  if (threadIdx.x == 0) {
-    piv[0] = bi[0];
-    const double pv = A[(size_t)bi[0] * p + j];
-    pval[0] = pv;
-    if (!(pv != 0.0) || !isfinite(pv)) atomicOr(status, MDA_ST_NOT_SPD);
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = tid + NT * i;
+    if (r >= j0 && r < j0 + nb) {
+#pragma unroll
+      for (int c = 0; c < NB; ++c) LU[r - j0][c] = a[i][c];
+    }
   }
-}
-
-// swap rows j and piv of [A | B] and divide row j by the pivot (columns >= j
-// of A, all of B); one thread per column
-__global__ void k_gj_swap_scale(int64_t p, int64_t m, int64_t j, double* __restrict__ A,
-                                double* __restrict__ B, const int64_t* __restrict__ piv,
-                                const double* __restrict__ pval) {
-  const int64_t r = piv[0];
-  const double inv = 1.0 / pval[0];
-  const int64_t ncols = (p - j) + m;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < ncols;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    double* M;
-    int64_t ld, cidx;
-    if (t < p - j) { M = A; ld = p; cidx = j + t; } else { M = B; ld = m; cidx = t - (p - j); }
-    double* rowj = M + (size_t)j * ld + cidx;
-    double* rowr = M + (size_t)r * ld + cidx;
-    const double vj = *rowj, vr = *rowr;
-    *rowr = vj;
-    *rowj = vr * inv;
+  __syncthreads();  // piv
+  if (tid == NT - 1) {
+    // the exchanges j0 + t <-> piv[t], one after the other, as moves of rows:
+    // row content of the block's positions, and of the positions below it
+    int n = 0;
+    for (int t = 0; t < nb; ++t) mv.pivot[t] = j0 + t;
+    for (int t = 0; t < nb; ++t) {
+      const int q = piv[t];
+      if (q == j0 + t) continue;
+      const int mine = mv.pivot[t];
+      if (q < j0 + nb) {
+        mv.pivot[t] = mv.pivot[q - j0];
+        mv.pivot[q - j0] = mine;
+        continue;
+      }
+      int at = 0;
+      while (at < n && mv.to[at] != q) ++at;
+      mv.pivot[t] = at < n ? mv.from[at] : q;
+      mv.to[at] = q;
+      mv.from[at] = mine;
+      if (at == n) ++n;
+    }
+    mv.ndisp = n;
   }
-}
-
-// row r != j:  X[r][c] -= A[r][j] X[j][c]  for c > j in A and every c of B
-// (column j of A itself is left as it is: later steps never read it)
-__global__ void k_gj_eliminate(int64_t p, int64_t m, int64_t j, double* __restrict__ A,
-                               double* __restrict__ B) {
-  const int64_t nca = p - j - 1, ncols = nca + m;
-  const int64_t total = p * ncols;
-  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = t / ncols, cc = t % ncols;
-    if (r == j) continue;
-    const double f = A[(size_t)r * p + j];
-    if (cc < nca) {
-      const int64_t c = j + 1 + cc;
-      A[(size_t)r * p + c] = fma(-f, A[(size_t)j * p + c], A[(size_t)r * p + c]);
-    } else {
-      const int64_t c = cc - nca;
-      B[(size_t)r * m + c] = fma(-f, B[(size_t)j * m + c], B[(size_t)r * m + c]);
+  __syncthreads();
+  if (tid < nb) moves->pivot[tid] = mv.pivot[tid];
+  if (tid < mv.ndisp) {
+    moves->to[tid] = mv.to[tid];
+    moves->from[tid] = mv.from[tid];
+  }
+  if (tid == 0) moves->ndisp = mv.ndisp;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int r = tid + NT * i;
+    if (r >= p) continue;
+    const bool pr = r >= j0 && r < j0 + nb;
+    if (pr) {  // y U = e_t
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        double y = r - j0 == c ? 1.0 : 0.0;
+        if (c < nb) {
+#pragma unroll
+          for (int q = 0; q < c; ++q) y = fma(-a[i][q], LU[q][c], y);
+          y /= LU[c][c];
+        }
+        a[i][c] = c < nb ? y : 0.0;
+      }
+    }
+    // x L = l_r (or y), unit lower L
+#pragma unroll
+    for (int c = NB - 1; c >= 0; --c) {
+      if (c < nb) {
+        double x = a[i][c];
+#pragma unroll
+        for (int q = c + 1; q < NB; ++q)
+          if (q < nb) x = fma(-a[i][q], LU[q][c], x);
+        a[i][c] = x;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < GJ_NB; ++c) {
+      const double x = c < NB && c < nb ? a[i][c < NB ? c : 0] : 0.0;
+      W[(size_t)r * GJ_NB + c] = pr ? x : -x;
     }
   }
 }
 
-void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* B,
-                        int64_t* piv, double* pval, int* status) {
+__global__ __launch_bounds__(512) void k_gj_strip(int p, int m, int j0, int nb,
+                                                  double* __restrict__ A, double* __restrict__ B,
+                                                  const double* __restrict__ W,
+                                                  const gj_moves* __restrict__ moves, int na) {
+  __shared__ double rows[GJ_NB][GJ_W + 2], disp[GJ_NB][GJ_W + 2];
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, i16 = lane & 15, kk = lane >> 4;
+  // strip of A's columns right of the block, or of B
+  const bool in_a = (int)blockIdx.x < na;
+  double* M = in_a ? A : B;
+  const int ld = in_a ? p : m;
+  const int c0 = in_a ? j0 + nb + GJ_W * blockIdx.x : GJ_W * ((int)blockIdx.x - na);
+  const int nc = ld - c0 < GJ_W ? ld - c0 : GJ_W;
+  const int nd = moves->ndisp;
+  {
+    const int t = tid / GJ_W, c = tid % GJ_W;  // 16 rows of 32 columns
+    rows[t][c] = t < nb && c < nc ? M[(size_t)moves->pivot[t] * ld + c0 + c] : 0.0;
+    disp[t][c] = t < nd && c < nc ? M[(size_t)moves->from[t] * ld + c0 + c] : 0.0;
+    __syncthreads();
+    if (t < nd && c < nc) M[(size_t)moves->to[t] * ld + c0 + c] = disp[t][c];
+    __syncthreads();
+  }
+  for (int r0 = 16 * wv; r0 < p; r0 += 16 * 8) {
+    double w[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      w[s] = r0 + i16 < p ? W[(size_t)(r0 + i16) * GJ_NB + 4 * s + kk] : 0.0;
+#pragma unroll
+    for (int u = 0; u < GJ_W / 16; ++u) {
+      const int c = 16 * u + i16;
+      d4 acc;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = r0 + kk + 4 * q;
+        acc[q] = r < p && c < nc && (r < j0 || r >= j0 + nb) ? M[(size_t)r * ld + c0 + c] : 0.0;
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(w[s], rows[4 * s + kk][c], acc, 0, 0, 0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = r0 + kk + 4 * q;
+        if (r < p && c < nc) M[(size_t)r * ld + c0 + c] = acc[q];
+      }
+    }
+  }
+}
+
+size_t dense_gauss_jordan_work(int64_t p) {
+  return (size_t)p * GJ_NB + (sizeof(gj_moves) + 7) / 8;
+}
+
+void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* B, double* work,
+                        int* status) {
   MDA_REQUIRE(p >= 1 && p <= MDA_DENSE_MAX && m >= 1, "dense solve size out of range");
-  for (int64_t j = 0; j < p; ++j) {
-    hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(1024), 0, s, p, j, A, piv, pval, status);
+  const int n = (int)p;
+  double* W = work;
+  gj_moves* mv = reinterpret_cast<gj_moves*>(work + (size_t)p * GJ_NB);
+  // blocks of 16 columns while a thread holds one row, of 8 beyond (more
+  // exceeds the registers of 1024 threads)
+  const int nbmax = p <= 1024 ? 16 : 8;
+  for (int j0 = 0; j0 < n; j0 += nbmax) {
+    const int nb = n - j0 < nbmax ? n - j0 : nbmax;
+#define MDA_GJ(NT, R, NB) \
+  hipLaunchKernelGGL((k_gj_panel<NT, R, NB>), dim3(1), dim3(NT), 0, s, n, j0, nb, A, W, mv, status)
+    if (p <= 256) MDA_GJ(256, 1, 16);
+    else if (p <= 512) MDA_GJ(512, 1, 16);
+    else if (p <= 1024) MDA_GJ(1024, 1, 16);
+    else if (p <= 2048) MDA_GJ(1024, 2, 8);
+    else MDA_GJ(1024, 4, 8);
+#undef MDA_GJ
     MDA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_gj_swap_scale, dim3(grid_for(p - j + m, 256, 1024)), dim3(256), 0, s, p,
-                       m, j, A, B, piv, pval);
-    MDA_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_gj_eliminate, dim3(grid_for(p * (p - j - 1 + m), 256, 8192)), dim3(256),
-                       0, s, p, m, j, A, B);
+    const int na = (n - j0 - nb + GJ_W - 1) / GJ_W, nbs = ((int)m + GJ_W - 1) / GJ_W;
+    hipLaunchKernelGGL(k_gj_strip, dim3(na + nbs), dim3(512), 0, s, n, (int)m, j0, nb, A, B, W, mv,
+                       na);
     MDA_LAUNCH_CHECK();
   }
 }

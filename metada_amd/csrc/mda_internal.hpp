@@ -516,8 +516,6 @@ void launch_idw4_stencil(hipStream_t s, int64_t p, int coord, const double* oa, 
 constexpr int64_t MDA_DENSE_MAX = 4096;
 void launch_form_enkf_S(hipStream_t s, const double* yp, const double* var, int k, int64_t p,
                         double* S);
-void dense_tridiagonalise(hipStream_t s, int64_t p, double* A, double* d, double* e, double* u,
-                          double* pv, double* w, double* sc);
 // enqueues the extreme eigenvalues of the symmetric device matrix A (destroyed
 // beyond 128 rows) into out [4] = lmin, lmax, |l|min, |l|max (device); lda: row
 // stride, 0 = p (rows beyond 128 are contiguous)
@@ -528,9 +526,10 @@ void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* o
 void lowrank_spd_extremes(mda_ctx* c, const double* yp, const double* var, const double* hvar,
                           int k, int64_t p, double* out);
 // B <- A^-1 B by Gauss-Jordan with partial pivoting (A destroyed); a zero
-// pivot sets MDA_ST_NOT_SPD in *status
-void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* B,
-                        int64_t* piv, double* pval, int* status);
+// pivot sets MDA_ST_NOT_SPD in *status; work: dense_gauss_jordan_work(p) doubles
+size_t dense_gauss_jordan_work(int64_t p);
+void dense_gauss_jordan(hipStream_t s, int64_t p, int64_t m, double* A, double* B, double* work,
+                        int* status);
 
 // LWEnKF (kernels_lw.hip)
 // sumsq[j] = sum over the state of (x_j - mean)^2; part: LW_SUMSQ_BLOCKS * k

@@ -235,6 +235,50 @@ def test_lwenkf_update_matches_oracle(mda, ctx, orc, k, n, p, fn):
         assert abs(r[key] - d[key]) <= 1e-9 * scale, (key, r[key], d[key])
 
 
+# ---- dense S of the LWEnKF: LDS reduction to p = 128, a launch per column beyond; elimination
+# ---- in blocks of 16 columns (8 beyond p = 1024), a thread per row to 1024, two to 2048 -------
+@pytest.mark.parametrize("p", [1, 2, 3, 15, 16, 17, 127, 129, 130, 255, 257, 512, 513, 1023, 1025,
+                               2047, 2049])
+def test_lwenkf_dense_algebra_with_pivoting(mda, ctx, orc, p):
+    # observations of very different scale, strongly correlated: the largest entry of a column
+    # of S is off the diagonal in some steps of each size above 3
+    k, n = 6, 40
+    rng = np.random.default_rng(p)
+    scale = 10.0 ** rng.uniform(-0.75, 0.75, p)
+    X = 2.0 + rng.standard_normal((k, n))
+    Yb = scale * (rng.standard_normal((k, 1)) + 0.1 * rng.standard_normal((k, p)))
+    yo, var = scale * rng.standard_normal(p), 0.2 * scale ** 2
+    Z = rng.standard_normal((p, k))
+    cfg = mda.Config({"analysis": {"inflation": 1.1, "localization_radius": 5.0 * p,
+                                   "localization_function": "gaussian",
+                                   "weighting_scheme": "uniform"}})
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    f = mda.LWEnKF(ens, mda.Observation(yo, var, np.zeros(p), np.zeros(p)),
+                   mda.ObsOperator(hx=Yb), cfg, ctx=ctx, gc_form="standard")
+    f.Analyse(Z=Z)
+    if p <= 257:
+        Xo, _, d, _ = orc.lwenkf_analyse(X, Yb, yo, var, Z, f.inflation_factor,
+                                         f.localization_radius, "gaussian", "uniform",
+                                         gc_standard=True)
+        cond = d["condition_number"]
+    else:  # the oracle's singular values take minutes there
+        def taper(rows, size):
+            d = np.abs(np.arange(rows)[:, None] - np.arange(p)) / size
+            return np.exp(-0.5 * (d / f.localization_radius) ** 2)
+        Y, Xp = Yb - Yb.mean(0), (X - X.mean(0)) * np.sqrt(f.inflation_factor)
+        S = taper(p, p) * (Y.T @ Y / k) + np.diag(var)
+        K = np.linalg.solve(S, Y.T @ Xp).T / (k - 1) * taper(n, max(n, p))
+        Xo = X.mean(0) + Xp + (yo + np.sqrt(var) * Z.T - Yb) @ K.T
+        ev = np.linalg.eigvalsh(S)
+        cond = ev[-1] / ev[0]
+    # cond(S) eps per solve and per singular value, over p-term sums; growth of 100
+    tol = 100 * np.finfo(float).eps * cond * max(4.0, np.sqrt(p))
+    assert tol < 1e-5
+    assert rel_err(ens.data, Xo) < tol
+    r = f.getAnalysisResults()
+    assert abs(r["condition_number"] / cond - 1.0) < tol
+
+
 # ---- verification scores: members held in registers, and the general form beyond 128 --------
 @pytest.mark.parametrize("k,n", [(2, 1), (7, 300), (8, 255), (9, 257), (40, 1000), (41, 64),
                                  (63, 500), (65, 33), (97, 100), (128, 270), (129, 50)])
