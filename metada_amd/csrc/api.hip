@@ -350,28 +350,30 @@ int mda_obs_innovations(mda_ctx* c, const mda_ensemble* ens, const mda_obs* obs,
 //                             eigenvalue of E = Y'^T R^-1 Y' (from [E | b]);
 //   otherwise                 both extremes by multisection on k x k
 //                             factorisations (p <= MDA_DENSE_MAX, NaN beyond).
-// Enqueues what the device computes of it into res [4]; the value follows from
-// enkf_condition_value.
+// Enqueues what the device computes of it into res [4], as a branch beside the
+// solve, the gain and the update; the value follows from enkf_condition_value.
 enum { COND_NONE, COND_INF, COND_DENSE, COND_CONSTANT, COND_LOWRANK };
 
-static int enqueue_enkf_condition(mda_ctx* c, const double* yp, const double* var,
-                                  const double* hv, int k, int64_t p, double* EB, double* res) {
+static int enqueue_enkf_condition(mda_ctx* c, side_branch& br, const double* yp,
+                                  const double* var, const double* hv, int k, int64_t p,
+                                  double* EB, double* res) {
   // invalid variances end the analysis with an error (status word)
   if (std::any_of(hv, hv + p, [](double v) { return !(v > 0.0); })) return COND_NONE;
   // an invalid observation (var = +inf) is an infinite singular value of S
   if (std::any_of(hv, hv + p, [](double v) { return std::isinf(v); })) return COND_INF;
   if (p <= 128) {
     double* S = c->get<double>("enkf_S", (size_t)128 * 128);
-    launch_form_enkf_S(c->stream, yp, var, k, p, S);
-    dense_sym_extremes(c, S, p, 0, res);
+    hipStream_t s = br.fork();
+    launch_form_enkf_S(s, yp, var, k, p, S);
+    dense_sym_extremes(c, s, S, p, 0, res);
     return COND_DENSE;
   }
   if (std::all_of(hv, hv + p, [&](double v) { return v == hv[0]; })) {
-    dense_sym_extremes(c, EB, k, k + 1, res);
+    dense_sym_extremes(c, br.fork(), EB, k, k + 1, res);
     return COND_CONSTANT;
   }
   if (p > MDA_DENSE_MAX) return COND_NONE;
-  lowrank_spd_extremes(c, yp, var, hv, k, p, res);
+  lowrank_spd_extremes(c, br, yp, var, hv, k, p, res);
   return COND_LOWRANK;
 }
 
@@ -479,11 +481,15 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
     double* EB = c->get<double>("gg_EB", (size_t)k * (k + 1));
     double* F = c->get<double>("gg_F", (size_t)k * k);
     launch_global_gram(s, yp, dd, o.var, nullptr, k, p, 0, part, nb, EB);
+    // cond(S) = ratio of the extreme singular values of the SPD
+    // S = Y'Y'^T/(k-1) + R (EnKF.hpp:205-209)
+    side_branch beside(c);
+    const int cond =
+        diag ? enqueue_enkf_condition(c, beside, yp, o.var, hv, k, p, EB, res + 8) : COND_NONE;
     launch_global_gram(s, yp, dd, o.var, dZ, k, p, 1, part, nb, F);
     double* T = c->get<double>("gT", (size_t)k * k);
     double* Minv = c->get<double>("gMinv", (size_t)k * k);
     launch_enkf_solve_ws(s, k, EB, F, T, Minv, st);
-    int cond = COND_NONE;
     if (diag) {
       enqueue_sumsq(c, dd, p, res + 12);
       // max / min Kalman gain over the n x p entries of K (EnKF.hpp:202-203;
@@ -492,14 +498,12 @@ int mda_enkf_analyse(mda_ctx* c, double inflation, int32_t method, mda_ensemble*
       double* Gf = c->get<double>("enkf_G", gs.gf_doubles());
       double* mm = c->get<double>("enkf_mm", gs.partial_doubles());
       launch_enkf_gain_minmax(s, de.X, k, n, scale, Minv, yp, o.var, p, gs, Gf, mm, res);
-      // cond(S) = ratio of the extreme singular values of the SPD
-      // S = Y'Y'^T/(k-1) + R (EnKF.hpp:205-209)
-      cond = enqueue_enkf_condition(c, yp, o.var, hv, k, p, EB, res + 8);
       double* pa = c->get<double>("enkf_xa_part", (size_t)4 * transform_global_blocks(n));
       launch_transform_global(s, de.X, k, n, scale, T, st, pa, res + 4);
     } else {
       launch_transform_global(s, de.X, k, n, scale, T, st);
     }
+    beside.join();
     double hr[14];
     d2h(c, hr, res, sizeof(hr));
     int hs = 0;
@@ -632,12 +636,9 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     double* St = c->get<double>("lw_St", (size_t)p * p);
     launch_lw_form_S(s, yp, dw, o.var, k, p, radius, prm->localization, prm->gc_form, S, St);
     mda_lwenkf_diag dg{};
-    if (diag) {
-      // cond(S) = sigma_max / sigma_min (:280-284); S is symmetric, so its
-      // singular values are the |eigenvalues|
-      dense_sym_extremes(c, S, p, 0, res + 4);
-      enqueue_sumsq(c, dd, p, res + 8);
-    }
+    if (diag) enqueue_sumsq(c, dd, p, res + 8);
+    side_branch cond(c);
+    hipStream_t beside = diag ? cond.fork() : nullptr;
     // G^T = S^-T Y' (p x k), in place of Y'
     double* gj = c->get<double>("lw_gj", dense_gauss_jordan_work(p));
     MDA_HIP(hipEventRecord(c->ev[0], s));
@@ -654,6 +655,11 @@ int mda_lwenkf_analyse(mda_ctx* c, const mda_lwenkf_params* prm, mda_ensemble* e
     launch_lw_update(s, de.X, scale, yp, D, k, n, p, radius, prm->localization, prm->gc_form, us,
                      Gf, Df, tap, mm, res, st);
     MDA_HIP(hipEventRecord(c->ev[3], s));
+    // cond(S) = sigma_max / sigma_min (:280-284); S is symmetric, so its
+    // singular values are the |eigenvalues|.  A chain of small launches, beside
+    // the update.
+    if (diag) dense_sym_extremes(c, beside, S, p, 0, res + 4);
+    cond.join();
     d2h(c, hres.data(), res, sizeof(double) * 10);
     std::memcpy(hst, &hres[9], sizeof(hst));
     if (hst[0] & MDA_ST_NOT_SPD)  // the update has left the ensemble alone

@@ -401,8 +401,8 @@ __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restri
   }
 }
 
-void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* out) {
-  hipStream_t s = c->stream;
+void dense_sym_extremes(mda_ctx* c, hipStream_t s, double* A, int64_t p, int64_t lda,
+                        double* out) {
   if (lda == 0) lda = p;
   double* d = c->get<double>("dense_d", p);
   double* e = c->get<double>("dense_e", p);
@@ -631,16 +631,16 @@ __global__ __launch_bounds__(256) void k_ce_final(const double* __restrict__ rs,
   }
 }
 
-void lowrank_spd_extremes(mda_ctx* c, const double* yp, const double* var, const double* hvar,
-                          int k, int64_t p, double* out) {
+void lowrank_spd_extremes(mda_ctx* c, side_branch& br, const double* yp, const double* var,
+                          const double* hvar, int k, int64_t p, double* out) {
   MDA_REQUIRE(k >= 2 && k <= 128 && p >= 1, "condition number: size out of range");
-  hipStream_t s = c->stream;
   std::vector<uint32_t> order(p);
   std::iota(order.begin(), order.end(), 0u);
   std::stable_sort(order.begin(), order.end(),
                    [&](uint32_t a, uint32_t b) { return hvar[a] < hvar[b]; });
   uint32_t* dord = c->get<uint32_t>("ce_order", p);
   h2d(c, dord, order.data(), sizeof(uint32_t) * p);
+  hipStream_t s = br.fork();
   const int kt = (k + 15) / 16;
   const int64_t nstep = (p + 3) / 4;
   double* Yf = c->get<double>("ce_rows", (size_t)nstep * kt * 64);

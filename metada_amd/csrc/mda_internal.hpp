@@ -220,6 +220,43 @@ const T* to_device(mda_ctx* c, const std::string& name, const T* src, size_t cou
   return d;
 }
 
+// Work beside the context's stream: what fork() returns runs after everything
+// enqueued so far, and what is enqueued after join(), or after the branch has
+// gone out of scope, runs after the branch's work.
+struct side_branch {
+  mda_ctx* c;
+  bool open = false;
+  explicit side_branch(mda_ctx* ctx) : c(ctx) {
+    if (c->side.empty()) {
+      hipStream_t st = nullptr;
+      MDA_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
+      c->side.push_back(st);
+    }
+    while (c->fj.size() < 2) {
+      hipEvent_t e = nullptr;
+      MDA_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+      c->fj.push_back(e);
+    }
+  }
+  side_branch(const side_branch&) = delete;
+  side_branch& operator=(const side_branch&) = delete;
+  hipStream_t fork() {
+    MDA_HIP(hipEventRecord(c->fj[0], c->stream));
+    MDA_HIP(hipStreamWaitEvent(c->side[0], c->fj[0], 0));
+    open = true;
+    return c->side[0];
+  }
+  void join() {
+    if (!open) return;
+    open = false;
+    MDA_HIP(hipEventRecord(c->fj[1], c->side[0]));
+    MDA_HIP(hipStreamWaitEvent(c->stream, c->fj[1], 0));
+  }
+  ~side_branch() {  // an error is on its way out
+    if (open) (void)hipStreamSynchronize(c->side[0]);
+  }
+};
+
 inline unsigned grid_for(int64_t n, int block, int64_t cap = 1 << 20) {
   int64_t g = (n + block - 1) / block;
   if (g < 1) g = 1;
@@ -519,12 +556,12 @@ void launch_form_enkf_S(hipStream_t s, const double* yp, const double* var, int 
 // enqueues the extreme eigenvalues of the symmetric device matrix A (destroyed
 // beyond 128 rows) into out [4] = lmin, lmax, |l|min, |l|max (device); lda: row
 // stride, 0 = p (rows beyond 128 are contiguous)
-void dense_sym_extremes(mda_ctx* c, double* A, int64_t p, int64_t lda, double* out);
+void dense_sym_extremes(mda_ctx* c, hipStream_t s, double* A, int64_t p, int64_t lda, double* out);
 // enqueues lambda_max and lambda_min of S = Y'Y'^T/(k-1) + diag(var), through
 // k x k factorisations, into out [2] (device); hvar: the variances on the host,
 // finite and > 0
-void lowrank_spd_extremes(mda_ctx* c, const double* yp, const double* var, const double* hvar,
-                          int k, int64_t p, double* out);
+void lowrank_spd_extremes(mda_ctx* c, side_branch& br, const double* yp, const double* var,
+                          const double* hvar, int k, int64_t p, double* out);
 // B <- A^-1 B by Gauss-Jordan with partial pivoting (A destroyed); a zero
 // pivot sets MDA_ST_NOT_SPD in *status; work: dense_gauss_jordan_work(p) doubles
 size_t dense_gauss_jordan_work(int64_t p);
