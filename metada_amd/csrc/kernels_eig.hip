@@ -221,40 +221,6 @@ void k_trd(int64_t ncol, const double* __restrict__ C, int c32,
 // wave-uniform branch.  Ascending output by an odd-even merge network.
 // ---------------------------------------------------------------------------
 
-// sqrt(f^2 + g^2) without the library hypot; rescaled only when the squares
-// would leave the normal range.
-__device__ inline double hyp2(double f, double g) {
-  const double a = fabs(f), b = fabs(g);
-  const double t = fmax(a, b);
-  double r = sqrt(fma(f, f, g * g));
-  if (t > 1e150 || (t < 1e-150 && t > 0.0)) {
-    const double u = fmin(a, b) / t;
-    r = t * sqrt(fma(u, u, 1.0));
-  }
-  return r;
-}
-
-// r = sqrt(f^2 + g^2) and 1/r from one reciprocal square root: the hardware
-// estimate y (about 2^-24 relative) refined by one third-order step
-// y <- y (1 + e/2 + 3e^2/8), e = 1 - t y^2 (the Taylor series of
-// (1 - e)^(-1/2)), as accurate as two Newton steps (about 1 ulp, measured
-// on the part) with a shorter dependency chain, and far shorter than a
-// square root followed by a division.  Sums of squares outside the normal
-// range (including 0) take the rescaled route.
-__device__ inline void hyp_rinv(double f, double g, double& r, double& inv) {
-  const double t2 = fma(f, f, g * g);
-  if (t2 > 1e-290 && t2 < 1e290) {
-    double y = __builtin_amdgcn_rsq(t2);
-    const double e = fma(-t2 * y, y, 1.0);
-    y = fma(y * e, fma(e, 0.375, 0.5), y);
-    r = t2 * y;
-    inv = y;
-  } else {
-    r = hyp2(f, g);
-    inv = 1.0 / r;
-  }
-}
-
 __device__ inline bool wave_any(bool v) { return __builtin_amdgcn_ballot_w64(v) != 0; }
 
 // Smallest / largest v in [0, 64) over the lanes where p holds, wave-uniform,
@@ -320,6 +286,17 @@ void k_trd_eigvals(int64_t ncol, const int* __restrict__ nloc, const double* __r
     d[i] = active ? dg[i] : 0.0;
     e[i] = (active && i < n - 1) ? dg[n + i] : 0.0;
   }
+  // scaled by a power of two to largest entry in [1/2, 1): no square below
+  // overflows, and one that leaves the normal range is zero beside the rest
+  double big = 0.0;
+#pragma unroll
+  for (int i = 0; i < n; ++i) big = fmax(big, fmax(fabs(d[i]), fabs(e[i])));
+  const int sc = __builtin_amdgcn_frexp_exp(big);  // 0 for 0, infinity and NaN
+#pragma unroll
+  for (int i = 0; i < n; ++i) {
+    d[i] = __builtin_amdgcn_ldexp(d[i], -sc);
+    e[i] = __builtin_amdgcn_ldexp(e[i], -sc);
+  }
   // e_i is negligible below tol (|d_i| + |d_{i+1}|): deflating there moves
   // the eigenvalues by O(e_i^2 / gap), far inside the 1e-12 ||T|| residual
   // the eigenvector checks accept, and it can save the last sweep of an
@@ -374,32 +351,36 @@ void k_trd_eigvals(int64_t ncol, const int* __restrict__ nloc, const double* __r
     ++wit;
     // shift from the leading 2x2 of the block
     double gg = (dl1 - dl) / (2.0 * el);
-    double rr = hyp2(gg, 1.0);
+    const double rr = sqrt(fma(gg, gg, 1.0));
     gg = dm - dl + el / (gg + (gg >= 0.0 ? rr : -rr));
     double s = 1.0, c = 1.0, p = 0.0;
-    bool run = !done;  // cleared when this lane's sweep ends early (underflow)
+    unsigned len = done ? 0u : (unsigned)(m - l);  // 0 once this lane's sweep has ended
 #pragma unroll
     for (int i = n - 2; i >= 0; --i) {
       if (i < lo || i >= hi) continue;
-      const bool act = run && l <= i && i < m;
-      const double f = s * e[i], b = c * e[i];
-      double r, inv;
-      hyp_rinv(f, gg, r, inv);
-      const bool under = act && r == 0.0;     // split and restart the block
-      const bool rot = act && r != 0.0;
-      if (act) e[i + 1] = (i == m - 1 || under) ? 0.0 : r;  // e_m ends at zero
-      if (under) { d[i + 1] -= p; run = false; }
-      const double sn = f * inv, cn = gg * inv;
-      const double g2 = d[i + 1] - p;
-      const double r2 = (d[i] - g2) * sn + 2.0 * cn * b;
-      const double pn = sn * r2;
-      if (rot) {
-        d[i + 1] = g2 + pn;
-        gg = cn * r2 - b;
-        s = sn;
-        c = cn;
-        p = pn;
-        if (i == l) {  // end of the sweep
+      if ((unsigned)(i - l) < len) {
+        const double f = s * e[i], b = c * e[i];
+        // r = sqrt(f^2 + gg^2) and 1/r from one reciprocal square root: the
+        // hardware estimate y (about 2^-24 relative) refined by one third-order
+        // step y <- y (1 + e/2 + 3e^2/8), e = 1 - t y^2 (the Taylor series of
+        // (1 - e)^(-1/2)), about 1 ulp.  Where the rotation vanishes (y = 0)
+        // the block splits and the sweep ends.
+        const double t2 = fma(f, f, gg * gg);
+        double y = __builtin_amdgcn_rsq(t2);
+        const double er = fma(-t2 * y, y, 1.0);
+        y = fma(y * er, fma(er, 0.375, 0.5), y);
+        const bool zero = !(t2 > 1e-290);
+        y = zero ? 0.0 : y;
+        e[i + 1] = i == m - 1 ? 0.0 : t2 * y;  // e_m ends at zero
+        s = f * y;
+        c = gg * y;
+        const double g2 = d[i + 1] - p;
+        const double r2 = (d[i] - g2) * s + 2.0 * c * b;
+        p = s * r2;
+        d[i + 1] = g2 + p;
+        gg = c * r2 - b;
+        if (zero) len = 0;
+        if (i == l && !zero) {  // end of the sweep
           d[i] -= p;
           e[i] = gg;
         }
@@ -411,7 +392,7 @@ void k_trd_eigvals(int64_t ncol, const int* __restrict__ nloc, const double* __r
   if (active) {
     double* lg = lam + (size_t)g * n;
 #pragma unroll
-    for (int i = 0; i < n; ++i) lg[i] = d[i];
+    for (int i = 0; i < n; ++i) lg[i] = __builtin_amdgcn_ldexp(d[i], sc);
     if (fail) flag[g] = 1;  // QL did not converge
   }
 }
