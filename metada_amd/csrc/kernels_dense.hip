@@ -301,39 +301,9 @@ __global__ __launch_bounds__(512) void k_sym_tridiag_lds(const double* __restric
 // Extreme eigenvalues of a symmetric tridiagonal (d, e), one workgroup:
 // multisection on Sturm counts, 128 points a round for each of the smallest,
 // the largest, the largest negative and the smallest non-negative eigenvalue.
-// count(x) = number of eigenvalues < x = sign changes of the leading
-// minors of T - x I, from their three-term recurrence: one fused multiply-add
-// deep per row, where the pivots' quotients are a division deep.  T is scaled by a
-// power of two to unit span, the pair of minors to unit size every 4 rows; a zero
-// minor counts as a pivot of -1e-40.  n = 512: 0.25 ms (0.5 ms by quotients).  out = [lmin, lmax, |l|min, |l|max].
+// out = [lmin, lmax, |l|min, |l|max].  Bound by the chain of the counts, n = 512:
+// 0.25 ms (0.5 ms with the counts by quotients).
 // ---------------------------------------------------------------------------
-typedef double d2 __attribute__((ext_vector_type(2)));
-
-// de[i] = (d_i, e_{i-1}^2), n rounded up to whole groups of 8 rows by rows (2, 0)
-__device__ inline int sturm_count(const d2* de, int n, double x) {
-  double m0 = 0.0, m1 = 1.0;  // the last two minors; e_{-1} = 0
-  int cnt = 0;
-  for (int i0 = 0; i0 < n; i0 += 8) {
-    d2 r[8];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) r[q] = de[i0 + q];
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      double m = fma(r[q][0] - x, m1, -r[q][1] * m0);
-      if (m == 0.0) m = -1e-40 * m1;
-      cnt += (int)((unsigned)(__double2hiint(m) ^ __double2hiint(m1)) >> 31);
-      m0 = m1;
-      m1 = m;
-      if (q == 3 || q == 7) {
-        const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(m0), fabs(m1)));
-        m0 = __builtin_amdgcn_ldexp(m0, ex);
-        m1 = __builtin_amdgcn_ldexp(m1, ex);
-      }
-    }
-  }
-  return cnt;
-}
-
 __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restrict__ dg,
                                                           const double* __restrict__ eg, int n,
                                                           double* __restrict__ out) {
@@ -362,12 +332,16 @@ __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restri
   const int sc = span > 0.0 && isfinite(span) ? -ilogb(span) - 1 : 0;
   for (int i = tid; i < (n + 7) / 8 * 8; i += 512) {
     const double ei = i > 0 && i < n ? ldexp(eg[i - 1], sc) : 0.0;
-    de[i] = d2{i < n ? ldexp(dg[i], sc) : 2.0, ei * ei};
+    de[i] = i < n ? sturm_row(ldexp(dg[i], sc), ei) : d2{2.0, 0.0};
   }
   __syncthreads();
   lo = ldexp(lo, sc) - 1e-14;
   hi = ldexp(hi, sc) + 1e-14;
-  const int neg = sturm_count(de, n, 0.0);
+  const int n8 = (n + 7) / 8 * 8;
+  const double zero[1] = {0.0};
+  int neg1[1];
+  sturm_counts(de, n8, zero, neg1);
+  const int neg = neg1[0];
   const int tg = tid >> 7, t = tid & 127;
   const int idx = tg == 0 ? 0 : tg == 1 ? n - 1 : tg == 2 ? neg - 1 : neg;
   if (t == 0) {
@@ -377,8 +351,10 @@ __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restri
   __syncthreads();
   for (int round = 0; round < 10; ++round) {
     const double a = slo[tg], b = shi[tg], w = b - a;
-    const int cnt = sturm_count(de, n, a + w * ((double)(t + 1) / 129.0));
-    const uint64_t above = __ballot(idx >= 0 && idx < n && cnt > idx);
+    const double x[1] = {a + w * ((double)(t + 1) / 129.0)};
+    int cnt[1];
+    sturm_counts(de, n8, x, cnt);
+    const uint64_t above = __ballot(idx >= 0 && idx < n && cnt[0] > idx);
     if (lane == 0) bal[wv] = above;
     __syncthreads();
     if (t == 0) {  // f: first point above the eigenvalue

@@ -112,7 +112,7 @@ __device__ inline double fast_rcp(double t) {
 // from the chunk's first row index on).  tau = 1 / (|x|^2 + |x_0| |x|).
 // Bound by the issue of vector instructions (85% of the cycles at k = 64).
 // With the norm and tau by refined estimates: k = 40, 32,768 columns 521 ->
-// 472 us; k = 64, 131,072 columns 17.4 -> 15.9 ms.  Both sums on FP64 MFMA (a
+// 472 us; k = 64, 524,288 columns 17.4 -> 15.9 ms.  Both sums on FP64 MFMA (a
 // product with ones, 5 instructions for 20): 588 us and 18.6 ms, the matrix
 // product holds the vector unit's FP64 pipe.
 // ---------------------------------------------------------------------------
@@ -964,11 +964,12 @@ __global__ __launch_bounds__(256) void k_trd_vectors_x(
 constexpr int E1W_CH = 8;  // step chunk of the k = 128 E1 (static column ranges)
 
 // E2 by bisection on Sturm counts (one wavefront per column, lane j owns
-// eigenvalues j, j + 64, ...): count(x) = #{i : q_i < 0} with
-// q_0 = d_0 - x, q_i = (d_i - x) - e_{i-1}^2 / q_{i-1}, |q_i| kept >= pivmin
-// (Golub & Van Loan, sec. 8.4.1).  Starts from the Gershgorin interval cut
-// into 65 cells by one multisection sweep and halves until the interval is
-// within 1e-13 of the eigenvalue (relative).  Ascending by construction.
+// eigenvalues j, j + 64, ...): counts by sign changes of the leading minors
+// (sturm_counts).  Starts from the Gershgorin interval cut into 65 cells by one
+// multisection sweep and halves until the interval is within 1e-13 of the
+// eigenvalue (relative).  Ascending by construction.  Bound by the issue of
+// vector instructions: k = 128, 18,432 columns 2.5 ms, 5.0 ms with the counts by
+// the quotients of the pivots.
 template <int N>
 __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
                                                             const int* __restrict__ nloc,
@@ -976,50 +977,47 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
                                                             double* __restrict__ lam,
                                                             int* __restrict__ flag) {
   constexpr int n = N, NQ = (N + 63) / 64;
-  __shared__ double sd[4][N], se2[4][N], msx[4][64];
+  static_assert(N % 8 == 0, "rows are counted in groups of 8");
+  __shared__ d2 sde[4][N];
+  __shared__ double msx[4][64];
   __shared__ int msc[4][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const int64_t g = (int64_t)blockIdx.x * 4 + wv;
   if (g >= ncol || nloc[g] == 0) return;  // whole wavefront; no block barriers below
   const double* dg = de + (size_t)g * 2 * n;
-  double* d = sd[wv];
-  double* e2 = se2[wv];
+  d2* row = sde[wv];
+  double lo = INFINITY, hi = -INFINITY;
   for (int i = lane; i < n; i += 64) {
-    d[i] = dg[i];
-    const double e = i < n - 1 ? dg[n + i] : 0.0;
-    e2[i] = e * e;
+    const double d = dg[i], r = (i > 0 ? fabs(dg[n + i - 1]) : 0.0) +
+                                (i < n - 1 ? fabs(dg[n + i]) : 0.0);
+    lo = fmin(lo, d - r);
+    hi = fmax(hi, d + r);
   }
+  for (int off = 32; off > 0; off >>= 1) {
+    lo = fmin(lo, __shfl_xor(lo, off));
+    hi = fmax(hi, __shfl_xor(hi, off));
+  }
+  // scaled by a power of two to unit Gershgorin radius
+  const int sc = __builtin_amdgcn_frexp_exp(fmax(fabs(lo), fabs(hi)));
+  for (int i = lane; i < n; i += 64)
+    row[i] = sturm_row(__builtin_amdgcn_ldexp(dg[i], -sc),
+                       i > 0 ? __builtin_amdgcn_ldexp(dg[n + i - 1], -sc) : 0.0);
   wave_lds_sync();
-  double lo = 0.0, hi = 0.0, emax = 0.0;
-  for (int i = 0; i < n; ++i) {
-    const double r = sqrt(e2[i]) + (i > 0 ? sqrt(e2[i - 1]) : 0.0);
-    lo = i == 0 ? d[i] - r : fmin(lo, d[i] - r);
-    hi = i == 0 ? d[i] + r : fmax(hi, d[i] + r);
-    emax = fmax(emax, e2[i]);
-  }
-  const double eps = 2.220446049250313e-16;
+  const double eps = 2.220446049250313e-16, least = 1e-290;
+  lo = __builtin_amdgcn_ldexp(lo, -sc);
+  hi = __builtin_amdgcn_ldexp(hi, -sc);
   const double tnorm = fmax(fabs(lo), fabs(hi));
-  const double pivmin = 2.2250738585072014e-308 * fmax(1.0, emax);
-  lo -= 2.0 * eps * tnorm + pivmin;
-  hi += 2.0 * eps * tnorm + pivmin;
+  lo -= 2.0 * eps * tnorm + least;
+  hi += 2.0 * eps * tnorm + least;
   // one multisection sweep: lane L counts the eigenvalues below the L-th of
   // 64 interior points, and every eigenvalue starts from the cell between
   // the points whose counts bracket it (six halvings for one sweep)
   {
-    const double xl = lo + (hi - lo) * ((double)(lane + 1) / 65.0);
-    double qv = 1.0;
-    int cnt = 0;
-    for (int i = 0; i < n; ++i) {
-      const double ei = i > 0 ? e2[i - 1] : 0.0;
-      double rq = __builtin_amdgcn_rcp(qv);
-      rq = fma(rq, fma(-qv, rq, 1.0), rq);
-      double v = (d[i] - xl) - ei * rq;
-      if (fabs(v) < pivmin) v = -pivmin;
-      qv = v;
-      cnt += v < 0.0;
-    }
-    msx[wv][lane] = xl;
-    msc[wv][lane] = cnt;
+    const double xl[1] = {lo + (hi - lo) * ((double)(lane + 1) / 65.0)};
+    int cnt[1];
+    sturm_counts(row, n, xl, cnt);
+    msx[wv][lane] = xl[0];
+    msc[wv][lane] = cnt[0];
   }
   wave_lds_sync();
   double a[NQ], b[NQ];
@@ -1043,30 +1041,16 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
   const double rel = 1e-13;
   for (int it = 0; it < 128; ++it) {
     bool open = false;
-    double x[NQ], qv[NQ];
+    double x[NQ];
     int cnt[NQ];
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       x[q] = 0.5 * (a[q] + b[q]);
-      open |= (lane + 64 * q < n) && b[q] - a[q] > rel * fmax(fabs(a[q]), fabs(b[q])) + pivmin
+      open |= (lane + 64 * q < n) && b[q] - a[q] > rel * fmax(fabs(a[q]), fabs(b[q])) + least
               && x[q] != a[q] && x[q] != b[q];
-      qv[q] = 1.0;
-      cnt[q] = 0;
     }
     if (!wave_any(open)) break;
-    for (int i = 0; i < n; ++i) {
-      const double di = d[i], ei = i > 0 ? e2[i - 1] : 0.0;
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        // 1/q by the hardware reciprocal and one Newton step
-        double rq = __builtin_amdgcn_rcp(qv[q]);
-        rq = fma(rq, fma(-qv[q], rq, 1.0), rq);
-        double v = (di - x[q]) - ei * rq;
-        if (fabs(v) < pivmin) v = -pivmin;
-        qv[q] = v;
-        cnt[q] += v < 0.0;
-      }
-    }
+    sturm_counts(row, n, x, cnt);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       if (cnt[q] > lane + 64 * q) b[q] = x[q];
@@ -1079,7 +1063,7 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
   for (int q = 0; q < NQ; ++q) {
     const int j = lane + 64 * q;
     if (j < n) {
-      const double v = 0.5 * (a[q] + b[q]);
+      const double v = __builtin_amdgcn_ldexp(0.5 * (a[q] + b[q]), sc);
       lg[j] = v;
       bad |= !(fabs(v) <= 1.7e308);
     }
@@ -1180,9 +1164,10 @@ __global__ __launch_bounds__(2 * N, 2) void k_trd_wr(int64_t ncol, const double*
       }
       const double nrm2 = block_total<NW>(h == 0 ? s2 : 0.0, red[0]);
       const double x0 = xs[0];
-      const bool nz = nrm2 > 0.0;
-      const double alpha = nz ? (x0 > 0.0 ? -1.0 : 1.0) * sqrt(nrm2) : 0.0;
-      const double tau = nz ? 2.0 / (nrm2 - 2.0 * alpha * x0 + alpha * alpha) : 0.0;
+      const bool nz = nrm2 > 1e-290;
+      const double nrm = fast_sqrt(nrm2);
+      const double alpha = nz ? (x0 > 0.0 ? -nrm : nrm) : 0.0;
+      const double tau = nz ? fast_rcp(fma(fabs(x0), nrm, nrm2)) : 0.0;
       double u[R];
 #pragma unroll
       for (int i = 0; i < R; ++i) u[i] = nz ? xi[i] - (rb + i == j + 1 ? alpha : 0.0) : 0.0;

@@ -62,6 +62,7 @@ __device__ inline float gaspari_cohn_f32(float z) {
 }
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------------------
 // FP64 MFMA over state points (v_mfma_f64_16x16x4f64, one wavefront per
@@ -351,6 +352,53 @@ __device__ inline int block_jacobi(double* A, int lda, double* V, int ldv, int n
     }
   }
   return sweep;
+}
+
+// Sturm counts: cnt[m] = number of eigenvalues below x[m] of the symmetric
+// tridiagonal with rows de[i] = (d_i, e_{i-1}^2), as the sign changes of the leading
+// minors of T - x I by their three-term recurrence: one multiply-add deep and five
+// instructions per row, where the pivots' quotients (a reciprocal and its
+// refinement) are ten deep.  Requires T scaled to largest entry of about 1 (sturm_row);
+// n a multiple of 8, filled up with rows (2, 0), which change no sign.  The pair of
+// minors is brought to unit size every 4 rows; e^2 is at least 1e-70, so a zero
+// minor is followed by a nonzero one of the sign opposite to the one before it, and
+// the two steps count one change whatever sign the zero has.
+__device__ inline d2 sturm_row(double d, double e) { return d2{d, fmax(e * e, 1e-70)}; }
+
+template <int M>
+__device__ inline void sturm_counts(const d2* de, int n, const double (&x)[M], int (&cnt)[M]) {
+  double m0[M], m1[M];  // the last two minors
+#pragma unroll
+  for (int t = 0; t < M; ++t) {
+    m0[t] = 0.0;  // what row 0's e^2 multiplies
+    m1[t] = 1.0;
+    cnt[t] = 0;
+  }
+  for (int i0 = 0; i0 < n; i0 += 8) {
+    unsigned bits[M];
+    d2 r[8];
+#pragma unroll
+    for (int t = 0; t < M; ++t) bits[t] = 0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) r[q] = de[i0 + q];
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+#pragma unroll
+      for (int t = 0; t < M; ++t) {
+        const double m = fma(r[q][0] - x[t], m1[t], -r[q][1] * m0[t]);
+        bits[t] = __builtin_amdgcn_alignbit(
+            bits[t], (unsigned)(__double2hiint(m) ^ __double2hiint(m1[t])), 31);
+        m0[t] = m1[t];
+        m1[t] = m;
+        if (q == 3 || q == 7) {
+          const int ex = -__builtin_amdgcn_frexp_exp(fmax(fabs(m0[t]), fabs(m1[t])));
+          m0[t] = __builtin_amdgcn_ldexp(m0[t], ex);
+          m1[t] = __builtin_amdgcn_ldexp(m1[t], ex);
+        }
+      }
+#pragma unroll
+    for (int t = 0; t < M; ++t) cnt[t] += __popc(bits[t]);
+  }
 }
 
 }  // namespace mda
