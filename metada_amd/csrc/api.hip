@@ -934,7 +934,7 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   }
 
   letkf_solve_args& sa = P.sa;
-  sa.k = k; sa.ks = ks; sa.ncol = ncol; sa.C = ga.C; sa.c32 = ga.c32; sa.b = ga.b; sa.nloc = ga.nloc;
+  sa.k = k; sa.ks = ks; sa.ncol = ncol; sa.all_cols = ncol; sa.C = ga.C; sa.c32 = ga.c32; sa.b = ga.b; sa.nloc = ga.nloc;
   sa.rho = prm->inflation; sa.rho_col = rho_col;
   sa.inflation_form = prm->inflation_form; sa.sqrt_form = prm->sqrt_form;
   sa.combine = prm->combine;

@@ -6,7 +6,8 @@
 //       the Householder vectors u_j and tau_j go to the reflector buffer U.
 //   E2  k_trd_eigvals: eigenvalues of T by implicit QL with Wilkinson shifts,
 //       one LANE per column so the serial scalar recurrence of 64 columns runs
-//       side by side, d and e in registers.
+//       side by side, d and e in registers; for few columns, and for k = 128,
+//       k_trd_eigvals_bisect: bisection, one wavefront per column.
 //   E3  k_trd_vectors: eigenvector s_j of T for eigenvalue lambda_j by a
 //       twisted factorisation of T - lambda_j I (one lane per eigenvalue),
 //       residual and near-pair orthogonality checks, back-transformation
@@ -976,9 +977,8 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
                                                             const double* __restrict__ de,
                                                             double* __restrict__ lam,
                                                             int* __restrict__ flag) {
-  constexpr int n = N, NQ = (N + 63) / 64;
-  static_assert(N % 8 == 0, "rows are counted in groups of 8");
-  __shared__ d2 sde[4][N];
+  constexpr int n = N, n8 = (N + 7) / 8 * 8, NQ = (N + 63) / 64;
+  __shared__ d2 sde[4][n8];
   __shared__ double msx[4][64];
   __shared__ int msc[4][64];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -999,9 +999,10 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
   }
   // scaled by a power of two to unit Gershgorin radius
   const int sc = __builtin_amdgcn_frexp_exp(fmax(fabs(lo), fabs(hi)));
-  for (int i = lane; i < n; i += 64)
-    row[i] = sturm_row(__builtin_amdgcn_ldexp(dg[i], -sc),
-                       i > 0 ? __builtin_amdgcn_ldexp(dg[n + i - 1], -sc) : 0.0);
+  for (int i = lane; i < n8; i += 64)
+    row[i] = i < n ? sturm_row(__builtin_amdgcn_ldexp(dg[i], -sc),
+                               i > 0 ? __builtin_amdgcn_ldexp(dg[n + i - 1], -sc) : 0.0)
+                   : d2{2.0, 0.0};
   wave_lds_sync();
   const double eps = 2.220446049250313e-16, least = 1e-290;
   lo = __builtin_amdgcn_ldexp(lo, -sc);
@@ -1015,7 +1016,7 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
   {
     const double xl[1] = {lo + (hi - lo) * ((double)(lane + 1) / 65.0)};
     int cnt[1];
-    sturm_counts(row, n, xl, cnt);
+    sturm_counts(row, n8, xl, cnt);
     msx[wv][lane] = xl[0];
     msc[wv][lane] = cnt[0];
   }
@@ -1035,10 +1036,11 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
       else b[q] = fmin(b[q], xm);
     }
   }
-  // converged at a relative width of 1e-13: the eigenvector checks ask for a
-  // residual within 1e-12 of ||T|| and the transform for 1e-10, and the last
-  // eight halvings to 2 eps would add 14 % to the sweeps
-  const double rel = 1e-13;
+  // k = 128 converges at a relative width of 1e-13: the eigenvector checks ask
+  // for a residual within 1e-12 of ||T|| and the transform for 1e-10, and the last
+  // eight halvings to 2 eps would add 14 % to the sweeps.  Where QL is the other
+  // way, the result is as close as QL's.
+  const double rel = N > 64 ? 1e-13 : 4.0 * eps;
   for (int it = 0; it < 128; ++it) {
     bool open = false;
     double x[NQ];
@@ -1050,7 +1052,7 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
               && x[q] != a[q] && x[q] != b[q];
     }
     if (!wave_any(open)) break;
-    sturm_counts(row, n, x, cnt);
+    sturm_counts(row, n8, x, cnt);
 #pragma unroll
     for (int q = 0; q < NQ; ++q) {
       if (cnt[q] > lane + 64 * q) b[q] = x[q];
@@ -1680,6 +1682,14 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
 }
 
 // ---------------------------------------------------------------------------
+// Eigenvalues of few columns by bisection, a wavefront per column: QL takes the
+// time of its slowest wavefront of 64 columns up to some 65,000 of them (337 us
+// at N = 32, 180 to 474 us by spectrum at N = 40, 1,367 us at N = 64), bisection
+// 22, 27 and 43 ns a column (118 us at N = 40 and 4,000 columns), so it is the
+// shorter up to 6,000 to 30,000 columns.  By the whole analysis, so that every
+// chunk of it takes the same way.
+constexpr int64_t EIG_BISECT_COLS = 128;  // per row of T
+
 template <int N>
 static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, double* lam,
                          int* flag) {
@@ -1691,8 +1701,12 @@ static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, d
                      a.rho, a.rho_col, prior, de, a.U);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[0]) MDA_HIP(hipEventRecord(a.ev_stage[0], s));
-  hipLaunchKernelGGL(k_trd_eigvals<N>, dim3((unsigned)((a.ncol + 63) / 64)), dim3(64), 0, s,
-                     a.ncol, nloc, de, lam, flag);
+  if (a.all_cols <= EIG_BISECT_COLS * N)
+    hipLaunchKernelGGL(k_trd_eigvals_bisect<N>, dim3((unsigned)((a.ncol + 3) / 4)), dim3(256), 0,
+                       s, a.ncol, nloc, de, lam, flag);
+  else
+    hipLaunchKernelGGL(k_trd_eigvals<N>, dim3((unsigned)((a.ncol + 63) / 64)), dim3(64), 0, s,
+                       a.ncol, nloc, de, lam, flag);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[1]) MDA_HIP(hipEventRecord(a.ev_stage[1], s));
   if constexpr (N % 16 == 0) {

@@ -459,6 +459,7 @@ struct letkf_solve_args {
   int k;
   int ks;  // size of the per-column blocks C, T, U, b, lam (letkf_gram_args::ks)
   int64_t ncol;
+  int64_t all_cols;  // of the whole analysis, where this is one chunk of it
   const double* C;
   int c32;  // C holds FP32 entries (letkf_gram_args::c32)
   const double* b;

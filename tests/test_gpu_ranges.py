@@ -88,6 +88,21 @@ def test_letkf_every_k_matches_oracle(mda, ctx, orc, k):
     assert rel_err(_latlon(mda, ctx, case, case["X"], 3000.0)[1], Xo) < TOL
 
 
+@pytest.mark.parametrize("over", [0, 1])
+@pytest.mark.parametrize("k,ks", [(7, 8), (16, 16), (19, 20), (32, 32), (40, 40), (47, 48),
+                                  (64, 64)])
+def test_letkf_eigenvalue_kernels_match_jacobi(mda, ctx, k, ks, over):
+    """Bisection up to 128 columns per row of the block, QL beyond."""
+    nlon, nlat = 2 * ks, 64 + over
+    case = latlon_case(nlon=nlon, nlat=nlat, nlev=1, k=k, p=500, seed=700 + k, nmodes=96)
+    L = mda._lib
+    f, X = _latlon(mda, ctx, case, case["X"], 4000.0)
+    _, Xj = _latlon(mda, ctx, case, case["X"], 4000.0, eig_method=L.EIG_JACOBI)
+    # near-degenerate columns may fail the eigenvector checks: a few in ten thousand
+    assert f.diag["n_fallback_columns"] <= nlon * nlat // 100
+    assert rel_err(X, Xj) < TOL
+
+
 @pytest.mark.parametrize("prec", ["FP32", "BF16X3"])
 @pytest.mark.parametrize("k,radius", [(10, 500.0), (25, 3000.0), (50, 1500.0), (50, 6000.0),
                                       (100, 1500.0), (100, 9000.0)])
