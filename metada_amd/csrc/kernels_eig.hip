@@ -85,15 +85,7 @@ __device__ inline double wave_total(double v) {
   return readlane_f64(v, 63);
 }
 
-// sqrt(t) for t in the normal range: the hardware reciprocal square root
-// (about 2^-24 relative) refined by one third-order step
-__device__ inline double fast_sqrt(double t) {
-  const double y = __builtin_amdgcn_rsq(t);
-  const double e = fma(-t * y, y, 1.0);
-  return t * fma(y * e, fma(e, 0.375, 0.5), y);
-}
-
-// 1 / t likewise
+// 1 / t: the hardware estimate refined by one third-order step
 __device__ inline double fast_rcp(double t) {
   const double y = __builtin_amdgcn_rcp(t);
   const double e = fma(-t, y, 1.0);
@@ -168,7 +160,7 @@ void k_trd(int64_t ncol, const double* __restrict__ C, int c32,
         const double nrm2 = wave_total(xi * xi);
         const double x0 = readlane_f64(xc, j + 1);
         const bool nz = nrm2 > 1e-290;
-        const double nrm = fast_sqrt(nrm2);
+        const double nrm = nrm2 * refined_rsqrt(nrm2);
         const double alpha = nz ? (x0 > 0.0 ? -nrm : nrm) : 0.0;
         const double ui = nz ? xi - (lane == j + 1 ? alpha : 0.0) : 0.0;
         const double tau = nz ? fast_rcp(fma(fabs(x0), nrm, nrm2)) : 0.0;
@@ -382,15 +374,10 @@ void k_trd_eigvals(int64_t ncol, const int* __restrict__ nloc, const double* __r
       if (i < lo || i >= hi) continue;
       if ((unsigned)(i - l) < len) {
         const double f = s * e[i], b = c * e[i];
-        // r = sqrt(f^2 + gg^2) and 1/r from one reciprocal square root: the
-        // hardware estimate y (about 2^-24 relative) refined by one third-order
-        // step y <- y (1 + e/2 + 3e^2/8), e = 1 - t y^2 (the Taylor series of
-        // (1 - e)^(-1/2)), about 1 ulp.  Where the rotation vanishes (y = 0)
-        // the block splits and the sweep ends.
+        // r = sqrt(f^2 + gg^2) and 1/r from one reciprocal square root.  Where
+        // the rotation vanishes (y = 0) the block splits and the sweep ends.
         const double t2 = fma(f, f, gg * gg);
-        double y = __builtin_amdgcn_rsq(t2);
-        const double er = fma(-t2 * y, y, 1.0);
-        y = fma(y * er, fma(er, 0.375, 0.5), y);
+        double y = refined_rsqrt(t2);
         const bool zero = !(t2 > 1e-290);
         y = zero ? 0.0 : y;
         e[i + 1] = i == m - 1 ? 0.0 : t2 * y;  // e_m ends at zero
@@ -1167,7 +1154,7 @@ __global__ __launch_bounds__(2 * N, 2) void k_trd_wr(int64_t ncol, const double*
       const double nrm2 = block_total<NW>(h == 0 ? s2 : 0.0, red[0]);
       const double x0 = xs[0];
       const bool nz = nrm2 > 1e-290;
-      const double nrm = fast_sqrt(nrm2);
+      const double nrm = nrm2 * refined_rsqrt(nrm2);
       const double alpha = nz ? (x0 > 0.0 ? -nrm : nrm) : 0.0;
       const double tau = nz ? fast_rcp(fma(fabs(x0), nrm, nrm2)) : 0.0;
       double u[R];
