@@ -2296,13 +2296,6 @@ void k_letkf_transform_bf16x3(double* __restrict__ X, int64_t ncol, int64_t nlev
   }
 }
 
-bool letkf_transform_reg_supported(int ks) {
-  switch (ks) {
-    case 8: case 16: case 20: case 32: case 40: case 48: case 64: return true;
-    default: return false;
-  }
-}
-
 void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t ncol,
                             int64_t nlev, const double* T, int* status, int64_t col0, int64_t nc,
                             int precision, const int* only) {
@@ -2345,7 +2338,7 @@ void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t nco
     MDA_LAUNCH_CHECK();
     return;
   }
-  if (letkf_transform_reg_supported(ks)) {
+  if (ks == 8 || ks == 20 || ks == 40) {
     MDA_REQUIRE((nc + XT_C - 1) / XT_C < (int64_t)1 << 31, "transform grid too large");
     const unsigned nbr = (unsigned)(((nc + XT_C - 1) / XT_C + 7) / 8 * 8);
     const size_t shr = sizeof(double) * XT_L * XT_C * (ks + 2);
@@ -2354,7 +2347,7 @@ void launch_letkf_transform(hipStream_t s, double* X, int k, int ks, int64_t nco
     hipLaunchKernelGGL(k_letkf_transform_reg<KK>, dim3(nbr), dim3(256), shr, s, X, k, ncol, nlev,  \
                        T, col0, nc, status);                                                 \
     break;
-    switch (ks) { MDA_XT(8) MDA_XT(16) MDA_XT(20) MDA_XT(32) MDA_XT(40) MDA_XT(48) MDA_XT(64) }
+    switch (ks) { MDA_XT(8) MDA_XT(20) MDA_XT(40) }
 #undef MDA_XT
     MDA_LAUNCH_CHECK();
     return;
