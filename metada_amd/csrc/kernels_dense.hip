@@ -302,7 +302,7 @@ __global__ __launch_bounds__(512) void k_sym_tridiag_lds(const double* __restric
 // multisection on Sturm counts, 128 points a round for each of the smallest,
 // the largest, the largest negative and the smallest non-negative eigenvalue.
 // out = [lmin, lmax, |l|min, |l|max].  Bound by the chain of the counts, n = 512:
-// 0.25 ms (0.5 ms with the counts by quotients).
+// 0.16 ms (0.5 ms with the counts by quotients).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(512) void k_tridiag_extremes(const double* __restrict__ dg,
                                                           const double* __restrict__ eg, int n,
@@ -411,8 +411,8 @@ void dense_sym_extremes(mda_ctx* c, hipStream_t s, double* A, int64_t p, int64_t
 // (256 workgroups, one per CU): the weighted Gram on FP64 MFMA, the rows of
 // Y_- carried through the factorisation of A, all in LDS.  Eight rounds narrow
 // each bracket by 129^8 = 8e16.  At p = 1,500, k = 80 the dense reduction of S
-// took 33 ms (four launches per column, before
-// the steps above shared one), this 1.8 ms.
+// took 33 ms with four launches per column, this 1.8 ms, on the second stream
+// beside the gain.
 // ---------------------------------------------------------------------------
 constexpr int CE_PTS = 128, CE_ROUNDS = 8;
 
