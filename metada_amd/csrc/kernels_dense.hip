@@ -518,7 +518,8 @@ __global__ __launch_bounds__(256) void k_ce_round(const double* __restrict__ Yf,
     d4 acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = d4{0.0, 0.0, 0.0, 0.0};
-    // one step's rows ahead of the products
+    // one step's rows ahead of the products, where the registers hold them
+    constexpr bool AHEAD = KT < 8;
     double nr = INFINITY, ny[KT];
     auto load = [&](int64_t st) {
       if (st >= nstep) return;
@@ -526,13 +527,14 @@ __global__ __launch_bounds__(256) void k_ce_round(const double* __restrict__ Yf,
 #pragma unroll
       for (int t = 0; t < KT; ++t) ny[t] = Yf[(size_t)(st * KT + t) * 64 + lane];
     };
-    load(wv);
+    if (AHEAD) load(wv);
     for (int64_t st = wv; st < nstep; st += 4) {
+      if (!AHEAD) load(st);
       const double r = nr;
       double y[KT];
 #pragma unroll
       for (int t = 0; t < KT; ++t) y[t] = ny[t];
-      load(st + 4);
+      if (AHEAD) load(st + 4);
       // past p: r = +inf, weight 0
       const double w = kind == 0 ? (r < INFINITY ? 1.0 / (x - r) : 0.0)
                                  : (r > x ? 1.0 / (r - x) : 0.0);
