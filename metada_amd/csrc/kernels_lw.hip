@@ -151,8 +151,9 @@ __global__ void k_lw_innovations(const double* __restrict__ yo, const double* __
 // reaches LDS, and X is read and written once.  The result's members match
 // the fragments of X'_rho lane by lane as well.
 // The taper depends on |s - b| alone: a table of every index distance (one
-// evaluation each, instead of one per state point and observation) is read
-// in windows of p + 32 entries.  Fragments go through two LDS buffers shared
+// evaluation each, instead of one per state point and observation), up to the
+// ends of the last block and the last tile, is read in windows of p + 32
+// entries.  Fragments go through two LDS buffers shared
 // by the block's four wavefronts, and they and the tapers are fetched one tile
 // ahead (read where they are used, they left one wavefront per SIMD waiting on
 // L2 and HBM: 20.9 ms).
@@ -370,7 +371,9 @@ lw_update_shape lw_update_plan(int k, int64_t n, int64_t p) {
   g.ns = (k + 15) / 16 * 4;
   g.ntile = (p + 15) / 16;
   g.nblk = (n + 127) / 128;
-  g.ntap = (n > p ? n : p) + 64;  // padded points and observations look past the ends
+  // whole blocks of points and whole tiles of observations look their distances
+  // up: |s - b| < 128 nblk for s >= b, and < 16 ntile otherwise
+  g.ntap = std::max(128 * g.nblk, 16 * g.ntile);
   return g;
 }
 
@@ -380,6 +383,7 @@ void launch_lw_update(hipStream_t s, double* X, double scale, const double* Gt, 
                       double* partial, double* out4, const int* status) {
   MDA_REQUIRE(k >= 2 && k <= 128, "LWEnKF supports 2 <= k <= 128");
   MDA_REQUIRE(g.nblk < (int64_t)1 << 31, "LWEnKF state too large");
+  MDA_REQUIRE(g.ntap >= 128 * g.nblk && g.ntap >= 16 * g.ntile, "LWEnKF taper table too short");
   hipLaunchKernelGGL(k_lw_fragments, dim3(grid_for(std::max(g.frag_doubles(), g.ntap), 256, 4096)),
                      dim3(256), 0, s, Gt, D, k, p, g.ns, g.ntile, n, g.ntap, radius, fn, gc_form,
                      Gf, Df, tap);

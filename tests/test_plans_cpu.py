@@ -1,0 +1,45 @@
+"""Workspace plans and host paths of the library, without a GPU."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "metada_amd")
+
+
+def _build(tmp, src, out, *link):
+    so = os.path.join(str(tmp), out)
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I", "/opt/rocm/include", "-I", os.path.join(ROOT, "include"),
+                    "-I", os.path.join(PKG, "csrc"), os.path.join(ROOT, "tests", "cpp", src),
+                    "-o", so, *link], check=True, capture_output=True)
+    return so
+
+
+@pytest.fixture(scope="module")
+def ntap(tmp_path_factory):
+    so = _build(tmp_path_factory.mktemp("lw"), "lw_plan_capi.cpp", "liblwplan.so",
+                "-L", PKG, "-l:libmetada_amd.so", "-Wl,-rpath," + PKG)
+    f = C.CDLL(so).lw_plan_ntap
+    f.restype, f.argtypes = C.c_int64, [C.c_int, C.c_int64, C.c_int64]
+    return f
+
+
+@pytest.mark.parametrize("n", [1, 5, 31, 63, 64, 65, 127, 128, 129, 191, 192, 193, 257, 1000, 1153])
+@pytest.mark.parametrize("p", [1, 3, 15, 16, 17, 33, 64, 100, 150, 512, 1025])
+def test_lwenkf_taper_table_covers_every_distance(ntap, n, p):
+    """The update kernel looks up |s - b| for every point s of its blocks (four
+    wavefronts of 32 points) and every observation b of its tiles of 16, those
+    past the ends too: the largest index lies inside the table."""
+    blk, wv, t, lane = np.ogrid[0:(n + 127) // 128, 0:4, 0:2, 0:64]
+    i16, kk = lane & 15, lane >> 4
+    i0 = (blk * 4 + wv) * 32
+    reach = 0
+    for tile in (0, (p + 15) // 16 - 1):
+        for r in range(4):
+            m = i0 + i16 - 16 * tile - kk + 16 * t - 4 * r
+            reach = max(reach, int(np.abs(m).max()))
+    assert reach < ntap(64, n, p)
