@@ -760,6 +760,10 @@ struct letkf_plan {
   int* sweeps = nullptr;
   int64_t* stats = nullptr;
   bool eig_path = false;
+  // false: the observations alone (inflation features).  The column buffers
+  // then stay as the last analysis left them: its transforms, counts and
+  // flags are read from them.
+  bool columns = true;
   // work-queue Gram: cost keys, column order and the counter
   bool queue = false;
   uint32_t *ckeys = nullptr, *ccols = nullptr, *ckeys2 = nullptr, *ccols2 = nullptr,
@@ -784,14 +788,14 @@ static void check_letkf_params(const mda_letkf_params* prm, const mda_geometry* 
 
 static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemble* ens,
                              const mda_geometry* geom, const mda_obs* obs, const mda_hop* hop,
-                             const std::string& pre, bool queue) {
+                             const std::string& pre, bool queue, bool columns = true) {
   check_letkf_params(prm, geom);
   letkf_plan P;
   // argument blocks with zero padding: the batch's graph key holds their bytes
   std::memset(&P.ga, 0, sizeof(P.ga));
   std::memset(&P.sa, 0, sizeof(P.sa));
   std::memset(&P.bg, 0, sizeof(P.bg));
-  P.prm = prm; P.ens = ens; P.geom = geom;
+  P.prm = prm; P.ens = ens; P.geom = geom; P.columns = columns;
   P.de = stage_ensemble(c, ens);
   P.o = stage_obs(c, obs, true, /*allow_empty=*/true);
   if (P.o.p > 0) P.h = stage_hop(c, hop, P.de.k, P.o.p, P.de.n);
@@ -903,6 +907,11 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
     ga.uy = c->get<double>(pre + "s_uy", p);
     ga.uz = c->get<double>(pre + "s_uz", p);
   }
+  if (!columns) {
+    P.sa.status = c->get<int>(pre + "obs_status", 1);
+    c->send_staged();
+    return P;
+  }
   // Column passes: at k > 64 the per-column k x k buffers of the whole grid
   // would not fit in HBM next to the ensemble (3 x 69 GB at k = 128 and
   // 524,288 columns), so the columns run in passes of 65,536.
@@ -988,12 +997,16 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
 // its rows are moved into bucket order afterwards.  Both idempotent.
 static void enqueue_buckets(hipStream_t s, letkf_plan& P) {
   letkf_gram_args& ga = P.ga;
-  letkf_begin_args b{};
-  b.ncol = P.ncol; b.npass = n_passes(P);
-  b.status = P.sa.status; b.sweeps = P.sweeps; b.flag = P.sa.flag;
-  b.nloc = P.p == 0 ? ga.nloc : nullptr;
-  b.stats = P.stats; b.wcount = P.sa.wcount; b.shell_count = ga.shell_count;
-  launch_letkf_begin(s, b);
+  if (P.columns) {
+    letkf_begin_args b{};
+    b.ncol = P.ncol; b.npass = n_passes(P);
+    b.status = P.sa.status; b.sweeps = P.sweeps; b.flag = P.sa.flag;
+    b.nloc = P.p == 0 ? ga.nloc : nullptr;
+    b.stats = P.stats; b.wcount = P.sa.wcount; b.shell_count = ga.shell_count;
+    launch_letkf_begin(s, b);
+  } else {
+    launch_zero(s, P.sa.status, sizeof(int));
+  }
   if (P.p == 0) return;  // every column takes the empty-column branch
   obs_prepare_args q{};
   q.p = P.p; q.nxy = P.nx * P.ny;
@@ -1018,7 +1031,7 @@ static void enqueue_buckets(hipStream_t s, letkf_plan& P) {
                     const_cast<double*>(ga.ux), const_cast<double*>(ga.uy),
                     const_cast<double*>(ga.uz), P.ipos);
   // window geometry of every column for the Gram
-  launch_column_setup(s, ga);
+  if (P.columns) launch_column_setup(s, ga);
 }
 
 static void enqueue_local(hipStream_t s, letkf_plan& P) {
@@ -1563,8 +1576,8 @@ int mda_letkf_inflation_features(mda_ctx* c, const mda_letkf_params* prm,
     mda_letkf_params fp = *prm;
     fp.precision = MDA_PREC_FP64;
     fp.rho_column = nullptr;
-    letkf_plan P = plan_letkf(c, &fp, const_cast<mda_ensemble*>(ens), geom, obs, hop, "",
-                              false);
+    letkf_plan P = plan_letkf(c, &fp, const_cast<mda_ensemble*>(ens), geom, obs, hop, "", false,
+                              /*columns=*/false);
     MDA_REQUIRE(P.p > 0, "inflation features need observations");
     enqueue_buckets(s, P);
     enqueue_local(s, P);

@@ -135,6 +135,7 @@ struct mda_ctx {
       // a cached graph may hold the old address: drop them all (their keys
       // hold every address they use, so none would match again anyway)
       drop_graphs();
+      forget_results(b.ptr);
       if (b.ptr) MDA_HIP(hipFree(b.ptr));
       b.ptr = nullptr;
       b.bytes = 0;
@@ -147,6 +148,12 @@ struct mda_ctx {
   template <class T>
   T* get(const std::string& name, size_t count) {
     return static_cast<T*>(get(name, count * sizeof(T)));
+  }
+  // results of the last LETKF call that lie in a buffer about to be freed
+  void forget_results(const void* ptr) {
+    if (last_T == ptr) last_T = nullptr;
+    if (last_nloc == ptr) last_nloc = nullptr;
+    if (last_flag == ptr) last_flag = nullptr;
   }
   void drop_graphs() {
     for (auto& kv : graphs)
