@@ -231,26 +231,23 @@ int mda_ctx_create(int device, mda_ctx** out) {
   int ndev = 0;
   if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return MDA_E_DEVICE;
   if (device < 0 || device >= ndev) return MDA_E_ARG;
+  int prev = 0;
+  if (hipGetDevice(&prev) != hipSuccess) return MDA_E_DEVICE;
   mda_ctx* c = new mda_ctx();
   c->device = device;
-  int prev = 0;
-  if (hipGetDevice(&prev) != hipSuccess || hipSetDevice(device) != hipSuccess ||
-      hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
-    delete c;
-    return MDA_E_DEVICE;
-  }
-  for (auto& e : c->ev) {
-    if (hipEventCreate(&e) != hipSuccess) {
-      delete c;
-      return MDA_E_DEVICE;
-    }
-  }
+  auto created = [](hipError_t e) {
+    if (e != hipSuccess) throw mda_error(MDA_E_DEVICE, hipGetErrorString(e));
+  };
   try {
+    created(hipSetDevice(device));
+    created(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
+    for (auto& e : c->ev) created(hipEventCreate(&e));
     c->create_staging();
   } catch (const mda_error& e) {
-    c->destroy_staging();
-    delete c;
-    return e.code;
+    const int rc = e.code;
+    (void)mda_ctx_destroy(c);  // what there is of it
+    (void)hipSetDevice(prev);
+    return rc;
   }
   (void)hipSetDevice(prev);
   *out = c;

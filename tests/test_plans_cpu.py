@@ -2,6 +2,7 @@
 import ctypes as C
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -43,3 +44,33 @@ def test_lwenkf_taper_table_covers_every_distance(ntap, n, p):
             m = i0 + i16 - 16 * tile - kk + 16 * t - 4 * r
             reach = max(reach, int(np.abs(m).max()))
     assert reach < ntap(64, n, p)
+
+
+CTX_CREATE = """
+import ctypes as C, sys
+mock = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+lib = C.CDLL(sys.argv[2])
+h = C.c_void_p()
+mock.mock_refuse(0)
+assert lib.mda_ctx_create(0, C.byref(h)) == 0 and mock.mock_device() == 1
+n = mock.mock_calls()
+assert lib.mda_ctx_destroy(h) == 0 and mock.mock_alive() == 0
+for i in range(1, n + 1):
+    mock.mock_refuse(i)
+    rc = lib.mda_ctx_create(0, C.byref(h))
+    print(i, rc, mock.mock_alive(), mock.mock_device(), h.value)
+"""
+
+
+def test_context_creation_that_fails_leaves_nothing_behind(tmp_path):
+    """Whichever stream, event or staging buffer cannot be had: nothing stays
+    allocated and the thread is back on its device."""
+    so = _build(tmp_path, "hip_mock.cpp", "libhipmock.so")
+    out = subprocess.run([sys.executable, "-c", CTX_CREATE, so,
+                          os.path.join(PKG, "libmetada_amd.so")],
+                         check=True, capture_output=True, text=True).stdout.splitlines()
+    got = [line.split() for line in out]
+    assert len(got) == 16  # stream, twelve events, two pinned buffers, one on the device
+    for i, (_, rc, alive, dev, h) in enumerate(got):
+        assert int(rc) == (-3 if i >= 13 else -2), got[i]
+        assert (alive, dev, h) == ("0", "1", "None"), got[i]
