@@ -498,7 +498,7 @@ __global__ __launch_bounds__(256) void k_fold_extremes(const double* __restrict_
                                                        int64_t nb, double* __restrict__ out) {
   __shared__ double r0[256], r1[256], r2[256], r3[256];
   const int tid = threadIdx.x;
-  double mx = -1.0e308, mn = 1.0e308, s2 = 0.0, s3 = 0.0;
+  double mx = -INFINITY, mn = INFINITY, s2 = 0.0, s3 = 0.0;
 #pragma unroll 4
   for (int64_t b = tid; b < nb; b += 256) {
     mx = fmax(mx, partial[4 * b]);

@@ -80,3 +80,21 @@ def test_features_leave_the_last_analysis_readable(mda, ctx, k, prec):
     e2.data[:] = ens.data
     np.testing.assert_array_equal(_features(c2, f2), feat)
     c2.close()
+
+
+# ---- gain extremes when no entry of the gain is a number ------------------------------------
+def test_lwenkf_extremes_of_a_gain_without_numbers(mda, ctx):
+    """A background of NaN with finite H(x): the LWEnKF has no gain entry to
+    compare and reports the empty maximum and minimum, -inf and +inf."""
+    k, n, p = 8, 200, 20
+    rng = np.random.default_rng(3)
+    ens = mda.Ensemble(np.full((k, n), np.nan), n, 1, 1)
+    f = mda.LWEnKF(ens, mda.Observation(rng.standard_normal(p), np.ones(p), np.zeros(p),
+                                        np.zeros(p)),
+                   mda.ObsOperator(hx=rng.standard_normal((k, p))),
+                   mda.Config({"analysis": {"inflation": 1.1, "localization_radius": 0.3,
+                                            "localization_function": "gaussian",
+                                            "weighting_scheme": "uniform"}}), ctx=ctx)
+    f.Analyse(Z=rng.standard_normal((p, k)))
+    r = f.getAnalysisResults()
+    assert r["max_kalman_gain"] == -np.inf and r["min_kalman_gain"] == np.inf
