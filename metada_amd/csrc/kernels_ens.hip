@@ -773,14 +773,14 @@ void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, d
 // Metrics::CalculateAll (Metrics.hpp:74-94): per-block partial sums of
 // [rmse^2, bias, sum mean, sum truth, sum mean*truth, sum mean^2,
 //  sum truth^2, spread, crps].
-// One point per thread.  Up to 128 members sit in registers (KM of them; the
-// entries past k repeat member 0), and the CRPS's k^2 differences take each
-// member once more from the cache against all the registers: two FP64
+// One point per thread.  Up to 128 members sit in registers (KM of them), and
+// the CRPS's k^2 differences take each member once more from the cache against
+// all the registers, against itself in place of the entries past k: two FP64
 // operations a pair and X read from HBM once.  n = 1,048,576, k = 40: 192 us
 // (3.56 ms with both members of every pair loaded).  Beyond 128 members
 // (KM = 0) that form remains.
 // ---------------------------------------------------------------------------
-template <int KM>
+template <int KM, bool WHOLE>  // WHOLE: k = KM
 __global__ __launch_bounds__(256) void k_metrics(const double* __restrict__ X, int k, int64_t n,
                                                  const double* __restrict__ truth,
                                                  double* __restrict__ partial) {
@@ -793,22 +793,20 @@ __global__ __launch_bounds__(256) void k_metrics(const double* __restrict__ X, i
     if constexpr (KM > 0) {
       double x[KM];
 #pragma unroll
-      for (int j = 0; j < KM; ++j) x[j] = j < k ? X[(size_t)j * n + i] : 0.0;
+      for (int j = 0; j < KM; ++j) x[j] = WHOLE || j < k ? X[(size_t)j * n + i] : 0.0;
 #pragma unroll
       for (int j = 0; j < KM; ++j) m += x[j];
       m /= (double)k;  // Metrics.hpp:111-113 divides
-      double s0 = 0.0;  // sum over members of |x_j - x_0|
 #pragma unroll
       for (int j = 0; j < KM; ++j) {
         const double df = x[j] - m;
-        if (j < k) {
+        if (WHOLE || j < k) {
           sp += df * df;
           st += fabs(x[j] - t);
-          s0 += fabs(x[j] - x[0]);
-        } else {
-          x[j] = x[0];
         }
       }
+      // entries that every k of this kernel fills
+      constexpr int FULL = WHOLE ? KM : KM - (KM > 64 ? 16 : 8) + 1;
       double d0 = 0.0, d1 = 0.0;
       double xn = x[0];
       for (int a = 0; a < k; ++a) {
@@ -816,11 +814,11 @@ __global__ __launch_bounds__(256) void k_metrics(const double* __restrict__ X, i
         if (a + 1 < k) xn = X[(size_t)(a + 1) * n + i];  // in flight during the pairs
 #pragma unroll
         for (int b = 0; b < KM; b += 2) {
-          d0 += fabs(xa - x[b]);
-          d1 += fabs(xa - x[b + 1]);
+          d0 += fabs(xa - (b < FULL || b < k ? x[b] : xa));
+          d1 += fabs(xa - (b + 1 < FULL || b + 1 < k ? x[b + 1] : xa));
         }
       }
-      sd = (d0 + d1) - (double)(KM - k) * s0;
+      sd = d0 + d1;
     } else {
       for (int j = 0; j < k; ++j) m += X[(size_t)j * n + i];
       m /= (double)k;
@@ -849,22 +847,30 @@ __global__ __launch_bounds__(256) void k_metrics(const double* __restrict__ X, i
 void launch_metrics(hipStream_t s, const double* X, int k, int64_t n, const double* truth,
                     double* partial, double* out9) {
   const unsigned nb = grid_for(n, 256, METRICS_BLOCKS);
-#define MDA_MT(KM) \
-  hipLaunchKernelGGL(k_metrics<KM>, dim3(nb), dim3(256), 0, s, X, k, n, truth, partial)
-  if (k <= 8) MDA_MT(8);
-  else if (k <= 16) MDA_MT(16);
-  else if (k <= 24) MDA_MT(24);
-  else if (k <= 32) MDA_MT(32);
-  else if (k <= 40) MDA_MT(40);
-  else if (k <= 48) MDA_MT(48);
-  else if (k <= 56) MDA_MT(56);
-  else if (k <= 64) MDA_MT(64);
-  else if (k <= 80) MDA_MT(80);
-  else if (k <= 96) MDA_MT(96);
-  else if (k <= 112) MDA_MT(112);
-  else if (k <= 128) MDA_MT(128);
-  else MDA_MT(0);
+#define MDA_MTL(KM, WHOLE)                                                                 \
+  hipLaunchKernelGGL((k_metrics<KM, WHOLE>), dim3(nb), dim3(256), 0, s, X, k, n, truth, partial)
+#define MDA_MT(KM)                \
+  {                               \
+    if (k == KM)                  \
+      MDA_MTL(KM, true);          \
+    else                          \
+      MDA_MTL(KM, false);         \
+  }
+  if (k <= 8) MDA_MT(8)
+  else if (k <= 16) MDA_MT(16)
+  else if (k <= 24) MDA_MT(24)
+  else if (k <= 32) MDA_MT(32)
+  else if (k <= 40) MDA_MT(40)
+  else if (k <= 48) MDA_MT(48)
+  else if (k <= 56) MDA_MT(56)
+  else if (k <= 64) MDA_MT(64)
+  else if (k <= 80) MDA_MT(80)
+  else if (k <= 96) MDA_MT(96)
+  else if (k <= 112) MDA_MT(112)
+  else if (k <= 128) MDA_MT(128)
+  else MDA_MTL(0, false);
 #undef MDA_MT
+#undef MDA_MTL
   MDA_LAUNCH_CHECK();
   launch_reduce_partials(s, partial, (int)nb, 9, out9);
 }

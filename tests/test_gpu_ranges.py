@@ -390,3 +390,17 @@ def test_host_arrays_equal_device_arrays(mda, ctx, nx, p):
     for where in ("device", "host again"):
         for u, v in zip(out["host"], out[where]):
             np.testing.assert_array_equal(u, v)
+
+
+@pytest.mark.parametrize("k", [2, 3, 9, 17, 65, 81, 97])
+def test_metrics_crps_with_an_outlying_first_member(mda, ctx, k):
+    """One point, member 0 at the power of two V, the others at zero, V so large
+    that its 2 (k - 1) differences add up to at most 1.2e308: whole multiples
+    of V, exact.  The score is V / k - (k - 1) V / k^2 = V / k^2, off by the
+    rounding of the two quotients (eps / 2 of V / k each) and of their
+    difference; a pair sum with more copies of member 0 would overflow."""
+    V = 2.0 ** np.floor(np.log2(0.6e308 / (k - 1)))
+    X = np.zeros((k, 1))
+    X[0] = V
+    m = mda.metrics(mda.Ensemble(X, 1, 1, 1), np.zeros(1), ctx=ctx)
+    assert abs(m["crps"] / (V / k / k) - 1.0) <= (k + 3) * np.finfo(float).eps
