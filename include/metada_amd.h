@@ -250,8 +250,8 @@ typedef struct {
                                   (split-precision bf16 products, FP32 accumulation; k a
                                   multiple of 16, at most 64) */
   int32_t keep_transforms;     /* 1: keep every column's T for mda_letkf_last_transforms.
-                                  0 (the default): at k in 9..16 and 21..64 but 33..40
-                                  with the tridiagonal eigensolver, the matrix combination and an
+                                  0 (the default): at k in {16, 32, 48, 64} with the
+                                  tridiagonal eigensolver, the matrix combination and an
                                   FP64 transform, the eigenvector kernel applies
                                   X_a = X T' itself and T is not stored */
 } mda_letkf_params;

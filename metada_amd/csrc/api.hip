@@ -978,8 +978,10 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
     sa.null_rel = 0.0;
     sa.eig_nloc = c->get<int>(pre + "eig_nloc", ncol);
   }
-  // E3 applies the transform itself unless T is to be kept
-  sa.fuse = P.eig_path && !sa.eig_nloc && letkf_eig_fusable(ks) && prm->combine == MDA_COMBINE_MATRIX &&
+  // E3 applies the transform itself unless T is to be kept.  An ensemble in a
+  // larger block keeps T: mda_letkf_last_transforms answers there without
+  // keep_transforms.
+  sa.fuse = P.eig_path && ks == k && letkf_eig_fusable(ks) && prm->combine == MDA_COMBINE_MATRIX &&
             prm->transform_precision == MDA_PREC_FP64 && !prm->keep_transforms;
   c->send_staged();
   return P;

@@ -98,3 +98,21 @@ def test_lwenkf_extremes_of_a_gain_without_numbers(mda, ctx):
     f.Analyse(Z=rng.standard_normal((p, k)))
     r = f.getAnalysisResults()
     assert r["max_kalman_gain"] == -np.inf and r["min_kalman_gain"] == np.inf
+
+
+# ---- transforms without keep_transforms ------------------------------------------------------
+@pytest.mark.parametrize("prec", ["FP64", "FP32", "BF16X3"])
+@pytest.mark.parametrize("k", [7, 10, 15, 21, 25, 31, 41, 47, 49, 50, 63, 80])
+def test_transforms_between_block_sizes_are_readable(mda, ctx, k, prec):
+    """Only k in {16, 32, 48, 64} need keep_transforms: elsewhere the default
+    stores T, the same one, and the analysis is the same to the bit."""
+    case = latlon_case(nlon=18, nlat=9, nlev=3, k=k, p=400, seed=800 + k)
+    kw = {"precision": getattr(mda._lib, "PREC_" + prec)}
+    cols = np.array([0, 40, 80, 161])
+    f, ens = _letkf(mda, ctx, case, 2500.0, **kw)
+    f.Analyse()
+    T = f.transforms(cols)
+    g, ens_kept = _letkf(mda, ctx, case, 2500.0, keep_transforms=True, **kw)
+    g.Analyse()
+    np.testing.assert_array_equal(T, g.transforms(cols))
+    np.testing.assert_array_equal(ens.data, ens_kept.data)
