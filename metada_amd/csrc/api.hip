@@ -978,6 +978,9 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
     sa.null_rel = 0.0;
     sa.eig_nloc = c->get<int>(pre + "eig_nloc", ncol);
   }
+  // An FP64 ensemble in a larger block is as close to 64 bits as Jacobi leaves
+  // it (E4)
+  sa.refine = P.eig_path && ks != k && prm->precision == MDA_PREC_FP64;
   // E3 applies the transform itself unless T is to be kept.  An ensemble in a
   // larger block keeps T: mda_letkf_last_transforms answers there without
   // keep_transforms.

@@ -16,13 +16,16 @@
 // A column that fails a check (or QL non-convergence) is flagged and
 // re-solved by the parallel-order Jacobi kernel.
 //
+//   E4  k_trd_root: for an FP64 ensemble in a block larger than k, Z = A^-1/2
+//       corrected against A, and T from it (E3 writes Z alone then).
+//
 // The kernels are compiled for block sizes N; an ensemble of km < N members
 // runs in the next larger block.  The Gram's zeros past km make the block
 // diag(A, sigma I): the padding decouples (zero reflector entries, e_i = 0),
 // its eigenvalues are sigma exactly, which E3 leaves out as it does the null
-// space, and km enters only sigma and the scale of W.  Measured at 200 x 160
-// columns of 30 levels, k = 50 (N = 64): Jacobi and the stored transform took
-// 68.4 ms, these kernels with the transform in E3 take 4.5 ms.
+// space, and km enters only sigma and the scale of W.  200 x 160 columns of
+// 30 levels, k = 50 (N = 64): Jacobi and the stored transform take 68.4 ms,
+// these kernels with E4 and the stored transform 7.9 ms.
 #include "mda_device.hpp"
 #include "mda_internal.hpp"
 #include "mda_xform.hpp"
@@ -433,6 +436,9 @@ __device__ inline double fast_div(double a, double b) {
   return fma(q, fma(e, e, e), q);
 }
 
+// in place of a combination: T = A^-1/2 alone, for E4
+constexpr int EIG_ROOT_ONLY = -1;
+
 constexpr int E3_SUB = 4;  // reflectors per static range in the back-transform
 
 // global_load_lds instructions that stage chunk c of the Householder rows in
@@ -767,7 +773,8 @@ __device__ __forceinline__ bool e3_column(
     for (int e2 = 0; e2 < N; ++e2) acc += Z[lane * ld + e2] * sy[e2];
     wbar = sc * (sb[lane] / sigma - acc);
   }
-  const double coef = sqrt((double)(km - 1)) * sqrt(sc);
+  const double coef =
+      combine == EIG_ROOT_ONLY ? 1.0 : sqrt((double)(km - 1)) * sqrt(sc);
   const double fs = 1.0 / sqrt(sigma);
   if (combine == MDA_COMBINE_ELEMENTWISE) {
     // t_i = wbar_i + coef (f(sigma) - sum_a U_s[i][a] (sum_j U_s[j][a]))
@@ -790,7 +797,7 @@ __device__ __forceinline__ bool e3_column(
     return false;
   }
   wave_lds_sync();
-  sy[lane] = wbar;
+  sy[lane] = combine == EIG_ROOT_ONLY ? 0.0 : wbar;
   wave_lds_sync();
   // ---- W = coef (f(sigma) I - U_s U_s^T) on FP64 MFMA (lower tiles, mirrored) ----
   constexpr int nt = NP / 16;
@@ -954,14 +961,15 @@ constexpr int E1W_CH = 8;  // step chunk of the k = 128 E1 (static column ranges
 // E2 by bisection on Sturm counts (one wavefront per column, lane j owns
 // eigenvalues j, j + 64, ...): counts by sign changes of the leading minors
 // (sturm_counts).  Starts from the Gershgorin interval cut into 65 cells by one
-// multisection sweep and halves until the interval is within 1e-13 of the
-// eigenvalue (relative).  Ascending by construction.  Bound by the issue of
+// multisection sweep and halves until the interval is within rel of the
+// eigenvalue.  Ascending by construction.  Bound by the issue of
 // vector instructions: k = 128, 18,432 columns 2.5 ms, 5.0 ms with the counts by
 // the quotients of the pivots.
 template <int N>
 __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
                                                             const int* __restrict__ nloc,
                                                             const double* __restrict__ de,
+                                                            double rel,
                                                             double* __restrict__ lam,
                                                             int* __restrict__ flag) {
   constexpr int n = N, n8 = (N + 7) / 8 * 8, NQ = (N + 63) / 64;
@@ -1023,11 +1031,6 @@ __global__ __launch_bounds__(256) void k_trd_eigvals_bisect(int64_t ncol,
       else b[q] = fmin(b[q], xm);
     }
   }
-  // k = 128 converges at a relative width of 1e-13: the eigenvector checks ask
-  // for a residual within 1e-12 of ||T|| and the transform for 1e-10, and the last
-  // eight halvings to 2 eps would add 14 % to the sweeps.  Where QL is the other
-  // way, the result is as close as QL's.
-  const double rel = N > 64 ? 1e-13 : 4.0 * eps;
   for (int it = 0; it < 128; ++it) {
     bool open = false;
     double x[NQ];
@@ -1617,7 +1620,8 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
     }
   }
   __syncthreads();
-  const double coef = sqrt((double)(km - 1)) * sqrt(sc);
+  const double coef =
+      combine == EIG_ROOT_ONLY ? 1.0 : sqrt((double)(km - 1)) * sqrt(sc);
   const double fs = 1.0 / sqrt(sigma);
   // wbar_j = s [ b_j / sigma - sum_e U_s[j][e] y'_e ], row j by its pair
   double wbar;
@@ -1641,7 +1645,7 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
     }
   }
   __syncthreads();  // sy (y') reads done
-  if (h == 0) sy[j] = wbar;
+  if (h == 0) sy[j] = combine == EIG_ROOT_ONLY ? 0.0 : wbar;
   __syncthreads();
   // ---- W = coef (f(sigma) I - U_s U_s^T) on FP64 MFMA, tiles round-robin ----
   constexpr int nt = N / 16;
@@ -1669,6 +1673,268 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
 }
 
 // ---------------------------------------------------------------------------
+// E4: the inverse square root corrected against the matrix itself, then T, for
+// ensembles in a block larger than k (in their place Jacobi was used before).
+// An eigensolution through a tridiagonal matrix carries eps ||A|| into every
+// eigenvalue, which is eps ||A|| / sigma relative to the smallest; Jacobi's
+// rounding is relative to each.  With Z from E3, R = I - Z A Z and W = Z R Z,
+//   Z <- Z + sqrt(sigma) (1/2 + 1/a) W - sigma / (2 a) (Z W + W Z),  a = 0.7,
+// multiplies an error of Z in the direction of eigenvectors i and j by
+// (1 - s / 2)(1 - s / a), s = sqrt(sigma / lambda_i) + sqrt(sigma / lambda_j):
+// zero at sigma, where that error lies, within 0.3 up to lambda = 8 sigma, and
+// nowhere above 1.  R holds eps sqrt(||A|| / sigma) of rounding.  Error of the
+// analysis against 64 bits (200 x 160 columns, k = 50): 5.8e-14 from E3, 2.0e-15
+// here, 3.8e-15 by Jacobi.  wbar = s A^-1 b from the corrected Z, by Z (Z b) and one
+// step on its residual.
+// On FP64 MFMA, a wavefront per 16 columns of Z: register r of tile t of a
+// product (rows 16 t + kk + 4 r) is the right operand of the step over the
+// rows 16 t + 4 r .. + 3, so Z (A Z) and Z (R Z) run from register to
+// register, and as Z, A and R are symmetric their left operands are read by
+// rows.  Z in LDS (and R for N <= 64, in U[g] beyond), A = C + sigma I from
+// the cache.  Seven products of N^3; bound by them and, with two columns a CU, by
+// the loads and barriers between them: N = 64, 32,000 columns 2.46 ms (1.6 ms of
+// matrix products), N = 128, 2,592 columns 2.3 ms.
+// ---------------------------------------------------------------------------
+constexpr double E4_A = 0.7;
+
+// hi + lo += a b, the rounding of the product and of the sum kept in lo
+__device__ __forceinline__ void two_add(double& hi, double& lo, double a, double b) {
+#pragma clang fp contract(off)
+  const double p = a * b, pe = fma(a, b, -p), s = hi + p, t = s - hi;
+  lo += ((hi - (s - t)) + (p - t)) + pe;
+  hi = s;
+}
+
+template <int N>
+struct e4_shape {
+  static constexpr int NP = (N + 15) / 16 * 16, NT = NP / 16, NS = NP / 4;
+  static constexpr bool R_LDS = N <= 64;
+  static constexpr bool AHEAD = N <= 64;  // a lane's entries of A fit in its registers
+  static constexpr size_t LDS = sizeof(double) * ((R_LDS ? 2 : 1) * NP * NP + 12 * NP);
+  // entry (r, c) of a matrix in LDS: rows of an even number of tiles are 0 mod
+  // 64 banks apart, so odd rows have neighbouring tiles changed over
+  static __device__ __forceinline__ int at(int r, int c) {
+    return r * NP + (NT % 2 == 0 ? c ^ ((r & 1) << 4) : c);
+  }
+};
+
+template <int N>
+__global__ __launch_bounds__(64 * e4_shape<N>::NT) __attribute__((amdgpu_waves_per_eu(2)))
+void k_trd_root(
+    int64_t ncol, const double* __restrict__ C, const int* __restrict__ nloc,
+    const double* __restrict__ bvec, int km, double rho, const double* __restrict__ rho_col,
+    int prior, int combine, double* __restrict__ U, double* __restrict__ T,
+    const int* __restrict__ flag) {
+  using S = e4_shape<N>;
+  constexpr int NP = S::NP, NT = S::NT, NS = S::NS, THREADS = 64 * NT;
+  extern __shared__ double sh[];
+  double* zl = sh;
+  double* vec = sh + (S::R_LDS ? 2 : 1) * NP * NP;
+  double *sb = vec, *sy = vec + NP, *sw = vec + 2 * NP, *st = vec + 3 * NP;
+  double *red = vec + 4 * NP, *red2 = vec + 8 * NP;  // [4][NP]
+  const int64_t g = blockIdx.x;
+  if (g >= ncol || nloc[g] == 0 || flag[g]) return;  // block-uniform
+  const int tid = threadIdx.x, lane = tid & 63, i16 = lane & 15, kk = lane >> 4;
+  const int cj = 16 * (tid >> 6) + i16;  // this lane's column of Z
+  const double r = rho_col ? rho_col[g] : rho;
+  const double sigma = prior ? (double)(km - 1) / r : (double)(km - 1);
+  const double* Cg = C + (size_t)g * N * N;
+  double* Tg = T + (size_t)g * N * N;
+  double* Rg = S::R_LDS ? sh + NP * NP : U + (size_t)g * N * N;
+  // Rows 4 s + kk have the parity of kk.  Of such a row of Z: this lane's
+  // column (at row 0: zc), and its entries 16 ti + i16 (ze of the even, zo of the
+  // odd tiles); the same of R
+  const int sw16 = NT % 2 == 0 ? (kk & 1) << 4 : 0;
+  constexpr int RS = S::R_LDS ? NP : N;  // row stride of R
+  const int rsw = S::R_LDS ? sw16 : 0;
+  double* zc = zl + kk * NP + (cj ^ sw16);
+  auto r_column = [&] {  // its addresses formed where they are used, not kept
+    int at = kk * RS + (cj ^ rsw);
+    __asm__ volatile("" : "+v"(at));
+    return Rg + at;
+  };
+  const double *ze = zl + kk * NP + i16 + sw16, *zo = zl + kk * NP + i16 + 16 - sw16;
+  const double *re = Rg + kk * RS + i16 + rsw, *ro = Rg + kk * RS + i16 + 16 - rsw;
+  auto zrow = [&](int s, int ti) {
+    return (NT % 2 == 0 && (ti & 1) ? zo : ze)[4 * s * NP + 16 * (NT % 2 == 0 ? ti & ~1 : ti)];
+  };
+  auto rrow = [&](int s, int ti) {
+    return (NT % 2 == 0 && (ti & 1) ? ro : re)[4 * s * RS + 16 * (NT % 2 == 0 ? ti & ~1 : ti)];
+  };
+  // A[4 s + kk][16 ti + i16]
+  auto entry = [&](int s, int ti) {
+    const int row = 4 * s + kk, col = 16 * ti + i16;
+    return (row < N && col < N ? Cg[row * N + col] : 0.0) + (row == col ? sigma : 0.0);
+  };
+  double av[S::AHEAD ? NS : 1][NT];
+  if constexpr (S::AHEAD) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti) av[s][ti] = entry(s, ti);
+  }
+#pragma unroll 16
+  for (int m = 0; m < NP / 4; ++m) {
+    const int i = 4 * m + tid / NP, c = tid % NP;
+    zl[S::at(i, c)] = i < N && c < N ? Tg[i * N + c] : i == c ? 1.0 / sqrt(sigma) : 0.0;
+  }
+  for (int i = tid; i < NP; i += THREADS) sb[i] = i < N ? bvec[(size_t)g * N + i] : 0.0;
+  __syncthreads();
+  // the wide form's registers: bounds what is loaded ahead
+  auto bound = [] {
+    if (!S::AHEAD) lds_reload_point();
+  };
+  d4 p[NT], q[NT];
+  // q = Z p, from p's registers
+  auto z_times_p = [&] {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) q[t] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if ((e & 1) == 0) bound();
+#pragma unroll
+        for (int ti = 0; ti < NT; ++ti)
+          q[ti] = __builtin_amdgcn_mfma_f64_16x16x4f64(zrow(4 * t + e, ti), p[t][e], q[ti], 0, 0, 0);
+      }
+  };
+  // p = A Z.  A z is far below A where z belongs to a small eigenvalue, so the
+  // leading 23 bits of both go into p, whose sums are exact, and the rest into q
+  double big = 0.0;
+  for (int i = lane; i < N; i += 64) big = fmax(big, Cg[i * (N + 1)]);
+  for (int off = 32; off > 0; off >>= 1) big = fmax(big, __shfl_xor(big, off));
+  const double ra = __builtin_amdgcn_ldexp(1.5, __builtin_amdgcn_frexp_exp(big + sigma) + 29),
+               rz = __builtin_amdgcn_ldexp(1.5, __builtin_amdgcn_frexp_exp(1.01 / sqrt(sigma)) + 29);
+#pragma unroll
+  for (int t = 0; t < NT; ++t) p[t] = q[t] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll S::AHEAD ? NS : 2
+  for (int s = 0; s < NS; ++s) {
+    bound();
+    const double b = zc[4 * s * NP], b1 = (b + rz) - rz, b2 = b - b1;
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti) {
+      const double a = S::AHEAD ? av[S::AHEAD ? s : 0][ti] : entry(s, ti), a1 = (a + ra) - ra;
+      p[ti] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, p[ti], 0, 0, 0);
+      q[ti] = __builtin_amdgcn_mfma_f64_16x16x4f64(a - a1, b, q[ti], 0, 0, 0);
+      q[ti] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b2, q[ti], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int t = 0; t < NT; ++t) p[t] += q[t];
+  z_times_p();
+  double* rc = r_column();
+#pragma unroll
+  for (int ti = 0; ti < NT; ++ti) {
+    bound();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      rc[(16 * ti + 4 * e) * RS] = (16 * ti + kk + 4 * e == cj ? 1.0 : 0.0) - q[ti][e];
+      p[ti][e] = 0.0;
+    }
+  }
+  __syncthreads();
+#pragma unroll S::AHEAD ? 4 : 2
+  for (int s = 0; s < NS; ++s) {  // p = R Z
+    bound();
+    const double b = zc[4 * s * NP];
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti)
+      p[ti] = __builtin_amdgcn_mfma_f64_16x16x4f64(rrow(s, ti), b, p[ti], 0, 0, 0);
+  }
+  z_times_p();
+  // q = W; then Z W and its transpose
+#pragma unroll
+  for (int ti = 0; ti < NT; ++ti) p[ti] = q[ti];
+  __syncthreads();  // R has been read
+  z_times_p();
+  rc = r_column();
+#pragma unroll
+  for (int ti = 0; ti < NT; ++ti) {
+    bound();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) rc[(16 * ti + 4 * e) * RS] = q[ti][e];
+  }
+  __syncthreads();  // Z has been read, Z W is there
+  const double c1 = sqrt(sigma) * (0.5 + 1.0 / E4_A), c2 = -sigma * (0.5 / E4_A);
+#pragma unroll
+  for (int ti = 0; ti < NT; ++ti) {
+    bound();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int row = 16 * ti + kk + 4 * e;
+      const double t = q[ti][e] + Rg[S::R_LDS ? S::at(cj, row) : cj * N + row];
+      double* z = zc + (16 * ti + 4 * e) * NP;
+      *z = fma(c1, p[ti][e], fma(c2, t, *z));
+    }
+  }
+  __syncthreads();
+  // out[i] = scale sum_c Z[c][i] in[c] (in = null: ones), four threads an entry
+  auto times_z = [&](const double* in, double scale, double* out) {
+    const int i = tid % NP, c0 = tid / NP * (NP / 4);
+    double s = 0.0;
+#pragma unroll 16
+    for (int c = c0; c < c0 + NP / 4; ++c) s = fma(zl[S::at(c, i)], in ? in[c] : 1.0, s);
+    red[tid] = s;
+    __syncthreads();
+    if (tid < NP)
+      out[tid] = scale * ((red[tid] + red[NP + tid]) + (red[2 * NP + tid] + red[3 * NP + tid]));
+    __syncthreads();
+  };
+  // w = A^-1 b, and its residual b - A w in twice the working precision: the
+  // entries of b - A w are far below those of b
+  times_z(sb, 1.0, sy);
+  times_z(sy, 1.0, sw);
+  {
+    const int i = tid % NP, c0 = tid / NP * (NP / 4);
+    double hi = 0.0, lo = 0.0;
+#pragma unroll 8
+    for (int m = 0; m < NP / 4; ++m)
+      two_add(hi, lo, i < N && c0 + m < N ? Cg[(c0 + m) * N + i] : 0.0, sw[c0 + m]);
+    red[tid] = hi;
+    red2[tid] = lo;
+    __syncthreads();
+    if (tid < NP) {
+      hi = sb[tid];
+      lo = 0.0;
+      two_add(hi, lo, -sigma, sw[tid]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        two_add(hi, lo, -1.0, red[q * NP + tid]);
+        lo -= red2[q * NP + tid];
+      }
+      sy[tid] = hi + lo;
+    }
+    __syncthreads();
+  }
+  times_z(sy, 1.0, st);
+  times_z(st, 1.0, sy);
+  const double sc = prior ? 1.0 : r, coef = sqrt((double)(km - 1)) * sqrt(sc);
+  if (tid < NP) sw[tid] = sc * (sw[tid] + sy[tid]);
+  __syncthreads();
+  if (combine == MDA_COMBINE_ELEMENTWISE) {
+    times_z(nullptr, coef, sy);
+    for (int idx = tid; idx < N * N; idx += THREADS)
+      Tg[idx] = idx / N == idx % N ? sw[idx / N] + sy[idx / N] : 0.0;
+    return;
+  }
+#pragma unroll 8
+  for (int m = 0; m < NP / 4; ++m) {
+    const int i = 4 * m + tid / NP, c = tid % NP;
+    if (i < N && c < N) Tg[i * N + c] = fma(coef, zl[S::at(i, c)], sw[i]);
+  }
+}
+
+template <int N>
+static void launch_root(hipStream_t s, const letkf_solve_args& a, int prior, const int* nloc,
+                        const int* flag) {
+  hipLaunchKernelGGL(k_trd_root<N>, dim3((unsigned)a.ncol), dim3(64 * e4_shape<N>::NT),
+                     e4_shape<N>::LDS, s, a.ncol, a.C, nloc, a.b, a.k, a.rho, a.rho_col, prior,
+                     a.combine, a.U, a.T, flag);
+  MDA_LAUNCH_CHECK();
+}
+
+// ---------------------------------------------------------------------------
 // Eigenvalues of few columns by bisection, a wavefront per column: QL takes the
 // time of its slowest wavefront of 64 columns up to some 65,000 of them (337 us
 // at N = 32, 180 to 474 us by spectrum at N = 40, 1,367 us at N = 64), bisection
@@ -1676,6 +1942,15 @@ __global__ __launch_bounds__(2 * N) void k_trd_vectors_w4(
 // shorter up to 6,000 to 30,000 columns.  By the whole analysis, so that every
 // chunk of it takes the same way.
 constexpr int64_t EIG_BISECT_COLS = 128;  // per row of T
+
+// Where bisection stops, relative.  At N = 128 within 1e-13: the eigenvector
+// checks ask for a residual within 1e-12 of ||T|| and the transform for 1e-10, and
+// the last eight halvings to rounding level would add 14 % to the sweeps.  At
+// rounding level where bisection stands in for QL, and at every N for E4 to start
+// from: below a block's own size eigenvalues are bisected whatever the number of
+// columns (200 x 160 columns, k = 50: 0.5 ms more than QL, whose sweeps leave
+// entries of the analysis 1.8e-14 off 64 bits after E4, against 4.0e-15 here).
+constexpr double EIG_REL = 1e-13, EIG_REL_ROUNDING = 4 * 2.220446049250313e-16;
 
 template <int N>
 static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, double* lam,
@@ -1688,9 +1963,9 @@ static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, d
                      a.rho, a.rho_col, prior, de, a.U);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[0]) MDA_HIP(hipEventRecord(a.ev_stage[0], s));
-  if (a.all_cols <= EIG_BISECT_COLS * N)
+  if (a.refine || a.all_cols <= EIG_BISECT_COLS * N)
     hipLaunchKernelGGL(k_trd_eigvals_bisect<N>, dim3((unsigned)((a.ncol + 3) / 4)), dim3(256), 0,
-                       s, a.ncol, nloc, de, lam, flag);
+                       s, a.ncol, nloc, de, EIG_REL_ROUNDING, lam, flag);
   else
     hipLaunchKernelGGL(k_trd_eigvals<N>, dim3((unsigned)((a.ncol + 63) / 64)), dim3(64), 0, s,
                        a.ncol, nloc, de, lam, flag);
@@ -1714,8 +1989,10 @@ static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, d
   MDA_REQUIRE(!a.fuse, "fused eigenvector transform: no kernel for this block size");
   MDA_REQUIRE(a.ncol < (int64_t)1 << 31, "eigenvector grid too large");
   hipLaunchKernelGGL(k_trd_vectors<N>, dim3((unsigned)a.ncol), dim3(64), 0, s, a.ncol, nloc, de, lam, a.b,
-                     a.k, a.rho, a.rho_col, prior, a.combine, a.null_rel, a.U, a.T, flag);
+                     a.k, a.rho, a.rho_col, prior, a.refine ? EIG_ROOT_ONLY : a.combine,
+                     a.null_rel, a.U, a.T, flag);
   MDA_LAUNCH_CHECK();
+  if (a.refine) launch_root<N>(s, a, prior, nloc, flag);
   if (a.ev_stage[2]) MDA_HIP(hipEventRecord(a.ev_stage[2], s));
 }
 
@@ -1733,13 +2010,15 @@ static void launch_eig_w(hipStream_t s, const letkf_solve_args& a, double* de, d
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[0]) MDA_HIP(hipEventRecord(a.ev_stage[0], s));
   hipLaunchKernelGGL(k_trd_eigvals_bisect<N>, dim3((unsigned)((a.ncol + 3) / 4)), dim3(256), 0,
-                     s, a.ncol, nloc, de, lam, flag);
+                     s, a.ncol, nloc, de, a.refine ? EIG_REL_ROUNDING : EIG_REL, lam, flag);
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[1]) MDA_HIP(hipEventRecord(a.ev_stage[1], s));
   MDA_REQUIRE(a.ncol < (int64_t)1 << 31, "eigenvector grid too large");
   hipLaunchKernelGGL(k_trd_vectors_w4<N>, dim3((unsigned)a.ncol), dim3(2 * N), 0, s, a.ncol, nloc, de, lam, a.b,
-                     a.k, a.rho, a.rho_col, prior, a.combine, a.null_rel, a.U, a.T, flag);
+                     a.k, a.rho, a.rho_col, prior, a.refine ? EIG_ROOT_ONLY : a.combine,
+                     a.null_rel, a.U, a.T, flag);
   MDA_LAUNCH_CHECK();
+  if (a.refine) launch_root<N>(s, a, prior, nloc, flag);
   if (a.ev_stage[2]) MDA_HIP(hipEventRecord(a.ev_stage[2], s));
 }
 

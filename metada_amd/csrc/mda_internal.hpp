@@ -495,6 +495,8 @@ struct letkf_solve_args {
   // nloc >= k and 0 elsewhere; the others with observations go to the
   // fallback (k < ks with a reduced-precision Gram, see launch_letkf_solve)
   int* eig_nloc;
+  // set: T from the inverse square root corrected against C (k < ks, FP64)
+  int refine;
   hipEvent_t ev_stage[3];  // recorded after E1, E2, E3 when set (timing)
   // Reduced-precision Gram: eigenvalues within null_rel * ||A|| of (k-1)/rho
   // are treated as the null space of Y'^T R^-1 Y' (0 for FP64)

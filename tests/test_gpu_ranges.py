@@ -1,5 +1,7 @@
 """Analyses at the sizes where a kernel's tiles, its search or the rule that
 chooses it can go wrong, against the oracle."""
+import math
+
 import numpy as np
 import pytest
 
@@ -404,3 +406,97 @@ def test_metrics_crps_with_an_outlying_first_member(mda, ctx, k):
     X[0] = V
     m = mda.metrics(mda.Ensemble(X, 1, 1, 1), np.zeros(1), ctx=ctx)
     assert abs(m["crps"] / (V / k / k) - 1.0) <= (k + 3) * np.finfo(float).eps
+
+
+# ---- FP64 ensembles between the block sizes: as close to 64 bits as Jacobi ------------------
+S = 120  # binary places of the whole numbers below
+
+
+def _fixed(v):
+    """A float64 array as whole numbers of 2^-S, without rounding above 2^-S."""
+    return np.array([int(np.ldexp(x, 60)) << (S - 60) if abs(x) > 1e-2 else int(np.ldexp(x, S))
+                     for x in np.ravel(v)], object).reshape(np.shape(v))
+
+
+def _float(v, places):
+    return np.array([float(x) for x in np.ravel(v)]).reshape(np.shape(v)) * 2.0 ** -places
+
+
+def _exact_transform(A, b, k, factor):
+    """A^-1 b 1^T + factor sqrt(k-1) A^-1/2 in whole numbers of 2^-S, for
+    whole-number A and b: float64 steps on residuals without rounding."""
+    lam, V = np.linalg.eigh(A.astype(float))
+    root = np.sqrt(lam)
+    Z, w = _fixed((V / root) @ V.T), _fixed(np.zeros(k))
+    eye = np.array([[(1 << 2 * S) * int(i == j) for j in range(k)] for i in range(k)], object)
+    for _ in range(3):
+        R = _float(eye - Z.dot(A.dot(Z)), 2 * S)
+        Z = Z + _fixed(V @ ((V.T @ R @ V) / (root[:, None] + root)) @ V.T)
+        w = w + _fixed(V @ ((V.T @ _float((b << S) - A.dot(w), S)) / lam))
+    assert np.abs(R).max() < 1e-9  # of the last but one; the last step squares it
+    return w[:, None] + (factor * math.isqrt((k - 1) << 2 * S) * Z >> S)
+
+
+@pytest.mark.parametrize("var", [16.0, 1.0, 2.0 ** -6])
+@pytest.mark.parametrize("p", [5, 300])
+@pytest.mark.parametrize("k", [2, 7, 9, 15, 17, 21, 31, 33, 39, 41, 47, 50, 63, 65, 100, 127])
+def test_letkf_between_blocks_is_as_accurate_as_jacobi(mda, ctx, k, p, var):
+    """Whole-number H(x) of mean zero, a cutoff of weight one and a power of two
+    as variance make Gram and right-hand side exact, so T = wbar 1^T + W can be
+    held against its exact value: no further off than Jacobi's, or at rounding
+    level."""
+    L = mda._lib
+    rng = np.random.default_rng(k * 1000 + p)
+    Yb = rng.integers(-8, 9, (k, p)).astype(float)
+    Yb[:, 1:] += 2 * Yb[:, :1]  # correlated: eigenvalues far apart
+    Yb[-1] -= Yb.sum(0)
+    yo = rng.integers(-20, 21, p).astype(float)
+    out = {}
+    for method in ("AUTO", "JACOBI"):
+        ens = mda.Ensemble(rng.standard_normal((k, 12)), 4, 3, 1)
+        f = mda.LETKF(ens, mda.Observation(yo, np.full(p, var), np.ones(p), np.ones(p)),
+                      mda.ObsOperator(hx=Yb), mda.Config({"inflation": 1.0,
+                                                          "localization_radius": 50.0}),
+                      ctx=ctx, eig_method=getattr(L, "EIG_" + method), keep_transforms=True)
+        f.params.localization = L.LOC_CUTOFF
+        f.Analyse()
+        out[method] = f.transforms([0, 11])
+    # whole numbers: unit A and unit b, unit = 16 or 1, with the root's factor 4 or 1
+    unit = max(var, 1.0)
+    A = (Yb @ Yb.T * (unit / var) + unit * (k - 1) * np.eye(k)).astype(np.int64).astype(object)
+    b = (Yb @ yo * (unit / var)).astype(np.int64).astype(object)
+    T = _exact_transform(A, b, k, math.isqrt(int(unit)))
+    size = np.sqrt((_float(T, S) ** 2).sum())
+    err = {m: max(np.sqrt((_float(_fixed(t) - T, S) ** 2).sum()) for t in v) / size
+           for m, v in out.items()}
+    # 8 eps: the rounding of T itself and of wbar's two products
+    assert err["AUTO"] <= max(err["JACOBI"], 8 * np.finfo(float).eps), err
+
+
+@pytest.mark.parametrize("combine", ["MATRIX", "ELEMENTWISE"])
+@pytest.mark.parametrize("form", ["PRIOR", "POSTERIOR"])
+@pytest.mark.parametrize("k", [5, 13, 18, 25, 36, 44, 50, 90])
+def test_letkf_between_blocks_every_form_matches_jacobi(mda, ctx, monkeypatch, k, form, combine):
+    """Inflation forms, combinations, an inflation per column, empty columns,
+    one pass and passes of 50 columns."""
+    L = mda._lib
+    case = latlon_case(nlon=18, nlat=9, nlev=3, k=k, p=350, seed=900 + k, cluster=True, nmodes=96)
+    rho = np.random.default_rng(k).uniform(1.0, 1.4, 162)
+    X = {}
+    for method, chunk in (("JACOBI", None), ("AUTO", None), ("AUTO", "50")):
+        if chunk:
+            monkeypatch.setenv("MDA_LETKF_CHUNK_COLS", chunk)
+        ens = mda.Ensemble(case["X"].copy(), 18, 9, 3)
+        f = mda.LETKF(ens, mda.Observation(case["yo"], case["var"], case["lat"], case["lon"],
+                                           coord=L.COORD_GEOGRAPHIC), case["H"],
+                      mda.Config({"inflation": 1.1, "localization_radius": 1800.0}),
+                      geometry=mda.ColumnGeometry(L.COORD_GEOGRAPHIC, case["col_lat"],
+                                                  case["col_lon"]), ctx=ctx, rho_column=rho,
+                      eig_method=getattr(L, "EIG_" + method))
+        f.params.inflation_form = getattr(L, "INFLFORM_" + form)
+        f.params.combine = getattr(L, "COMBINE_" + combine)
+        f.Analyse()
+        assert f.diag["n_empty_columns"] > 0
+        X[method, chunk] = ens.data.copy()
+    np.testing.assert_array_equal(X["AUTO", "50"], X["AUTO", None])
+    assert rel_err(X["AUTO", None], X["JACOBI", None]) < TOL
