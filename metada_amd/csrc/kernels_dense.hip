@@ -665,7 +665,9 @@ void lowrank_spd_extremes(mda_ctx* c, side_branch& br, const double* yp, const d
 //   panel   one workgroup, rows in registers (a thread owns positions tid,
 //           tid + NT, ...): LU with partial pivoting of the block's columns over
 //           the rows >= j0, the pivot of a column being the first row with the
-//           largest entry.  With A11 = L11 U11 the pivot rows and l_r the
+//           largest entry (entries within 2^-40 of each other count as equal: no
+//           multiplier exceeds 1 by more); an entry that is no finite number makes
+//           S singular.  With A11 = L11 U11 the pivot rows and l_r the
 //           multipliers of any other row, W[r] = -l_r L11^-1, and W[j0 + t] =
 //           row t of A11^-1.
 //   strips  a workgroup per 32 columns right of the block or of B: the row
@@ -709,17 +711,23 @@ __global__ __launch_bounds__(NT) void k_gj_panel(int p, int j0, int nb, const do
   for (int t = 0; t < NB; ++t) {
     if (t < nb) {
       // key: |value| with its last 12 bits replaced by 4095 - row, so that the
-      // first of the largest wins; a NaN is never taken
+      // first of the largest wins
       const int par = t & 1;
       double kv = -1.0;
+      bool bad = false;
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         const int r = tid + NT * i;
         const double v = fabs(a[i][0]);
-        if (r >= j0 + t && r < p && v == v)
-          kv = fmax(kv, __hiloint2double(__double2hiint(v),
-                                         (__double2loint(v) & ~4095) | (4095 - r)));
+        if (r >= j0 + t && r < p) {
+          if (v < INFINITY)
+            kv = fmax(kv, __hiloint2double(__double2hiint(v),
+                                           (__double2loint(v) & ~4095) | (4095 - r)));
+          else
+            bad = true;
+        }
       }
+      if (bad) atomicOr(status, MDA_ST_NOT_SPD);
       kv = wave_max(kv);
       const int rw = kv >= 0.0 ? 4095 - (__double2loint(kv) & 4095) : -1;
 #pragma unroll
@@ -740,7 +748,7 @@ __global__ __launch_bounds__(NT) void k_gj_panel(int p, int j0, int nb, const do
       if (lane == 0) key[par][wv] = kv;
       __syncthreads();
       const double best = read_lane(row_max(key[par][lane % NW]), 15);
-      // no comparable entry (NaN): no exchange, and no finite pivot
+      // no finite entry: no exchange, and no finite pivot
       const int bi = best >= 0.0 ? 4095 - (__double2loint(best) & 4095) : j0 + t;
       const int bw = (bi % NT) >> 6;
       const double(&prow)[NB] = cand[par][bw][0];

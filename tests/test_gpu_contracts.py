@@ -116,3 +116,27 @@ def test_transforms_between_block_sizes_are_readable(mda, ctx, k, prec):
     g.Analyse()
     np.testing.assert_array_equal(T, g.transforms(cols))
     np.testing.assert_array_equal(ens.data, ens_kept.data)
+
+
+# ---- elimination that meets no finite number -------------------------------------------------
+@pytest.mark.parametrize("p,where", [(5, 0), (16, 15), (40, 20), (300, 17), (1030, 1029)])
+@pytest.mark.parametrize("size", [1e160, 1e308])
+def test_lwenkf_infinite_covariance_is_an_error(mda, ctx, p, where, size):
+    """One observation whose spread overflows S (to infinities, or to NaN off
+    the diagonal): MDA_E_NUMERIC, and the ensemble as it was."""
+    k, n = 6, 50
+    rng = np.random.default_rng(p)
+    Yb = rng.standard_normal((k, p))
+    Yb[:, where] = size * np.array([1, -1, 1, -1, 1, -1])
+    X = rng.standard_normal((k, n))
+    ens = mda.Ensemble(X.copy(), n, 1, 1)
+    f = mda.LWEnKF(ens, mda.Observation(rng.standard_normal(p), np.ones(p), np.zeros(p),
+                                        np.zeros(p)),
+                   mda.ObsOperator(hx=Yb),
+                   mda.Config({"analysis": {"inflation": 1.1, "localization_radius": 0.3,
+                                            "localization_function": "gaussian",
+                                            "weighting_scheme": "uniform"}}), ctx=ctx)
+    with pytest.raises(mda._lib.MdaError) as e:
+        f.Analyse(Z=rng.standard_normal((p, k)))
+    assert e.value.code == -4
+    np.testing.assert_array_equal(ens.data, X)
