@@ -785,7 +785,8 @@ static void check_letkf_params(const mda_letkf_params* prm, const mda_geometry* 
 
 static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemble* ens,
                              const mda_geometry* geom, const mda_obs* obs, const mda_hop* hop,
-                             const std::string& pre, bool queue, bool columns = true) {
+                             const std::string& pre, bool queue, bool own_size,
+                             bool columns = true) {
   check_letkf_params(prm, geom);
   letkf_plan P;
   // argument blocks with zero padding: the batch's graph key holds their bytes
@@ -881,10 +882,10 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
   // BF16x3 Gram is symmetric only to its FP32 accumulation (hi lo^T + lo hi^T
   // rounds differently in the two triangles), so its result depends at 1e-9
   // on which entries a solver reads: sizes without a kernel of their own stay
-  // with Jacobi there.
+  // with Jacobi there, and with own_size all of them do.
   const int ke = letkf_eig_size(k);
   P.eig_path = prm->sqrt_form == MDA_SQRT_SYMMETRIC && prm->eig_method == MDA_EIG_AUTO &&
-               (ke == k || prm->precision != MDA_PREC_BF16X3);
+               (ke == k || (prm->precision != MDA_PREC_BF16X3 && !own_size));
   const int ks = P.ks = P.eig_path ? ke : k;
   letkf_gram_args& ga = P.ga;
   ga.k = k; ga.ks = ks; ga.ncol = ncol; ga.nx = P.nx; ga.coord = geom->coord;
@@ -988,6 +989,20 @@ static letkf_plan plan_letkf(mda_ctx* c, const mda_letkf_params* prm, mda_ensemb
             prm->transform_precision == MDA_PREC_FP64 && !prm->keep_transforms;
   c->send_staged();
   return P;
+}
+
+// plan(false), and where the device has not the memory for it plan(true): three
+// blocks of the eigensolver's size per column take up to 5.8 times (k = 65) the
+// two k x k ones that Jacobi works with, and what fits with those is analysed.
+static void plan_within_memory(mda_ctx* c, const std::function<void(bool)>& plan) {
+  try {
+    plan(false);
+  } catch (const mda_error& e) {
+    if (e.code != MDA_E_NOMEM) throw;
+    (void)hipGetLastError();  // the refused allocation's
+    for (const char* name : {"col_C", "col_T", "eig_U"}) c->release(name);
+    plan(true);
+  }
 }
 
 // Stages before the per-column work (LETKF.hpp:152-211).  The bucket index
@@ -1173,7 +1188,10 @@ int mda_letkf_analyse(mda_ctx* c, const mda_letkf_params* prm, mda_ensemble* ens
   return guarded(c, [&] {
     hipStream_t s = c->stream;
     MDA_HIP(hipEventRecord(c->ev[0], s));
-    letkf_plan P = plan_letkf(c, prm, ens, geom, obs, hop, "", false);
+    letkf_plan P;
+    plan_within_memory(c, [&](bool own_size) {
+      P = plan_letkf(c, prm, ens, geom, obs, hop, "", false, own_size);
+    });
     const int64_t npass = n_passes(P);
     while ((int64_t)c->evpool.size() < 7 * npass) {
       hipEvent_t e = nullptr;
@@ -1316,11 +1334,12 @@ int mda_letkf_analyse_batch(mda_ctx* c, int32_t nb, const mda_letkf_params* prm,
                   "batched analyses take device-resident ensembles, observations and H");
     const bool use_graph = flags & MDA_BATCH_GRAPH, use_queue = flags & MDA_BATCH_QUEUE;
     hipStream_t s = c->stream;
-    std::vector<letkf_plan> plans;
-    plans.reserve(nb);
-    for (int i = 0; i < nb; ++i)
-      plans.push_back(plan_letkf(c, &prm[i], &ens[i], &geom[i], &obs[i], &hop[i],
-                                 "b" + std::to_string(i) + ":", use_queue));
+    std::vector<letkf_plan> plans(nb);
+    plan_within_memory(c, [&](bool own_size) {
+      for (int i = 0; i < nb; ++i)
+        plans[i] = plan_letkf(c, &prm[i], &ens[i], &geom[i], &obs[i], &hop[i],
+                              "b" + std::to_string(i) + ":", use_queue, own_size);
+    });
     std::vector<std::pair<int, int>> cfg(nb, {0, use_queue ? 1 : 0});
     for (int i = 0; i < nb; ++i) {
       const std::string key = tune_key(plans[i]) + (use_queue ? ":q" : "");
@@ -1579,7 +1598,7 @@ int mda_letkf_inflation_features(mda_ctx* c, const mda_letkf_params* prm,
     fp.precision = MDA_PREC_FP64;
     fp.rho_column = nullptr;
     letkf_plan P = plan_letkf(c, &fp, const_cast<mda_ensemble*>(ens), geom, obs, hop, "", false,
-                              /*columns=*/false);
+                              /*own_size=*/false, /*columns=*/false);
     MDA_REQUIRE(P.p > 0, "inflation features need observations");
     enqueue_buckets(s, P);
     enqueue_local(s, P);

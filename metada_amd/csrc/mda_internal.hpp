@@ -149,6 +149,18 @@ struct mda_ctx {
   T* get(const std::string& name, size_t count) {
     return static_cast<T*>(get(name, count * sizeof(T)));
   }
+  // frees the buffers whose names end in `suffix`
+  void release(const std::string& suffix) {
+    drop_graphs();
+    for (auto& kv : ws) {
+      const std::string& n = kv.first;
+      if (n.size() < suffix.size() || n.compare(n.size() - suffix.size(), suffix.size(), suffix) != 0)
+        continue;
+      forget_results(kv.second.ptr);
+      if (kv.second.ptr) MDA_HIP(hipFree(kv.second.ptr));
+      kv.second = buf{};
+    }
+  }
   // results of the last LETKF call that lie in a buffer about to be freed
   void forget_results(const void* ptr) {
     if (last_T == ptr) last_T = nullptr;

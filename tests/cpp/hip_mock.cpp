@@ -1,10 +1,14 @@
-// A HIP runtime of two devices that counts what is alive and refuses the
-// call of a chosen number, for the creation and destruction of a context.
+// A HIP runtime of two devices that runs no kernel: it counts what is alive,
+// refuses the call of a chosen number or the device memory beyond a capacity.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdlib>
+#include <cstring>
+#include <map>
 
 namespace {
+std::map<void*, size_t> size;
+size_t used = 0, capacity = 0;
 int device = 1, streams = 0, events = 0, buffers = 0, calls = 0, refuse = 0;
 bool refused() { return ++calls == refuse; }
 template <class T>
@@ -38,10 +42,45 @@ hipError_t hipStreamDestroy(hipStream_t s) { return drop(s, streams); }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return make(e, events, hipErrorUnknown); }
 hipError_t hipEventDestroy(hipEvent_t e) { return drop(e, events); }
-hipError_t hipHostMalloc(void** p, size_t, unsigned) {
-  return make(p, buffers, hipErrorOutOfMemory);
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  const hipError_t e = make(p, buffers, hipErrorOutOfMemory);
+  if (e == hipSuccess) *p = std::realloc(*p, n), std::memset(*p, 0, n);
+  return e;
 }
 hipError_t hipHostFree(void* p) { return drop(p, buffers); }
-hipError_t hipMalloc(void** p, size_t) { return make(p, buffers, hipErrorOutOfMemory); }
-hipError_t hipFree(void* p) { return drop(p, buffers); }
+hipError_t hipMalloc(void** p, size_t n) {
+  if (capacity && used + n > capacity) return hipErrorOutOfMemory;
+  const hipError_t e = make(p, buffers, hipErrorOutOfMemory);
+  if (e == hipSuccess) used += size[*p] = n;
+  return e;
+}
+hipError_t hipFree(void* p) {
+  used -= size[p];
+  size.erase(p);
+  return drop(p, buffers);
+}
+
+void mock_capacity(size_t bytes) { capacity = bytes; }
+size_t mock_used() { return used; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  return make(e, events, hipErrorUnknown);
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { *ms = 0.f; return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+// device memory holds zeros
+hipError_t hipMemcpy(void* d, const void*, size_t n, hipMemcpyKind k) {
+  if (k == hipMemcpyDeviceToHost) std::memset(d, 0, n);
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void*, const void*, size_t, hipMemcpyKind, hipStream_t) {
+  return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3*, dim3*, size_t*, hipStream_t*) { return hipSuccess; }
+hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t) {
+  return hipSuccess;
+}
 }

@@ -74,3 +74,69 @@ def test_context_creation_that_fails_leaves_nothing_behind(tmp_path):
     for i, (_, rc, alive, dev, h) in enumerate(got):
         assert int(rc) == (-3 if i >= 13 else -2), got[i]
         assert (alive, dev, h) == ("0", "1", "None"), got[i]
+
+
+WITHIN_MEMORY = """
+import ctypes as C, importlib.util, sys
+mock = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+mock.mock_used.restype = C.c_size_t
+spec = importlib.util.spec_from_file_location("_lib", sys.argv[2])
+L = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(L)
+lib = L.load()
+DEV = 64  # some device address
+
+def analyse(k, method, prec, batch, capacity=0):
+    h = C.c_void_p()
+    mock.mock_capacity(C.c_size_t(0))
+    assert lib.mda_ctx_create(0, C.byref(h)) == 0
+    before = mock.mock_used()
+    mock.mock_capacity(C.c_size_t(before + capacity if capacity else 0))
+    prm, ens, geo, obs, hop = ((t * 2)() for t in (L.LetkfParams, L.Ensemble, L.Geometry, L.Obs,
+                                                   L.Hop))
+    for i in range(2):
+        lib.mda_letkf_params_standard(C.byref(prm[i]), 1.1, 1000.0)
+        prm[i].eig_method, prm[i].precision = method, prec
+        ens[i].k, ens[i].nx, ens[i].ny, ens[i].nlev, ens[i].data, ens[i].on_device = \\
+            k, 200, 100, 2, DEV, 1
+        geo[i].coord, geo[i].col_a, geo[i].col_b, geo[i].on_device = L.COORD_GEOGRAPHIC, DEV, DEV, 1
+        obs[i].p, obs[i].value, obs[i].variance, obs[i].loc_a, obs[i].loc_b, obs[i].on_device = \\
+            500, DEV, DEV, DEV, DEV, 1
+        hop[i].kind, hop[i].row_ptr, hop[i].col, hop[i].weight, hop[i].nnz, hop[i].on_device = \\
+            L.HOP_CSR, DEV, DEV, DEV, 2000, 1
+    args = h, prm, ens, geo, obs, hop, None
+    if batch:
+        rc = lib.mda_letkf_analyse_batch(h, 2, prm, ens, geo, obs, hop, None, 0, None)
+    else:
+        rc = lib.mda_letkf_analyse(h, C.byref(prm[0]), C.byref(ens[0]), C.byref(geo[0]),
+                                   C.byref(obs[0]), C.byref(hop[0]), None)
+    used = mock.mock_used() - before
+    lib.mda_ctx_destroy(h)
+    return rc, used
+
+for k in (21, 41, 49, 65):
+    for prec in (L.PREC_FP64, L.PREC_FP32):
+        for batch in (0, 1):
+            rc, own = analyse(k, L.EIG_JACOBI, prec, batch)
+            rc2, block = analyse(k, L.EIG_AUTO, prec, batch)
+            assert rc == rc2 == 0
+            rc3, used = analyse(k, L.EIG_AUTO, prec, batch, own + own // 8)
+            rc4, _ = analyse(k, L.EIG_JACOBI, prec, batch, own // 2)
+            print(k, prec, batch, own, block, rc3, used, rc4)
+"""
+
+
+def test_ensembles_between_block_sizes_fit_where_jacobi_does(tmp_path):
+    """Blocks of the next larger size need up to 5.8 times the memory (k = 65):
+    on a device that holds the k x k ones and an eighth more, single analyses
+    and batches still run; half of it is MDA_E_NOMEM."""
+    so = _build(tmp_path, "hip_mock.cpp", "libhipmock.so")
+    out = subprocess.run([sys.executable, "-c", WITHIN_MEMORY, so, os.path.join(PKG, "_lib.py")],
+                         capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    rows = [tuple(map(int, line.split())) for line in out.stdout.splitlines()]
+    assert len(rows) == 16
+    for k, prec, batch, own, block, rc, used, rc_half in rows:
+        assert block > 1.3 * own, (k, prec, batch)
+        assert rc == 0 and used <= own + own // 8, (k, prec, batch)
+        assert rc_half == -3
