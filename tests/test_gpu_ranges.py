@@ -500,3 +500,33 @@ def test_letkf_between_blocks_every_form_matches_jacobi(mda, ctx, monkeypatch, k
         X[method, chunk] = ens.data.copy()
     np.testing.assert_array_equal(X["AUTO", "50"], X["AUTO", None])
     assert rel_err(X["AUTO", None], X["JACOBI", None]) < TOL
+
+
+@pytest.mark.parametrize("prec", ["FP32", "BF16X3"])
+@pytest.mark.parametrize("k,radius,few_columns", [(10, 500.0, True), (25, 1500.0, True),
+                                                  (50, 1500.0, True), (50, 9000.0, False),
+                                                  (100, 9000.0, False)])
+def test_letkf_reduced_precision_between_blocks_solver(mda, ctx, orc, k, radius, few_columns, prec):
+    """Which solver a reduced-precision Gram gets at a size between the blocks:
+    BF16x3 Jacobi for every column, FP32 the tridiagonal one, which columns with
+    fewer than k observations leave at once (and others by its checks); the
+    analysis within the 1e-4 of the FP64 oracle that these contractions are
+    stated to keep."""
+    L = mda._lib
+    case = latlon_case(nlon=18, nlat=9, nlev=2, k=k, p=700, seed=400 + k, nmodes=96)
+    f, X = _latlon(mda, ctx, case, case["X"], radius, precision=getattr(L, "PREC_" + prec))
+    nloc = f.local_counts()
+    few = int(((nloc > 0) & (nloc < k)).sum())
+    assert (few > 0) == few_columns
+    if prec == "BF16X3":
+        assert f.diag["n_fallback_columns"] == 0 and f.diag["max_jacobi_sweeps"] > 0
+        assert not f.column_flags().any()
+    else:
+        assert few <= f.diag["n_fallback_columns"]
+        assert (f.column_flags()[(nloc > 0) & (nloc < k)] == 16).all()
+    prob = orc.Problem(k, 18, 9, 2, orc.COORD_GEOGRAPHIC, case["col_lat"], case["col_lon"],
+                       case["lat"], case["lon"], case["yo"], case["var"],
+                       float(np.float32(1.05)), float(np.float32(radius)))
+    Xo, _, _ = orc.letkf_standard(prob, case["X"], case["H"].apply_host(case["X"]))
+    inc = Xo - case["X"]
+    assert np.sqrt(((X - Xo) ** 2).mean()) < 1e-4 * np.sqrt((inc ** 2).mean())
