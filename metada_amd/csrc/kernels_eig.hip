@@ -904,7 +904,7 @@ constexpr int E3_PRE = 2;  // 16-level chunks of X loaded during E3's W products
 template <int N>
 __global__ __launch_bounds__(256) void k_trd_vectors_x(
     int64_t ncol, const int* __restrict__ nloc, const double* __restrict__ de,
-    const double* __restrict__ lam, const double* __restrict__ bvec, int km, double rho,
+    const double* __restrict__ lam, const double* __restrict__ bvec, double rho,
     const double* __restrict__ rho_col, int prior, double null_rel,
     const double* __restrict__ Ug, int* __restrict__ flag, double* __restrict__ X,
     int64_t x_ncol, int64_t nlev, int64_t col0, int* __restrict__ status) {
@@ -933,12 +933,12 @@ __global__ __launch_bounds__(256) void k_trd_vectors_x(
     if (loaded) return;
 #pragma unroll
     for (int ci = 0; ci < E3_PRE; ++ci)
-      xm_load<N>(pre[ci], X, km, x_ncol, nlev, col0 + g0, ncl, (int64_t)XM_L * ci);
+      xm_load<N>(pre[ci], X, N, x_ncol, nlev, col0 + g0, ncl, (int64_t)XM_L * ci);
     loaded = true;
   };
   bool ok = false;
   if (wv < ncl)
-    ok = e3_column<N, true>(g0 + wv, lds + wv * SL, nloc, de, lam, bvec, km, rho, rho_col, prior,
+    ok = e3_column<N, true>(g0 + wv, lds + wv * SL, nloc, de, lam, bvec, N, rho, rho_col, prior,
                             MDA_COMBINE_MATRIX, null_rel, Ug, nullptr, flag, tb, preload);
   preload();
   if ((tid & 63) == 0) sok[wv] = ok ? 1 : 0;
@@ -946,8 +946,8 @@ __global__ __launch_bounds__(256) void k_trd_vectors_x(
   unsigned store = 0u;
   for (int c = 0; c < ncl; ++c) store |= sok[c] ? 1u << c : 0u;
   if (store == 0u || (*status & MDA_ST_SKIP_UPDATE)) return;  // block-uniform
-  xm_tprime<N>(tb, km);
-  xm_apply<N, E3_PRE>(X, km, x_ncol, nlev, col0 + g0, ncl, store, tb, lds, status, pre);
+  xm_tprime<N>(tb, N);
+  xm_apply<N, E3_PRE>(X, N, x_ncol, nlev, col0 + g0, ncl, store, tb, lds, status, pre);
 }
 
 // ---------------------------------------------------------------------------
@@ -1937,10 +1937,13 @@ static void launch_root(hipStream_t s, const letkf_solve_args& a, int prior, con
 // ---------------------------------------------------------------------------
 // Eigenvalues of few columns by bisection, a wavefront per column: QL takes the
 // time of its slowest wavefront of 64 columns up to some 65,000 of them (337 us
-// at N = 32, 180 to 474 us by spectrum at N = 40, 1,367 us at N = 64), bisection
-// 22, 27 and 43 ns a column (118 us at N = 40 and 4,000 columns), so it is the
-// shorter up to 6,000 to 30,000 columns.  By the whole analysis, so that every
-// chunk of it takes the same way.
+// at N = 32, 180 to 474 us by spectrum at N = 40, 855 to 1,367 us at N = 64),
+// bisection 22, 27 and 43 ns a column (118 us at N = 40 and 4,000 columns).  It is
+// the shorter up to 15,000 columns at N = 32, 6,000 to 17,000 at N = 40 and 20,000
+// to 32,000 at N = 64, by spectrum; the line is where it is the shorter at
+// N = 40 whatever the spectrum (5,120), and leaves some of that unused at the
+// other sizes.  By the whole analysis, so that every chunk of it takes the same
+// way.
 constexpr int64_t EIG_BISECT_COLS = 128;  // per row of T
 
 // Where bisection stops, relative.  At N = 128 within 1e-13: the eigenvector
@@ -1972,14 +1975,14 @@ static void launch_eig_n(hipStream_t s, const letkf_solve_args& a, double* de, d
   MDA_LAUNCH_CHECK();
   if (a.ev_stage[1]) MDA_HIP(hipEventRecord(a.ev_stage[1], s));
   if constexpr (N % 16 == 0) {
-    if (a.fuse) {
+    if (a.fuse) {  // k = N
       MDA_REQUIRE(a.combine == MDA_COMBINE_MATRIX && a.X && a.status,
                   "fused eigenvector transform needs the matrix combination and X");
       const int64_t ngrp = (a.ncol + XM_C - 1) / XM_C;
       MDA_REQUIRE(ngrp < (int64_t)1 << 31, "eigenvector grid too large");
       const unsigned nbx = (unsigned)((ngrp + 7) / 8 * 8);
       hipLaunchKernelGGL(k_trd_vectors_x<N>, dim3(nbx), dim3(256), 0, s, a.ncol, nloc, de, lam,
-                         a.b, a.k, a.rho, a.rho_col, prior, a.null_rel, a.U, flag, a.X, a.x_ncol,
+                         a.b, a.rho, a.rho_col, prior, a.null_rel, a.U, flag, a.X, a.x_ncol,
                          a.x_nlev, a.x_col0, a.status);
       MDA_LAUNCH_CHECK();
       if (a.ev_stage[2]) MDA_HIP(hipEventRecord(a.ev_stage[2], s));

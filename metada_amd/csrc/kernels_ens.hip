@@ -48,7 +48,7 @@ void launch_mean_pert(hipStream_t s, const double* X, int k, int64_t n, double s
   MDA_LAUNCH_CHECK();
 }
 
-// sum of squares, one partial per block (reduced on the host in block order)
+// sum of squares, one partial per block (launch_reduce_partials adds them in order)
 __global__ void k_sumsq(const double* __restrict__ X, int64_t count, double* partial) {
   __shared__ double red[256];
   double acc = 0.0;
@@ -361,7 +361,7 @@ void launch_global_gram(hipStream_t s, const double* yp_om, const double* d,
 // the factorisation, so that W = L^-T (upper triangular) comes with it.  Both
 // triangles packed in LDS (132 KB at k = 128).  The matrix in global memory,
 // a barrier per column and a serial inverse took 545 us (ETKF, k = 64) and
-// 960 us (EnKF, k = 80); this takes 74 and 182 us.
+// 960 us (EnKF, k = 80); this takes 62 and 182 us.
 // ---------------------------------------------------------------------------
 constexpr int KS_THREADS = 512;
 __host__ __device__ inline size_t ks_tri(int k) { return (size_t)k * (k + 1) / 2; }
@@ -776,7 +776,7 @@ void launch_enkf_gain_minmax(hipStream_t s, const double* X, int k, int64_t n, d
 // One point per thread.  Up to 128 members sit in registers (KM of them), and
 // the CRPS's k^2 differences take each member once more from the cache against
 // all the registers, against itself in place of the entries past k: two FP64
-// operations a pair and X read from HBM once.  n = 1,048,576, k = 40: 192 us
+// operations a pair and X read from HBM once.  n = 1,048,576, k = 40: 184 us
 // (3.56 ms with both members of every pair loaded).  Beyond 128 members
 // (KM = 0) that form remains.
 // ---------------------------------------------------------------------------

@@ -85,9 +85,9 @@ struct mda_ctx {
   int* last_flag = nullptr;  // device, [ncol] (tridiagonal path only)
 
   // Staging of small host arrays (create_staging): a pinned buffer with a
-  // device buffer of the same layout.  stage() copies an array into the pinned
-  // one and returns its device address; one asynchronous copy (send_staged)
-  // carries everything staged since the last, before the first kernel that
+  // device buffer of the same layout.  An array goes to its place (stage_place)
+  // in the pinned one, its device address lies at the same place in the other;
+  // one asynchronous copy (send_staged) carries everything staged since the last, before the first kernel that
   // reads it.  Offsets start again with every entry point, once the stream has
   // drained.  `result` is the pinned end of small copies back.
   static constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MAX = 512u << 10, RESULT_BYTES = 1u << 20;
