@@ -87,12 +87,15 @@ struct mda_ctx {
   // Staging of small host arrays (create_staging): a pinned buffer with a
   // device buffer of the same layout.  An array goes to its place (stage_place)
   // in the pinned one, its device address lies at the same place in the other;
-  // one asynchronous copy (send_staged) carries everything staged since the last, before the first kernel that
-  // reads it.  Offsets start again with every entry point, once the stream has
-  // drained.  `result` is the pinned end of small copies back.
+  // one asynchronous copy (send_staged) carries everything staged since the last,
+  // before the first kernel that reads it.  Offsets start again with the first
+  // array that an entry point stages, once the stream has drained; one that
+  // stages nothing does not wait.  `result` is the pinned end of small copies
+  // back.
   static constexpr size_t STAGE_BYTES = 4u << 20, STAGE_MAX = 512u << 10, RESULT_BYTES = 1u << 20;
   char *stage_host = nullptr, *stage_dev = nullptr, *result = nullptr;
   size_t stage_off = 0, stage_sent = 0;
+  bool stage_begun = false;  // by the entry point that runs
   int depth = 0;  // nested entry points
 
   void create_staging() {
@@ -108,7 +111,14 @@ struct mda_ctx {
   // place for `bytes` in both buffers (offset), or SIZE_MAX when the array is
   // too large or the buffers are full
   size_t stage_place(size_t bytes) {
-    if (bytes > STAGE_MAX || stage_off + bytes > STAGE_BYTES) return SIZE_MAX;
+    if (bytes > STAGE_MAX) return SIZE_MAX;
+    if (!stage_begun) {
+      // no copy or kernel of the calls before is left
+      if (stage_off) MDA_HIP(hipStreamSynchronize(stream));
+      stage_off = stage_sent = 0;
+      stage_begun = true;
+    }
+    if (stage_off + bytes > STAGE_BYTES) return SIZE_MAX;
     const size_t at = stage_off;
     stage_off = (stage_off + bytes + 255) & ~(size_t)255;
     return at;
@@ -120,9 +130,8 @@ struct mda_ctx {
     stage_sent = stage_off;
   }
   void begin_call() {
-    if (stage_off == 0) return;
-    MDA_HIP(hipStreamSynchronize(stream));  // no copy or kernel of the last call is left
-    stage_off = stage_sent = 0;
+    stage_begun = false;
+    stage_sent = stage_off;  // what a call that failed left unsent
   }
 
   // returns a device buffer of at least `bytes`; contents are unspecified.

@@ -9,6 +9,7 @@
 namespace {
 std::map<void*, size_t> size;
 size_t used = 0, capacity = 0;
+int syncs = 0;
 int device = 1, streams = 0, events = 0, buffers = 0, calls = 0, refuse = 0;
 bool refused() { return ++calls == refuse; }
 template <class T>
@@ -39,7 +40,8 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
   return make(s, streams, hipErrorUnknown);
 }
 hipError_t hipStreamDestroy(hipStream_t s) { return drop(s, streams); }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+int mock_syncs() { return syncs; }
+hipError_t hipStreamSynchronize(hipStream_t) { ++syncs; return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) { return make(e, events, hipErrorUnknown); }
 hipError_t hipEventDestroy(hipEvent_t e) { return drop(e, events); }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {

@@ -140,3 +140,39 @@ def test_ensembles_between_block_sizes_fit_where_jacobi_does(tmp_path):
         assert block > 1.3 * own, (k, prec, batch)
         assert rc == 0 and used <= own + own // 8, (k, prec, batch)
         assert rc_half == -3
+
+
+NO_WAIT = """
+import ctypes as C, importlib.util, sys
+mock = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+spec = importlib.util.spec_from_file_location("_lib", sys.argv[2])
+L = importlib.util.module_from_spec(spec)
+spec.loader.exec_module(L)
+lib = L.load()
+h = C.c_void_p()
+assert lib.mda_ctx_create(0, C.byref(h)) == 0
+par, feat, rho = (C.c_float * 4801)(), (C.c_float * 64)(), (C.c_float * 8)()
+a = [C.cast(v, C.c_void_p) for v in (par, feat, rho)]
+waits = []
+for call in ("host", "adam", "adam", "host", "host", "adam"):
+    n = mock.mock_syncs()
+    if call == "host":
+        assert lib.mda_mlp_forward(h, a[0], a[1], 8, a[2], 0) == 0
+    else:
+        assert lib.mda_mlp_adam_step(h, 64, 64, 64, 64, 1, 1e-3, 0.9, 0.999, 1e-8, 1) == 0
+    waits.append(mock.mock_syncs() - n)
+print(*waits)
+"""
+
+
+def test_calls_without_host_arrays_do_not_wait(tmp_path):
+    """An entry point that only launches (the Adam step on device arrays, which a
+    caller may capture) waits for nothing, also after calls with host arrays;
+    those wait for the stream before they use the staging buffer again."""
+    so = _build(tmp_path, "hip_mock.cpp", "libhipmock.so")
+    out = subprocess.run([sys.executable, "-c", NO_WAIT, so, os.path.join(PKG, "_lib.py")],
+                         capture_output=True, text=True)
+    assert out.returncode == 0, out.stderr
+    waits = list(map(int, out.stdout.split()))
+    assert waits[1] == waits[2] == waits[5] == 0
+    assert waits[3] == waits[4] == waits[0] + 1
